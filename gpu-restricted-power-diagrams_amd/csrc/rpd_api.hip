@@ -50,7 +50,7 @@
 struct rpd_domain {
     int device = 0;
     DomainDev dev;
-    DevBuf flags, centre, pts, tris, tlist, toffs, tvoffs, tvox, tinfo, dist, dvox;
+    DevBuf flags, centre, pts, tris, tlist, toffs, tvoffs, tvox, tinfo, vfoffs, vface, dist, dvox;
     int64_t bytes = 0;
 };
 
@@ -298,6 +298,129 @@ void domain_distance(const rpd_grid_desc *g, std::vector<uint8_t> &dist) {
                     q.push_back(int(u));
                 }
     }
+}
+
+// The faces of a domain made of voxel faces (DomainDev::vface), or false: the
+// triangles are not exactly the two halves of lattice squares (corner
+// coordinates i * vs, bit for bit), oriented alike, each in the lists of the
+// voxels on both sides; or a voxel's class is unknown.  The finish kernel then
+// keeps to the triangle lists.
+bool voxel_faces(const rpd_grid_desc *g, const std::vector<int> &tvoffs, const std::vector<uint32_t> &tvox,
+                 std::vector<int> &offs, std::vector<uint32_t> &faces) {
+    const int G = g->size;
+    if (!g->centre || G > 1023) return false;
+    const size_t nv = size_t(G) * G * G, nt = size_t(g->num_triangles);
+    for (size_t v = 0; v < nv; ++v)
+        if (g->centre[v] != 0 && g->centre[v] != 2) return false;
+    const double vs = 1000.0 / double(G);
+    // lattice coordinates of the points
+    std::vector<uint16_t> pt(3 * size_t(g->num_points));
+    for (size_t p = 0; p < size_t(g->num_points); ++p)
+        for (int k = 0; k < 3; ++k) {
+            const double x = g->points[4 * p + size_t(k)];
+            if (!(x >= 0.0 && x <= 1000.0 + vs)) return false;
+            const int i = int(std::lround(x / vs));
+            if (i > G || i * vs != x) return false;
+            pt[3 * p + size_t(k)] = uint16_t(i);
+        }
+    // each triangle: its face (lowest corner, axis), the corner of its right
+    // angle (2 bits) and the sign of its normal
+    const size_t G1 = size_t(G) + 1;
+    struct Half {
+        uint32_t at;  // x | y << 10 | z << 20 | axis << 30
+        uint8_t corner, up;
+    };
+    std::vector<Half> half(nt);
+    offs.assign(G1 * G1 * G1 + 1, 0);
+    for (size_t t = 0; t < nt; ++t) {
+        int p[3][3], lo[3], hi[3];
+        for (int c = 0; c < 3; ++c)
+            for (int k = 0; k < 3; ++k) p[c][k] = pt[3 * size_t(g->triangles[3 * t + size_t(c)]) + size_t(k)];
+        int ax = -1;
+        for (int k = 0; k < 3; ++k) {
+            lo[k] = std::min(p[0][k], std::min(p[1][k], p[2][k]));
+            hi[k] = std::max(p[0][k], std::max(p[1][k], p[2][k]));
+            if (hi[k] == lo[k]) {
+                if (ax >= 0) return false;
+                ax = k;
+            } else if (hi[k] != lo[k] + 1) {
+                return false;
+            }
+        }
+        if (ax < 0) return false;
+        const int u = ax == 0 ? 1 : 0, v = ax == 2 ? 1 : 2;
+        // the square's corner that the triangle does not have, opposite its right angle
+        int seen = 0;
+        for (int c = 0; c < 3; ++c) seen |= 1 << ((p[c][u] - lo[u]) + 2 * (p[c][v] - lo[v]));
+        int missing = -1;
+        for (int c = 0; c < 4; ++c)
+            if (!(seen >> c & 1)) missing = missing < 0 ? c : 4;
+        if (missing < 0 || missing > 3) return false;
+        const int cr = (p[1][u] - p[0][u]) * (p[2][v] - p[0][v]) - (p[1][v] - p[0][v]) * (p[2][u] - p[0][u]);
+        // (e_u x e_v is +e_axis for x and z, -e_axis for y)
+        const bool up = (cr > 0) != (ax == 1);
+        // in the lists of the voxels on both sides
+        for (int side = 0; side < 2; ++side) {
+            int w[3] = {lo[0], lo[1], lo[2]};
+            w[ax] -= side;
+            if (w[ax] < 0 || w[ax] >= G) continue;
+            const uint32_t pv = (uint32_t(w[2]) << 20) | (uint32_t(w[1]) << 10) | uint32_t(w[0]);
+            if (!std::binary_search(tvox.begin() + tvoffs[t], tvox.begin() + tvoffs[t + 1], pv)) return false;
+        }
+        half[t] = Half{(uint32_t(lo[2]) << 20) | (uint32_t(lo[1]) << 10) | uint32_t(lo[0]) | (uint32_t(ax) << 30),
+                       uint8_t(missing), uint8_t(up)};
+    }
+    auto point_of = [&](uint32_t at) {
+        return size_t(at & 1023u) + G1 * (size_t((at >> 10) & 1023u) + G1 * size_t((at >> 20) & 1023u));
+    };
+    // the halves by lattice point
+    for (const Half &h : half) offs[point_of(h.at) + 1]++;
+    for (size_t i = 0; i + 1 < offs.size(); ++i) offs[i + 1] += offs[i];
+    std::vector<int> cur(offs.begin(), offs.end() - 1), by(nt);
+    for (size_t t = 0; t < nt; ++t) by[size_t(cur[point_of(half[t].at)]++)] = int(t);
+    // two halves each, of one orientation, with opposite right angles
+    faces.clear();
+    faces.reserve(nt);
+    std::vector<int> foffs(offs.size(), 0);
+    for (size_t i = 0; i + 1 < offs.size(); ++i) {
+        for (uint32_t ax = 0; ax < 3; ++ax) {
+            const Half *h[2] = {nullptr, nullptr};
+            int n = 0;
+            for (int q = offs[i]; q < offs[i + 1]; ++q) {
+                const Half &x = half[size_t(by[size_t(q)])];
+                if (x.at >> 30 != ax) continue;
+                if (n == 2) return false;
+                h[n++] = &x;
+            }
+            if (n == 0) continue;
+            if (n != 2 || h[0]->up != h[1]->up || (h[0]->corner ^ h[1]->corner) != 3) return false;
+            faces.push_back(h[0]->at);
+            faces.push_back(h[0]->up ? 1u : 0u);
+        }
+        foffs[i + 1] = int(faces.size() / 2);
+    }
+    offs.swap(foffs);
+    // runs along x (faces across y or z) or y (faces across x), from the end
+    auto find = [&](size_t i, uint32_t ax) -> int {
+        for (int q = offs[i]; q < offs[i + 1]; ++q)
+            if (faces[2 * size_t(q)] >> 30 == ax) return q;
+        return -1;
+    };
+    for (size_t i = offs.size() - 1; i-- > 0;)
+        for (int q = offs[i]; q < offs[i + 1]; ++q) {
+            const uint32_t at = faces[2 * size_t(q)], ax = at >> 30;
+            const size_t next = i + (ax == 0 ? G1 : 1);
+            uint32_t run = 1;
+            if (((ax == 0 ? at >> 10 : at) & 1023u) < uint32_t(G)) {
+                const int r = find(next, ax);
+                if (r >= 0 && (faces[2 * size_t(r) + 1] & 1u) == (faces[2 * size_t(q) + 1] & 1u)) {
+                    run += faces[2 * size_t(r) + 1] >> 2;
+                    faces[2 * size_t(r) + 1] |= 2u;
+                }
+            }
+            faces[2 * size_t(q) + 1] |= run << 2;
+        }
+    return true;
 }
 
 // The lanes of a wave that hold one status add their count once (a ballot
@@ -652,6 +775,13 @@ int rpd_domain_create(rpd_ctx *c, const rpd_grid_desc *g, rpd_domain **out) {
     if (r == RPD_OK) r = up(d->tvoffs, tvoffs.data(), tvoffs.size() * 4);
     if (r == RPD_OK) r = up(d->tvox, tvox.data(), tvox.size() * 4);
     if (r == RPD_OK) r = up(d->tinfo, tinfo.data(), tinfo.size() * 4);
+    std::vector<int> vfoffs;
+    std::vector<uint32_t> vface;
+    const bool vox = r == RPD_OK && voxel_faces(g, tvoffs, tvox, vfoffs, vface);
+    if (vox) {
+        r = up(d->vfoffs, vfoffs.data(), vfoffs.size() * 4);
+        if (r == RPD_OK) r = up(d->vface, vface.data(), vface.size() * 4);
+    }
     std::vector<uint8_t> dist;
     domain_distance(g, dist);
     if (r == RPD_OK) r = up(d->dist, dist.data(), nv);
@@ -675,6 +805,10 @@ int rpd_domain_create(rpd_ctx *c, const rpd_grid_desc *g, rpd_domain **out) {
     d->dev.tvoffs = d->tvoffs.as<int>();
     d->dev.tvox = d->tvox.as<uint32_t>();
     d->dev.tinfo = d->tinfo.as<uint4>();
+    if (vox) {
+        d->dev.vfoffs = d->vfoffs.as<int>();
+        d->dev.vface = d->vface.as<uint2>();
+    }
     d->dev.dist = d->dist.as<uint8_t>();
     d->dev.dvox = d->dvox.as<int>();
     d->dev.n_dvox = int(dvox.size());
@@ -895,6 +1029,9 @@ static int solve_impl(rpd_ctx *c, rpd_domain *dom, const rpd_params *prm, rpd_st
                                    : nullptr;
     };
     const DomainDev *dd = dom ? &dom->dev : nullptr;
+    // the restriction goes by voxel faces when every domain has them
+    bool vox = !dd || dd->vface;
+    for (const auto &q : c->batch) vox = vox && (!q.dom || q.dom->dev.vface);
     // the weight minimum the kernels subtract, and whether there are walls
     // (border seeds): known here unless the minima are new (then at settle)
     double wmin = 0;
@@ -1041,6 +1178,7 @@ static int solve_impl(rpd_ctx *c, rpd_domain *dom, const rpd_params *prm, rpd_st
         L.wmin = wmin;
         L.cull = prm->cull != 0;
         L.dom = dd;
+        L.vox = vox;
         L.out = c->out.as<double4>();
         L.status = c->status.as<int>();
         L.kused = c->kused.as<int>();
@@ -1463,6 +1601,7 @@ static int solve_impl(rpd_ctx *c, rpd_domain *dom, const rpd_params *prm, rpd_st
         L.wmin = wmin;
         L.cull = prm->cull != 0;
         L.dom = dd;
+        L.vox = vox;
         L.out = c->out.as<double4>();
         L.status = c->status.as<int>();
         L.kused = c->kused.as<int>();
@@ -1717,6 +1856,8 @@ int rpd_solve_batch(rpd_ctx *c, int32_t nreq, rpd_domain *const *doms, const dou
             d.tvoffs = dv.tvoffs;
             d.tvox = dv.tvox;
             d.tinfo = dv.tinfo;
+            d.vfoffs = dv.vfoffs;
+            d.vface = dv.vface;
             d.dist = prm->cull ? dv.dist : nullptr;
         }
         kdesc[size_t(r)] = KnnReq{cnt, q.dim};

@@ -85,6 +85,8 @@ struct ClipArgs {
     const int *tvoffs;    // per triangle: offsets into tvox
     const uint32_t *tvox; // per triangle: sorted voxels whose list holds it, z<<20 | y<<10 | x
     const uint4 *tinfo;   // per triangle-list entry: its voxel, earlier near voxels holding it
+    const int *vfoffs;    // voxel domain: per lattice point, offsets into vface
+    const uint2 *vface;   // voxel domain: faces, by the lattice point of their lowest corner
     int security_mode;    // 0 exact power stop, 1 reference stop
     double wmin;          // minimum weight over non-border seeds
     const uint8_t *dist;  // Chebyshev voxel distance to the nearest domain voxel (nullable)
@@ -118,6 +120,7 @@ struct ClipArgs {
     int *hids;
     int H, hc;
     int *dcnt;  // debug counters of this pass (kDcStride ints), nullable
+    int count_only;  // finish kernel, triangle lists: only the union counters of the cells whose union fits
     // packed batch (nullable): the fields of request req_of[sid] replace
     // n_seeds, wmin and the domain's
     const ReqDesc *reqs;
@@ -155,6 +158,8 @@ __device__ __forceinline__ void bind_request(ClipArgs &a, int sid) {
     a.tvoffs = d.tvoffs;
     a.tvox = d.tvox;
     a.tinfo = d.tinfo;
+    a.vfoffs = d.vfoffs;
+    a.vface = d.vface;
     a.dist = d.dist;
 }
 
@@ -590,13 +595,22 @@ struct VtxRec {
 };
 constexpr size_t kVtxRecBytes = 40;  // sizeof(VtxRec<double>), the larger one
 
-// LDS bytes of one wave (pl: bytes of one stored plane; corners: the finish
-// kernel's triangle corners and vertex copy)
-__host__ __device__ constexpr size_t finish_wave_lds(int P, int S, int T, size_t pl, bool corners = false) {
+// LDS bytes of one wave (pl: bytes of one stored plane; tail: bytes after the
+// cone planes and flags)
+__host__ __device__ constexpr size_t wave_lds(int P, int S, int T, size_t pl, size_t tail) {
     return ((((((P * pl + 15) & ~size_t(15)) + ((4 * size_t(P) + 15) & ~size_t(15)) + 4 * 64 * size_t(S) +
                256 + 4 * size_t(P) * size_t((P + 31) >> 5) + 4 * size_t(T)) +
-              15) & ~size_t(15)) + 64 * pl + 64 + (corners ? 16 * 9 * 8 + 64 * size_t(S) * kVtxRecBytes : 0) +
-            15) & ~size_t(15);
+              15) & ~size_t(15)) + 64 * pl + 64 + tail + 15) & ~size_t(15);
+}
+// (corners: the finish kernel's triangle corners and vertex copy)
+__host__ __device__ constexpr size_t finish_wave_lds(int P, int S, int T, size_t pl, bool corners = false) {
+    return wave_lds(P, S, T, pl, corners ? 16 * 9 * 8 + 64 * size_t(S) * kVtxRecBytes : 0);
+}
+// The voxel form of the finish kernel: room for one plane more (a strip has
+// five cone planes, a triangle four), no corners, the vertex copy in the test
+// precision (vr bytes each).
+__host__ __device__ constexpr size_t finish_vox_wave_lds(int P, int S, int T, size_t vr) {
+    return wave_lds(P + 1, S, T, 32, 64 * size_t(S) * vr);
 }
 // LDS the Hessian adds to a finish-kernel wave: per plane 4 sums, per vertex
 // slot 4 values and a plane id
@@ -989,6 +1003,14 @@ void clip_cells_kernel(ClipArgs a) {
     }
 }
 
+// vface[q] of a voxel domain's face: x, y, z (10 bits each) of its lowest
+// lattice point and, in bits 30-31 of .x, the axis it lies across; .y holds
+// kVfaceUp when its triangles' normal points along that axis, kVfacePrev when
+// the face before it (along x, or along y for faces across x) exists with the
+// same normal, and from bit 2 the number of faces from it on that do, itself
+// included.
+constexpr uint32_t kVfaceUp = 1u, kVfacePrev = 2u;
+
 // tinfo[q] of a triangle-list entry (voxel v): x is v packed as
 // z<<20 | y<<10 | x; (z << 32 | y) a 64-bit mask with bit
 // (dz+2)*25 + (dy+2)*5 + (dx+2) set when the voxel v + (dx, dy, dz), within 2
@@ -1039,12 +1061,24 @@ __device__ __forceinline__ uint64_t box_near(int x, int y, int z, const int *mn,
 // only when the caps guarantee that those earlier clips could not overflow
 // either (at most 3 more planes, at most 2 more vertices per clip), so the
 // outcome is the reference's.
+//
+// VOX: a domain of voxel faces.  What bounds this kernel is the work per
+// boundary triangle (cone planes, skip tests, clips, one integration per
+// clipped one: 81% of its time on the 1M-seed torus), so a cell is cut by
+// strips of faces instead: the faces come from one entry each (a triangle is
+// listed by 9 to 12 voxels), side by side ones are one convex unit, their cone
+// planes have two components, and five clips and one integration serve two
+// triangles or more.  The apex lies in the middle of the cell's box, not in
+// its first voxel: cones then only meet the cell where the boundary does.
+// Alone on 1M seeds / torus 128^3 the launch went from 1.43 to 0.87 ms
+// (mixed); 1,000 seeds in a sphere at 96^3, where a cell meets hundreds of
+// triangles, from 3.3 to 1.16 ms for the whole solve.
 // ---------------------------------------------------------------------------
-template <typename R, typename RP, bool FILTER, int S, bool HESS, bool BATCH>
+template <typename R, typename RP, bool FILTER, int S, bool HESS, bool BATCH, bool VOX>
 // 4 waves per SIMD for S = 1 (128 VGPRs): measured at 1M seeds against 5 and
 // 6, whose spills cost more than the extra residency gives.  HESS: the
 // Hessian variant (one wave per cell).
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(S == 1 && !HESS ? 4 : 1)))
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(S > 1 ? 1 : (HESS ? 3 : 4))))
 void finish_cells_kernel(ClipArgs a, int nq, int W) {
     extern __shared__ __attribute__((aligned(16))) char lds_raw[];
     const int lane = lane_id();
@@ -1063,12 +1097,14 @@ void finish_cells_kernel(ClipArgs a, int nq, int W) {
     int *tu = nullptr, *goo = nullptr;
     Pl<RP> *cpl = nullptr;
     double *tcor = nullptr;
-    bind_lds(lds_raw + size_t(cpb) * a.cell_stride + size_t(wv) * a.lds_stride, a.P, a.T, c, nullptr, &tu,
+    // VOX: a strip's fifth cone plane has room of its own, so that no cap is
+    // met earlier than with triangles
+    const int P = VOX ? a.P + 1 : a.P;
+    bind_lds(lds_raw + size_t(cpb) * a.cell_stride + size_t(wv) * a.lds_stride, P, a.T, c, nullptr, &tu,
              &cpl, &goo, &tcor);
-    c.P = a.P;
+    c.P = P;
     c.V = a.V;
     c.lane = lane;
-    const int P = a.P;
 
     const char *rec = a.rec + size_t(slot) * size_t(a.rec_stride);
     const RecHeader hd = *reinterpret_cast<const RecHeader *>(rec);
@@ -1134,13 +1170,16 @@ void finish_cells_kernel(ClipArgs a, int nq, int W) {
     // ---- integration (CCExportBaryVolume): factor/6 * (volume, moments) of
     // the current cell in the local frame, FP64 wave sums --------------------
     const RP vol_eps2 = sizeof(RP) == 8 ? RP(1e-12) : RP(1e-6);  // voronoi.cpp:919-922
+    // the vertex copy of the skip tests
+    VtxRec<R> *vtx = reinterpret_cast<VtxRec<R> *>(VOX ? tcor : tcor + 16 * 9);
     // Hessian sums: per record plane 4 doubles (area-weighted centroid in the
     // local frame, area), per vertex slot staging for their reduction
     double *hacc = nullptr, *hval = nullptr;
     int *hpid = nullptr;
     const int nbk = c.nb_plane;  // the record's planes; cone planes come after
     if (HESS) {
-        hacc = reinterpret_cast<double *>(reinterpret_cast<char *>(tcor + 16 * 9) + 64 * size_t(S) * kVtxRecBytes);
+        hacc = reinterpret_cast<double *>(reinterpret_cast<char *>(vtx) +
+                                          64 * size_t(S) * (VOX ? sizeof(VtxRec<R>) : kVtxRecBytes));
         hval = hacc + 4 * size_t(P);
         hpid = reinterpret_cast<int *>(hval + 4 * 64);
         for (int i = lane; i < 4 * nbk; i += 64) hacc[i] = 0.0;
@@ -1160,55 +1199,111 @@ void finish_cells_kernel(ClipArgs a, int nq, int W) {
             if (vok) {
                 RP Ax, Ay, Az;
                 vertex_rp(s, Ax, Ay, Az);
-                const RP ACx = -Ax, ACy = -Ay, ACz = -Az;  // seed at the origin
                 const Pl<RP> pl[3] = {c.planes[t0(tr)], c.planes[t1(tr)], c.planes[t2(tr)]};
-                RP opx[3], opy[3], opz[3], olx[3], oly[3], olz[3];
-    #pragma unroll
-                for (int k = 0; k < 3; ++k) {
-                    const RP nn = pl[k].x * pl[k].x + pl[k].y * pl[k].y + pl[k].z * pl[k].z;
-                    const RP f = (ACx * pl[k].x + ACy * pl[k].y + ACz * pl[k].z) / nn;
-                    opx[k] = ACx - f * pl[k].x;
-                    opy[k] = ACy - f * pl[k].y;
-                    opz[k] = ACz - f * pl[k].z;
-                }
-    #pragma unroll
-                for (int k = 0; k < 3; ++k) {
-                    const Pl<RP> &p = pl[k], &q = pl[(k + 1) % 3];
-                    const RP cx = p.y * q.z - p.z * q.y, cy = p.z * q.x - p.x * q.z, cz = p.x * q.y - p.y * q.x;
-                    const RP c2 = cx * cx + cy * cy + cz * cz;
-                    const RP pp = p.x * p.x + p.y * p.y + p.z * p.z, qq = q.x * q.x + q.y * q.y + q.z * q.z;
-                    if (c2 < vol_eps2 * pp * qq) {
-                        olx[k] = oly[k] = olz[k] = RP(0);
-                    } else {
-                        const RP f = (ACx * cx + ACy * cy + ACz * cz) / c2;
-                        olx[k] = f * cx;
-                        oly[k] = f * cy;
-                        olz[k] = f * cz;
-                    }
-                }
-    #pragma unroll
-                for (int k = 0; k < 3; ++k) {
-    #pragma unroll
-                    for (int st = 0; st < 2; ++st) {
-                        const int j = (k + 3 - st) % 3;
-                        // det3 of rows AC, onPlane_k, onLine_j (ConvexCell.cl:72-77)
-                        const RP d = ACx * (opy[k] * olz[j] - opz[k] * oly[j]) - opx[k] * (ACy * olz[j] - ACz * oly[j]) +
-                                     olx[j] * (ACy * opz[k] - ACz * opy[k]);
-                        const RP w = st ? d : -d;
-                        sw += w;
-                        sx += w * (Ax + RP(0.25) * (ACx + opx[k] + olx[j]));
-                        sy += w * (Ay + RP(0.25) * (ACy + opy[k] + oly[j]));
-                        sz += w * (Az + RP(0.25) * (ACz + opz[k] + olz[j]));
+                if constexpr (sizeof(RP) == 8) {
+                    // The reference's six tetrahedra (seed, its foot on plane
+                    // i, its foot on the line of planes i and j, vertex A) are
+                    // path simplices: the three legs are orthogonal.  With
+                    // unit normals, a_i = n_i.A, t = n_k x n_q and T =
+                    // (t.A)/|t|^2, the line (k, q) gives the two volumes
+                    // (times 6) a_k (a_q - a_k n_k.n_q) T and a_q (a_k - a_q
+                    // n_k.n_q) T, and the feet are a_i n_i and A - T t: three
+                    // divisions instead of six, and no determinants.
+                    RP av[3], ws[3] = {0, 0, 0};
+#pragma unroll
+                    for (int k = 0; k < 3; ++k) av[k] = pl[k].x * Ax + pl[k].y * Ay + pl[k].z * Az;
+                    RP lx = 0, ly = 0, lz = 0;
+#pragma unroll
+                    for (int k = 0; k < 3; ++k) {
+                        const int q = (k + 1) % 3;
+                        const Pl<RP> &p = pl[k], &r = pl[q];
+                        const RP tx = p.y * r.z - p.z * r.y, ty = p.z * r.x - p.x * r.z, tz = p.x * r.y - p.y * r.x;
+                        const RP c2 = tx * tx + ty * ty + tz * tz;
+                        const RP d = p.x * r.x + p.y * r.y + p.z * r.z;
+                        // (nearly) parallel planes: the reference's foot on the line is the seed
+                        const RP T = c2 < vol_eps2 ? RP(0) : (tx * Ax + ty * Ay + tz * Az) / c2;
+                        const RP ek = (av[q] - av[k] * d) * T, eq = (av[k] - av[q] * d) * T;
+                        const RP wk = av[k] * ek, wq = av[q] * eq;
+                        ws[k] += wk;
+                        ws[q] += wq;
+                        const RP wt = (wk + wq) * T;
+                        lx += wt * tx;
+                        ly += wt * ty;
+                        lz += wt * tz;
                         if (HESS) {
-                            // det3 of rows onPlane_k, onLine_j, n_k, halved
-                            const double dt = double(opx[k]) * (double(oly[j]) * pl[k].z - double(olz[j]) * pl[k].y) -
-                                              double(opy[k]) * (double(olx[j]) * pl[k].z - double(olz[j]) * pl[k].x) +
-                                              double(opz[k]) * (double(olx[j]) * pl[k].y - double(oly[j]) * pl[k].x);
-                            const double ar = (st ? 0.5 : -0.5) * factor * dt;
-                            ha[k] += ar;
-                            hx[k] += ar * (double(Ax) + (double(opx[k]) + double(olx[j])) / 3.0);
-                            hy[k] += ar * (double(Ay) + (double(opy[k]) + double(oly[j])) / 3.0);
-                            hz[k] += ar * (double(Az) + (double(opz[k]) + double(olz[j])) / 3.0);
+                            // per plane of the line, the triangle (foot on the
+                            // plane, foot on the line, A): its area and centroid
+                            const double f2 = -0.5 * factor;
+                            const double ak = f2 * ek, aq = f2 * eq;
+                            const double Lx = Ax - (T * tx) * 0.5, Ly = Ay - (T * ty) * 0.5, Lz = Az - (T * tz) * 0.5;
+                            ha[k] += ak;
+                            hx[k] += ak * (2.0 * Lx + av[k] * p.x) / 3.0;
+                            hy[k] += ak * (2.0 * Ly + av[k] * p.y) / 3.0;
+                            hz[k] += ak * (2.0 * Lz + av[k] * p.z) / 3.0;
+                            ha[q] += aq;
+                            hx[q] += aq * (2.0 * Lx + av[q] * r.x) / 3.0;
+                            hy[q] += aq * (2.0 * Ly + av[q] * r.y) / 3.0;
+                            hz[q] += aq * (2.0 * Lz + av[q] * r.z) / 3.0;
+                        }
+                    }
+                    // centroid of (seed, a n, A - T t, A)
+                    const RP w = ws[0] + ws[1] + ws[2];
+                    const RP b0 = ws[0] * av[0], b1 = ws[1] * av[1], b2 = ws[2] * av[2];
+                    sw += w;
+                    sx += RP(0.5) * w * Ax + RP(0.25) * (b0 * pl[0].x + b1 * pl[1].x + b2 * pl[2].x - lx);
+                    sy += RP(0.5) * w * Ay + RP(0.25) * (b0 * pl[0].y + b1 * pl[1].y + b2 * pl[2].y - ly);
+                    sz += RP(0.5) * w * Az + RP(0.25) * (b0 * pl[0].z + b1 * pl[1].z + b2 * pl[2].z - lz);
+                } else {
+                    // FP32 form: the reference's evaluation
+                    const RP ACx = -Ax, ACy = -Ay, ACz = -Az;  // seed at the origin
+                    RP opx[3], opy[3], opz[3], olx[3], oly[3], olz[3];
+    #pragma unroll
+                    for (int k = 0; k < 3; ++k) {
+                        const RP nn = pl[k].x * pl[k].x + pl[k].y * pl[k].y + pl[k].z * pl[k].z;
+                        const RP f = (ACx * pl[k].x + ACy * pl[k].y + ACz * pl[k].z) / nn;
+                        opx[k] = ACx - f * pl[k].x;
+                        opy[k] = ACy - f * pl[k].y;
+                        opz[k] = ACz - f * pl[k].z;
+                    }
+    #pragma unroll
+                    for (int k = 0; k < 3; ++k) {
+                        const Pl<RP> &p = pl[k], &q = pl[(k + 1) % 3];
+                        const RP cx = p.y * q.z - p.z * q.y, cy = p.z * q.x - p.x * q.z, cz = p.x * q.y - p.y * q.x;
+                        const RP c2 = cx * cx + cy * cy + cz * cz;
+                        const RP pp = p.x * p.x + p.y * p.y + p.z * p.z, qq = q.x * q.x + q.y * q.y + q.z * q.z;
+                        if (c2 < vol_eps2 * pp * qq) {
+                            olx[k] = oly[k] = olz[k] = RP(0);
+                        } else {
+                            const RP f = (ACx * cx + ACy * cy + ACz * cz) / c2;
+                            olx[k] = f * cx;
+                            oly[k] = f * cy;
+                            olz[k] = f * cz;
+                        }
+                    }
+    #pragma unroll
+                    for (int k = 0; k < 3; ++k) {
+    #pragma unroll
+                        for (int st = 0; st < 2; ++st) {
+                            const int j = (k + 3 - st) % 3;
+                            // det3 of rows AC, onPlane_k, onLine_j (ConvexCell.cl:72-77)
+                            const RP d = ACx * (opy[k] * olz[j] - opz[k] * oly[j]) - opx[k] * (ACy * olz[j] - ACz * oly[j]) +
+                                         olx[j] * (ACy * opz[k] - ACz * opy[k]);
+                            const RP w = st ? d : -d;
+                            sw += w;
+                            sx += w * (Ax + RP(0.25) * (ACx + opx[k] + olx[j]));
+                            sy += w * (Ay + RP(0.25) * (ACy + opy[k] + oly[j]));
+                            sz += w * (Az + RP(0.25) * (ACz + opz[k] + olz[j]));
+                            if (HESS) {
+                                // det3 of rows onPlane_k, onLine_j, n_k, halved
+                                const double dt = double(opx[k]) * (double(oly[j]) * pl[k].z - double(olz[j]) * pl[k].y) -
+                                                  double(opy[k]) * (double(olx[j]) * pl[k].z - double(olz[j]) * pl[k].x) +
+                                                  double(opz[k]) * (double(olx[j]) * pl[k].y - double(oly[j]) * pl[k].x);
+                                const double ar = (st ? 0.5 : -0.5) * factor * dt;
+                                ha[k] += ar;
+                                hx[k] += ar * (double(Ax) + (double(opx[k]) + double(olx[j])) / 3.0);
+                                hy[k] += ar * (double(Ay) + (double(opy[k]) + double(oly[j])) / 3.0);
+                                hz[k] += ar * (double(Az) + (double(opz[k]) + double(olz[j])) / 3.0);
+                            }
                         }
                     }
                 }
@@ -1252,6 +1347,7 @@ void finish_cells_kernel(ClipArgs a, int nq, int W) {
     int ntri = 0;
     double rcell = 0;  // largest distance of a vertex from the seed (FP64)
     double P0x = 0, P0y = 0, P0z = 0;  // apex, global frame
+    int vmx[3] = {0, 0, 0};
     if (a.g > 0) {
         const int g = a.g;
         const double vs = a.vs;
@@ -1271,201 +1367,299 @@ void finish_cells_kernel(ClipArgs a, int nq, int W) {
             bmx[2] = fmax(bmx[2], gz);
         }
         rcell = sqrt(wave_max(vr2));
-        int vmn[3], vmx[3];
+        int vmn[3];
+        double mid[3];  // middle of the box, in voxels (VOX)
 #pragma unroll
         for (int d = 0; d < 3; ++d) {
             // (int)(b / vs) clamped to [0, g-1] (ConvexCell.cl:939-940); the
             // clamp is applied in floating point first so that inf/NaN from a
             // degenerate vertex cannot produce an out-of-grid range
             const double lo = wave_min(bmn[d]) / vs, hi = wave_max(bmx[d]) / vs;
-            vmn[d] = int(fmin(fmax(lo, 0.0), double(g - 1)));
-            vmx[d] = int(fmin(fmax(hi, 0.0), double(g - 1)));
+            vmn[d] = uni(int(fmin(fmax(lo, 0.0), double(g - 1))));
+            vmx[d] = uni(int(fmin(fmax(hi, 0.0), double(g - 1))));
             if (vmx[d] < vmn[d]) vmx[d] = vmn[d];
+            mid[d] = fmin(fmax(0.5 * (lo + hi), double(vmn[d])), double(vmx[d]));
         }
-        const int nx = vmx[0] - vmn[0] + 1, ny = vmx[1] - vmn[1] + 1, nz = vmx[2] - vmn[2] + 1;
-        const int nvox = nx * ny * nz;
-        // First voxel of the box, in scan order (x fastest, then y, z),
-        // whose flag is not 1 (the reference corner rule) or whose class is
-        // known (apex_mode 1); usually the first voxel already.
-        int first_ref = -1, first_c = -1, ref_flag = 1, c_flag = 1;
-        for (int vb = 0; vb < nvox && (a.apex_mode == 1 ? first_c < 0 : first_ref < 0); vb += 64) {
-            const int v = vb + lane;
-            const bool in = v < nvox;
-            int f = 1, cf = 1;
-            if (in) {
-                const int x = vmn[0] + v % nx, y = vmn[1] + (v / nx) % ny, z = vmn[2] + v / (nx * ny);
-                const int id = x + y * g + z * g * g;
-                f = a.flags[id];
-                cf = a.centre ? a.centre[id] : (a.toffs[id + 1] == a.toffs[id] ? f : 1);
+        if constexpr (VOX) {
+            // ---- voxel domain: every boundary face is a voxel face, and the
+            // class of every voxel is known -------------------------------
+            // Apex: near the middle of the cell's box, off the lattice and
+            // off the middle planes of voxels, in a voxel of known class.
+            // From inside the cell the cones only meet it where the boundary
+            // does, so fewer strips are clipped than from the box's first
+            // voxel.
+            int va[3];
+#pragma unroll
+            for (int d = 0; d < 3; ++d) {
+                va[d] = uni(min(int(mid[d]), vmx[d]));
+                const double fr = fmin(fmax(mid[d] - double(va[d]), 0.25), 0.75);
+                const double P0 = (double(va[d]) + fr + (kApexFrac[d] - 0.5)) * vs;
+                if (d == 0) P0x = P0;
+                if (d == 1) P0y = P0;
+                if (d == 2) P0z = P0;
             }
-            const uint64_t mr = ballot(in && f != 1);
-            if (first_ref < 0 && mr) {
-                const int l = lowest_bit(mr);
-                first_ref = vb + l;
-                ref_flag = rlane(f, l);
-            }
-            const uint64_t mc = ballot(in && cf != 1);
-            if (first_c < 0 && mc) {
-                const int l = lowest_bit(mc);
-                first_c = vb + l;
-                c_flag = rlane(cf, l);
-            }
-        }
-        // Union of the voxels' lists (merge, ConvexCell.cl:722-749).  The
-        // list entries of one row of the box are one range of tlist; the
-        // rows' ranges are spread over the lanes.  An entry is kept in the
-        // first voxel of the box, in scan order, whose list holds its
-        // triangle: tinfo holds the entry's voxel and a mask of the voxels
-        // within 2 of it per axis that precede it and hold the triangle too
-        // (or kTinfoFar when one farther away does: then the triangle's own
-        // voxel list is read).  Entries are kept in scan order.
-        int nu = 0;
-        const uint32_t pmn = (uint32_t(vmn[2]) << 20) | (uint32_t(vmn[1]) << 10) | uint32_t(vmn[0]);
-        const uint32_t pmx = (uint32_t(vmx[2]) << 20) | (uint32_t(vmx[1]) << 10) | uint32_t(vmx[0]);
-        int *seg_off = reinterpret_cast<int *>(cpl), *seg_a = seg_off + 64;
-        const int nrows = ny * nz;
-        for (int rb = 0; rb < nrows; rb += 64) {
-            const int r = rb + lane;
-            int sa = 0, len = 0;
-            if (r < nrows) {
-                const int id0 = vmn[0] + (vmn[1] + r % ny) * g + (vmn[2] + r / ny) * g * g;
-                sa = a.toffs[id0];
-                len = a.toffs[id0 + nx] - sa;
-            }
-            const int off = wave_excl_scan(len);
-            const int total = uni(rlane(off + len, 63));
-            if (total == 0) continue;
-            seg_off[lane] = off;
-            seg_a[lane] = sa;
-            wsync();
-            for (int base = 0; base < total; base += 64) {
-                const int e = base + lane;
-                bool keep = false;
-                int t = -1;
-                if (e < total) {
-                    // last row whose offset is <= e (empty rows never win)
-                    int lo = 0, hi = 63;
-                    while (lo < hi) {
-                        const int mid = (lo + hi + 1) >> 1;
-                        if (seg_off[mid] <= e)
-                            lo = mid;
-                        else
-                            hi = mid - 1;
-                    }
-                    const int q = seg_a[lo] + (e - seg_off[lo]);
-                    t = a.tlist[q];
-                    const uint4 inf = a.tinfo[q];
-                    const uint32_t pv = inf.x;
-                    const uint64_t near = (uint64_t(inf.z) << 32) | inf.y;
-                    if (near & kTinfoFar) {
-                        keep = true;
-                        for (int u = a.tvoffs[t], ue = a.tvoffs[t + 1]; u < ue; ++u) {
-                            const uint32_t w = a.tvox[u];
-                            if (w >= pv) break;
-                            const uint32_t ux = w & 1023u, uy = (w >> 10) & 1023u, uz = w >> 20;
-                            if (ux >= (pmn & 1023u) && ux <= (pmx & 1023u) && uy >= ((pmn >> 10) & 1023u) &&
-                                uy <= ((pmx >> 10) & 1023u) && uz >= (pmn >> 20) && uz <= (pmx >> 20)) {
-                                keep = false;  // an earlier voxel of the box holds it
-                                break;
-                            }
-                        }
-                    } else {
-                        const int x = int(pv & 1023u), y = int((pv >> 10) & 1023u), z = int(pv >> 20);
-                        keep = (near & box_near(x, y, z, vmn, vmx)) == 0;
-                    }
+            const int in_domain = uni(int(a.centre[va[0] + va[1] * g + va[2] * g * g]));
+            // Strips: the faces of one orientation side by side along x (faces
+            // across y or z) or y (faces across x) within the box.  Faces are
+            // listed once, at their lowest lattice point, so the box's faces
+            // are one range per row of lattice points; a face whose neighbour
+            // before it lies in the box too belongs to that one's strip.
+            // Faces on a side of the box inside the frame only touch the
+            // cell, which lies on one side of them.
+            int nu = 0;
+            const int g1 = g + 1;
+            const int nx = vmx[0] - vmn[0] + 2, ny = vmx[1] - vmn[1] + 2, nz = vmx[2] - vmn[2] + 2;
+            int *seg_off = reinterpret_cast<int *>(cpl), *seg_a = seg_off + 64;
+            const int nrows = ny * nz;
+            for (int rb = 0; rb < nrows; rb += 64) {
+                const int r = rb + lane;
+                int sa = 0, len = 0;
+                if (r < nrows) {
+                    const int id0 = vmn[0] + (vmn[1] + r % ny) * g1 + (vmn[2] + r / ny) * g1 * g1;
+                    sa = a.vfoffs[id0];
+                    len = a.vfoffs[id0 + nx] - sa;
                 }
-                const uint64_t m = ballot(keep);
-                if (keep && nu + mbcnt(m) < a.T) tu[nu + mbcnt(m)] = t;
-                nu += __popcll(m);
+                const int off = wave_excl_scan(len);
+                const int total = uni(rlane(off + len, 63));
+                if (total == 0) continue;
+                seg_off[lane] = off;
+                seg_a[lane] = sa;
+                wsync();
+                for (int base = 0; base < total; base += 64) {
+                    const int e = base + lane;
+                    bool keep = false;
+                    int q = -1;
+                    if (e < total) {
+                        // last row whose offset is <= e (empty rows never win)
+                        int lo = 0, hi = 63;
+                        while (lo < hi) {
+                            const int m = (lo + hi + 1) >> 1;
+                            if (seg_off[m] <= e)
+                                lo = m;
+                            else
+                                hi = m - 1;
+                        }
+                        q = seg_a[lo] + (e - seg_off[lo]);
+                        const uint2 ent = a.vface[q];
+                        const int p[3] = {int(ent.x & 1023u), int((ent.x >> 10) & 1023u), int((ent.x >> 20) & 1023u)};
+                        const int ax = int(ent.x >> 30);
+                        const bool prev = (ent.y & kVfacePrev) != 0;
+                        keep = true;
+#pragma unroll
+                        for (int d = 0; d < 3; ++d)
+                            keep = keep && (d == ax ? (p[d] > vmn[d] || p[d] == 0) && (p[d] <= vmx[d] || p[d] == g)
+                                                    : p[d] <= vmx[d]);
+                        const bool first = ax == 0 ? p[1] == vmn[1] : p[0] == vmn[0];
+                        keep = keep && (first || !prev);
+                    }
+                    const uint64_t m = ballot(keep);
+                    if (keep && nu + mbcnt(m) < a.T) tu[nu + mbcnt(m)] = q;
+                    nu += __popcll(m);
+                }
+                wsync();  // the next rows overwrite seg_off / seg_a
             }
-            wsync();  // the next rows overwrite seg_off / seg_a
-        }
-        if (nu > a.T) {
-            // the cap a re-queue pass needs for this cell
-            if (sub == 0 && lane == 0 && a.fl_cnt) atomicMax(a.fl_cnt + 13, nu);
-            fail(RPD_TRIANGLE_OVERFLOW);
-            return;
-        }
-        if (a.dcnt && sub == 0 && lane == 0) {  // ConvexCell.cl:981-982
-            atomicMax(a.dcnt + kDcMax + 3, nu);
-            atomicAdd(a.dcnt + kDcHistT + min(nu, kDcUnionMax), 1);
-        }
-        wsync();
-        ntri = nu;
-        // apex
-        int in_domain = 1;
-        auto vox_xyz = [&](int v, int &x, int &y, int &z) {
-            x = vmn[0] + v % nx;
-            y = vmn[1] + (v / nx) % ny;
-            z = vmn[2] + v / (nx * ny);
-        };
-        if (a.apex_mode == 1 && first_c >= 0) {
-            int x, y, z;
-            vox_xyz(first_c, x, y, z);
-            P0x = (x + kApexFrac[0]) * vs;
-            P0y = (y + kApexFrac[1]) * vs;
-            P0z = (z + kApexFrac[2]) * vs;
-            in_domain = c_flag;
-        } else if (first_ref >= 0) {
-            int x, y, z;
-            vox_xyz(first_ref, x, y, z);
-            P0x = x * vs;
-            P0y = y * vs;
-            P0z = z * vs;
-            in_domain = ref_flag;
+            if (nu > a.T) {
+                // the cap a re-queue pass needs for this cell
+                if (sub == 0 && lane == 0 && a.fl_cnt) atomicMax(a.fl_cnt + 13, nu);
+                fail(RPD_TRIANGLE_OVERFLOW);
+                return;
+            }
+            wsync();
+            ntri = nu;
+            add_volume = in_domain == 2;
         } else {
-            // GRID_OUT_DOMAIN fallback (ConvexCell.cl:985-1051)
-            auto flag = [&](int x, int y, int z) { return int(a.flags[x + y * g + z * g * g]); };
-            auto setc = [&](int x, int y, int z) {
+            const int nx = vmx[0] - vmn[0] + 1, ny = vmx[1] - vmn[1] + 1, nz = vmx[2] - vmn[2] + 1;
+            const int nvox = nx * ny * nz;
+            // First voxel of the box, in scan order (x fastest, then y, z),
+            // whose flag is not 1 (the reference corner rule) or whose class is
+            // known (apex_mode 1); usually the first voxel already.
+            int first_ref = -1, first_c = -1, ref_flag = 1, c_flag = 1;
+            for (int vb = 0; vb < nvox && (a.apex_mode == 1 ? first_c < 0 : first_ref < 0); vb += 64) {
+                const int v = vb + lane;
+                const bool in = v < nvox;
+                int f = 1, cf = 1;
+                if (in) {
+                    const int x = vmn[0] + v % nx, y = vmn[1] + (v / nx) % ny, z = vmn[2] + v / (nx * ny);
+                    const int id = x + y * g + z * g * g;
+                    f = a.flags[id];
+                    cf = a.centre ? a.centre[id] : (a.toffs[id + 1] == a.toffs[id] ? f : 1);
+                }
+                const uint64_t mr = ballot(in && f != 1);
+                if (first_ref < 0 && mr) {
+                    const int l = lowest_bit(mr);
+                    first_ref = vb + l;
+                    ref_flag = rlane(f, l);
+                }
+                const uint64_t mc = ballot(in && cf != 1);
+                if (first_c < 0 && mc) {
+                    const int l = lowest_bit(mc);
+                    first_c = vb + l;
+                    c_flag = rlane(cf, l);
+                }
+            }
+            // Union of the voxels' lists (merge, ConvexCell.cl:722-749).  The
+            // list entries of one row of the box are one range of tlist; the
+            // rows' ranges are spread over the lanes.  An entry is kept in the
+            // first voxel of the box, in scan order, whose list holds its
+            // triangle: tinfo holds the entry's voxel and a mask of the voxels
+            // within 2 of it per axis that precede it and hold the triangle too
+            // (or kTinfoFar when one farther away does: then the triangle's own
+            // voxel list is read).  Entries are kept in scan order.
+            int nu = 0;
+            const uint32_t pmn = (uint32_t(vmn[2]) << 20) | (uint32_t(vmn[1]) << 10) | uint32_t(vmn[0]);
+            const uint32_t pmx = (uint32_t(vmx[2]) << 20) | (uint32_t(vmx[1]) << 10) | uint32_t(vmx[0]);
+            int *seg_off = reinterpret_cast<int *>(cpl), *seg_a = seg_off + 64;
+            const int nrows = ny * nz;
+            for (int rb = 0; rb < nrows; rb += 64) {
+                const int r = rb + lane;
+                int sa = 0, len = 0;
+                if (r < nrows) {
+                    const int id0 = vmn[0] + (vmn[1] + r % ny) * g + (vmn[2] + r / ny) * g * g;
+                    sa = a.toffs[id0];
+                    len = a.toffs[id0 + nx] - sa;
+                }
+                const int off = wave_excl_scan(len);
+                const int total = uni(rlane(off + len, 63));
+                if (total == 0) continue;
+                seg_off[lane] = off;
+                seg_a[lane] = sa;
+                wsync();
+                for (int base = 0; base < total; base += 64) {
+                    const int e = base + lane;
+                    bool keep = false;
+                    int t = -1;
+                    if (e < total) {
+                        // last row whose offset is <= e (empty rows never win)
+                        int lo = 0, hi = 63;
+                        while (lo < hi) {
+                            const int mid = (lo + hi + 1) >> 1;
+                            if (seg_off[mid] <= e)
+                                lo = mid;
+                            else
+                                hi = mid - 1;
+                        }
+                        const int q = seg_a[lo] + (e - seg_off[lo]);
+                        t = a.tlist[q];
+                        const uint4 inf = a.tinfo[q];
+                        const uint32_t pv = inf.x;
+                        const uint64_t near = (uint64_t(inf.z) << 32) | inf.y;
+                        if (near & kTinfoFar) {
+                            keep = true;
+                            for (int u = a.tvoffs[t], ue = a.tvoffs[t + 1]; u < ue; ++u) {
+                                const uint32_t w = a.tvox[u];
+                                if (w >= pv) break;
+                                const uint32_t ux = w & 1023u, uy = (w >> 10) & 1023u, uz = w >> 20;
+                                if (ux >= (pmn & 1023u) && ux <= (pmx & 1023u) && uy >= ((pmn >> 10) & 1023u) &&
+                                    uy <= ((pmx >> 10) & 1023u) && uz >= (pmn >> 20) && uz <= (pmx >> 20)) {
+                                    keep = false;  // an earlier voxel of the box holds it
+                                    break;
+                                }
+                            }
+                        } else {
+                            const int x = int(pv & 1023u), y = int((pv >> 10) & 1023u), z = int(pv >> 20);
+                            keep = (near & box_near(x, y, z, vmn, vmx)) == 0;
+                        }
+                    }
+                    const uint64_t m = ballot(keep);
+                    if (keep && nu + mbcnt(m) < a.T) tu[nu + mbcnt(m)] = t;
+                    nu += __popcll(m);
+                }
+                wsync();  // the next rows overwrite seg_off / seg_a
+            }
+            if (a.count_only) {
+                if (lane == 0 && a.status[orig] != RPD_TRIANGLE_OVERFLOW) {
+                    atomicMax(a.dcnt + kDcMax + 3, nu);
+                    atomicAdd(a.dcnt + kDcHistT + min(nu, kDcUnionMax), 1);
+                }
+                return;
+            }
+            if (nu > a.T) {
+                // the cap a re-queue pass needs for this cell
+                if (sub == 0 && lane == 0 && a.fl_cnt) atomicMax(a.fl_cnt + 13, nu);
+                fail(RPD_TRIANGLE_OVERFLOW);
+                return;
+            }
+            if (a.dcnt && sub == 0 && lane == 0) {  // ConvexCell.cl:981-982
+                atomicMax(a.dcnt + kDcMax + 3, nu);
+                atomicAdd(a.dcnt + kDcHistT + min(nu, kDcUnionMax), 1);
+            }
+            wsync();
+            ntri = nu;
+            // apex
+            int in_domain = 1;
+            auto vox_xyz = [&](int v, int &x, int &y, int &z) {
+                x = vmn[0] + v % nx;
+                y = vmn[1] + (v / nx) % ny;
+                z = vmn[2] + v / (nx * ny);
+            };
+            if (a.apex_mode == 1 && first_c >= 0) {
+                int x, y, z;
+                vox_xyz(first_c, x, y, z);
+                P0x = (x + kApexFrac[0]) * vs;
+                P0y = (y + kApexFrac[1]) * vs;
+                P0z = (z + kApexFrac[2]) * vs;
+                in_domain = c_flag;
+            } else if (first_ref >= 0) {
+                int x, y, z;
+                vox_xyz(first_ref, x, y, z);
                 P0x = x * vs;
                 P0y = y * vs;
                 P0z = z * vs;
-            };
-            if (vmx[2] + 1 < g) {
-                const int z = vmx[2] + 1;
-                for (int y = vmn[1]; y <= vmx[1] + 1 && y < g && in_domain == 1; y++)
-                    for (int x = vmn[0]; x <= vmx[0] + 1 && x < g; x++)
-                        if (flag(x, y, z) != 1) {
-                            in_domain = flag(x, y, z);
-                            setc(x, y, z);
-                            break;
-                        }
+                in_domain = ref_flag;
             } else {
-                in_domain = 0;
-                setc(vmn[0], vmn[1], vmx[2] + 1);
+                // GRID_OUT_DOMAIN fallback (ConvexCell.cl:985-1051)
+                auto flag = [&](int x, int y, int z) { return int(a.flags[x + y * g + z * g * g]); };
+                auto setc = [&](int x, int y, int z) {
+                    P0x = x * vs;
+                    P0y = y * vs;
+                    P0z = z * vs;
+                };
+                if (vmx[2] + 1 < g) {
+                    const int z = vmx[2] + 1;
+                    for (int y = vmn[1]; y <= vmx[1] + 1 && y < g && in_domain == 1; y++)
+                        for (int x = vmn[0]; x <= vmx[0] + 1 && x < g; x++)
+                            if (flag(x, y, z) != 1) {
+                                in_domain = flag(x, y, z);
+                                setc(x, y, z);
+                                break;
+                            }
+                } else {
+                    in_domain = 0;
+                    setc(vmn[0], vmn[1], vmx[2] + 1);
+                }
+                if (in_domain == 1 && vmx[1] + 1 < g) {
+                    const int y = vmx[1] + 1;
+                    for (int z = vmn[2]; z <= vmx[2] && in_domain == 1; z++)
+                        for (int x = vmn[0]; x <= vmx[0] + 1 && x < g; x++)
+                            if (flag(x, y, z) != 1) {
+                                in_domain = flag(x, y, z);
+                                setc(x, y, z);
+                                break;
+                            }
+                } else if (in_domain == 1) {
+                    in_domain = 0;
+                    setc(vmn[0], vmx[1] + 1, vmn[2]);
+                }
+                if (in_domain == 1 && vmx[0] + 1 < g) {
+                    const int x = vmx[0] + 1;
+                    for (int z = vmn[2]; z <= vmx[2] && in_domain == 1; z++)
+                        for (int y = vmn[1]; y <= vmx[1]; y++)
+                            if (flag(x, y, z) != 1) {
+                                in_domain = flag(x, y, z);
+                                setc(x, y, z);
+                                break;
+                            }
+                } else if (in_domain == 1) {
+                    in_domain = 0;
+                    setc(vmx[0] + 1, vmn[1], vmn[2]);
+                }
+                if (in_domain == 1) {
+                    fail(RPD_FIND_ANOTHER_BEGINNING_VERTEX);
+                    return;
+                }
             }
-            if (in_domain == 1 && vmx[1] + 1 < g) {
-                const int y = vmx[1] + 1;
-                for (int z = vmn[2]; z <= vmx[2] && in_domain == 1; z++)
-                    for (int x = vmn[0]; x <= vmx[0] + 1 && x < g; x++)
-                        if (flag(x, y, z) != 1) {
-                            in_domain = flag(x, y, z);
-                            setc(x, y, z);
-                            break;
-                        }
-            } else if (in_domain == 1) {
-                in_domain = 0;
-                setc(vmn[0], vmx[1] + 1, vmn[2]);
-            }
-            if (in_domain == 1 && vmx[0] + 1 < g) {
-                const int x = vmx[0] + 1;
-                for (int z = vmn[2]; z <= vmx[2] && in_domain == 1; z++)
-                    for (int y = vmn[1]; y <= vmx[1]; y++)
-                        if (flag(x, y, z) != 1) {
-                            in_domain = flag(x, y, z);
-                            setc(x, y, z);
-                            break;
-                        }
-            } else if (in_domain == 1) {
-                in_domain = 0;
-                setc(vmx[0] + 1, vmn[1], vmn[2]);
-            }
-            if (in_domain == 1) {
-                fail(RPD_FIND_ANOTHER_BEGINNING_VERTEX);
-                return;
-            }
+            add_volume = in_domain == 2;
         }
-        add_volume = in_domain == 2;
     }
     double4 cadd = make_double4(0.0, 0.0, 0.0, 0.0);
     if (add_volume && sub == 0) cadd = integrate(1.0);
@@ -1479,13 +1673,15 @@ void finish_cells_kernel(ClipArgs a, int nq, int W) {
     if (ntri > 0) {
         // backup (ConvexCell.cl:692-715): the vertex registers and the plane count
         const WaveCell<R, RP, FILTER, S> bk = c;
-        const bool may_skip = c.nb_plane + 4 <= P && nvalid + 6 <= a.V;
+        constexpr int kPl = VOX ? 5 : 4;    // cone planes of a unit (strip or triangle)
+        constexpr int kUB = VOX ? 12 : 16;  // units of a batch
+        constexpr uint64_t kUm = (1ull << kPl) - 1;
+        const bool may_skip = c.nb_plane + kPl <= P && nvalid + (VOX ? 8 : 6) <= a.V;
         const double lx0 = P0x - S0.x, ly0 = P0y - S0.y, lz0 = P0z - S0.z;
         const double face_margin = sizeof(RP) == 8 ? 1e-7 : 1e-3;
         // The cell's vertices, compacted, for the lane-parallel tests: a cone
         // plane removes every vertex (with the margin of removes_all) when
         // each one is strictly on its removed side.
-        VtxRec<R> *vtx = reinterpret_cast<VtxRec<R> *>(tcor + 16 * 9);
         int nvc = 0;
 #pragma unroll
         for (int s = 0; s < S; ++s) {
@@ -1499,13 +1695,68 @@ void finish_cells_kernel(ClipArgs a, int nq, int W) {
         // removes every vertex (kept side n.y + d >= 0), with a margin far
         // above the rounding of d and rcell.
         const double rsk = rcell * (1.0 + 1e-9) + 1e-9;
-        for (int jb = sub; jb < ntri; jb += 16 * W) {
-            // cone planes (A,B,C), (A,D,B), (A,C,D), (C,D,B), A = apex
-            // (CCClipTetFromPointsInfinite): lane = 4 * triangle + plane
-            const int i = lane >> 2, f = lane & 3;
-            const int k = jb + W * i;
+        // VOX: wave sub takes the batches sub, sub + W, ... of 12 strips in
+        // list order; else the triangles sub, sub + W, ...
+        for (int jb = VOX ? sub * kUB : sub; jb < ntri; jb += kUB * W) {
+            // cone planes, lane = kPl * unit + plane
+            const int i = VOX ? lane / 5 : lane >> 2, f = VOX ? lane - 5 * i : lane & 3;
+            const int k = VOX ? (i < kUB ? jb + i : ntri) : jb + W * i;
             Pl<RP> pl{RP(0), RP(0), RP(0), RP(0)};
-            if (k < ntri) {
+            uint64_t gom = 0;  // VOX: strips whose region counts positive, at lane 5 * strip
+            // VOX: the strip in the local frame, across axis ax at rc, from
+            // (ru0, rv0) to (ru1, rv1) along its two other axes
+            int ax = 0;
+            double rc = 0, ru0 = 0, ru1 = 0, rv0 = 0, rv1 = 0;
+            if constexpr (VOX) {
+                // Cone of a strip from the apex A: for each side, the plane
+                // through A and that side, which is parallel to an axis, so
+                // its normal has two components; and the strip's own plane.
+                bool go = false;
+                if (k < ntri) {
+                    const uint2 ent = a.vface[tu[k]];
+                    const int p0 = int(ent.x & 1023u), p1 = int((ent.x >> 10) & 1023u), p2 = int((ent.x >> 20) & 1023u);
+                    ax = int(ent.x >> 30);
+                    const int run = int(ent.y >> 2);
+                    // axes (u, v) of the strip: x across: (y, z); y: (x, z); z: (x, y)
+                    const int pc = ax == 0 ? p0 : (ax == 1 ? p1 : p2);
+                    const int pu = ax == 0 ? p1 : p0, pv = ax == 2 ? p1 : p2;
+                    const int pu1 = min(pu + run, (ax == 0 ? vmx[1] : vmx[0]) + 1);
+                    const double Sc = ax == 0 ? S0.x : (ax == 1 ? S0.y : S0.z), Su = ax == 0 ? S0.y : S0.x,
+                                 Sv = ax == 2 ? S0.y : S0.z;
+                    const double Ac = ax == 0 ? lx0 : (ax == 1 ? ly0 : lz0), Au = ax == 0 ? ly0 : lx0,
+                                 Av = ax == 2 ? ly0 : lz0;
+                    rc = pc * a.vs - Sc;
+                    ru0 = pu * a.vs - Su;
+                    ru1 = pu1 * a.vs - Su;
+                    rv0 = pv * a.vs - Sv;
+                    rv1 = (pv + 1) * a.vs - Sv;
+                    const double da = rc - Ac;  // not 0: the apex is inside a voxel
+                    go = (ent.y & kVfaceUp) ? da > 0.0 : da < 0.0;
+                    const double sg = da > 0.0 ? 1.0 : -1.0;
+                    double nc, nt = 0, nd;
+                    if (f < 4) {
+                        // sides v0, v1, u0, u1
+                        const double At = f < 2 ? Av : Au;
+                        const double dt = (f == 0 ? rv0 : (f == 1 ? rv1 : (f == 2 ? ru0 : ru1))) - At;
+                        const double il = ((f & 1) ? -1.0 : 1.0) / sqrt(da * da + dt * dt);
+                        nt = fabs(da) * il;
+                        nc = -sg * dt * il;
+                        nd = -(nt * At + nc * Ac);
+                    } else {
+                        nc = sg;
+                        nd = -sg * rc;
+                    }
+                    // back to x, y, z
+                    const bool tu_ = f >= 2;  // the side's axis t is u (else v)
+                    const double nu_ = tu_ ? nt : 0.0, nv_ = tu_ ? 0.0 : nt;
+                    pl = Pl<RP>{RP(ax == 0 ? nc : nu_), RP(ax == 0 ? nu_ : (ax == 1 ? nc : nv_)),
+                                RP(ax == 2 ? nc : nv_), RP(nd)};
+                }
+                gom = ballot(go);
+            }
+            // general domain: planes (A,B,C), (A,D,B), (A,C,D), (C,D,B), A =
+            // apex (CCClipTetFromPointsInfinite)
+            if (!VOX && k < ntri) {
                 const int tid = tu[k];
                 const double4 G1 = a.gpts[a.tris[3 * tid]];
                 double4 G2 = a.gpts[a.tris[3 * tid + 1]], G3 = a.gpts[a.tris[3 * tid + 2]];
@@ -1611,7 +1862,28 @@ void finish_cells_kernel(ClipArgs a, int nq, int W) {
             // triangle i.
             {
                 bool sep = false;
-                if (may_skip && k < ntri && ((skipm >> (4 * i)) & 0xfull) == 0) {
+                if constexpr (VOX) {
+                    if (may_skip && k < ntri && ((skipm >> (kPl * i)) & kUm) == 0) {
+                        // the strip's corner farthest along the plane's normal
+                        // decides for all four
+                        for (int j = f; j < c.nb_plane && !sep; j += 10) {
+                            Pl<RP> q2[2];
+#pragma unroll
+                            for (int u = 0; u < 2; ++u) q2[u] = c.planes[min(j + 5 * u, c.nb_plane - 1)];
+#pragma unroll
+                            for (int u = 0; u < 2; ++u) {
+                                const double nx = double(q2[u].x), ny = double(q2[u].y), nz = double(q2[u].z),
+                                             nw = double(q2[u].w);
+                                const double nc = ax == 0 ? nx : (ax == 1 ? ny : nz), nu_ = ax == 0 ? ny : nx,
+                                             nv_ = ax == 2 ? ny : nz;
+                                const double far = nc * rc + fmax(nu_ * ru0, nu_ * ru1) + fmax(nv_ * rv0, nv_ * rv1);
+                                const double m = face_margin * (1.0 + fabs(nw));
+                                sep = sep || (far + nw < -m && far - (nx * lx0 + ny * ly0 + nz * lz0) <= 0.0);
+                            }
+                        }
+                    }
+                }
+                if (!VOX && may_skip && k < ntri && ((skipm >> (4 * i)) & 0xfull) == 0) {
                     double px[3], py[3], pz[3];
 #pragma unroll
                     for (int v = 0; v < 3; ++v) {
@@ -1647,25 +1919,27 @@ void finish_cells_kernel(ClipArgs a, int nq, int W) {
             // lanes skipped them
             uint32_t todo = 0;
 #pragma unroll
-            for (int t = 0; t < 16; ++t)
-                if (jb + W * t < ntri && ((skipm >> (4 * t)) & 0xfull) == 0) todo |= 1u << t;
-            if (W > 1 && lane < 16 && jb + W * lane < ntri) contrib[jb + W * lane] = make_double4(0.0, 0.0, 0.0, 0.0);
+            for (int t = 0; t < kUB; ++t)
+                if (jb + (VOX ? t : W * t) < ntri && ((skipm >> (kPl * t)) & kUm) == 0) todo |= 1u << t;
+            if (W > 1 && lane < kUB && jb + (VOX ? lane : W * lane) < ntri)
+                contrib[jb + (VOX ? lane : W * lane)] = make_double4(0.0, 0.0, 0.0, 0.0);
             // in increasing k: the running sums add the contributions in order
             // (a skipped triangle adds +0, which leaves them unchanged)
             while (todo) {
                 const int t = __builtin_ctz(todo);
                 todo &= todo - 1;
-                const int kk = jb + W * t;
-                const int tid = uni(tu[kk]);
+                const int kk = jb + (VOX ? t : W * t);
+                // (a strip stands for several triangles: its place in the list)
+                const int tid = VOX ? kk : uni(tu[kk]);
                 if (tid > fail_t) continue;
                 double4 ck = make_double4(0.0, 0.0, 0.0, 0.0);
                 int res = kNoClip;
                 // each cone plane read from LDS just before its clip: the four
                 // held at once would take 32 registers through the clips
 #pragma unroll
-                for (int f2 = 0; f2 < 4; ++f2) {
+                for (int f2 = 0; f2 < kPl; ++f2) {
                     if (res < 0) {
-                        const Pl<RP> q = cpl[4 * t + f2];
+                        const Pl<RP> q = cpl[kPl * t + f2];
                         res = c.nb_plane >= P ? int(RPD_PLANE_OVERFLOW) : c.template clip<false>(cvt<R>(q), -1, q);
                     }
                 }
@@ -1673,7 +1947,7 @@ void finish_cells_kernel(ClipArgs a, int nq, int W) {
                     fail_t = tid;
                     fail_st = res;
                 } else if (res != RPD_EMPTY_CELL) {
-                    ck = integrate(goo[t] ? 1.0 : -1.0);
+                    ck = integrate((VOX ? ((gom >> (kPl * t)) & 1) != 0 : goo[t] != 0) ? 1.0 : -1.0);
                 }
                 c = bk;
                 if (W == 1) {
@@ -1864,6 +2138,8 @@ static int make_args(int form, const ClipLaunch &L, ClipArgs &a) {
         a.tvoffs = L.dom->tvoffs;
         a.tvox = L.dom->tvox;
         a.tinfo = L.dom->tinfo;
+        a.vfoffs = L.dom->vfoffs;
+        a.vface = L.dom->vface;
         a.dist = L.cull ? L.dom->dist : nullptr;
     }
     a.security_mode = L.security_mode;
@@ -1998,64 +2274,79 @@ int rpd_launch_finish(hipStream_t st, int form, const ClipLaunch &L, int nq, int
     const int S = L.V <= 64 ? 1 : (L.V <= 128 ? 2 : 4);
     // kernel B: restriction + integration of the queued cells.  Short queues
     // (re-queue passes) spread each cell over W waves.
-    {
-        const size_t pl = plane_bytes(form);
-        const bool hess = a.H > 0;
-        const size_t wstride = finish_wave_lds(L.P, S, a.T, pl, true) + (hess ? hessian_wave_lds(L.P, S) : 0);
+    const size_t pl = plane_bytes(form);
+    const bool hess = a.H > 0;
+    // Domains of voxel faces (of every request of a batch) restrict by strips;
+    // the FP32 form and the reference's corner apex take the triangle lists.
+    // The debug counters count triangles: with strips, a launch of the
+    // triangle form for the union's counters alone follows.
+    const bool vox = L.vox && form != RPD_PREC_FP32 && a.apex_mode == 1;
+    // waves per cell from the cells that share the device: this queue's and
+    // those of finish kernels running beside it (the Hessian variant: one wave
+    // per cell)
+    const int64_t load = int64_t(nq) + std::max(beside, 0);
+    auto launch = [&](bool vx, bool hs) -> int {
+        const size_t wstride =
+            (vx ? finish_vox_wave_lds(L.P, S, a.T, form == RPD_PREC_FP64 ? sizeof(VtxRec<double>) : sizeof(VtxRec<float>))
+                : finish_wave_lds(L.P, S, a.T, pl, true)) +
+            (hs ? hessian_wave_lds(L.P + (vx ? 1 : 0), S) : 0);
         const size_t kLdsMax = lds_limit();
         if (finish_cell_stride(a.T, 1) + wstride > kLdsMax) return RPD_E_LIMIT;
-        // waves per cell from the cells that share the device: this queue's
-        // and those of finish kernels running beside it (the Hessian variant:
-        // one wave per cell)
-        const int64_t load = int64_t(nq) + std::max(beside, 0);
-        int W = hess || load > 32768 ? 1 : (load <= 2048 ? 8 : (load <= 8192 ? 4 : 2));
+        int W = hs || a.count_only || load > 32768 ? 1 : (load <= 2048 ? 8 : (load <= 8192 ? 4 : 2));
         while (W > 1 && finish_cell_stride(a.T, W) + W * wstride > kLdsMax) W >>= 1;
-        const size_t cstride = finish_cell_stride(a.T, W);
         a.lds_stride = int(wstride);
-        a.cell_stride = int(cstride);
+        a.cell_stride = int(finish_cell_stride(a.T, W));
         // One cell per workgroup: a workgroup keeps its LDS until its last
         // wave ends, and cell costs are skewed (interior cells are cheap), so
         // several cells per workgroup would hold the LDS of finished cells for
         // the slowest one.  LDS bounds the residency of this kernel.
-        const int wpb = W;
-        const int cpb = 1;
-        const unsigned blocks = unsigned((nq + cpb - 1) / cpb);
-        const size_t shm = size_t(cpb) * cstride + size_t(wpb) * wstride;
-#define RPD_CLIP_B1(R, RP, F, HS, B)                                                                 \
-    do {                                                                                             \
-        if (S == 1)                                                                                  \
-            finish_cells_kernel<R, RP, F, 1, HS, B><<<blocks, dim3(64 * wpb), shm, st>>>(a, nq, W);  \
-        else if (S == 2)                                                                             \
-            finish_cells_kernel<R, RP, F, 2, HS, B><<<blocks, dim3(64 * wpb), shm, st>>>(a, nq, W);  \
-        else                                                                                         \
-            finish_cells_kernel<R, RP, F, 4, HS, B><<<blocks, dim3(64 * wpb), shm, st>>>(a, nq, W);  \
+        const dim3 tb(64 * W);
+        const size_t shm = size_t(a.cell_stride) + size_t(W) * wstride;
+#define RPD_CLIP_B2(R, RP, F, HS, B, X)                                                    \
+    do {                                                                                   \
+        if (S == 1)                                                                        \
+            finish_cells_kernel<R, RP, F, 1, HS, B, X><<<unsigned(nq), tb, shm, st>>>(a, nq, W); \
+        else if (S == 2)                                                                   \
+            finish_cells_kernel<R, RP, F, 2, HS, B, X><<<unsigned(nq), tb, shm, st>>>(a, nq, W); \
+        else                                                                               \
+            finish_cells_kernel<R, RP, F, 4, HS, B, X><<<unsigned(nq), tb, shm, st>>>(a, nq, W); \
+    } while (0)
+// (the FP32 form has no strips)
+#define RPD_CLIP_B1(R, RP, F, HS, B)                       \
+    do {                                                   \
+        if (sizeof(RP) == 8 && vx)                         \
+            RPD_CLIP_B2(R, RP, F, HS, B, sizeof(RP) == 8); \
+        else                                               \
+            RPD_CLIP_B2(R, RP, F, HS, B, false);           \
     } while (0)
 // a packed batch has no Hessian
-#define RPD_CLIP_B(R, RP, F, HS)                  \
-    do {                                          \
-        if (!HS && a.reqs)                        \
-            RPD_CLIP_B1(R, RP, F, false, true);   \
-        else                                      \
-            RPD_CLIP_B1(R, RP, F, HS, false);     \
+#define RPD_CLIP_B(R, RP, F)                    \
+    do {                                        \
+        if (hs)                                 \
+            RPD_CLIP_B1(R, RP, F, true, false); \
+        else if (a.reqs)                        \
+            RPD_CLIP_B1(R, RP, F, false, true); \
+        else                                    \
+            RPD_CLIP_B1(R, RP, F, false, false); \
     } while (0)
-        if (form == RPD_PREC_FP64) {
-            if (hess)
-                RPD_CLIP_B(double, double, false, true);
-            else
-                RPD_CLIP_B(double, double, false, false);
-        } else if (form == RPD_PREC_MIXED) {
-            if (hess)
-                RPD_CLIP_B(float, double, true, true);
-            else
-                RPD_CLIP_B(float, double, true, false);
-        } else {
-            if (hess)
-                RPD_CLIP_B(float, float, false, true);
-            else
-                RPD_CLIP_B(float, float, false, false);
-        }
+        if (form == RPD_PREC_FP64)
+            RPD_CLIP_B(double, double, false);
+        else if (form == RPD_PREC_MIXED)
+            RPD_CLIP_B(float, double, true);
+        else
+            RPD_CLIP_B(float, float, false);
 #undef RPD_CLIP_B
 #undef RPD_CLIP_B1
+#undef RPD_CLIP_B2
+        return RPD_OK;
+    };
+    const int rl = launch(vox, hess);
+    if (rl != RPD_OK) return rl;
+    if (vox && a.dcnt) {
+        a.count_only = 1;
+        a.T = 0;
+        const int rc = launch(false, false);
+        if (rc != RPD_OK) return rc;
     }
     return hipGetLastError() == hipSuccess ? RPD_OK : RPD_E_DEVICE;
 }

@@ -121,6 +121,13 @@ struct DomainDev {
     const int *tvoffs = nullptr;     // per triangle: offsets into tvox
     const uint32_t *tvox = nullptr;  // per triangle: sorted voxels (z<<20 | y<<10 | x) whose list holds it
     const uint4 *tinfo = nullptr;    // per triangle-list entry: its voxel, earlier near voxels holding it
+    // A domain whose triangles are the two halves of voxel faces, in the lists
+    // of the voxels they bound, and whose voxel classes are all known: its
+    // faces, by the lattice point of their lowest corner (rpd_clip.hip,
+    // kVface*), and per lattice point ((size + 1)^3, x fastest) the offsets
+    // into them.  Else null.
+    const int *vfoffs = nullptr;
+    const uint2 *vface = nullptr;
     const uint8_t *dist = nullptr;   // Chebyshev voxel distance to domain voxels
     const int *dvox = nullptr;       // the domain voxels (distance 0), ascending
     int n_dvox = 0;
@@ -143,6 +150,8 @@ struct ReqDesc {
     const int *tvoffs;
     const uint32_t *tvox;
     const uint4 *tinfo;
+    const int *vfoffs;
+    const uint2 *vface;
     const uint8_t *dist;  // nullptr: no cull
 };
 
@@ -159,6 +168,7 @@ struct ClipLaunch {
     double wmin;
     bool cull;
     const DomainDev *dom;  // nullptr: no domain
+    bool vox;              // every domain of the launch has voxel faces (DomainDev::vface)
     double4 *out;          // original order
     int *status;           // original order
     int *kused;            // original order (nullable)
