@@ -54,9 +54,17 @@ struct rpd_domain {
     int64_t bytes = 0;
 };
 
-// work buffers of one pass: neighbour lists, queued-cell records, queue length
+// work buffers of one pass: neighbour lists, cell records, how each cell left
+// the bisector kernel, its queue counter and ticket (FailLists::q)
 struct PassBufs {
-    DevBuf knn, rec, qcount;
+    DevBuf knn, rec, code, q;
+    int ensure(int64_t n_ids, int K, size_t rec_bytes) {
+        const size_t n = size_t(std::max<int64_t>(n_ids, 1));
+        int r = knn.ensure(n * size_t(K) * 4);
+        if (r == RPD_OK) r = rec.ensure(n * rec_bytes);
+        if (r == RPD_OK) r = code.ensure((n + 15) & ~size_t(15));
+        return r;
+    }
 };
 // failed cells handed to the next pass: counters, then stored ids of the
 // exact-predicate failures and the overflows (eo, 2n entries: exact ones
@@ -127,15 +135,17 @@ struct rpd_ctx {
     };
     std::vector<BatchReq> batch;
     DevBuf req_desc, knn_req, req_of;
-    // pass work buffers: up to three passes may run at once, one per stream
-    PassBufs pb[4];
+    // pass work buffers: up to three passes may run at once, one per stream;
+    // pass 1's own (its records keep the states of its resumable cells and
+    // serve the finish failures' first pass)
+    PassBufs pb[4], pb1;
     // pass 1 writes lists 0 (bisector kernel) and 1 (finish kernel); the
     // re-queue chains 2, 3 and 4, 5
     FailBufs fl[6];
     DevBuf knn, ids1, cnt, wred, cull_scratch;
-    // states of resumable cells (two record buffers per chain, their
-    // counters) and, per stored id, the record slot and the last neighbour
-    DevBuf rs[4], rs_cnt, rslot, lastnb;
+    // states of resumable cells of the re-queue passes (two record buffers per
+    // chain) and, per stored id, the record slot and the last neighbour
+    DevBuf rs[4], rslot, lastnb;
     // record slots of pass 1's finish-kernel failures (laid out as their list)
     DevBuf fslot;
     bool solved = false;
@@ -508,7 +518,7 @@ __global__ __launch_bounds__(256) void ring_select_kernel(const int *__restrict_
     if (sel) ids[atomicAdd(count, 1)] = int(s);
 }
 
-// One wave per queued cell record (FP64 planes): the neighbours of the
+// One wave per cell record (FP64 planes; a negative id: none): the neighbours of the
 // planes of its vertices that carry no mark get d (CCUpdateUsedCell,
 // ConvexCell.cl:680-690).  Every writer of a ring writes the same d.
 __global__ __launch_bounds__(256) void mark_neighbours_kernel(const char *__restrict__ rec, int stride, int P,
@@ -517,6 +527,7 @@ __global__ __launch_bounds__(256) void mark_neighbours_kernel(const char *__rest
     const int lane = int(threadIdx.x & 63);
     if (q >= nq) return;
     const char *r = rec + size_t(q) * size_t(stride);
+    if (reinterpret_cast<const int *>(r)[0] < 0) return;  // no cell
     const int nvalid = reinterpret_cast<const int *>(r)[2];  // RecHeader{sid, nb_plane, nvalid, kused}
     const uint32_t *tri = reinterpret_cast<const uint32_t *>(r + 16 + size_t(P) * 32);
     const int *nid = reinterpret_cast<const int *>(tri + 64 * S);
@@ -977,17 +988,17 @@ static int solve_impl(rpd_ctx *c, rpd_domain *dom, const rpd_params *prm, rpd_st
         RPDCHK(c, l.eo.ensure(size_t(n) * 8), "alloc failure list");
         RPDCHK(c, l.sec.ensure(size_t(n) * 4), "alloc failure list");
     }
-    RPDCHK(c, c->rs_cnt.ensure(4 * sizeof(int)), "alloc resume counters");
     RPDCHK(c, c->rslot.ensure(size_t(n) * 4), "alloc resume slots");
     RPDCHK(c, c->lastnb.ensure(size_t(n) * 4), "alloc resume slots");
     RPDCHK(c, c->fslot.ensure(size_t(n) * 8), "alloc failure slots");
     RPDCHK(c, c->cnt.ensure(64), "alloc cnt");
-    for (auto &b : c->pb) RPDCHK(c, b.qcount.ensure(sizeof(int)), "alloc qcount");
+    for (auto &b : c->pb) RPDCHK(c, b.q.ensure(2 * sizeof(int)), "alloc queue counter");
+    RPDCHK(c, c->pb1.q.ensure(2 * sizeof(int)), "alloc queue counter");
     // The counters the solve starts from, cleared by one launch: the final
-    // status histogram's, every failure list's, the resume buffers' and the
-    // queue lengths.  A list, resume buffer or queue counter stays "fresh"
-    // (known zero) until a pass writes it; clearing a fresh one is skipped.
-    bool fresh_fl[6], fresh_rs[4], fresh_q[4];
+    // status histogram's, every failure list's and the queue counters.  A
+    // list stays "fresh" (known zero) until a pass writes it; clearing a fresh
+    // one is skipped.
+    bool fresh_fl[6];
     {
         ZeroSet z{};
         z.p[z.k] = c->cnt.as<int>();
@@ -997,12 +1008,9 @@ static int solve_impl(rpd_ctx *c, rpd_domain *dom, const rpd_params *prm, rpd_st
             z.n[z.k++] = kFailCounters;
             fresh_fl[i] = true;
         }
-        z.p[z.k] = c->rs_cnt.as<int>();
-        z.n[z.k++] = 4;
-        for (int i = 0; i < 4; ++i) {
-            z.p[z.k] = c->pb[i].qcount.as<int>();
-            z.n[z.k++] = 1;
-            fresh_rs[i] = fresh_q[i] = true;
+        for (PassBufs *b : {&c->pb1, &c->pb[0], &c->pb[1], &c->pb[2], &c->pb[3]}) {
+            z.p[z.k] = b->q.as<int>();
+            z.n[z.k++] = 2;
         }
         zero_words_kernel<<<1, 64, 0, c->stream>>>(z);
         HIPCHK(c, hipGetLastError());
@@ -1123,17 +1131,15 @@ static int solve_impl(rpd_ctx *c, rpd_domain *dom, const rpd_params *prm, rpd_st
     const KnnReq *kreqs = batch ? c->knn_req.as<KnnReq>() : nullptr;
     const uint16_t *req_of = batch ? c->req_of.as<uint16_t>() : nullptr;
 
-    // One pass = kNN + bisector kernel (which waits for the queue length)
-    // on a stream, then the finish kernel queued behind them.  Failed cells
-    // go to failure list fl_out; fl_cnt_host receives the list's counters
-    // as they stand once the bisector kernel is done.
+    // One pass = kNN + bisector kernel + finish kernel on a stream, then the
+    // lists of its failed cells (fl_out).
     struct Pass {
         int index = 0;  // pass number (0 the first), for the debug counters
         int slot = 0;  // stream, events and buffers
         int form = 0;
         int64_t n_ids = 0;
         int caps[4] = {0, 0, 0, 0};
-        int nq = 0;
+        int nq = 0;    // queued cells (pass 1)
         bool finish_only = false;  // a finish kernel over earlier records (events 1 and 3 only)
     };
     // resumable cells: records read (in, FP64 passes) and written (out)
@@ -1141,20 +1147,24 @@ static int solve_impl(rpd_ctx *c, rpd_domain *dom, const rpd_params *prm, rpd_st
         const char *in = nullptr;  // the cells of this pass resume from here
         int in_stride = 0, in_P = 0;
         int out = -1;              // rs buffer written, -1: none
-        int out_stride = 0, out_cap = 0;
+        int out_stride = 0, out_base = 0;
     };
     // device address of a pinned word (nullptr: no mapping)
     auto pin_d = [&](const int *host) -> int * { return c->pin_dev ? c->pin_dev + (host - c->pin) : nullptr; };
-    // kNN + bisector kernel, the queue length copied to the host (not waited for)
-    auto pass_front = [&](Pass &ps, const int *ids, int fl_out, int *fl_cnt_host, const Resume &rz,
-                          ClipLaunch &L) -> int {
+    // The FP64 passes of a mixed solve finish in the mixed form: over the
+    // same records (FP64 planes), its finish kernel decides in FP64, in
+    // place, the tests its filter leaves open and those of ill-conditioned
+    // vertices, so a cell gets the FP64 form's combinatorics for less work.
+    const int finish_form_fp64 = form0 == RPD_PREC_MIXED && !hess ? RPD_PREC_MIXED : RPD_PREC_FP64;
+    // A re-queue pass's kernels: kNN, bisector kernel and finish kernel (over
+    // every cell of the pass: those the bisector kernel did not queue are left
+    // out on the device, so nothing waits for a count).
+    auto pass_run = [&](Pass &ps, const int *ids, int fl_out, const Resume &rz, int beside, ClipLaunch &L) -> int {
         const int sl = ps.slot;
         hipStream_t s = c->streams[sl];
         PassBufs &b = c->pb[sl];
         const int K_ = ps.caps[0], P_ = ps.caps[1], V_ = ps.caps[2], T_ = ps.caps[3];
-        int r = b.knn.ensure(size_t(ps.n_ids) * K_ * 4);
-        if (r == RPD_OK) r = b.rec.ensure(size_t(ps.n_ids) * rpd_clip_record_bytes(ps.form, P_, V_));
-        if (r == RPD_OK) r = b.qcount.ensure(sizeof(int));
+        int r = b.ensure(ps.n_ids, K_, rpd_clip_record_bytes(ps.form, P_, V_));
         if (r != RPD_OK) return r;
         if (hipEventRecord(c->ev[sl][0], s) != hipSuccess) return RPD_E_DEVICE;
         // (re-queue passes run beside a finish kernel: one-wave workgroups)
@@ -1183,19 +1193,16 @@ static int solve_impl(rpd_ctx *c, rpd_domain *dom, const rpd_params *prm, rpd_st
         L.status = c->status.as<int>();
         L.kused = c->kused.as<int>();
         L.rec = b.rec.ptr;
-        L.qcount = b.qcount.as<int>();
+        L.code = b.code.as<uint8_t>();
         L.ev_mid = c->ev[sl][2];
         L.fl_cnt = c->fl[fl_out].cnt.as<int>();
         L.fl_eo = c->fl[fl_out].eo.as<int>() + n;
-        L.fl_sec = c->fl[fl_out].sec.as<int>();
-        L.fl_cnt_host = fl_cnt_host;
         L.rs_in = rz.in;
         L.rs_in_stride = rz.in_stride;
         L.rs_in_P = rz.in_P;
         L.rs_out = rz.out >= 0 ? static_cast<char *>(c->rs[rz.out].ptr) : nullptr;
         L.rs_out_stride = rz.out_stride;
-        L.rs_cap = rz.out_cap;
-        L.rs_count = c->rs_cnt.as<int>() + std::max(rz.out, 0);
+        L.rs_base = rz.out_base;
         L.rslot = c->rslot.as<int>();
         L.lastnb = c->lastnb.as<int>();
         if (hess) {
@@ -1207,25 +1214,28 @@ static int solve_impl(rpd_ctx *c, rpd_domain *dom, const rpd_params *prm, rpd_st
         L.dcnt = dcnt_of(ps.index);
         L.reqs = reqs;
         L.req_of = req_of;
-        L.qcount_zeroed = fresh_q[sl];
-        fresh_q[sl] = false;
-        L.nq_dev_out = pin_d(c->pin + sl);
-        L.fl_cnt_dev_out = fl_cnt_host ? pin_d(fl_cnt_host) : nullptr;
-        return rpd_launch_cells(s, ps.form, L, c->pin + sl, false);
-    };
-    // the finish kernel of a pass whose bisector kernel (and queue length) is done
-    // The FP64 passes of a mixed solve finish in the mixed form: over the
-    // same records (FP64 planes), its finish kernel decides in FP64, in
-    // place, the tests its filter leaves open and those of ill-conditioned
-    // vertices, so a cell gets the FP64 form's combinatorics for less work.
-    const int finish_form_fp64 = form0 == RPD_PREC_MIXED && !hess ? RPD_PREC_MIXED : RPD_PREC_FP64;
-    auto pass_back = [&](Pass &ps, const ClipLaunch &L, int beside) -> int {
-        hipStream_t s = c->streams[ps.slot];
-        ps.nq = c->pin[ps.slot];
-        const int r =
-            rpd_launch_finish(s, ps.form == RPD_PREC_FP64 ? finish_form_fp64 : ps.form, L, ps.nq, beside);
+        r = rpd_launch_cells(s, ps.form, L);
+        if (r == RPD_OK)
+            r = rpd_launch_finish(s, ps.form == RPD_PREC_FP64 ? finish_form_fp64 : ps.form, L, int(ps.n_ids), beside);
         if (r != RPD_OK) return r;
-        return hipEventRecord(c->ev[ps.slot][3], s) == hipSuccess ? RPD_OK : RPD_E_DEVICE;
+        return hipEventRecord(c->ev[sl][3], s) == hipSuccess ? RPD_OK : RPD_E_DEVICE;
+    };
+    // Failure list fl from the codes of a pass's bisector kernel, on its
+    // stream; with copy, its counters then go to their pinned words (cnt_pin
+    // below), with copy_q (pass 1) the number of queued cells too.
+    auto pass_lists = [&](const Pass &ps, const ClipLaunch &L, PassBufs &b, int fl, bool copy, int *q_pin) -> int {
+        hipStream_t s = c->streams[ps.slot];
+        int *cnt_p = c->pin + kPinCounters + kFailCounters * fl;
+        FailLists F{c->fl[fl].cnt.as<int>(), c->fl[fl].eo.as<int>() + n, c->fl[fl].sec.as<int>(), b.q.as<int>(),
+                    q_pin ? pin_d(q_pin) : nullptr, copy ? pin_d(cnt_p) : nullptr};
+        const int r = rpd_launch_lists(s, L, F);
+        if (r != RPD_OK || c->pin_dev || (!copy && !q_pin)) return r;
+        // no mapped pinned memory: the copy engine
+        if (q_pin && hipMemcpyAsync(q_pin, F.q, sizeof(int), hipMemcpyDeviceToHost, s) != hipSuccess)
+            return RPD_E_DEVICE;
+        if (copy && hipMemcpyAsync(cnt_p, F.cnt, kFailCounters * sizeof(int), hipMemcpyDeviceToHost, s) != hipSuccess)
+            return RPD_E_DEVICE;
+        return RPD_OK;
     };
     double ms_knn = 0, ms_fb_knn = 0, ms_fb = 0;
     auto account = [&](const Pass &ps, int index) {
@@ -1281,20 +1291,11 @@ static int solve_impl(rpd_ctx *c, rpd_domain *dom, const rpd_params *prm, rpd_st
         }
         return rpd_zero_ints(s, c->fl[fl].cnt.as<int>(), kFailCounters) == RPD_OK;
     };
-    // Record buffer `which` for cap records of stride bytes, counter cleared.
-    auto resume_buf = [&](int which, int64_t cap, int stride, hipStream_t s) -> int {
-        const int r = c->rs[which].ensure(size_t(std::max<int64_t>(cap, 1)) * size_t(stride));
-        if (r != RPD_OK) return r;
-        if (fresh_rs[which]) {
-            fresh_rs[which] = false;
-            return RPD_OK;
-        }
-        return rpd_zero_ints(s, c->rs_cnt.as<int>() + which, 1);
-    };
     // Where the previous pass of a chain left the states of its resumable
-    // cells (rs buffer, stride, plane room), or which = -1.
+    // cells (records, stride, plane room), or null.
     struct Left {
-        int which = -1, stride = 0, P = 0;
+        const char *rec = nullptr;
+        int stride = 0, P = 0;
     };
     // 1: done, 0: still running, -1: error
     auto done = [&](hipStream_t s) {
@@ -1316,13 +1317,13 @@ static int solve_impl(rpd_ctx *c, rpd_domain *dom, const rpd_params *prm, rpd_st
         Caps cap{0, 0, 0, 0}, nc{0, 0, 0, 0};
         Left left;
         int k = 0, nxt = 0;
-        int phase = 0;  // 0 idle, 1 bisector kernels queued, 2 finish kernels queued, 3 done, 4 waiting for pass 1
+        int phase = 0;  // 0 idle, 2 a pass queued, 3 done, 4 waiting for pass 1
+        hipStream_t end = nullptr;  // the stream on which the queued pass's counters come last
         int64_t n_res = 0, n_scr = 0;
         Pass pr, pz;
         ClipLaunch Lr, Lz;
         Resume rz;
         bool from_finish = false;  // the chain of pass 1's finish-kernel failures
-        bool back_r = false, back_z = false;  // phase 1: the finish kernel of pr / pz queued
     };
     ClipLaunch L1{};  // pass 1's launch; its finish kernel's records serve chain B's first pass
     auto cnt_pin = [&](int list) { return c->pin + kPinCounters + kFailCounters * list; };
@@ -1333,8 +1334,10 @@ static int solve_impl(rpd_ctx *c, rpd_domain *dom, const rpd_params *prm, rpd_st
         return hipMemcpyAsync(cnt_pin(list), c->fl[list].cnt.ptr, kFailCounters * sizeof(int), hipMemcpyDeviceToHost,
                               s) == hipSuccess;
     };
-    // plans the chain's next pass from the counters and queues its kNN and
-    // bisector kernels (phase 1), or ends the chain (phase 3)
+    Pass p1;                 // pass 1 (stream 0)
+    bool p1_running = true;  // its finish kernel is not known to be done
+    // plans the chain's next pass from the counters and queues it (phase 2),
+    // or ends the chain (phase 3)
     auto chain_front = [&](Chain &ch) -> int {
         if (ch.k >= prm->max_extra_steps) {
             ch.phase = 3;
@@ -1347,7 +1350,7 @@ static int solve_impl(rpd_ctx *c, rpd_domain *dom, const rpd_params *prm, rpd_st
         // exact-predicate failures (only listed from the FP32 forms) always
         // go to FP64; overflows only when a cap grew; kept states when K grew
         // (else they would run out again: they end as they are)
-        ch.n_res = n_sec > 0 && ch.left.which >= 0 && nc.K > ch.cap.K ? n_sec : 0;
+        ch.n_res = n_sec > 0 && ch.left.rec && nc.K > ch.cap.K ? n_sec : 0;
         ch.n_scr = n_exact + (caps_changed ? n_over : 0);
         if (ch.n_res + ch.n_scr == 0) {
             ch.phase = 3;
@@ -1392,8 +1395,6 @@ static int solve_impl(rpd_ctx *c, rpd_domain *dom, const rpd_params *prm, rpd_st
             L.fl_slot = nullptr;
             L.fl_cnt = c->fl[ch.nxt].cnt.as<int>();
             L.fl_eo = c->fl[ch.nxt].eo.as<int>() + n;
-            L.fl_sec = c->fl[ch.nxt].sec.as<int>();
-            L.fl_cnt_host = nullptr;
             L.rs_out = nullptr;
             L.rs_in = nullptr;
             L.ev_mid = nullptr;
@@ -1403,14 +1404,14 @@ static int solve_impl(rpd_ctx *c, rpd_domain *dom, const rpd_params *prm, rpd_st
             int r = rpd_launch_finish(s, RPD_PREC_FP64, L, int(ch.n_scr), 0);
             if (r != RPD_OK) return r;
             if (hipEventRecord(c->ev[ch.sl][3], s) != hipSuccess || !copy_counts(ch.nxt, s)) return RPD_E_DEVICE;
+            ch.end = s;
             ch.phase = 2;
             return RPD_OK;
         }
         ch.rz = Resume{};
         ch.rz.out = ch.rsb[ch.k & 1];
         ch.rz.out_stride = int(rpd_clip_record_bytes(RPD_PREC_FP64, nc.P, nc.V));
-        ch.rz.out_cap = int(ch.n_res + ch.n_scr);
-        int r = resume_buf(ch.rz.out, ch.rz.out_cap, ch.rz.out_stride, s);
+        int r = c->rs[ch.rz.out].ensure(size_t(ch.n_res + ch.n_scr) * size_t(ch.rz.out_stride));
         if (r != RPD_OK) return r;
         ch.pr = Pass{};
         ch.pz = Pass{};
@@ -1430,76 +1431,51 @@ static int solve_impl(rpd_ctx *c, rpd_domain *dom, const rpd_params *prm, rpd_st
         ch.pr.caps[1] = ch.pz.caps[1] = nc.P;
         ch.pr.caps[2] = ch.pz.caps[2] = nc.V;
         ch.pr.caps[3] = ch.pz.caps[3] = nc.T;
-        // the recomputed cells start once the list and the record counter are cleared
+        // pass 1's finish kernel may still run beside this pass
+        const int beside = p1_running ? p1.nq : 0;
+        // the recomputed cells start once the list is cleared
         if (ch.n_scr > 0 && (hipEventRecord(c->dep[ch.dep], s) != hipSuccess ||
                              hipStreamWaitEvent(s2, c->dep[ch.dep], 0) != hipSuccess))
             return RPD_E_DEVICE;
         if (ch.n_res > 0) {
             Resume rr = ch.rz;
-            rr.in = static_cast<const char *>(c->rs[ch.left.which].ptr);
+            rr.in = ch.left.rec;
             rr.in_stride = ch.left.stride;
             rr.in_P = ch.left.P;
-            r = pass_front(ch.pr, c->fl[ch.cur].sec.as<int>(), ch.nxt, nullptr, rr, ch.Lr);
+            r = pass_run(ch.pr, c->fl[ch.cur].sec.as<int>(), ch.nxt, rr, beside, ch.Lr);
             if (r != RPD_OK) return r;
         }
         if (ch.n_scr > 0) {
+            Resume rr = ch.rz;
+            rr.out_base = int(ch.n_res);
             // exact entries and (when recomputed) the overflows are one range
-            r = pass_front(ch.pz, c->fl[ch.cur].eo.as<int>() + n - n_exact, ch.nxt, nullptr, ch.rz, ch.Lz);
+            r = pass_run(ch.pz, c->fl[ch.cur].eo.as<int>() + n - n_exact, ch.nxt, rr, beside, ch.Lz);
+            if (r == RPD_OK) r = pass_lists(ch.pz, ch.Lz, c->pb[ch.sl2], ch.nxt, ch.n_res == 0, nullptr);
             if (r != RPD_OK) return r;
+            ch.end = s2;
         }
-        ch.back_r = ch.n_res == 0;
-        ch.back_z = ch.n_scr == 0;
-        ch.phase = 1;
-        return RPD_OK;
-    };
-    Pass p1;                 // pass 1 (stream 0)
-    bool p1_running = true;  // its finish kernel is not known to be done
-    // advances the chain as far as its streams allow, without waiting
-    auto chain_poll = [&](Chain &ch, bool &progress) -> int {
-        hipStream_t s = c->streams[ch.sl], s2 = c->streams[ch.sl2];
-        if (ch.phase == 1) {
-            // each finish kernel as soon as its own bisector kernel is done;
-            // pass 1's finish kernel may still run beside them
-            const int beside = p1_running ? p1.nq : 0;
-            bool s_done = false;  // s found idle by this poll, before any launch on it
-            if (!ch.back_r) {
-                const int d = done(s);
-                if (d < 0) return RPD_E_DEVICE;
-                if (d) {
-                    s_done = true;
-                    if (pass_back(ch.pr, ch.Lr, beside) != RPD_OK) return RPD_E_DEVICE;
-                    ch.back_r = true;
-                    progress = true;
-                }
-            }
-            if (!ch.back_z) {
-                // one stream for both (two-stream contexts): pz's bisector
-                // kernel was queued after pr's, so s idle covers it
-                const int d = s2 == s && s_done ? 1 : done(s2);
-                if (d < 0) return RPD_E_DEVICE;
-                if (d) {
-                    if (pass_back(ch.pz, ch.Lz, beside) != RPD_OK) return RPD_E_DEVICE;
-                    ch.back_z = true;
-                    progress = true;
-                }
-            }
-            if (!ch.back_r || !ch.back_z) return RPD_OK;
-            // the counters of the pass, once both finish kernels are done
+        if (ch.n_res > 0) {
+            // its lists, and the counters of both halves, come last
             if (ch.n_scr > 0 && (hipEventRecord(c->dep[ch.dep], s2) != hipSuccess ||
                                  hipStreamWaitEvent(s, c->dep[ch.dep], 0) != hipSuccess))
                 return RPD_E_DEVICE;
-            if (!copy_counts(ch.nxt, s)) return RPD_E_DEVICE;
-            ch.phase = 2;
-            progress = true;
+            r = pass_lists(ch.pr, ch.Lr, c->pb[ch.sl], ch.nxt, true, nullptr);
+            if (r != RPD_OK) return r;
+            ch.end = s;
         }
+        ch.phase = 2;
+        return RPD_OK;
+    };
+    // advances the chain as far as its streams allow, without waiting
+    auto chain_poll = [&](Chain &ch, bool &progress) -> int {
         if (ch.phase == 2) {
-            const int d = done(s);
+            const int d = done(ch.end);
             if (d < 0) return RPD_E_DEVICE;
             if (!d) return RPD_OK;
             if (ch.n_res > 0) account(ch.pr, 1 + ch.k);
             if (ch.n_scr > 0) account(ch.pz, 1 + ch.k);
             ch.cap = ch.nc;
-            ch.left.which = ch.rz.out;
+            ch.left.rec = ch.rz.out >= 0 ? static_cast<const char *>(c->rs[ch.rz.out].ptr) : nullptr;
             ch.left.stride = ch.rz.out_stride;
             ch.left.P = ch.nc.P;
             ch.cur = ch.nxt;
@@ -1524,7 +1500,7 @@ static int solve_impl(rpd_ctx *c, rpd_domain *dom, const rpd_params *prm, rpd_st
     Left left1;
     {
         hipStream_t s = c->streams[0];
-        PassBufs &b = c->pb[0];
+        PassBufs &b = c->pb1;
         // pass 1's kNN: over the kept cells, their count read on the device
         // while the host does not know it yet.  The launch covers the last
         // solve's count over as many seeds, with a margin (n rows at most, or
@@ -1573,18 +1549,16 @@ static int solve_impl(rpd_ctx *c, rpd_domain *dom, const rpd_params *prm, rpd_st
         p1.caps[1] = P;
         p1.caps[2] = V;
         p1.caps[3] = T;
+        const size_t rec_bytes = rpd_clip_record_bytes(form0, P, V);
+        RPDCHK(c, b.ensure(n1, K, rec_bytes), "alloc records");
         // states of pass 1's cells whose K neighbours do not reach their
-        // security radius are kept (FP64 planes: FP64 and mixed forms), for
-        // up to 40% of the cells; the others are recomputed from scratch
-        const int64_t cap_rs1 = std::min<int64_t>(n1, n1 * 2 / 5 + 1024);
+        // security radius are kept (FP64 planes: FP64 and mixed forms), in
+        // the records the finish kernel leaves out
         if (form0 != RPD_PREC_FP32 && prm->max_extra_steps > 0 && n1 > 0) {
-            left1.which = 0;
-            left1.stride = int(rpd_clip_record_bytes(form0, P, V));
+            left1.rec = static_cast<const char *>(b.rec.ptr);
+            left1.stride = int(rec_bytes);
             left1.P = P;
-            RPDCHK(c, resume_buf(0, cap_rs1, left1.stride, c->streams[0]), "alloc resume records");
         }
-        RPDCHK(c, b.rec.ensure(size_t(std::max<int64_t>(n1, 1)) * rpd_clip_record_bytes(form0, P, V)), "alloc records");
-        RPDCHK(c, b.qcount.ensure(sizeof(int)), "alloc qcount");
         ClipLaunch &L = L1;
         L.seeds = c->stored64.as<double4>();
         L.perm = c->perm.as<int>();
@@ -1606,57 +1580,42 @@ static int solve_impl(rpd_ctx *c, rpd_domain *dom, const rpd_params *prm, rpd_st
         L.status = c->status.as<int>();
         L.kused = c->kused.as<int>();
         L.rec = b.rec.ptr;
-        L.qcount = b.qcount.as<int>();
+        L.code = b.code.as<uint8_t>();
         L.ev_mid = c->ev[0][2];
-        L.fl_cnt = c->fl[0].cnt.as<int>();
-        L.fl_eo = c->fl[0].eo.as<int>() + n;
-        L.fl_sec = c->fl[0].sec.as<int>();
-        L.fl_cnt_host = cnt_pin(0);
         if (hess) {
             L.hess = c->hess.as<double>();
             L.hids = c->hids.as<int>();
             L.H = prm->H;
             L.hc = prm->HC;
         }
-        if (left1.which == 0) {
-            L.rs_out = static_cast<char *>(c->rs[0].ptr);
+        if (left1.rec) {
+            L.rs_out = static_cast<char *>(b.rec.ptr);
             L.rs_out_stride = left1.stride;
-            L.rs_cap = int(cap_rs1);
-            L.rs_count = c->rs_cnt.as<int>();
             L.rslot = c->rslot.as<int>();
             L.lastnb = c->lastnb.as<int>();
         }
         L.dcnt = dcnt_of(0);
         L.reqs = reqs;
         L.req_of = req_of;
-        L.qcount_zeroed = fresh_q[0];
-        fresh_q[0] = false;
-        L.nq_dev_out = pin_d(c->pin + 0);
-        L.fl_cnt_dev_out = pin_d(cnt_pin(0));
-        RPDCHK(c, rpd_launch_cells(s, form0, L, c->pin + 0, false), "pass 1 cells");
-        L.nq_dev_out = L.fl_cnt_dev_out = nullptr;
-        L.qcount_zeroed = false;
+        RPDCHK(c, rpd_launch_cells(s, form0, L), "pass 1 cells");
+        RPDCHK(c, pass_lists(p1, L, b, 0, true, c->pin + 0), "pass 1 lists");
         HIPCHK(c, hipEventRecord(c->dep[2], s));  // queue length and failure counters copied
         L.fl_cnt = c->fl[1].cnt.as<int>();
         L.fl_eo = c->fl[1].eo.as<int>() + n;
-        L.fl_sec = c->fl[1].sec.as<int>();
-        L.fl_cnt_host = nullptr;
         L.fl_slot = c->fslot.as<int>() + n;  // the finish kernel's failures keep their record slots
-        // The finish kernel is queued at once, over the n1 cells the queue
-        // can hold at most, reading its length on the device: no host round
-        // trip between the two kernels.  Chain A's first pass follows once
-        // the host has the bisector kernel's failure counters; its kNN uses
-        // one-wave workgroups, which fit beside the finish kernel's.
-        L.nq_dev = L.qcount;
+        // The finish kernel is queued at once, over the n1 cells' records: no
+        // host round trip between the two kernels.  Chain A's first pass
+        // follows once the host has the bisector kernel's failure counters;
+        // its kNN uses one-wave workgroups, which fit beside the finish
+        // kernel's.
         RPDCHK(c, rpd_launch_finish(s, form0, L, int(n1), 0), "pass 1 finish");
         HIPCHK(c, hipEventRecord(c->ev[0][3], s));
         if (!copy_counts(1, s)) return set_err(c, RPD_E_DEVICE, "pass 1 counters");
         HIPCHK(c, hipEventSynchronize(c->dep[2]));
-        p1.nq = c->pin[0];
+        p1.nq = n1 > 0 ? c->pin[0] : 0;
         // no cell to clip (every one skipped): the bisector kernel did not
         // run and copied no failure counters
         if (n1 <= 0) std::fill(cnt_pin(0), cnt_pin(0) + kFailCounters, 0);
-        L.nq_dev = nullptr;
     }
     const Caps caps1{K, P, V, T};
     Chain ca, cb;
@@ -1720,7 +1679,7 @@ static int solve_impl(rpd_ctx *c, rpd_domain *dom, const rpd_params *prm, rpd_st
         RPDCHK(c, chain_poll(cb, progress), "re-queue chain (finish failures)");
         const Chain *last = ca.phase == 3 && cb.phase == 2 ? &cb : (cb.phase == 3 && ca.phase == 2 ? &ca : nullptr);
         if (last && !(hist_for == last && hist_k == last->k)) {
-            RPDCHK(c, queue_hist(c->streams[last->sl]), "status histogram");
+            RPDCHK(c, queue_hist(last->end), "status histogram");
             hist_for = last;
             hist_k = last->k;
         }
@@ -1736,7 +1695,7 @@ static int solve_impl(rpd_ctx *c, rpd_domain *dom, const rpd_params *prm, rpd_st
     // final status histogram, unless the one queued early covers every pass
     hipStream_t hist_s = c->stream;
     if (hist_for && hist_for->k == hist_k + 1)
-        hist_s = c->streams[hist_for->sl];
+        hist_s = hist_for->end;
     else
         RPDCHK(c, queue_hist(c->stream), "status histogram");
     HIPCHK(c, hipStreamSynchronize(hist_s));
@@ -2006,9 +1965,7 @@ int compact_device(rpd_ctx *c, double keep_volume, int32_t keep_distance) {
         for (int step = 0; cnt > 0 && step <= std::max(c->last_steps, 0); ++step) {
             PassBufs &b = c->pb[0];
             const size_t stride = rpd_clip_record_bytes(RPD_PREC_FP64, P, V);
-            RPDCHK(c, b.knn.ensure(size_t(cnt) * K * 4), "alloc knn");
-            RPDCHK(c, b.rec.ensure(size_t(cnt) * stride), "alloc records");
-            RPDCHK(c, b.qcount.ensure(sizeof(int)), "alloc qcount");
+            RPDCHK(c, b.ensure(cnt, K, stride), "alloc records");
             HIPCHK(c, hipMemsetAsync(c->fl[0].cnt.ptr, 0, kFailCounters * sizeof(int), s));
             RPDCHK(c,
                    rpd_launch_knn(s, c->bin_prec, c->stored.ptr, c->perm.as<int>(), c->counters.as<int>(), c->dim,
@@ -2033,17 +1990,18 @@ int compact_device(rpd_ctx *c, double keep_volume, int32_t keep_distance) {
             L.out = c->bout.as<double4>();
             L.status = c->bstatus.as<int>();
             L.rec = b.rec.ptr;
-            L.qcount = b.qcount.as<int>();
-            L.fl_cnt = c->fl[0].cnt.as<int>();
-            L.fl_eo = c->fl[0].eo.as<int>() + n;
-            L.fl_sec = c->fl[0].sec.as<int>();
-            L.fl_cnt_host = c->pin + kPinCounters;
-            RPDCHK(c, rpd_launch_cells(s, RPD_PREC_FP64, L, c->pin + 0, true), "bordering cells");
-            const int nq = c->pin[0];
+            L.code = b.code.as<uint8_t>();
+            RPDCHK(c, rpd_launch_cells(s, RPD_PREC_FP64, L), "bordering cells");
+            RPDCHK(c,
+                   rpd_launch_lists(s, L, FailLists{c->fl[0].cnt.as<int>(), c->fl[0].eo.as<int>() + n,
+                                                    c->fl[0].sec.as<int>(), b.q.as<int>(), nullptr, nullptr}),
+                   "bordering cells");
+            HIPCHK(c, hipMemcpyAsync(c->pin + kPinCounters, c->fl[0].cnt.ptr, kFailCounters * sizeof(int),
+                                     hipMemcpyDeviceToHost, s));
             const int S = V <= 64 ? 1 : (V <= 128 ? 2 : 4);
-            if (nq > 0)
-                mark_neighbours_kernel<<<unsigned((nq + 3) / 4), 256, 0, s>>>(
-                    static_cast<const char *>(b.rec.ptr), int(stride), P, S, nq, c->used.as<int>(), k + 1);
+            mark_neighbours_kernel<<<unsigned((cnt + 3) / 4), 256, 0, s>>>(
+                static_cast<const char *>(b.rec.ptr), int(stride), P, S, cnt, c->used.as<int>(), k + 1);
+            HIPCHK(c, hipStreamSynchronize(s));
             // cells that overflowed or ran out of neighbours: again with grown caps
             const int *h = c->pin + kPinCounters + 2;
             const int n_over = c->pin[kPinCounters + 1];

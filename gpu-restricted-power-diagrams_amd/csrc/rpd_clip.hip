@@ -90,30 +90,35 @@ struct ClipArgs {
     int security_mode;    // 0 exact power stop, 1 reference stop
     double wmin;          // minimum weight over non-border seeds
     const uint8_t *dist;  // Chebyshev voxel distance to the nearest domain voxel (nullable)
-    char *rec;            // queue of finished cells (records of rec_stride bytes)
+    // Records of the cells (rec_stride bytes, item t's at slot t); one whose
+    // header holds no cell (sid -1) is not for the finish kernel.  code[t] is
+    // how item t left the bisector kernel (kCode*), from which
+    // list_failures_kernel makes the lists: with one wave per cell, counters
+    // that every cell adds to cost 9 ns a cell (atomics of one address), more
+    // than the cell itself where most cells fail.
+    char *rec;
     int rec_stride;
-    int *qcount;          // number of queued records
-    // failed cells for the next pass (nullable): fl_cnt[0] exact-predicate
-    // entries, stored at fl_eo[-1], fl_eo[-2], ..., [1] overflow entries at
-    // fl_eo[0], fl_eo[1], ... (so that both kinds together are one range),
-    // [2 + s] cells that ended with status s, [13] the largest triangle union
-    // of a cell that overflowed T
+    uint8_t *code;
+    // finish kernel: failed cells for the next pass (nullable): fl_cnt[0]
+    // exact-predicate entries, stored at fl_eo[-1], fl_eo[-2], ..., [1]
+    // overflow entries at fl_eo[0], fl_eo[1], ... (so that both kinds together
+    // are one range), [2 + s] cells that ended with status s, [13] the largest
+    // triangle union of a cell that overflowed T
     int *fl_cnt, *fl_eo;
     int exact_final;      // FP64 form: exact-predicate failures are final
     // A cell whose list runs out before its security radius is reached can be
-    // resumed: its state goes to rs_out (records of rs_out_stride bytes, slot
-    // from *rs_count below rs_cap, kept in rslot[sid]), the stored id of its
-    // last neighbour to lastnb[sid], the cell to fl_sec (counter fl_cnt[14]).
-    // rs_out null, or the buffer full: a plain overflow.  With rs_in set
-    // (FP64 form), every cell resumes from record rs_in[rslot[sid]] (written
-    // with rs_in_P planes) and its list holds only the neighbours after the
-    // ones it has used.
+    // resumed: its state goes to slot rs_base + t of rs_out (records of
+    // rs_out_stride bytes; the slot is kept in rslot[sid]), the stored id of
+    // its last neighbour to lastnb[sid].  rs_out may be rec itself (rs_base
+    // 0): an item has one record, for the finish kernel or to resume from.
+    // rs_out null: a plain overflow.  With rs_in set (FP64 form), every cell
+    // resumes from record rs_in[rslot[sid]] (written with rs_in_P planes) and
+    // its list holds only the neighbours after the ones it has used.
     char *rs_out;
-    int rs_out_stride, rs_cap;
-    int *rs_count;
+    int rs_out_stride, rs_base;
     const char *rs_in;
     int rs_in_stride, rs_in_P;
-    int *rslot, *lastnb, *fl_sec;
+    int *rslot, *lastnb;
     // Hessian (finish kernel, H > 0): per original seed up to H entries of
     // hc values in hess and the neighbours' original indices in hids
     double *hess;
@@ -134,9 +139,6 @@ struct ClipArgs {
     // slots they were written with (the finish kernel's own P and S may be
     // larger)
     int rec_P, rec_S;
-    // finish kernel (nullable): the queue length in device memory, read when
-    // the launch covers an upper bound of it
-    const int *nq_dev;
 };
 
 // The cell of stored id sid reads its request's seed count, weight minimum
@@ -163,21 +165,31 @@ __device__ __forceinline__ void bind_request(ClipArgs &a, int sid) {
     a.dist = d.dist;
 }
 
-// Appends a failed cell (stored id sid) to the failure list: overflows
-// (vertex, plane, K, triangle) always; needs_exact_predicates,
+// How an item leaves the bisector kernel: done (no list), queued for the
+// finish kernel, or failed with status code - kCodeFailed (code -
+// kCodeResume: its state kept, to be resumed).
+constexpr uint32_t kCodeDone = 0, kCodeQueued = 1, kCodeFailed = 16, kCodeResume = 32;
+
+__device__ __forceinline__ bool exact_failure(int st) {
+    return st == RPD_NEEDS_EXACT_PREDICATES || st == RPD_INCONSISTENT_BOUNDARY ||
+           st == RPD_FIND_ANOTHER_BEGINNING_VERTEX;
+}
+
+// Whether a cell that ended with status st goes to the failure list:
+// overflows (vertex, plane, K, triangle) always; needs_exact_predicates,
 // inconsistent_boundary and find_another_beginning_vertex when the form was
-// not FP64 (in FP64 a recomputation would fail the same way).  One lane.
-__device__ __forceinline__ void note_failure(const ClipArgs &a, int sid, int st, bool resumable = false,
-                                             int rslot = -1) {
-    if (!a.fl_cnt || st == RPD_SUCCESS || st == RPD_EMPTY_CELL || st == RPD_HESSIAN_OVERFLOW) return;
-    const bool exact = st == RPD_NEEDS_EXACT_PREDICATES || st == RPD_INCONSISTENT_BOUNDARY ||
-                       st == RPD_FIND_ANOTHER_BEGINNING_VERTEX;
-    if (exact && a.exact_final) return;
+// not FP64 (in FP64 a recomputation would fail the same way).
+__device__ __forceinline__ bool listed_failure(const ClipArgs &a, int st) {
+    if (st == RPD_SUCCESS || st == RPD_EMPTY_CELL || st == RPD_HESSIAN_OVERFLOW) return false;
+    return !(exact_failure(st) && a.exact_final);
+}
+
+// Finish kernel: appends a failed cell (stored id sid, record slot rslot) to
+// the failure list.  One lane.  (Few cells fail here.)
+__device__ __forceinline__ void note_failure(const ClipArgs &a, int sid, int st, int rslot) {
+    if (!a.fl_cnt || !listed_failure(a, st)) return;
+    const bool exact = exact_failure(st);
     atomicAdd(a.fl_cnt + 2 + st, 1);
-    if (resumable) {
-        a.fl_sec[atomicAdd(a.fl_cnt + 14, 1)] = sid;
-        return;
-    }
     const int k = atomicAdd(a.fl_cnt + (exact ? 0 : 1), 1);
     a.fl_eo[exact ? -1 - k : k] = sid;
     if (a.fl_slot) a.fl_slot[exact ? -1 - k : k] = rslot;
@@ -698,7 +710,9 @@ void clip_cells_kernel(ClipArgs a) {
             a.out[orig] = make_double4(m0, m1, m2, m3);
             a.status[orig] = st;
             if (a.kused) a.kused[orig] = kbase + ku;
-            note_failure(a, sid, st, resumable);
+            reinterpret_cast<RecHeader *>(a.rec + size_t(t) * size_t(a.rec_stride))->sid = -1;
+            a.code[t] = uint8_t(!listed_failure(a, st) ? kCodeDone
+                                                       : uint32_t(st) + (resumable ? kCodeResume : kCodeFailed));
         }
     };
     auto fail = [&](int st, int ku) { finish(st, 0.0, 0.0, 0.0, 0.0, ku); };
@@ -944,17 +958,8 @@ void clip_cells_kernel(ClipArgs a) {
     // list ran out keeps its state when there is room, so that the next pass
     // goes on from here with the neighbours after the last one used.
     const bool ran_out = !reached && !complete;
-    int slot = -1;
-    if (lane == 0) {
-        if (!ran_out) {
-            slot = atomicAdd(a.qcount, 1);
-        } else if (a.rs_out) {
-            slot = atomicAdd(a.rs_count, 1);
-            if (slot >= a.rs_cap) slot = -1;
-        }
-    }
-    slot = rlane(slot, 0);
-    if (slot >= 0) {
+    if (!ran_out || a.rs_out) {
+        const int64_t slot = ran_out ? a.rs_base + t : t;
         // the cell's state as a record: header, planes in the geometry
         // precision (rebuilt from their sources when the test precision is
         // lower), vertex triples; P planes' room.  (Written in line: as a
@@ -971,7 +976,15 @@ void clip_cells_kernel(ClipArgs a) {
 #pragma unroll
         for (int s = 0; s < S; ++s) nv += __popcll(c.valid[s]);
         if (ran_out) nv = 64 * S;
-        if (lane == 0) *reinterpret_cast<RecHeader *>(rec) = RecHeader{sid, c.nb_plane, nv, kbase + kused};
+        if (lane == 0) {
+            *reinterpret_cast<RecHeader *>(rec) = RecHeader{sid, c.nb_plane, nv, kbase + kused};
+            if (ran_out) {
+                a.rslot[sid] = int(slot);
+                a.lastnb[sid] = nrow[K - 1];
+            } else {
+                a.code[t] = kCodeQueued;
+            }
+        }
         wsync();
         for (int p = lane; p < c.nb_plane; p += 64) {
             if (sizeof(R) == sizeof(RP)) {
@@ -994,13 +1007,105 @@ void clip_cells_kernel(ClipArgs a) {
             carry += __popcll(c.valid[s]);
         }
     }
-    if (ran_out) {
-        if (slot >= 0 && lane == 0) {
-            a.rslot[sid] = slot;
-            a.lastnb[sid] = nrow[K - 1];
-        }
-        finish(RPD_SECURITY_RADIUS_NOT_REACHED, 0.0, 0.0, 0.0, 0.0, kused, slot >= 0);
+    if (ran_out) finish(RPD_SECURITY_RADIUS_NOT_REACHED, 0.0, 0.0, 0.0, 0.0, kused, a.rs_out != nullptr);
+}
+
+// The failure lists of a bisector kernel's items, from their codes: one
+// atomic per list and workgroup of 4096 items, entries in item order within a
+// workgroup.  Counters as in ClipArgs (cnt[14]: cells to resume, listed in
+// sec); *q counts the queued items.  The last workgroup to end copies *q and
+// the counters to mapped pinned host memory (nullable) and clears *q, which is
+// otherwise left to the caller; q[1], its ticket, it leaves cleared.
+struct ListArgs {
+    const uint8_t *code;  // room for whole 16-byte groups
+    const int *ids;       // nullable: item t is stored id t
+    int64_t n;
+    int *cnt, *eo, *sec, *q;
+    int *q_host, *cnt_host;
+};
+constexpr int kListPer = 16;    // items of a thread
+constexpr int kListBlock = 256;
+__global__ __launch_bounds__(kListBlock) void list_failures_kernel(ListArgs a) {
+    __shared__ int tot[4][kListBlock / 64], base[3], hist[16], last;
+    const int tid = int(threadIdx.x), lane = lane_id(), wv = tid >> 6;
+    if (tid < 16) hist[tid] = 0;
+    __syncthreads();
+    const int64_t i0 = (int64_t(blockIdx.x) * kListBlock + tid) * kListPer;
+    uint32_t w[4] = {0, 0, 0, 0};
+    if (i0 < a.n) {
+        const uint4 v = *reinterpret_cast<const uint4 *>(a.code + i0);
+        w[0] = v.x, w[1] = v.y, w[2] = v.z, w[3] = v.w;
     }
+    auto code = [&](int j) -> uint32_t { return i0 + j < a.n ? (w[j >> 2] >> (8 * (j & 3))) & 255u : 0u; };
+    // exact, overflow, resume, queued
+    int num[4] = {0, 0, 0, 0};
+#pragma unroll
+    for (int j = 0; j < kListPer; ++j) {
+        const uint32_t cd = code(j);
+        const bool failed = cd >= kCodeFailed, resume = cd >= kCodeResume, exact = exact_failure(int(cd & 15u));
+        num[0] += failed && !resume && exact;
+        num[1] += failed && !resume && !exact;
+        num[2] += resume;
+        num[3] += cd == kCodeQueued;
+        if (failed) atomicAdd(&hist[cd & 15u], 1);
+    }
+    int at[3];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const int incl = wave_incl_scan_op(num[k], 0, [](int x, int y) { return x + y; });
+        if (k < 3) at[k] = incl - num[k];
+        if (lane == 63) tot[k][wv] = incl;
+    }
+    __syncthreads();
+    if (tid < 4) {
+        int n = 0;
+        for (int v = 0; v < kListBlock / 64; ++v) {
+            const int m = tot[tid][v];
+            tot[tid][v] = n;
+            n += m;
+        }
+        if (tid == 3) {
+            if (n) atomicAdd(a.q, n);
+        } else {
+            base[tid] = n ? atomicAdd(a.cnt + (tid == 2 ? 14 : tid), n) : 0;
+        }
+    } else if (tid >= 64 && tid < 64 + RPD_STATUS_NUM) {
+        const int st = tid - 64;
+        if (hist[st]) atomicAdd(a.cnt + 2 + st, hist[st]);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 3; ++k) at[k] += base[k] + tot[k][wv];
+#pragma unroll
+    for (int j = 0; j < kListPer; ++j) {
+        const uint32_t cd = code(j);
+        if (cd < kCodeFailed) continue;
+        const int sid = a.ids ? a.ids[i0 + j] : int(i0 + j);
+        if (cd >= kCodeResume)
+            a.sec[at[2]++] = sid;
+        else if (exact_failure(int(cd & 15u)))
+            a.eo[-1 - at[0]++] = sid;
+        else
+            a.eo[at[1]++] = sid;
+    }
+    if (!a.q_host && !a.cnt_host) return;
+    // the last workgroup's copy to the host
+    __threadfence();
+    __syncthreads();
+    if (tid == 0) last = atomicAdd(a.q + 1, 1) == int(gridDim.x) - 1;
+    __syncthreads();
+    if (!last) return;
+    __threadfence();
+    if (a.cnt_host && tid < kFailCounters)
+        a.cnt_host[tid] = __hip_atomic_load(a.cnt + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (tid == 0) {
+        if (a.q_host) {
+            *a.q_host = __hip_atomic_load(a.q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            a.q[0] = 0;
+        }
+        a.q[1] = 0;
+    }
+    __threadfence_system();
 }
 
 // vface[q] of a voxel domain's face: x, y, z (10 bits each) of its lowest
@@ -1087,8 +1192,10 @@ void finish_cells_kernel(ClipArgs a, int nq, int W) {
     const int cpb = wpb / W;  // cells per block; W > 1 implies cpb == 1
     const int ci = wv / W, sub = wv - ci * W;
     const int item = int(blockIdx.x) * cpb + ci;
-    if (item >= nq || (a.nq_dev && item >= uni(*a.nq_dev))) return;  // uniform over the waves of a cell
+    if (item >= nq) return;  // uniform over the waves of a cell
     const int slot = a.slots ? uni(a.slots[item]) : item;
+    if (reinterpret_cast<const RecHeader *>(a.rec + size_t(slot) * size_t(a.rec_stride))->sid < 0)
+        return;  // not queued
 
     char *cell_l = lds_raw + size_t(ci) * a.cell_stride;
     int *fails = reinterpret_cast<int *>(cell_l);                  // [W][2]
@@ -1142,7 +1249,7 @@ void finish_cells_kernel(ClipArgs a, int nq, int W) {
             a.out[orig] = make_double4(m0, m1, m2, m3);
             a.status[orig] = st;
             if (a.kused) a.kused[orig] = kused;
-            note_failure(a, sid, st, false, slot);
+            note_failure(a, sid, st, slot);
         }
     };
     auto fail = [&](int st) { finish(st, 0.0, 0.0, 0.0, 0.0); };
@@ -2112,7 +2219,7 @@ size_t rpd_clip_record_bytes(int form, int P, int V) {
 static int make_args(int form, const ClipLaunch &L, ClipArgs &a) {
     if (L.P < 7 || L.P > 255 || L.V < 8 || L.K < 1) return RPD_E_ARG;
     if (L.V > 256) return RPD_E_LIMIT;
-    if (!L.rec || !L.qcount) return RPD_E_ARG;
+    if (!L.rec) return RPD_E_ARG;
     if (L.reqs && (!L.req_of || (L.hess && L.H > 0))) return RPD_E_ARG;
     a = ClipArgs{};
     a.seeds = L.seeds;
@@ -2153,14 +2260,12 @@ static int make_args(int form, const ClipLaunch &L, ClipArgs &a) {
     a.rec_stride = int(rpd_clip_record_bytes(form, rec_P, rec_V));
     a.rec_P = rec_P;
     a.rec_S = rec_V <= 64 ? 1 : (rec_V <= 128 ? 2 : 4);
-    a.qcount = L.qcount;
+    a.code = L.code;
     a.fl_cnt = L.fl_cnt;
     a.fl_eo = L.fl_eo;
-    a.fl_sec = L.fl_sec;
-    a.rs_out = L.fl_sec ? L.rs_out : nullptr;
+    a.rs_out = L.rs_out;
     a.rs_out_stride = L.rs_out_stride;
-    a.rs_cap = L.rs_cap;
-    a.rs_count = L.rs_count;
+    a.rs_base = L.rs_base;
     a.rs_in = form == RPD_PREC_FP64 ? L.rs_in : nullptr;
     a.rs_in_stride = L.rs_in_stride;
     a.rs_in_P = L.rs_in_P;
@@ -2175,20 +2280,17 @@ static int make_args(int form, const ClipLaunch &L, ClipArgs &a) {
     a.reqs = L.reqs;
     a.req_of = L.req_of;
     a.slots = L.slots;
-    a.nq_dev = L.nq_dev;
     a.fl_slot = L.fl_slot;
     return RPD_OK;
 }
 
-int rpd_launch_cells(hipStream_t st, int form, const ClipLaunch &L, int *nq_out, bool wait) {
-    *nq_out = 0;
+int rpd_launch_cells(hipStream_t st, int form, const ClipLaunch &L) {
     if (L.n_ids <= 0) return RPD_OK;
+    if (!L.code) return RPD_E_ARG;
     ClipArgs a;
     const int r = make_args(form, L, a);
     if (r != RPD_OK) return r;
     const int S = L.V <= 64 ? 1 : (L.V <= 128 ? 2 : 4);
-    if (!L.qcount_zeroed && rpd_zero_ints(st, L.qcount, 1) != RPD_OK) return RPD_E_DEVICE;
-
     // kernel A: the bisector loop of every cell
     {
         const size_t stride = finish_wave_lds(L.P, S, 0, form == RPD_PREC_FP64 ? 32 : 16);  // planes in R
@@ -2224,21 +2326,24 @@ int rpd_launch_cells(hipStream_t st, int form, const ClipLaunch &L, int *nq_out,
         if (hipGetLastError() != hipSuccess) return RPD_E_DEVICE;
     }
     if (L.ev_mid && hipEventRecord(L.ev_mid, st) != hipSuccess) return RPD_E_DEVICE;
-    if (L.nq_dev_out) {
-        const bool fl = L.fl_cnt && L.fl_cnt_host && L.fl_cnt_dev_out;
-        if (rpd_pin_copy(st, L.qcount, L.nq_dev_out, 1, fl ? L.fl_cnt : nullptr, fl ? L.fl_cnt_dev_out : nullptr,
-                         fl ? kFailCounters : 0) != RPD_OK)
-            return RPD_E_DEVICE;
-    } else {
-        if (hipMemcpyAsync(nq_out, L.qcount, sizeof(int), hipMemcpyDeviceToHost, st) != hipSuccess)
-            return RPD_E_DEVICE;
-        if (L.fl_cnt && L.fl_cnt_host &&
-            hipMemcpyAsync(L.fl_cnt_host, L.fl_cnt, kFailCounters * sizeof(int), hipMemcpyDeviceToHost, st) !=
-                hipSuccess)
-            return RPD_E_DEVICE;
-    }
-    if (!wait) return RPD_OK;
-    return hipStreamSynchronize(st) == hipSuccess ? RPD_OK : RPD_E_DEVICE;
+    return RPD_OK;
+}
+
+int rpd_launch_lists(hipStream_t st, const ClipLaunch &L, const FailLists &F) {
+    if (L.n_ids <= 0) return RPD_OK;
+    ListArgs a{};
+    a.code = L.code;
+    a.ids = L.ids;
+    a.n = L.n_ids;
+    a.cnt = F.cnt;
+    a.eo = F.eo;
+    a.sec = F.sec;
+    a.q = F.q;
+    a.q_host = F.q_host_dev;
+    a.cnt_host = F.cnt_host_dev;
+    const int64_t per = int64_t(kListBlock) * kListPer;
+    list_failures_kernel<<<unsigned((L.n_ids + per - 1) / per), kListBlock, 0, st>>>(a);
+    return hipGetLastError() == hipSuccess ? RPD_OK : RPD_E_DEVICE;
 }
 
 namespace rpd {

@@ -172,25 +172,15 @@ struct ClipLaunch {
     double4 *out;          // original order
     int *status;           // original order
     int *kused;            // original order (nullable)
-    void *rec;             // n_ids * rpd_clip_record_bytes(form, P, V) bytes
-    int *qcount;           // one device int: queued cells
-    bool qcount_zeroed;    // the caller has cleared qcount (rpd_launch_cells does not)
+    void *rec;             // n_ids * rpd_clip_record_bytes(form, P, V) bytes, item t's record at slot t
+    uint8_t *code;         // n_ids bytes, rounded up to whole 16: how each item left the bisector kernel
     hipEvent_t ev_mid;     // recorded after the bisector kernel (nullable)
-    // failure list the kernels append to (nullable): kFailCounters counters
-    // ([0] exact entries, [1] overflow entries, [2 + s] cells per status s,
-    // [13] largest triangle union over T, [14] resumable entries), then the
-    // stored ids: exact entries at fl_eo[-1 - k], overflows at fl_eo[k],
-    // resumable cells at fl_sec[k]
-    int *fl_cnt, *fl_eo, *fl_sec;
-    int *fl_cnt_host;      // host copy of the counters, filled by rpd_launch_cells (nullable)
-    // nullable: device addresses of nq_out / fl_cnt_host (mapped pinned
-    // memory), written by a one-wave copy kernel instead of copy engine
-    // blits, which wait for room beside a running finish kernel
-    int *nq_dev_out, *fl_cnt_dev_out;
+    // failure list the finish kernel appends to (nullable): counters and
+    // entries as in FailLists
+    int *fl_cnt, *fl_eo;
     // resumable cells (security radius not reached), see ClipArgs in rpd_clip.hip
-    char *rs_out;          // records written by this pass (nullable)
-    int rs_out_stride, rs_cap;
-    int *rs_count;
+    char *rs_out;          // records written by this pass (nullable), item t's at slot rs_base + t
+    int rs_out_stride, rs_base;
     const char *rs_in;     // records this pass resumes from (nullable; FP64 form)
     int rs_in_stride, rs_in_P;
     int *rslot, *lastnb;   // per stored id
@@ -210,12 +200,19 @@ struct ClipLaunch {
     int *fl_slot;
     // finish kernel: the P and V the records were written with (0: P, V)
     int rec_P, rec_V;
-    // finish kernel (nullable): the queue length in device memory, at most
-    // the nq it is launched with (items past it exit)
-    const int *nq_dev;
 };
 
 constexpr int kFailCounters = 16;
+// A failure list: kFailCounters counters ([0] exact entries, [1] overflow
+// entries, [2 + s] cells per status s, [13] largest triangle union over T,
+// [14] resumable entries), the stored ids (exact entries at eo[-1 - k],
+// overflows at eo[k], resumable cells at sec[k]); q: two device ints, queued
+// items and a ticket, both 0.  The nullable host pointers are device addresses
+// of mapped pinned memory, which receive *q (then cleared) and the counters.
+struct FailLists {
+    int *cnt, *eo, *sec, *q;
+    int *q_host_dev, *cnt_host_dev;
+};
 
 // Debug counters of one pass (the reference's debugCounter0..4,
 // ConvexCell.cl:15-39, 887-911, 981-982, 1128-1150): [kDcMax + 0..4] largest
@@ -270,8 +267,6 @@ int rpd_clip_max_T(int form, int P, int V, bool hess = false);
 // kernels keep their residency (LDS per CU) for one-slot cells (V <= 64)
 // with T triangle entries; P itself otherwise.
 int rpd_clip_plane_room(int form, int P, int V, int T, int floor);
-// form: RPD_PREC_FP64 / RPD_PREC_MIXED / RPD_PREC_FP32.  The bisector-loop
-// kernel of L.n_ids cells, then copies to the host the number of cells it
 // Copies n0 ints src0 -> dst0 and n1 src1 -> dst1 with one one-wave kernel
 // (dst: device addresses of mapped pinned host memory; n1 may be 0).  Small
 // copies of counters to the host this way need one free wave slot, where a
@@ -281,10 +276,13 @@ int rpd_pin_copy(hipStream_t st, const int *src0, int *dst0, int n0, const int *
 // Clears n device ints with one one-wave kernel (a fill blit, like a copy,
 // waits for room beside a running finish kernel).
 int rpd_zero_ints(hipStream_t st, int *p, int n);
-// queued (and the failure counters when L.fl_cnt_host is set); waits for
-// them unless wait is false (the caller synchronizes st before reading).
-int rpd_launch_cells(hipStream_t st, int form, const ClipLaunch &L, int *nq, bool wait = true);
-// The finish kernel over the nq records the bisector kernel queued (async);
-// beside: cells of other finish kernels expected to run at the same time
-// (they set how many waves each cell gets).
+// The bisector kernel of L.n_ids cells (form: RPD_PREC_FP64 / RPD_PREC_MIXED
+// / RPD_PREC_FP32).
+int rpd_launch_cells(hipStream_t st, int form, const ClipLaunch &L);
+// The failure lists of its items (added to F's counters), on the same stream.
+int rpd_launch_lists(hipStream_t st, const ClipLaunch &L, const FailLists &F);
+// The finish kernel over the records of nq items (those not queued are left
+// out), or over the records L.slots names (async); beside: cells of other
+// finish kernels expected to run at the same time (they set how many waves
+// each cell gets).
 int rpd_launch_finish(hipStream_t st, int form, const ClipLaunch &L, int nq, int beside = 0);

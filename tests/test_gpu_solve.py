@@ -211,3 +211,24 @@ def test_domain_outlives_its_context(rpd, ctx):
     ctx.solve(dom, K=50, P=30, V=40, precision=rpd.PREC_FP64)
     assert np.array_equal(ctx.moments(), ref)
     dom.close()
+
+
+@pytest.mark.parametrize("n", [2, 15, 16, 17, 4095, 4096, 4097, 8193])
+def test_failure_lists_at_group_edges(rpd, ctx, n):
+    """The failure lists are made from the cells' codes in groups of 16 and
+    workgroups of 4096.  Nearly every cell fails in pass 1 (12 planes; a
+    Hessian keeps the cap as asked), some run out of neighbours and are
+    resumed: the result is bit for bit that of ample caps, where no cell
+    fails."""
+    h = (1.0 / n) ** (1 / 3)
+    x = rpd.generate_seeds(rpd.SEEDS_UNIFORM, n, seed=n, wmax=0.8 * h * h * 1e6)
+    ctx.set_seeds(x)
+    ctx.solve(None, K=256, P=120, V=200, T=100, precision=rpd.PREC_FP64, H=60)
+    ref, ref_st = ctx.moments(), ctx.status()
+    st = ctx.solve(None, K=16, P=12, V=40, T=100, precision=rpd.PREC_FP64, H=60, max_extra_steps=12)
+    print("lists", n, st["passes"], st["pass_cells"], flush=True)
+    if n > 15:
+        assert st["pass_cells"][1] > n // 2
+    assert np.array_equal(ctx.status(), ref_st)
+    assert np.array_equal(ctx.moments(), ref)
+    assert abs(ref[:, 3].sum() - 1e9) <= 1e-11 * 1e9
