@@ -80,6 +80,8 @@ constexpr int kPinCounters = 16;
 constexpr int kPinBinFlag = kPinCounters - 4;
 // smallest triangle cap a solve uses
 constexpr int kTriangleFloor = 256;
+// smallest neighbour cap a solve uses (with re-queue passes, FP64 and mixed)
+constexpr int kNeighbourFloor = 64;
 // the plane cap a solve raises a lower one to, where that costs no residency
 constexpr int kPlaneFloor = 48;
 constexpr int kPinHist = kPinCounters + 6 * kFailCounters;
@@ -934,6 +936,17 @@ static int solve_impl(rpd_ctx *c, rpd_domain *dom, const rpd_params *prm, rpd_st
     const int form0 = prm->precision;
     const int kprec = form0 == RPD_PREC_FP64 ? 1 : 0;
     int K = std::min<int64_t>(prm->K, n - 1), P = prm->P, V = prm->V, T = prm->T;
+    // The neighbour cap is raised to a wavefront's 64 where it is lower: the
+    // kNN of 64 neighbours uses the same selection buffer as that of 20 (59
+    // against 48 us for 21,000 FP64 queries), the bisector kernel loads 64
+    // neighbours at once in any case, and a lower cap only sends cells to
+    // further passes (100,000 seeds in a torus at 100^3, K = 20: 87% of the
+    // cells a second time; solve 1.46 -> 0.98 ms, K = 25 0.90 of 1.29 ms,
+    // 300,000 seeds at K = 50 4.9 -> 4.7 ms).
+    // Only with re-queue passes allowed: without them, running out is the
+    // answer; and not in the FP32 form, whose re-queue passes are FP64.
+    if (prm->max_extra_steps > 0 && form0 != RPD_PREC_FP32 && K < kNeighbourFloor)
+        K = int(std::min<int64_t>(kNeighbourFloor, n - 1));
     // The triangle cap is raised to kTriangleFloor where it is lower: a cell
     // done by one wave keeps 4 bytes of LDS per union entry, which costs the
     // finish kernel no residency, and a cell's result does not depend on the

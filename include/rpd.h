@@ -152,7 +152,8 @@ typedef struct {
                                      no residency and changes no result: T to
                                      at least 256, V to its vertex slots'
                                      room (64/128/256) and, with
-                                     max_extra_steps > 0, P toward 48.  A
+                                     max_extra_steps > 0, P toward 48 and (FP64
+                                     and mixed forms) K to at least 64.  A
                                      cell's result does not depend on the cap
                                      it succeeds with; the caps a solve used
                                      are in rpd_stats.final_* / pass_caps    */
