@@ -530,11 +530,11 @@ __global__ __launch_bounds__(256) void mark_neighbours_kernel(const char *__rest
     if (q >= nq) return;
     const char *r = rec + size_t(q) * size_t(stride);
     if (reinterpret_cast<const int *>(r)[0] < 0) return;  // no cell
-    const int nvalid = reinterpret_cast<const int *>(r)[2];  // RecHeader{sid, nb_plane, nvalid, kused}
     const uint32_t *tri = reinterpret_cast<const uint32_t *>(r + 16 + size_t(P) * 32);
-    const int *nid = reinterpret_cast<const int *>(tri + 64 * S);
-    for (int j = lane; j < nvalid; j += 64) {
+    const int *nid = reinterpret_cast<const int *>(tri + 128 * S);  // after the triples and their adjacency
+    for (int j = lane; j < 64 * S; j += 64) {
         const uint32_t t = tri[j];
+        if (t == 0xffffffffu) continue;  // no vertex
         for (int k = 0; k < 3; ++k) {
             const int nb = nid[(t >> (8 * k)) & 0xff];
             if (nb >= 0 && used[nb] == 0) used[nb] = d;
@@ -1431,7 +1431,11 @@ static int solve_impl(rpd_ctx *c, rpd_domain *dom, const rpd_params *prm, rpd_st
         ch.pr.slot = ch.sl;
         ch.pz.slot = ch.sl2;
         ch.pr.index = ch.pz.index = 1 + ch.k;
-        ch.pr.form = ch.pz.form = RPD_PREC_FP64;
+        // resumed cells of a mixed solve go on in the mixed form, which decides
+        // its open tests in FP64 in place (the reference stop, whose near
+        // cases it leaves to the FP64 form, and the Hessian go on in FP64)
+        ch.pr.form = form0 == RPD_PREC_MIXED && prm->security_mode == 0 && !hess ? RPD_PREC_MIXED : RPD_PREC_FP64;
+        ch.pz.form = RPD_PREC_FP64;
         ch.pr.n_ids = ch.n_res;
         ch.pz.n_ids = ch.n_scr;
         ch.pr.caps[0] = nc.K - ch.cap.K;  // the neighbours after the ones used

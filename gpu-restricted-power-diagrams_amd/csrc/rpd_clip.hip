@@ -13,10 +13,10 @@
 // Because det4x4(pi1, pi2, pi3, e) == e . (X, Y, Z, W), the plane-side test
 // of CCVertexIsInHalfSpace is one 4-term dot product per lane.  Plane
 // equations live in LDS.  A clip removes the vertices with e.v > 0, finds the
-// cavity boundary as the edges of removed vertices whose reverse edge is not
-// also removed (checked to be one simple cycle, else inconsistent_boundary),
-// and places one new vertex (plane, a, b) per boundary edge a->b into free
-// lanes -- the same vertex set CCComputeBoundary + CCNewVertex build.
+// cavity boundary as the edges of removed vertices whose other end is kept
+// (checked to be one simple cycle, else inconsistent_boundary), and places one
+// new vertex (plane, a, b) per boundary edge a->b into free lanes -- the same
+// vertex set CCComputeBoundary + CCNewVertex build.
 //
 // Two kernels per pass:
 //   clip_cells_kernel   the bisector loop for every cell (light, high
@@ -34,13 +34,13 @@
 // Forms: FP64 (all double); mixed: the plane-side tests and the vertex
 // registers are FP32 and each test also evaluates a certified bound on its
 // FP32 error against the FP64 planes, 2^-18 * sum of |terms| of the det4x4
-// expansion.  In the bisector kernel (FP32 planes in LDS) a test inside the
-// bound or an ill-conditioned new vertex ends the cell with
-// needs_exact_predicates and the host re-runs it in FP64; in the finish kernel
-// (FP64 planes in LDS) a test inside the bound, and every test of an
-// ill-conditioned vertex, is decided in FP64 from the vertex's planes, as the
-// FP64 form decides it.  The
-// planes are stored in FP64, and the cell geometry that produces the results
+// expansion.  A test inside the bound, and every test of an ill-conditioned
+// vertex, is decided in FP64 from the vertex's planes, as the FP64 form
+// decides it: the finish kernel has FP64 planes in LDS, the bisector kernel
+// FP32 planes, beside which it makes FP64 ones when a test first needs them.
+// A cavity that such decisions leave inconsistent ends the cell with a status
+// that the host re-runs in FP64.  The records' planes are FP64; the
+// cell geometry that produces the results
 // (bbox, cone planes, volume and moments) is evaluated in FP64 from them, so
 // an unflagged mixed cell has the FP64 combinatorics and FP64 geometry.  FP32
 // form: everything in FP32, no filter.  Moments are accumulated in FP64.
@@ -141,6 +141,15 @@ struct ClipArgs {
     int rec_P, rec_S;
 };
 
+// The arguments in the kernel's argument area (its first parameter), for code
+// after the loops: loaded where they are used.
+using ColdArgs = const __attribute__((address_space(4))) ClipArgs;
+__device__ __forceinline__ ColdArgs *cold_args() {
+    auto p = (ColdArgs *)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(p));
+    return p;
+}
+
 // The cell of stored id sid reads its request's seed count, weight minimum
 // and domain (packed batch; wave-uniform, so the fields stay in SGPRs).  The
 // kernels take it as a template parameter, so that a single diagram's
@@ -179,15 +188,15 @@ __device__ __forceinline__ bool exact_failure(int st) {
 // overflows (vertex, plane, K, triangle) always; needs_exact_predicates,
 // inconsistent_boundary and find_another_beginning_vertex when the form was
 // not FP64 (in FP64 a recomputation would fail the same way).
-__device__ __forceinline__ bool listed_failure(const ClipArgs &a, int st) {
+__device__ __forceinline__ bool listed_failure(int exact_final, int st) {
     if (st == RPD_SUCCESS || st == RPD_EMPTY_CELL || st == RPD_HESSIAN_OVERFLOW) return false;
-    return !(exact_failure(st) && a.exact_final);
+    return !(exact_failure(st) && exact_final);
 }
 
 // Finish kernel: appends a failed cell (stored id sid, record slot rslot) to
 // the failure list.  One lane.  (Few cells fail here.)
 __device__ __forceinline__ void note_failure(const ClipArgs &a, int sid, int st, int rslot) {
-    if (!a.fl_cnt || !listed_failure(a, st)) return;
+    if (!a.fl_cnt || !listed_failure(a.exact_final, st)) return;
     const bool exact = exact_failure(st);
     atomicAdd(a.fl_cnt + 2 + st, 1);
     const int k = atomicAdd(a.fl_cnt + (exact ? 0 : 1), 1);
@@ -219,12 +228,10 @@ __device__ __forceinline__ Pl<T> cvt(const Pl<U> &p) {
 }
 
 // Homogeneous vertex of planes (p1, p2, p3): the cofactors of
-// CCComputeVertexCoordinates (ConvexCell.cl:344-362), plus (FILTER) the sums
-// of absolute values of their terms: MXYZ the largest of those of X, Y, Z,
-// MW that of W.
-template <typename R, bool FILTER>
+// CCComputeVertexCoordinates (ConvexCell.cl:344-362).
+template <typename R>
 __device__ __forceinline__ void vertex_from_planes(const Pl<R> &p1, const Pl<R> &p2, const Pl<R> &p3, R &X, R &Y,
-                                                   R &Z, R &W, float &MXYZ, float &MW) {
+                                                   R &Z, R &W) {
     const R m12 = p2.x * p3.y - p2.y * p3.x;
     const R m13 = p2.x * p3.z - p2.z * p3.x;
     const R m14 = p2.x * p3.w - p2.w * p3.x;
@@ -235,21 +242,6 @@ __device__ __forceinline__ void vertex_from_planes(const Pl<R> &p1, const Pl<R> 
     Y = p1.x * m34 + p1.w * m13 - p1.z * m14;
     Z = -p1.x * m24 + p1.y * m14 - p1.w * m12;
     W = p1.x * m23 - p1.y * m13 + p1.z * m12;
-    if (FILTER) {
-        const float x2 = fabsf(float(p2.x)), y2 = fabsf(float(p2.y)), z2 = fabsf(float(p2.z)),
-                    w2 = fabsf(float(p2.w));
-        const float x3 = fabsf(float(p3.x)), y3 = fabsf(float(p3.y)), z3 = fabsf(float(p3.z)),
-                    w3 = fabsf(float(p3.w));
-        const float a12 = fmaf(x2, y3, y2 * x3), a13 = fmaf(x2, z3, z2 * x3), a14 = fmaf(x2, w3, w2 * x3);
-        const float a23 = fmaf(y2, z3, z2 * y3), a24 = fmaf(y2, w3, w2 * y3), a34 = fmaf(z2, w3, w2 * z3);
-        const float ax = fabsf(float(p1.x)), ay = fabsf(float(p1.y)), az = fabsf(float(p1.z)),
-                    aw = fabsf(float(p1.w));
-        const float MX = aw * a23 + ay * a34 + az * a24;
-        const float MY = ax * a34 + aw * a13 + az * a14;
-        const float MZ = ax * a24 + ay * a14 + aw * a12;
-        MXYZ = fmaxf(MX, fmaxf(MY, MZ));
-        MW = ax * a23 + ay * a13 + az * a12;
-    }
 }
 
 // Whether the vertex of planes tr lies strictly outside plane e, in FP64:
@@ -258,20 +250,34 @@ __device__ __forceinline__ void vertex_from_planes(const Pl<R> &p1, const Pl<R> 
 // spills than inlined.)
 __device__ __forceinline__ bool outside64(const Pl<double> *planes, uint32_t tr, Pl<double> e) {
     double x, y, z, w;
-    float mx, mw;
-    vertex_from_planes<double, false>(planes[t0(tr)], planes[t1(tr)], planes[t2(tr)], x, y, z, w, mx, mw);
+    vertex_from_planes<double>(planes[t0(tr)], planes[t1(tr)], planes[t2(tr)], x, y, z, w);
     return e.x * x + e.y * y + e.z * z + e.w * w > 0.0;
+}
+
+// The squared distance from the seed of the vertex of planes tr, in FP64 from
+// its FP64 planes.
+__device__ __forceinline__ float vertex_r2_64(const Pl<double> *planes, uint32_t tr) {
+    double x, y, z, w;
+    vertex_from_planes<double>(planes[t0(tr)], planes[t1(tr)], planes[t2(tr)], x, y, z, w);
+    return float((x * x + y * y + z * z) / (w * w));
 }
 
 // Error bound factor of the mixed form: 64 units in the last place of FP32
 // (first-order analysis gives 13: 4 from rounding the FP64 planes, 9 from the
 // cofactor and dot-product evaluation).  The bound of a test e.v is
-// kappa * (|e.x| MX + |e.y| MY + |e.z| MZ + |e.w| MW), taken here as
-// kappa * ((|e.x| + |e.y| + |e.z|) MXYZ + |e.w| MW), which is not smaller.
+// kappa * (|e.x| MX + |e.y| MY + |e.z| MZ + |e.w| MW) with MX, MY, MZ, MW the
+// sums of absolute values of the cofactors' terms.  The planes' normals are
+// unit vectors, so by Cauchy-Schwarz MX, MY and MZ are at most M = |w1| + |w2|
+// + |w3| (the offsets), and MW, the permanent of three unit vectors, at most
+// 2 / sqrt(3): the test takes kappa * ((|e.x| + |e.y| + |e.z|) M + |e.w|
+// kMagW), which is not smaller.  M costs 3 instructions of the 28 that the
+// sums do; it is about twice as large, but a test it leaves open is decided
+// in FP64 in place.
 constexpr float kFilterKappa = 0x1.0p-18f;
-// vertices with |W| below this fraction of its term magnitude are
-// ill-conditioned in FP32 and sent to FP64
-constexpr float kFilterMinW = 1.0e-3f;
+constexpr float kMagW = 1.1548f;
+// vertices with |W| below this are ill-conditioned in FP32: all their tests are
+// decided in FP64, and their distance from the seed is taken in FP64
+constexpr float kFilterMinW = 1.0e-3f * kMagW;
 
 // apex_mode 1 puts the cone apex at this fraction of a voxel whose interior
 // has one known class (in or out).  Any interior point is valid; a generic
@@ -286,40 +292,72 @@ constexpr uint64_t kCube0 = 0x0402040405010502ull;  // 2 5 1 5 4 4 2 4
 constexpr uint64_t kCube1 = 0x0304000201050305ull;  // 5 3 5 1 2 0 4 3
 constexpr uint64_t kCube2 = 0x0101030003020000ull;  // 0 0 2 3 0 3 1 1
 
+// Adjacency of the cube's vertices: entry k of vertex i, 5 bits at 16 (i & 3) +
+// 5 k of word i >> 2, is (vertex << 2 | edge) of the reverse of edge k of i.
+struct CubeAdj {
+    uint64_t w[2];
+};
+constexpr CubeAdj cube_adjacency() {
+    CubeAdj c{};
+    const uint64_t t[3] = {kCube0, kCube1, kCube2};
+    for (int i = 0; i < 8; ++i)
+        for (int k = 0; k < 3; ++k) {
+            const uint64_t u = (t[k] >> (8 * i)) & 0xff, v = (t[(k + 1) % 3] >> (8 * i)) & 0xff;
+            for (int j = 0; j < 8; ++j)
+                for (int m = 0; m < 3; ++m)
+                    if (((t[m] >> (8 * j)) & 0xff) == v && ((t[(m + 1) % 3] >> (8 * j)) & 0xff) == u)
+                        c.w[i >> 2] |= uint64_t(j << 2 | m) << (16 * (i & 3) + 5 * k);
+        }
+    return c;
+}
+constexpr CubeAdj kCubeAdj = cube_adjacency();
+
+// A vertex's three adjacency entries as LDS holds them (16 bits each) and as a
+// record does (10 bits each).
+__device__ __forceinline__ uint2 adj_unpack(uint32_t a) {
+    return make_uint2((a & 0x3ffu) | ((a << 6) & 0x3ff0000u), a >> 20);
+}
+__device__ __forceinline__ uint32_t adj_pack(uint2 a) { return (a.x & 0x3ffu) | ((a.x >> 6) & 0xffc00u) | (a.y << 20); }
+
 // ---------------------------------------------------------------------------
 // The cell of one wavefront: vertices in lanes, planes in LDS.
 // ---------------------------------------------------------------------------
 // The cell of one wavefront.  Planes are stored in LDS in precision PS: the
 // bisector kernel keeps them in the test precision R, the finish kernel in
 // the geometry precision RP.
+//
+// Edge k of a vertex (p0, p1, p2) goes from plane p_k to p_(k+1); its reverse
+// belongs to the vertex at its other end.  adj holds, per vertex (64 slot +
+// lane) and edge, that vertex and which of its edges the reverse is (vertex <<
+// 2 | edge, 16 bits).  A clip's boundary edges are those of removed vertices
+// whose other end is kept: one LDS read and three bit tests.  (A bit matrix
+// of directed edges over pairs of planes, built by LDS atomics in every clip,
+// took three atomics, three reads and three writes with an address
+// computation each.)
 template <typename R, typename RP, bool FILTER, int S, typename PS = RP>
 struct WaveCell {
     Pl<PS> *planes;
     uint32_t *nvs;
-    uint8_t *nxt;
-    // bit matrix of directed edges, P rows of ceil(P / 32) words: bit v of
-    // row u set while a removed vertex's triangle holds the edge u -> v
-    // (all zero between clips)
-    uint32_t *em;
+    uint8_t *nxt;       // boundary successor of a plane (cycle check; 0xff between clips)
+    uint8_t *sta, *end;  // new vertex whose boundary edge starts / ends at a plane
+    uint2 *adj;
     int P, V, nb_plane, lane;
     uint32_t tri[S];
     R X[S], Y[S], Z[S], W[S], r2[S];
-    float MXYZ[S], MW[S];
+    float M[S];
     uint64_t valid[S];
-    // (mixed finish kernel) vertices whose tests are all decided in FP64:
-    // ill-conditioned in FP32 (|W| small against its terms)
+    // (FILTER) vertices whose tests are all decided in FP64: ill-conditioned
+    // in FP32 (small |W|)
     uint64_t x64[S];
     R maxr2;
-    // FP64 planes in LDS under the mixed filter (the finish kernel): tests
-    // the filter leaves open are decided in FP64 in place
-    static constexpr bool kInline64 = FILTER && sizeof(PS) == 8;
 
     // R2: also the vertex's squared distance from the seed (the bisector
     // loop's stop test reads it through maxr2; the finish kernel does not)
     template <bool R2 = true>
     __device__ void set_vertex(int s, uint32_t tr, const Pl<R> &p1, const Pl<R> &p2, const Pl<R> &p3) {
         tri[s] = tr;
-        vertex_from_planes<R, FILTER>(p1, p2, p3, X[s], Y[s], Z[s], W[s], MXYZ[s], MW[s]);
+        vertex_from_planes<R>(p1, p2, p3, X[s], Y[s], Z[s], W[s]);
+        if (FILTER) M[s] = fabsf(float(p1.w)) + fabsf(float(p2.w)) + fabsf(float(p3.w));
         if (R2) {
             // FP32: the hardware reciprocal (1 ulp); r2 is read only by the
             // stop and skip tests, whose radius margin (2e-4) is far larger
@@ -338,187 +376,154 @@ struct WaveCell {
         set_vertex<R2>(s, tr, cvt<R>(planes[t0(tr)]), cvt<R>(planes[t1(tr)]), cvt<R>(planes[t2(tr)]));
     }
 
+    // The vertices of a record of nent slots (triples rtr, adjacency radj) at
+    // their lanes.
+    template <bool R2, typename P64>
+    __device__ void load_vertices(const uint32_t *rtr, const uint32_t *radj, int nent, P64 planes64) {
+#pragma unroll
+        for (int s = 0; s < S; ++s) {
+            const int j = s * 64 + lane;
+            uint32_t tr = kNoTri;
+            if (j < nent) {
+                tr = rtr[j];
+                adj[j] = adj_unpack(radj[j]);
+            }
+            const bool v = tr != kNoTri;
+            if (v) set_vertex_lds<R2>(s, tr);
+            valid[s] = ballot(v);
+            if (FILTER) x64[s] = ballot(fabsf(float(W[s])) < kFilterMinW) & valid[s];
+            if constexpr (FILTER && R2)
+                if (x64[s]) {
+                    const Pl<double> *p64 = planes64();
+                    if (in_mask(x64[s])) r2[s] = vertex_r2_64(p64, tri[s]);
+                }
+        }
+        wsync();
+    }
+
+    __device__ void clear_vertices() {
+#pragma unroll
+        for (int s = 0; s < S; ++s) {
+            valid[s] = 0;
+            x64[s] = 0;
+            tri[s] = 0;
+            X[s] = Y[s] = Z[s] = R(0);
+            W[s] = R(1);
+            r2[s] = R(0);
+            M[s] = 0.f;
+        }
+    }
+
     __device__ void refresh_max_r2() {
         R m = R(0);
 #pragma unroll
-        for (int s = 0; s < S; ++s)
-            if ((valid[s] >> lane) & 1) m = r2[s] > m ? r2[s] : m;
-        maxr2 = wave_max(m);
-    }
-
-    // True when plane e removes every vertex with a margin: e.v above the
-    // certified FP32 error bound (mixed form) or above kSepTau times the sum
-    // of |terms| of e.v (FP64 and FP32 forms).
-    __device__ bool removes_all(const Pl<R> &e) const {
-        bool keep = false;
-        const float exyz = fabsf(float(e.x)) + fabsf(float(e.y)) + fabsf(float(e.z)), ew = fabsf(float(e.w));
-#pragma unroll
         for (int s = 0; s < S; ++s) {
-            const bool v = (valid[s] >> lane) & 1;
-            const R sv = e.x * X[s] + e.y * Y[s] + e.z * Z[s] + e.w * W[s];
-            R m;
-            if (FILTER)
-                m = R(kFilterKappa * (exyz * MXYZ[s] + ew * MW[s]));
-            else
-                m = R(sizeof(R) == 8 ? 0x1.0p-33 : 0x1.0p-16) *
-                    (fabs(e.x * X[s]) + fabs(e.y * Y[s]) + fabs(e.z * Z[s]) + fabs(e.w * W[s]));
-            bool k = !(sv > m);
-            if constexpr (kInline64) k = k || ((x64[s] >> lane) & 1);
-            keep |= v && k;
+            const R x = in_mask(valid[s]) ? r2[s] : R(0);
+            m = x > m ? x : m;
         }
-        return ballot(keep) == 0;
+        maxr2 = wave_max_pos(m);
     }
 
-    // One clip by plane e (wave-uniform, test precision).  Lane wl holds the
-    // same plane in the storage precision in eP (wl < 0: every lane does).
-    // Returns kNoClip, kClipped or a failure status.  R2: keep r2 and maxr2
-    // up to date.
-    template <bool R2 = true>
-    __device__ int clip(const Pl<R> &e, int wl, const Pl<PS> &eP) {
+    // One clip by plane e (wave-uniform, test precision), which the caller has
+    // put at planes[nb_plane].  Returns kNoClip, kClipped or a failure status.
+    // R2: keep r2 and maxr2 up to date.  planes64 (FILTER) gives the cell's
+    // FP64 planes, that of e at nb_plane.
+    //
+    // The scalar unit, which the four SIMDs of a CU share, bounds this code as
+    // much as the vector ALUs do: masks are combined as masks, edges that are
+    // not on the boundary write to a spare word instead of being branched
+    // around, and the wave-wide counts are scalar bit counts.
+    template <bool R2, typename P64>
+    __device__ __forceinline__ int clip(const Pl<R> &e, P64 planes64) {
         uint64_t rem[S], unsure[S];
-        int nr = 0, nvalid = 0;
         uint64_t flag = 0;
-        const float exyz = fabsf(float(e.x)) + fabsf(float(e.y)) + fabsf(float(e.z)), ew = fabsf(float(e.w));
+        const float ek = kFilterKappa * (fabsf(float(e.x)) + fabsf(float(e.y)) + fabsf(float(e.z))),
+                    ewk = kFilterKappa * kMagW * fabsf(float(e.w));
 #pragma unroll
         for (int s = 0; s < S; ++s) {
-            const bool v = (valid[s] >> lane) & 1;
             const R sv = e.x * X[s] + e.y * Y[s] + e.z * Z[s] + e.w * W[s];
-            rem[s] = ballot(v && sv > R(0));
+            rem[s] = ballot(sv > R(0)) & valid[s];
             unsure[s] = 0;
             if (FILTER) {
-                const float bound = kFilterKappa * (exyz * MXYZ[s] + ew * MW[s]);
-                unsure[s] = ballot(v && fabsf(float(sv)) <= bound);
-                if constexpr (kInline64) unsure[s] |= x64[s] & valid[s];
+                unsure[s] = (ballot(fabsf(float(sv)) <= fmaf(ek, M[s], ewk)) | x64[s]) & valid[s];
                 flag |= unsure[s];
             }
-            nr += __popcll(rem[s]);
-            nvalid += __popcll(valid[s]);
         }
         if (FILTER && flag) {
-            if constexpr (sizeof(PS) == 8) {
-                // FP64 planes at hand (the finish kernel): the vertices the
-                // filter leaves open are rebuilt from their planes in FP64
-                // and tested in FP64, the FP64 form's own evaluation, so the
-                // clip decides as the FP64 form does
+            // the vertices the filter leaves open are rebuilt from their
+            // planes in FP64 and tested in FP64, the FP64 form's own
+            // evaluation, so the clip decides as the FP64 form does
+            const Pl<double> *p64 = planes64();
+            const Pl<double> e64 = p64[nb_plane];
 #pragma unroll
-                for (int s = 0; s < S; ++s) {
-                    if (!unsure[s]) continue;
-                    const bool out = ((unsure[s] >> lane) & 1) && outside64(planes, tri[s], eP);
-                    const uint64_t now = ballot(out);
-                    nr += __popcll(now) - __popcll(rem[s] & unsure[s]);
-                    rem[s] = (rem[s] & ~unsure[s]) | now;
-                }
-            } else {
-                return RPD_NEEDS_EXACT_PREDICATES;
+            for (int s = 0; s < S; ++s) {
+                if (!unsure[s]) continue;
+                bool out = false;
+                if (in_mask(unsure[s])) out = outside64(p64, tri[s], e64);
+                rem[s] = (rem[s] & ~unsure[s]) | ballot(out);
             }
+        }
+        int nr = 0, nvalid = 0;
+#pragma unroll
+        for (int s = 0; s < S; ++s) {
+            nr += __popcll(rem[s]);
+            nvalid += __popcll(valid[s]);
         }
         if (nr == 0) return kNoClip;
         if (nr == nvalid) return RPD_EMPTY_CELL;
         const int pid = nb_plane;
-        if (lane == (wl < 0 ? 0 : wl)) planes[pid] = eP;
-        // boundary edges: an edge u->v of a removed triangle whose reverse
-        // v->u belongs to no removed triangle.  Every removed triangle marks
-        // its three directed edges in the bit matrix em (row u, bit v), reads
-        // the three reverse edges back, then clears the words it set.
-        uint32_t bm[S];
-        const uint32_t rw = uint32_t(P + 31) >> 5;  // words per row
-        // edge u -> v: word u * rw + v / 32, bit v % 32
-        auto edge_word = [&](uint32_t u, uint32_t v) { return em + (u * rw + (v >> 5)); };
-#pragma unroll
-        for (int s = 0; s < S; ++s) {
-            if ((rem[s] >> lane) & 1) {
-                const uint32_t tr = tri[s];
-                const uint32_t a0 = t0(tr), a1 = t1(tr), a2 = t2(tr);
-                atomicOr(edge_word(a0, a1), 1u << (a1 & 31));
-                atomicOr(edge_word(a1, a2), 1u << (a2 & 31));
-                atomicOr(edge_word(a2, a0), 1u << (a0 & 31));
-            }
-        }
-        wsync();
-#pragma unroll
-        for (int s = 0; s < S; ++s) {
-            bm[s] = 0;
-            if ((rem[s] >> lane) & 1) {
-                const uint32_t tr = tri[s];
-                const uint32_t a0 = t0(tr), a1 = t1(tr), a2 = t2(tr);
-                const bool h01 = (*edge_word(a1, a0) >> (a0 & 31)) & 1u;  // a1 -> a0 removed too
-                const bool h12 = (*edge_word(a2, a1) >> (a1 & 31)) & 1u;
-                const bool h20 = (*edge_word(a0, a2) >> (a2 & 31)) & 1u;
-                bm[s] = (h01 ? 0u : 1u) | (h12 ? 0u : 2u) | (h20 ? 0u : 4u);
-            }
-        }
-        wsync();
-#pragma unroll
-        for (int s = 0; s < S; ++s) {
-            if ((rem[s] >> lane) & 1) {
-                const uint32_t tr = tri[s];
-                const uint32_t a0 = t0(tr), a1 = t1(tr), a2 = t2(tr);
-                *edge_word(a0, a1) = 0;
-                *edge_word(a1, a2) = 0;
-                *edge_word(a2, a0) = 0;
-            }
-        }
-        // slot-major exclusive offsets of the new vertices
+        // boundary edges: edges of removed vertices whose other end is kept
+        uint32_t en[S][3];
+        uint64_t bd[S][3];
         int nb = 0;
-        int obase[S];
 #pragma unroll
         for (int s = 0; s < S; ++s) {
-            const int c = __popc(bm[s]);
-            const int incl = wave_incl_scan_op(c, 0, [](int x, int y) { return x + y; });
-            obase[s] = nb + incl - c;
-            nb += uni(rlane(incl, 63));
+            const uint2 ad = adj[s * 64 + lane];
+            en[s][0] = ad.x & 0xffffu;
+            en[s][1] = ad.x >> 16;
+            en[s][2] = ad.y;
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                const uint32_t v = en[s][k] >> 2;
+                uint64_t m = rem[0];
+#pragma unroll
+                for (int u = 1; u < S; ++u)
+                    if (v >> 6 == uint32_t(u)) m = rem[u];
+                bd[s][k] = ballot((uint32_t(m >> (v & 63u)) & 1u) == 0u) & rem[s];
+                nb += __popcll(bd[s][k]);
+            }
         }
-        int nkeep = 0;
-#pragma unroll
-        for (int s = 0; s < S; ++s) nkeep += __popcll(valid[s] & ~rem[s]);
-        if (nkeep + nb > V) return RPD_VERTEX_OVERFLOW;
-        // stage new triples (plane, a, b) and (unfiltered forms) the
-        // boundary successor map
+        if (nvalid - nr + nb > V) return RPD_VERTEX_OVERFLOW;
+        // stage the new vertices: (a, b) of the boundary edge and the kept end
+        int o = 0;
 #pragma unroll
         for (int s = 0; s < S; ++s) {
-            if (bm[s]) {
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
                 const uint32_t tr = tri[s];
-                const uint32_t v0 = t0(tr), v1 = t1(tr), v2 = t2(tr);
-                int o = obase[s];
-                if (bm[s] & 1u) {
-                    nvs[o++] = pack3(uint32_t(pid), v0, v1);
-                    if (!FILTER) nxt[v0] = uint8_t(v1);
-                }
-                if (bm[s] & 2u) {
-                    nvs[o++] = pack3(uint32_t(pid), v1, v2);
-                    if (!FILTER) nxt[v1] = uint8_t(v2);
-                }
-                if (bm[s] & 4u) {
-                    nvs[o++] = pack3(uint32_t(pid), v2, v0);
-                    if (!FILTER) nxt[v2] = uint8_t(v0);
-                }
+                const uint32_t a = k == 0 ? t0(tr) : (k == 1 ? t1(tr) : t2(tr)),
+                               b = k == 0 ? t1(tr) : (k == 1 ? t2(tr) : t0(tr));
+                nvs[in_mask(bd[s][k]) ? mbcnt(bd[s][k], o) : 64 * S + lane] = a | (b << 8) | (en[s][k] << 16);
+                o += __popcll(bd[s][k]);
             }
         }
         wsync();
         // The cavity must be a disk: its boundary one simple cycle.  With
-        // certified signs (FILTER) it always is: the removed vertices are
-        // those of a convex polytope strictly on one side of a plane, which,
-        // like the kept ones, form a connected set, and every face meets the
-        // plane's side in one contiguous arc, so no face is pinched.  The
-        // unfiltered forms check it, as CCComputeBoundary does: every start
-        // plane written once, and the walk from one start closes after
-        // exactly nb steps.
-        bool inconsistent = false;
-        if (!FILTER) {
+        // certified signs it always is: the removed vertices are those of a
+        // convex polytope strictly on one side of a plane, which, like the
+        // kept ones, form a connected set, and every face meets the plane's
+        // side in one contiguous arc, so no face is pinched.  Signs decided in
+        // FP64 are checked, as CCComputeBoundary does: every start plane
+        // written once, and the walk from one start closes after exactly nb
+        // steps.
+        if (!FILTER || flag) {
+            for (int q = lane; q < nb; q += 64) nxt[nvs[q] & 0xffu] = uint8_t(nvs[q] >> 8);
+            wsync();
             bool bad = false;
-#pragma unroll
-            for (int s = 0; s < S; ++s) {
-                if (bm[s]) {
-                    const uint32_t tr = tri[s];
-                    const uint32_t v0 = t0(tr), v1 = t1(tr), v2 = t2(tr);
-                    if (bm[s] & 1u) bad |= nxt[v0] != v1;
-                    if (bm[s] & 2u) bad |= nxt[v1] != v2;
-                    if (bm[s] & 4u) bad |= nxt[v2] != v0;
-                }
-            }
-            inconsistent = ballot(bad) != 0;
+            for (int q = lane; q < nb; q += 64) bad |= nxt[nvs[q] & 0xffu] != ((nvs[q] >> 8) & 0xffu);
+            bool inconsistent = ballot(bad) != 0;
             if (!inconsistent) {
-                const uint32_t start = t1(uni(nvs[0]));
+                const uint32_t start = uni(nvs[0]) & 0xffu;
                 uint32_t cur = start;
                 int steps = 0;
                 do {
@@ -528,91 +533,116 @@ struct WaveCell {
                 inconsistent = !(cur == start && steps == nb);
             }
             wsync();
-#pragma unroll
-            for (int s = 0; s < S; ++s) {
-                if (bm[s]) {
-                    const uint32_t tr = tri[s];
-                    if (bm[s] & 1u) nxt[t0(tr)] = 0xff;
-                    if (bm[s] & 2u) nxt[t1(tr)] = 0xff;
-                    if (bm[s] & 4u) nxt[t2(tr)] = 0xff;
-                }
-            }
+            for (int q = lane; q < nb; q += 64) nxt[nvs[q] & 0xffu] = 0xff;
+            if (inconsistent) return RPD_INCONSISTENT_BOUNDARY;
         }
-        if (inconsistent) return RPD_INCONSISTENT_BOUNDARY;
-        // new vertices fill the lowest free slots
+        // new vertices (plane, a, b) fill the lowest free slots
         int carry = 0;
-        uint64_t ill = 0;
+        uint32_t nw[S];
+        uint64_t newm[S];
 #pragma unroll
         for (int s = 0; s < S; ++s) {
             valid[s] &= ~rem[s];
             const uint64_t fr = ~valid[s];
-            const int q = carry + mbcnt(fr);
-            const bool take = ((fr >> lane) & 1) && q < nb;
-            const uint64_t newm = ballot(take);
-            if (take) {
-                const uint32_t tr = nvs[q];
-                set_vertex<R2>(s, tr, e, cvt<R>(planes[t1(tr)]), cvt<R>(planes[t2(tr)]));
+            const int q = mbcnt(fr, carry);
+            newm[s] = ballot(q < nb) & fr;
+            nw[s] = 0;
+            if (in_mask(newm[s])) {
+                const uint32_t w = nvs[q], a = w & 0xffu, b = (w >> 8) & 0xffu, v = uint32_t(s * 64 + lane);
+                nw[s] = w;
+                set_vertex<R2>(s, pack3(uint32_t(pid), a, b), e, cvt<R>(planes[a]), cvt<R>(planes[b]));
+                sta[a] = uint8_t(v);
+                end[b] = uint8_t(v);
+                // the kept end's edge now leads here (edge 1: a -> b)
+                reinterpret_cast<uint16_t *>(adj)[4 * (w >> 18) + ((w >> 16) & 3u)] = uint16_t(v << 2 | 1u);
+                if (S == 1) {
+                    // edge 0 (pid -> a) meets the new vertex that ends at a,
+                    // edge 2 (b -> pid) the one that starts at b
+                    wsync();
+                    adj[lane] = make_uint2((uint32_t(end[a]) << 2) | 2u | (w & 0xffff0000u), uint32_t(sta[b]) << 2);
+                }
             }
             if (FILTER) {
-                const uint64_t il = ballot(take && fabsf(float(W[s])) < kFilterMinW * MW[s]);
-                if constexpr (kInline64)
-                    x64[s] = (x64[s] & ~newm) | il;  // decided in FP64 from now on
-                else
-                    ill |= il;
+                const uint64_t il = ballot(fabsf(float(W[s])) < kFilterMinW) & newm[s];
+                x64[s] = (x64[s] & ~newm[s]) | il;
+                if constexpr (R2)
+                    if (il) {
+                        const Pl<double> *p64 = planes64();
+                        if (in_mask(il)) r2[s] = vertex_r2_64(p64, tri[s]);
+                    }
             }
             carry += __popcll(fr);
-            valid[s] |= newm;
+            valid[s] |= newm[s];
+        }
+        wsync();
+        if constexpr (S > 1) {
+#pragma unroll
+            for (int s = 0; s < S; ++s)
+                if (in_mask(newm[s])) {
+                    const uint32_t w = nw[s];
+                    adj[s * 64 + lane] = make_uint2((uint32_t(end[w & 0xffu]) << 2) | 2u | (w & 0xffff0000u),
+                                                    uint32_t(sta[(w >> 8) & 0xffu]) << 2);
+                }
+            wsync();
         }
         nb_plane = pid + 1;
-        if (FILTER && ill) return RPD_NEEDS_EXACT_PREDICATES;
         if (R2) refresh_max_r2();
         return kClipped;
     }
 };
 
-// LDS of one wave: planes[P] | plane sources src[P] (int32) | nvs[64S] |
-// nxt[256] | em[P][ceil(P / 32)] | tu[T] (finish kernel) | chunk / cone planes cpl[64] |
-// go_out flags[16] | triangle corners tcor[16][9] (finish kernel)
+// LDS of one wave: nvs[64S] and 64 spare words | adj[64S] (8 bytes) | chunk /
+// cone planes cpl[64] | go_out flags[16] | planes[P] | plane sources src[P]
+// (int32) | nxt, sta, end [P rounded up to 16 each] | tu[T] (finish kernel) |
+// tail (finish kernel: triangle corners tcor[16][9] and the vertex copy; mixed
+// bisector kernel: FP64 planes).  The parts of a fixed size come first: their
+// addresses are constants in the bisector kernel.
+__host__ __device__ constexpr size_t up16(size_t b) { return (b + 15) & ~size_t(15); }
 template <typename R, typename RP, bool FILTER, int S, typename PS>
 __device__ __forceinline__ void bind_lds(char *L, int P, int T, WaveCell<R, RP, FILTER, S, PS> &c,
                                          int **src = nullptr, int **tu = nullptr, Pl<PS> **cpl = nullptr,
-                                         int **goo = nullptr, double **tcor = nullptr) {
-    c.planes = reinterpret_cast<Pl<PS> *>(L);
-    size_t off = (size_t(P) * sizeof(Pl<PS>) + 15) & ~size_t(15);
-    if (src) *src = reinterpret_cast<int *>(L + off);
-    off += (4 * size_t(P) + 15) & ~size_t(15);
-    c.nvs = reinterpret_cast<uint32_t *>(L + off);
-    off += 4 * 64 * S;
-    c.nxt = reinterpret_cast<uint8_t *>(L + off);
-    off += 256;
-    c.em = reinterpret_cast<uint32_t *>(L + off);
-    off += 4 * size_t(P) * size_t((P + 31) >> 5);
-    if (tu) *tu = reinterpret_cast<int *>(L + off);
-    off += 4 * size_t(T);
-    off = (off + 15) & ~size_t(15);
+                                         int **goo = nullptr, char **tail = nullptr) {
+    c.nvs = reinterpret_cast<uint32_t *>(L);
+    size_t off = 4 * (64 * S + 64);
+    c.adj = reinterpret_cast<uint2 *>(L + off);
+    off += 8 * 64 * S;
     if (cpl) *cpl = reinterpret_cast<Pl<PS> *>(L + off);
     off += 64 * sizeof(Pl<PS>);
     if (goo) *goo = reinterpret_cast<int *>(L + off);
     off += 64;
-    if (tcor) *tcor = reinterpret_cast<double *>(L + off);
+    c.planes = reinterpret_cast<Pl<PS> *>(L + off);
+    off += up16(size_t(P) * sizeof(Pl<PS>));
+    if (src) *src = reinterpret_cast<int *>(L + off);
+    off += up16(4 * size_t(P));
+    c.nxt = reinterpret_cast<uint8_t *>(L + off);
+    c.sta = c.nxt + up16(P);
+    c.end = c.sta + up16(P);
+    off += 3 * up16(P);
+    if (tu) *tu = reinterpret_cast<int *>(L + off);
+    off += up16(4 * size_t(T));
+    if (tail) *tail = L + off;
 }
 
 // A vertex of the finish kernel's cell as the lane-parallel skip tests read
 // it: homogeneous coordinates in the test precision and, for the certified
-// form, the magnitudes of their terms.
+// form, the magnitude of their terms.
 template <typename R>
 struct VtxRec {
     R X, Y, Z, W;
-    float MXYZ, MW;
+    float M;
 };
 constexpr size_t kVtxRecBytes = 40;  // sizeof(VtxRec<double>), the larger one
 
 // LDS bytes of one wave (pl: bytes of one stored plane; tail: bytes after the
 // cone planes and flags)
 __host__ __device__ constexpr size_t wave_lds(int P, int S, int T, size_t pl, size_t tail) {
-    return ((((((P * pl + 15) & ~size_t(15)) + ((4 * size_t(P) + 15) & ~size_t(15)) + 4 * 64 * size_t(S) +
-               256 + 4 * size_t(P) * size_t((P + 31) >> 5) + 4 * size_t(T)) +
-              15) & ~size_t(15)) + 64 * pl + 64 + tail + 15) & ~size_t(15);
+    return 4 * (64 * size_t(S) + 64) + 8 * 64 * size_t(S) + 64 * pl + 64 + up16(P * pl) + up16(4 * size_t(P)) +
+           3 * up16(P) + up16(4 * size_t(T)) + up16(tail);
+}
+// (the bisector kernel; planes in the test precision, the mixed form with room
+// for the FP64 planes)
+__host__ __device__ constexpr size_t cells_wave_lds(int form, int P, int S) {
+    return wave_lds(P, S, 0, form == RPD_PREC_FP64 ? 32 : 16, form == RPD_PREC_MIXED ? 32 * size_t(P) : 0);
 }
 // (corners: the finish kernel's triangle corners and vertex copy)
 __host__ __device__ constexpr size_t finish_wave_lds(int P, int S, int T, size_t pl, bool corners = false) {
@@ -655,33 +685,43 @@ __device__ __forceinline__ Pl<double> cube_plane(int f, const double4 &S0, doubl
     return Pl<double>{ax == 0 ? sgn : 0.0, ax == 1 ? sgn : 0.0, ax == 2 ? sgn : 0.0, d};
 }
 
-// Record of a finished cell in the queue: header (sid, nb_plane, nvalid,
-// kused), planes[P] in the storage precision, vertex triples[64 * S].
+// Record of a cell: header (sid, nb_plane, nent = 64 * S, kused), planes[P] in
+// the storage precision, vertex triples[nent] (kNoTri where none) and their
+// adjacency[nent] (adj_pack), plane neighbours[P].  The vertices stay at the
+// lanes they have, so that a resumed cell has the lanes, and so the sums, of
+// one uninterrupted run, and the adjacency stays as it is.
 struct RecHeader {
-    int sid, nb_plane, nvalid, kused;
+    int sid, nb_plane, nent, kused;
 };
 
 // ---------------------------------------------------------------------------
 // Kernel A: the bisector loop (ConvexCell.cl:850-917)
 // ---------------------------------------------------------------------------
-// Minimum waves per SIMD the bisector kernel is compiled for (one vertex
-// slot per lane): its run time is set by latency, so occupancy pays more than
-// the few registers the compiler then spills (measured at 1M seeds: FP64 7,
-// 72 VGPRs and 12 bytes of spill, 2.10 ms against 2.35 at 5 waves and 2.27 at
-// 8; FP32 forms 8, which they reach without spills).  Wider cells (S > 1,
+// What bounds it: instruction issue.  The scalar unit serves the four SIMDs of
+// a CU, one instruction a cycle; with 4,200 (mixed form) scalar and 6,700
+// vector instructions a cell it was as busy as the vector ALUs, and a version
+// with fewer vector but more scalar ones (5,600 / 5,900) ran slower.  Hence the
+// adjacency (WaveCell), the masks instead of branches, the single exit of the
+// loop, and arguments read again after it instead of kept.  1M seeds in a
+// torus at 128^3: 1.50 -> 1.17 ms (mixed), 1.90 -> 1.45 ms (FP64); as a packed
+// batch of 300,000 cells, where the loop's branches had counted as divergent,
+// 3.45 -> 2.33 ms; 1M nearly cospherical seeds, whose cells all failed the
+// filter and went to a second kNN and FP64 pass, 15.5 -> 7.9 ms.
+//
+// Minimum waves per SIMD the bisector kernel is compiled for (one vertex slot
+// per lane): occupancy pays more than the few registers the compiler then
+// spills, all in the code of open tests (FP64 7 waves, 71 VGPRs; mixed 8, 64
+// VGPRs; FP32 form 8, 50; mixed at 7 waves 2% slower).  Wider cells (S > 1,
 // re-queue passes) are left unconstrained.
 template <typename R, int S>
 constexpr int kClipWaves = S > 1 ? 1 : (sizeof(R) == 8 ? 7 : 8);
 
 template <typename R, typename RP, bool FILTER, int S, bool BATCH>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kClipWaves<R, S>)))
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kClipWaves<R, S>)))
 void clip_cells_kernel(ClipArgs a) {
     extern __shared__ __attribute__((aligned(16))) char lds_raw[];
     const int lane = lane_id();
-    const int wv = uni(int(threadIdx.x >> 6));  // wave-uniform: lets ids, seeds and pointers live in SGPRs
-    const int wpb = blockDim.x >> 6;
-    const int64_t t = int64_t(blockIdx.x) * wpb + wv;
-    if (t >= a.n_ids) return;  // wave-uniform
+    const int64_t t = blockIdx.x;  // one wave per workgroup
 
     // planes in the test precision; src[p] records where plane p came from
     // (the neighbour's stored id, or -1 - f for cube face f), so that the
@@ -690,39 +730,58 @@ void clip_cells_kernel(ClipArgs a) {
     WaveCell<R, RP, FILTER, S, R> c;
     Pl<R> *chunk = nullptr;  // planes of the current 64 neighbours
     int *src = nullptr;
-    bind_lds(lds_raw + size_t(wv) * a.lds_stride, a.P, 0, c, &src, nullptr, &chunk);
+    char *tail = nullptr;
+    bind_lds(lds_raw, a.P, 0, c, &src, nullptr, &chunk, nullptr, &tail);
     c.P = a.P;
     c.V = a.V;
     c.lane = lane;
 
     const int sid = uni(a.ids ? a.ids[t] : int(t));
-    if constexpr (BATCH) bind_request(a, sid);
+    // the weight minimum and the domain, in a packed batch those of the
+    // cell's request
+    double wmin = a.wmin, vs = a.vs;
+    int g = a.g;
+    const uint8_t *dist = a.dist;
+    if constexpr (BATCH) {
+        const ReqDesc &d = a.reqs[uni(int(a.req_of[sid]))];
+        wmin = uni(d.wmin);
+        vs = uni(d.vs);
+        g = uni(d.g);
+        dist = d.dist;
+    }
     const double4 S0 = a.seeds[sid];
-    const int orig = a.perm[sid];
     const int K = a.K, P = a.P;
     // resumed cells: record of the state, neighbours used before this pass
-    const bool resume = sizeof(R) == 8 && a.rs_in != nullptr;
+    const bool resume = sizeof(RP) == 8 && a.rs_in != nullptr;
     const char *rs_rec = resume ? a.rs_in + size_t(a.rslot[sid]) * size_t(a.rs_in_stride) : nullptr;
     const int kbase = resume ? uni(reinterpret_cast<const RecHeader *>(rs_rec)->kused) : 0;
 
+    // The end of an item that is not queued: its outputs and code.  (The
+    // arguments are read again from the kernel's argument area: held in
+    // registers through the loop, these pointers were spilled to vector lanes
+    // and read back one by one.)
     auto finish = [&](int st, double m0, double m1, double m2, double m3, int ku, bool resumable = false) {
+        const auto *k = cold_args();
         if (lane == 0) {
-            a.out[orig] = make_double4(m0, m1, m2, m3);
-            a.status[orig] = st;
-            if (a.kused) a.kused[orig] = kbase + ku;
-            reinterpret_cast<RecHeader *>(a.rec + size_t(t) * size_t(a.rec_stride))->sid = -1;
-            a.code[t] = uint8_t(!listed_failure(a, st) ? kCodeDone
-                                                       : uint32_t(st) + (resumable ? kCodeResume : kCodeFailed));
+            const int orig = k->perm[sid];
+            k->out[orig] = make_double4(m0, m1, m2, m3);
+            k->status[orig] = st;
+            if (k->kused) k->kused[orig] = kbase + ku;
+            reinterpret_cast<RecHeader *>(k->rec + size_t(t) * size_t(k->rec_stride))->sid = -1;
+            k->code[t] = uint8_t(!listed_failure(k->exact_final, st)
+                                     ? kCodeDone
+                                     : uint32_t(st) + (resumable ? kCodeResume : kCodeFailed));
         }
     };
-    auto fail = [&](int st, int ku) { finish(st, 0.0, 0.0, 0.0, 0.0, ku); };
 
     if (S0.w <= RPD_NO_CELL_LIMITS) {  // border seed: copied (ConvexCell.cl:873-876)
         finish(RPD_SUCCESS, S0.x, S0.y, S0.z, S0.w, 0);
         return;
     }
-    for (int i = lane; i < 256; i += 64) c.nxt[i] = 0xff;
-    for (int i = lane; i < P * ((P + 31) >> 5); i += 64) c.em[i] = 0;
+    for (int i = lane; i < P; i += 64) {
+        c.nxt[i] = 0xff;
+        c.sta[i] = c.end[i] = 0;
+    }
 
     // Domain cull: a seed whose voxel is d >= 2 voxels (Chebyshev) from every
     // voxel that holds triangles or lies inside has no point of the domain
@@ -730,61 +789,58 @@ void clip_cells_kernel(ClipArgs a) {
     // below that, its restriction to the domain is empty (volume 0, as the
     // reference's apex-outside / no-triangle case, ConvexCell.cl:1067-1079).
     double cull_r2 = 0;
-    if (a.g > 0 && a.dist) {
-        const int g = a.g;
-        auto vox = [&](double x) { return int(fmin(fmax(x / a.vs, 0.0), double(g - 1))); };
-        const int d = a.dist[vox(S0.x) + vox(S0.y) * g + vox(S0.z) * g * g];
-        if (d >= 2) cull_r2 = double(d - 1) * a.vs * double(d - 1) * a.vs;
+    if (g > 0 && dist) {
+        auto vox = [&](double x) { return int(fmin(fmax(x / vs, 0.0), double(g - 1))); };
+        // (uni: a load through a pointer that is itself loaded, as in a packed
+        // batch, counts as differing by lane, and so would the loop's branches)
+        const int d = uni(int(dist[vox(S0.x) + vox(S0.y) * g + vox(S0.z) * g * g]));
+        if (d >= 2) cull_r2 = double(d - 1) * vs * double(d - 1) * vs;
     }
-    const double wgap = S0.w - a.wmin;  // >= 0 except for the lightest seeds
+    const double wgap = S0.w - wmin;  // >= 0 except for the lightest seeds
 
-    const double eps = a.g > 0 ? 0.1 : 0.0;  // CUBE_EPSILON, voronoi.cpp:929
-#pragma unroll
-    for (int s = 0; s < S; ++s) {
-        c.valid[s] = 0;
-        c.x64[s] = 0;
-        c.tri[s] = 0;
-        c.X[s] = c.Y[s] = c.Z[s] = R(0);
-        c.W[s] = R(1);
-        c.r2[s] = R(0);
-        c.MXYZ[s] = c.MW[s] = 0.f;
-    }
+    const double eps = g > 0 ? 0.1 : 0.0;  // CUBE_EPSILON, voronoi.cpp:929
+    c.clear_vertices();
+    // (mixed form) the FP64 planes: the first n64 of them are in p64, the
+    // others are made when a test or the record first needs them
+    Pl<double> *p64 = reinterpret_cast<Pl<double> *>(tail);
+    int n64 = 0;
     if (resume) {
         // ---- the state a previous pass left: planes, then the vertices at
         // their lanes (nent = 64 x the S of the pass that left it) ----------
         const RecHeader hd = *reinterpret_cast<const RecHeader *>(rs_rec);
-        const int nent = uni(hd.nvalid);
+        const int nent = uni(hd.nent);
         c.nb_plane = uni(hd.nb_plane);
         const Pl<RP> *rpl = reinterpret_cast<const Pl<RP> *>(rs_rec + sizeof(RecHeader));
         const uint32_t *rtr =
             reinterpret_cast<const uint32_t *>(rs_rec + sizeof(RecHeader) + size_t(a.rs_in_P) * sizeof(Pl<RP>));
-        const int *rnid = reinterpret_cast<const int *>(rtr + nent);
+        const int *rnid = reinterpret_cast<const int *>(rtr + 2 * nent);
         for (int p = lane; p < c.nb_plane; p += 64) {
             c.planes[p] = cvt<R>(rpl[p]);
+            if constexpr (FILTER) p64[p] = rpl[p];
             src[p] = rnid[p];
         }
+        n64 = c.nb_plane;
         wsync();
-#pragma unroll
-        for (int s = 0; s < S; ++s) {
-            const int j = s * 64 + lane;
-            const uint32_t tr = j < nent ? rtr[j] : kNoTri;
-            if (tr != kNoTri) c.set_vertex_lds(s, tr);
-            c.valid[s] = ballot(tr != kNoTri);
-        }
+        c.template load_vertices<true>(rtr, rtr + nent, nent, [&]() -> const Pl<double> * { return p64; });
     } else {
         // ---- CCInit: bounding cube in the local frame ----------------------
         if (lane < 6) {
-            c.planes[lane] = cvt<R>(cube_plane(lane, S0, eps));
+            const Pl<double> q = cube_plane(lane, S0, eps);
+            c.planes[lane] = cvt<R>(q);
+            if constexpr (FILTER) p64[lane] = q;
             src[lane] = -1 - lane;
         }
         wsync();
-        c.nb_plane = 6;
+        c.nb_plane = n64 = 6;
         if (lane < 8) {
             const uint32_t sh = 8 * uint32_t(lane);
             c.set_vertex_lds(0, pack3(uint32_t(kCube0 >> sh) & 0xff, uint32_t(kCube1 >> sh) & 0xff,
                                       uint32_t(kCube2 >> sh) & 0xff));
+            const uint32_t w = uint32_t(kCubeAdj.w[lane >> 2] >> (16 * (lane & 3)));
+            c.adj[lane] = make_uint2((w & 31u) | ((w & 0x3e0u) << 11), (w >> 10) & 31u);
         }
         c.valid[0] = 0xffull;
+        wsync();
     }
     c.refresh_max_r2();
 
@@ -800,12 +856,6 @@ void clip_cells_kernel(ClipArgs a) {
     // plane list fails at the next neighbour, ConvexCell.cl:316-319) are
     // those of the one-by-one loop.
     const int *nrow = a.knn + t * int64_t(K);
-    bool reached = false, complete = false;
-    int kused = 0;
-    double cdl = 0;
-    float ct = 0;
-    int cnb = -1;
-    int loaded = -1;
     const double rmarg = sizeof(R) == 8 ? 1.0 + 1e-9 : 1.0 + 2e-4;  // FP32 R may be low by ~1e-4
     // the cell's radius (FP32 forms: the hardware square root, 1 ulp, far
     // inside the radius margin)
@@ -816,198 +866,192 @@ void clip_cells_kernel(ClipArgs a) {
             return sqrt(double(c.maxr2));
     };
     double Rcur = radius();
-    auto stop_at = [&](double dl, double Rm) -> bool {
-        // CCIsSecurityRadiusReached (reference stop, weights ignored) or the
-        // exact power stop d (d - 2R) >= w_s - w_min
-        const double Rs = Rm * rmarg;
-        if (a.security_mode == 1 || wgap <= 0) return dl * dl > 4.0 * Rs * Rs;
-        return dl * (dl - 2.0 * Rs) >= wgap;
-    };
-    // The exact stop only ever holds when no later bisector can cut, so the
-    // FP32 radius's margin merely delays it.  The reference stop can hold
-    // while a later bisector of a lighter seed still cuts; there a delayed
-    // stop changes the cell.  So in the mixed form a reference-stop test
-    // within the FP32 radius's margin (2R / rmarg < d <= 2R rmarg) that the
-    // loop reaches ends the cell with needs_exact_predicates: the FP64 pass
-    // decides it, as an uncertain plane-side test.
+    // Stop test: CCIsSecurityRadiusReached (reference stop, weights ignored)
+    // or the exact power stop d (d - 2R) >= w_s - w_min.  The exact stop only
+    // ever holds when no later bisector can cut, so the FP32 radius's margin
+    // merely delays it.  The reference stop can hold while a later bisector of
+    // a lighter seed still cuts; there a delayed stop changes the cell.  So in
+    // the mixed form a reference-stop test within the FP32 radius's margin
+    // (2R / rmarg < d <= 2R rmarg) that the loop reaches ends the cell with
+    // needs_exact_predicates: the FP64 pass decides it.
+    const bool plain_stop = a.security_mode == 1 || wgap <= 0;
     const bool ref_stop = FILTER && a.security_mode == 1;
-    auto stop_near = [&](double dl, double Rm) -> bool {
-        const double Rl = Rm / rmarg;
-        return dl * dl > 4.0 * Rl * Rl && !stop_at(dl, Rm);
+    auto fill64 = [&](int upto) {
+        wsync();
+        for (int p = n64 + lane; p < upto; p += 64) {
+            double bl;
+            p64[p] = bisector_plane(S0, a.seeds[src[p]], bl);
+        }
+        wsync();
+        n64 = upto;
     };
-    int i = 0;
-    while (i < K) {
-        const int base = i & ~63;
-        if (base != loaded) {
-            const int j = base + lane;
-            cnb = j < K ? nrow[j] : -2;  // -1: list exhausted, -2: past K
-            Pl<R> cpl{R(0), R(0), R(0), R(0)};
-            cdl = 0;
-            ct = 0;
-            if (cnb >= 0) {
-                double bl;
-                const Pl<double> q = bisector_plane(S0, a.seeds[cnb], bl);
-                cpl = cvt<R>(q);
-                cdl = bl;
-                ct = float(q.w);
-            }
-            wsync();  // the previous chunk's planes are no longer read
-            chunk[lane] = cpl;
-            wsync();
-            loaded = base;
+    // (the plane about to be clipped by lies at nb_plane)
+    auto planes64 = [&]() -> const Pl<double> * {
+        if constexpr (FILTER) fill64(c.nb_plane + 1);
+        return p64;
+    };
+    // how the loop ends: the list ran out, the radius was reached, every other
+    // seed was used, culled, failed (with the status)
+    enum { kRanOut = -1, kReached = -2, kComplete = -3, kCulled = -4 };
+    int why = kRanOut, kused = 0;
+    for (int base = 0; base < K; base += 64) {
+        const int j = base + lane;
+        const int cnb = j < K ? nrow[j] : -2;  // -1: list exhausted, -2: past K
+        double cdl = 0;
+        float ct = 0;
+        wsync();  // the previous chunk's planes are no longer read
+        if (cnb >= 0) {
+            double bl;
+            const Pl<double> q = bisector_plane(S0, a.seeds[cnb], bl);
+            chunk[lane] = cvt<R>(q);
+            cdl = bl;
+            ct = float(q.w);
         }
-        const int l0 = i & 63;
-        const bool in = lane >= l0 && cnb != -2;
-        if (c.nb_plane >= P) {
-            // the next neighbour's plane cannot be stored
-            const uint64_t me = ballot(in && cnb == -1), mv = ballot(in && cnb >= 0);
-            if (mv && (!me || lowest_bit(mv) < lowest_bit(me))) {
-                fail(RPD_PLANE_OVERFLOW, base + lowest_bit(mv) + 1);
-                return;
+        wsync();
+        const uint64_t m_has = ballot(cnb >= 0), m_none = ballot(cnb == -1);
+        // the neighbours not visited yet, and the one clipped by last, whose
+        // stop test comes with the next choice
+        uint64_t left = ~0ull, last = 0;
+        for (;;) {
+            const double Rs = Rcur * rmarg;
+            uint64_t m_stop;
+            if (plain_stop)
+                m_stop = ballot(cdl * cdl > 4.0 * Rs * Rs);
+            else
+                m_stop = ballot(cdl * (cdl - 2.0 * Rs) >= wgap);
+            m_stop &= m_has & (left | last);
+            // skip test in FP32: t is rounded to FP32, so the radius gets a
+            // margin well above FP32 rounding (a false candidate only costs a
+            // no-op clip)
+            const float Rskip = float(Rs) * (1.0f + 1e-6f);
+            const uint64_t m_clip = ballot(ct < Rskip) & m_has & left;
+            const uint64_t m_end = m_none & left;
+            uint64_t m_any = m_stop | m_clip | m_end;
+            const bool full = c.nb_plane >= P;
+            // a full plane list: the next neighbour's plane cannot be stored
+            if (full) m_any = (m_stop & last) ? (m_stop & last) : ((m_has | m_none) & left);
+            if (FILTER && ref_stop && !full) {
+                const double Rl = Rcur / rmarg;
+                const uint64_t m_near = ballot(cdl * cdl > 4.0 * Rl * Rl) & ~m_stop & m_has & (left | last);
+                if (m_near && (!m_any || lowest_bit(m_near) < lowest_bit(m_any))) {
+                    why = RPD_NEEDS_EXACT_PREDICATES;
+                    kused = base + lowest_bit(m_near) + 1;
+                    break;
+                }
             }
-            if (me) {
-                complete = true;
+            if (!m_any) {
+                if (!full) kused = min(K, base + 64);
+                break;  // the next chunk
+            }
+            const int f = lowest_bit(m_any);
+            const uint64_t bit = 1ull << f;
+            if (full || !(m_clip & bit)) {
+                if (m_stop & bit & (full ? last : ~0ull)) {
+                    why = kReached;
+                    kused = base + f + 1;
+                } else if (m_end & bit) {
+                    why = kComplete;  // every other seed has been used
+                    if (!full) kused = base + f;
+                } else {
+                    why = RPD_PLANE_OVERFLOW;
+                    kused = base + f + 1;
+                }
                 break;
             }
-            i = base + 64;
-            continue;
-        }
-        // skip test in FP32: t is rounded to FP32, so the radius gets a margin
-        // well above FP32 rounding (a false candidate only costs a no-op clip)
-        const float Rskip = float(Rcur * rmarg) * (1.0f + 1e-6f);
-        const uint64_t m_end = ballot(in && cnb == -1);
-        const uint64_t m_clip = ballot(in && cnb >= 0 && ct < Rskip);
-        const uint64_t m_stop = ballot(in && cnb >= 0 && stop_at(cdl, Rcur));
-        const int f_end = m_end ? lowest_bit(m_end) : 64;
-        const int f_clip = m_clip ? lowest_bit(m_clip) : 64;
-        const int f_stop = m_stop ? lowest_bit(m_stop) : 64;
-        if (ref_stop) {
-            const uint64_t m_near = ballot(in && cnb >= 0 && stop_near(cdl, Rcur));
-            if (m_near && lowest_bit(m_near) < min(f_end, min(f_clip, f_stop))) {
-                fail(RPD_NEEDS_EXACT_PREDICATES, base + lowest_bit(m_near) + 1);
-                return;
+            // clip by the plane of neighbour base + f
+            const Pl<R> e = chunk[f];
+            const int nbid = rlane(cnb, f);
+            if (lane == 0) {
+                src[c.nb_plane] = nbid;
+                c.planes[c.nb_plane] = e;
             }
-        }
-        if (f_end < f_clip && f_end < f_stop) {
-            complete = true;  // every other seed has been used
-            kused = base + f_end;
-            break;
-        }
-        if (f_stop < f_clip) {
-            reached = true;
-            kused = base + f_stop + 1;
-            break;
-        }
-        if (f_clip == 64) {
-            i = base + 64;
-            kused = min(K, i);
-            continue;
-        }
-        // clip by the plane of neighbour base + f_clip
-        const Pl<R> e = chunk[f_clip];
-        const int nbid = rlane(cnb, f_clip);
-        if (lane == 0) src[c.nb_plane] = nbid;
-        const int res = c.clip(e, -1, e);
-        kused = base + f_clip + 1;
-        if (res >= 0) {
-            fail(res, kused);
-            return;
-        }
-        if (res == kClipped) {
-            Rcur = radius();
-            if (double(c.maxr2) * 1.001 < cull_r2) {
-                finish(RPD_SUCCESS, 0.0, 0.0, 0.0, 0.0, kused);
-                return;
-            }
-        }
-        {
-            const double dl = rlane(cdl, f_clip);
-            if (ref_stop && stop_near(dl, Rcur)) {
-                fail(RPD_NEEDS_EXACT_PREDICATES, kused);
-                return;
-            }
-            if (stop_at(dl, Rcur)) {
-                reached = true;
+            const int res = c.template clip<true>(e, planes64);
+            kused = base + f + 1;
+            if (res >= 0) {
+                why = res;
                 break;
             }
+            if (res == kClipped) {
+                Rcur = radius();
+                if (double(c.maxr2) * 1.001 < cull_r2) {
+                    why = kCulled;
+                    break;
+                }
+            } else if (FILTER) {
+                n64 = min(n64, c.nb_plane);  // the plane that did not cut gives way
+            }
+            left = ~1ull << f;  // past f
+            last = bit;
         }
-        i = base + f_clip + 1;
+        if (why != kRanOut) break;
     }
+    if (why >= 0 || why == kCulled) {
+        finish(why >= 0 ? why : int(RPD_SUCCESS), 0.0, 0.0, 0.0, 0.0, kused);
+        return;
+    }
+    const auto *k = cold_args();
     // a list that holds every other seed leaves nothing to test: the cell is
     // exact once the list is used up (the reference reads past the seeds there)
-    if (!reached && !complete && int64_t(kbase) + K >= a.n_seeds - 1) complete = true;
+    int64_t n_seeds = k->n_seeds;
+    if constexpr (BATCH) n_seeds = k->reqs[uni(int(k->req_of[sid]))].n_seeds;
+    if (why == kRanOut && int64_t(kbase) + K >= n_seeds - 1) why = kComplete;
 
     // debug counters (ConvexCell.cl:887-911): K used where the security
     // radius was reached, P and V once the neighbour loop is done
-    if (a.dcnt && lane == 0) {
-        if (reached) {
+    if (k->dcnt && lane == 0) {
+        if (why == kReached) {
             const int ku = min(kbase + kused, 256);
-            atomicMax(a.dcnt + kDcMax + 0, ku);
-            atomicAdd(a.dcnt + kDcHistK + ku, 1);
+            atomicMax(k->dcnt + kDcMax + 0, ku);
+            atomicAdd(k->dcnt + kDcHistK + ku, 1);
         }
         int nv = 0;
 #pragma unroll
         for (int s = 0; s < S; ++s) nv += __popcll(c.valid[s]);
-        atomicMax(a.dcnt + kDcMax + 1, c.nb_plane);
-        atomicAdd(a.dcnt + kDcHistP + min(c.nb_plane, 255), 1);
-        atomicMax(a.dcnt + kDcMax + 2, nv);
-        atomicAdd(a.dcnt + kDcHistV + min(nv, 256), 1);
+        atomicMax(k->dcnt + kDcMax + 1, c.nb_plane);
+        atomicAdd(k->dcnt + kDcHistP + min(c.nb_plane, 255), 1);
+        atomicMax(k->dcnt + kDcMax + 2, nv);
+        atomicAdd(k->dcnt + kDcHistV + min(nv, 256), 1);
     }
 
     // A finished cell is queued for restriction + integration.  A cell whose
     // list ran out keeps its state when there is room, so that the next pass
     // goes on from here with the neighbours after the last one used.
-    const bool ran_out = !reached && !complete;
-    if (!ran_out || a.rs_out) {
-        const int64_t slot = ran_out ? a.rs_base + t : t;
+    const bool ran_out = why == kRanOut;
+    if (!ran_out || k->rs_out) {
+        const int64_t slot = ran_out ? k->rs_base + t : t;
         // the cell's state as a record: header, planes in the geometry
-        // precision (rebuilt from their sources when the test precision is
-        // lower), vertex triples; P planes' room.  (Written in line: as a
-        // lambda the FP32-test kernel spills.)
-        char *rec = ran_out ? a.rs_out + size_t(slot) * size_t(a.rs_out_stride)
-                            : a.rec + size_t(slot) * size_t(a.rec_stride);
+        // precision, vertex triples and adjacency; P planes' room
+        char *rec = ran_out ? k->rs_out + size_t(slot) * size_t(k->rs_out_stride)
+                            : k->rec + size_t(slot) * size_t(k->rec_stride);
         Pl<RP> *rpl = reinterpret_cast<Pl<RP> *>(rec + sizeof(RecHeader));
         uint32_t *rtr = reinterpret_cast<uint32_t *>(rec + sizeof(RecHeader) + size_t(P) * sizeof(Pl<RP>));
-        int *rnid = reinterpret_cast<int *>(rtr + 64 * S);
-        // a queued cell's vertices are compacted; a kept state holds each
-        // triple at its lane (kNoTri where none), so that the resumed cell
-        // has the lanes, and so the sums, of one uninterrupted run
-        int nv = 0;
-#pragma unroll
-        for (int s = 0; s < S; ++s) nv += __popcll(c.valid[s]);
-        if (ran_out) nv = 64 * S;
+        int *rnid = reinterpret_cast<int *>(rtr + 128 * S);
         if (lane == 0) {
-            *reinterpret_cast<RecHeader *>(rec) = RecHeader{sid, c.nb_plane, nv, kbase + kused};
+            *reinterpret_cast<RecHeader *>(rec) = RecHeader{sid, c.nb_plane, 64 * S, kbase + kused};
             if (ran_out) {
-                a.rslot[sid] = int(slot);
-                a.lastnb[sid] = nrow[K - 1];
+                k->rslot[sid] = int(slot);
+                k->lastnb[sid] = nrow[K - 1];
             } else {
-                a.code[t] = kCodeQueued;
+                k->code[t] = kCodeQueued;
             }
         }
         wsync();
+        if constexpr (FILTER) fill64(c.nb_plane);
         for (int p = lane; p < c.nb_plane; p += 64) {
-            if (sizeof(R) == sizeof(RP)) {
+            if constexpr (FILTER)
+                rpl[p] = p64[p];
+            else
                 rpl[p] = cvt<RP>(c.planes[p]);
-            } else {
-                const int sj = src[p];
-                double bl;
-                rpl[p] = cvt<RP>(sj < 0 ? cube_plane(-1 - sj, S0, eps) : bisector_plane(S0, a.seeds[sj], bl));
-            }
             rnid[p] = src[p];
         }
-        int carry = 0;
 #pragma unroll
         for (int s = 0; s < S; ++s) {
-            const bool v = (c.valid[s] >> lane) & 1;
-            if (ran_out)
-                rtr[64 * s + lane] = v ? c.tri[s] : kNoTri;
-            else if (v)
-                rtr[carry + mbcnt(c.valid[s])] = c.tri[s];
-            carry += __popcll(c.valid[s]);
+            const bool v = in_mask(c.valid[s]);
+            rtr[64 * s + lane] = v ? c.tri[s] : kNoTri;
+            if (v) rtr[64 * S + 64 * s + lane] = adj_pack(c.adj[64 * s + lane]);
         }
     }
-    if (ran_out) finish(RPD_SECURITY_RADIUS_NOT_REACHED, 0.0, 0.0, 0.0, 0.0, kused, a.rs_out != nullptr);
+    if (ran_out) finish(RPD_SECURITY_RADIUS_NOT_REACHED, 0.0, 0.0, 0.0, 0.0, kused, k->rs_out != nullptr);
 }
 
 // The failure lists of a bisector kernel's items, from their codes: one
@@ -1203,12 +1247,13 @@ void finish_cells_kernel(ClipArgs a, int nq, int W) {
     WaveCell<R, RP, FILTER, S> c;
     int *tu = nullptr, *goo = nullptr;
     Pl<RP> *cpl = nullptr;
-    double *tcor = nullptr;
+    char *tail = nullptr;
     // VOX: a strip's fifth cone plane has room of its own, so that no cap is
     // met earlier than with triangles
     const int P = VOX ? a.P + 1 : a.P;
     bind_lds(lds_raw + size_t(cpb) * a.cell_stride + size_t(wv) * a.lds_stride, P, a.T, c, nullptr, &tu,
-             &cpl, &goo, &tcor);
+             &cpl, &goo, &tail);
+    double *tcor = reinterpret_cast<double *>(tail);  // (not VOX)
     c.P = P;
     c.V = a.V;
     c.lane = lane;
@@ -1218,27 +1263,22 @@ void finish_cells_kernel(ClipArgs a, int nq, int W) {
     const int sid = uni(hd.sid);
     if constexpr (BATCH) bind_request(a, sid);
     const int kused = uni(hd.kused);
-    const int nvalid = uni(hd.nvalid);
+    const int nent = uni(hd.nent);
     c.nb_plane = uni(hd.nb_plane);
     const Pl<RP> *rpl = reinterpret_cast<const Pl<RP> *>(rec + sizeof(RecHeader));
     const uint32_t *rtr =
         reinterpret_cast<const uint32_t *>(rec + sizeof(RecHeader) + size_t(a.rec_P) * sizeof(Pl<RP>));
     for (int p = lane; p < c.nb_plane; p += 64) c.planes[p] = rpl[p];
-    for (int i = lane; i < 256; i += 64) c.nxt[i] = 0xff;
-    for (int i = lane; i < P * ((P + 31) >> 5); i += 64) c.em[i] = 0;
-    wsync();
-#pragma unroll
-    for (int s = 0; s < S; ++s) {
-        const int j = s * 64 + lane;
-        c.tri[s] = 0;
-        c.X[s] = c.Y[s] = c.Z[s] = R(0);
-        c.W[s] = R(1);
-        c.r2[s] = R(0);
-        c.MXYZ[s] = c.MW[s] = 0.f;
-        if (j < nvalid) c.template set_vertex_lds<false>(s, rtr[j]);
-        c.valid[s] = ballot(j < nvalid);
-        c.x64[s] = 0;
+    for (int i = lane; i < P; i += 64) {
+        c.nxt[i] = 0xff;
+        c.sta[i] = c.end[i] = 0;
     }
+    wsync();
+    c.clear_vertices();
+    c.template load_vertices<false>(rtr, rtr + nent, nent, 0);
+    int nvalid = 0;
+#pragma unroll
+    for (int s = 0; s < S; ++s) nvalid += __popcll(c.valid[s]);
     // (the vertices' distances from the seed are not kept here: the
     // restriction takes the cell's radius in FP64 below)
 
@@ -1265,8 +1305,7 @@ void finish_cells_kernel(ClipArgs a, int nq, int W) {
         } else {
             const uint32_t tr = c.tri[s];
             RP X, Y, Z, W;
-            float d0, d1;
-            vertex_from_planes<RP, false>(c.planes[t0(tr)], c.planes[t1(tr)], c.planes[t2(tr)], X, Y, Z, W, d0, d1);
+            vertex_from_planes<RP>(c.planes[t0(tr)], c.planes[t1(tr)], c.planes[t2(tr)], X, Y, Z, W);
             const RP iw = RP(1) / W;
             Ax = X * iw;
             Ay = Y * iw;
@@ -1296,7 +1335,7 @@ void finish_cells_kernel(ClipArgs a, int nq, int W) {
         RP sw = 0, sx = 0, sy = 0, sz = 0;
 #pragma unroll
         for (int s = 0; s < S; ++s) {
-            const bool vok = (c.valid[s] >> lane) & 1;
+            const bool vok = in_mask(c.valid[s]);
             // per plane k of the vertex: area (CCExportBaryVolumeAndArea,
             // ConvexCell.cl:621-674) and area-weighted centroid
             double ha[3] = {0.0, 0.0, 0.0}, hx[3] = {0.0, 0.0, 0.0}, hy[3] = {0.0, 0.0, 0.0},
@@ -1461,7 +1500,7 @@ void finish_cells_kernel(ClipArgs a, int nq, int W) {
         double bmn[3] = {1000.0, 1000.0, 1000.0}, bmx[3] = {0.0, 0.0, 0.0}, vr2 = 0.0;
 #pragma unroll
         for (int s = 0; s < S; ++s) {
-            if (!((c.valid[s] >> lane) & 1)) continue;
+            if (!in_mask(c.valid[s])) continue;
             RP lx, ly, lz;
             vertex_rp(s, lx, ly, lz);
             vr2 = fmax(vr2, double(lx) * double(lx) + double(ly) * double(ly) + double(lz) * double(lz));
@@ -1778,8 +1817,16 @@ void finish_cells_kernel(ClipArgs a, int nq, int W) {
     int fail_t = 0x7fffffff, fail_st = 0;
     double sm = 0, sx = 0, sy = 0, sz = 0;  // running sums of the contributions (W = 1; wave-uniform)
     if (ntri > 0) {
-        // backup (ConvexCell.cl:692-715): the vertex registers and the plane count
+        // backup (ConvexCell.cl:692-715): the vertex registers, their adjacency
+        // and the plane count
         const WaveCell<R, RP, FILTER, S> bk = c;
+        uint2 bk_adj[S];
+#pragma unroll
+        for (int s = 0; s < S; ++s) bk_adj[s] = c.adj[s * 64 + lane];
+        auto planes64 = [&]() -> const Pl<double> * {
+            if constexpr (sizeof(RP) == 8) return c.planes;
+            return nullptr;
+        };
         constexpr int kPl = VOX ? 5 : 4;    // cone planes of a unit (strip or triangle)
         constexpr int kUB = VOX ? 12 : 16;  // units of a batch
         constexpr uint64_t kUm = (1ull << kPl) - 1;
@@ -1787,13 +1834,15 @@ void finish_cells_kernel(ClipArgs a, int nq, int W) {
         const double lx0 = P0x - S0.x, ly0 = P0y - S0.y, lz0 = P0z - S0.z;
         const double face_margin = sizeof(RP) == 8 ? 1e-7 : 1e-3;
         // The cell's vertices, compacted, for the lane-parallel tests: a cone
-        // plane removes every vertex (with the margin of removes_all) when
-        // each one is strictly on its removed side.
+        // plane removes every vertex when each one is strictly on its removed
+        // side, with a margin: above the certified FP32 error bound (mixed
+        // form) or above 2^-33 (FP64) or 2^-16 (FP32 form) times the sum of
+        // the test's |terms|.
         int nvc = 0;
 #pragma unroll
         for (int s = 0; s < S; ++s) {
-            if ((c.valid[s] >> lane) & 1)
-                vtx[nvc + mbcnt(c.valid[s])] = VtxRec<R>{c.X[s], c.Y[s], c.Z[s], c.W[s], c.MXYZ[s], c.MW[s]};
+            if (in_mask(c.valid[s]))
+                vtx[nvc + mbcnt(c.valid[s])] = VtxRec<R>{c.X[s], c.Y[s], c.Z[s], c.W[s], c.M[s]};
             nvc += __popcll(c.valid[s]);
         }
         wsync();
@@ -1925,14 +1974,14 @@ void finish_cells_kernel(ClipArgs a, int nq, int W) {
             }
             cpl[lane] = pl;
             // Skip tests, one lane per cone plane: the ball about the seed,
-            // then every vertex (the test of removes_all).
+            // then every vertex.
             bool gone = false;
             if (may_skip && k < ntri) {
                 gone = double(pl.w) < -rsk;
                 if (!gone) {
                     const Pl<R> e = cvt<R>(pl);
-                    const float exyz = fabsf(float(e.x)) + fabsf(float(e.y)) + fabsf(float(e.z)),
-                                ew = fabsf(float(e.w));
+                    const float ek = kFilterKappa * (fabsf(float(e.x)) + fabsf(float(e.y)) + fabsf(float(e.z))),
+                                ewk = kFilterKappa * kMagW * fabsf(float(e.w));
                     gone = true;
                     // U vertices a step, their loads issued together (the
                     // last vertex stands in past the end: testing it twice
@@ -1947,7 +1996,7 @@ void finish_cells_kernel(ClipArgs a, int nq, int W) {
                             const R sv = e.x * v[u].X + e.y * v[u].Y + e.z * v[u].Z + e.w * v[u].W;
                             R m;
                             if (FILTER)
-                                m = R(kFilterKappa * (exyz * v[u].MXYZ + ew * v[u].MW));
+                                m = R(fmaf(ek, v[u].M, ewk));
                             else
                                 m = R(sizeof(R) == 8 ? 0x1.0p-33 : 0x1.0p-16) *
                                     (fabs(e.x * v[u].X) + fabs(e.y * v[u].Y) + fabs(e.z * v[u].Z) +
@@ -2047,7 +2096,12 @@ void finish_cells_kernel(ClipArgs a, int nq, int W) {
                 for (int f2 = 0; f2 < kPl; ++f2) {
                     if (res < 0) {
                         const Pl<RP> q = cpl[kPl * t + f2];
-                        res = c.nb_plane >= P ? int(RPD_PLANE_OVERFLOW) : c.template clip<false>(cvt<R>(q), -1, q);
+                        if (c.nb_plane >= P) {
+                            res = RPD_PLANE_OVERFLOW;
+                        } else {
+                            if (lane == 0) c.planes[c.nb_plane] = q;
+                            res = c.template clip<false>(cvt<R>(q), planes64);
+                        }
                     }
                 }
                 if (res >= 0 && res != RPD_EMPTY_CELL) {
@@ -2057,6 +2111,9 @@ void finish_cells_kernel(ClipArgs a, int nq, int W) {
                     ck = integrate((VOX ? ((gom >> (kPl * t)) & 1) != 0 : goo[t] != 0) ? 1.0 : -1.0);
                 }
                 c = bk;
+#pragma unroll
+                for (int s = 0; s < S; ++s) c.adj[s * 64 + lane] = bk_adj[s];
+                wsync();
                 if (W == 1) {
                     sx = uni(sx + ck.x);
                     sy = uni(sy + ck.y);
@@ -2109,7 +2166,7 @@ void finish_cells_kernel(ClipArgs a, int nq, int W) {
     // H written
     int st_out = RPD_SUCCESS;
     if (HESS) {
-        const int *rnid = reinterpret_cast<const int *>(rtr + 64 * a.rec_S);
+        const int *rnid = reinterpret_cast<const int *>(rtr + 128 * a.rec_S);
         const int H = a.H;
         int cnt = 0;
         for (int pb = 0; pb < nbk; pb += 64) {
@@ -2201,19 +2258,18 @@ int rpd_clip_plane_room(int form, int P, int V, int T, int floor) {
     // finish kernel, kClipWaves for the bisector kernel (one cell a wave)
     const size_t fin_cells = 4 * 4;
     const size_t bis_cells = 4 * size_t(form == RPD_PREC_FP64 ? kClipWaves<double, 1> : kClipWaves<float, 1>);
-    const size_t bis_pl = form == RPD_PREC_FP64 ? 32 : 16;  // the bisector kernel's planes, in the test precision
     for (int p = std::min(floor, 255); p > P; --p)
         if (finish_cell_lds(form, p, V, T, false) * fin_cells <= kLdsPerCu &&
-            finish_wave_lds(p, S, 0, bis_pl) * bis_cells <= kLdsPerCu)
+            cells_wave_lds(form, p, S) * bis_cells <= kLdsPerCu)
             return p;
     return P;
 }
 
-// header | P planes | 64 S vertex triples | P plane neighbours (int)
+// header | P planes | 64 S vertex triples, 64 S adjacency words | P plane neighbours (int)
 size_t rpd_clip_record_bytes(int form, int P, int V) {
     const int S = V <= 64 ? 1 : (V <= 128 ? 2 : 4);
     const size_t pl = plane_bytes(form);
-    return (sizeof(RecHeader) + size_t(P) * pl + 4 * 64 * size_t(S) + 4 * size_t(P) + 15) & ~size_t(15);
+    return (sizeof(RecHeader) + size_t(P) * pl + 8 * 64 * size_t(S) + 4 * size_t(P) + 15) & ~size_t(15);
 }
 
 static int make_args(int form, const ClipLaunch &L, ClipArgs &a) {
@@ -2266,7 +2322,7 @@ static int make_args(int form, const ClipLaunch &L, ClipArgs &a) {
     a.rs_out = L.rs_out;
     a.rs_out_stride = L.rs_out_stride;
     a.rs_base = L.rs_base;
-    a.rs_in = form == RPD_PREC_FP64 ? L.rs_in : nullptr;
+    a.rs_in = form != RPD_PREC_FP32 ? L.rs_in : nullptr;
     a.rs_in_stride = L.rs_in_stride;
     a.rs_in_P = L.rs_in_P;
     a.rslot = L.rslot;
@@ -2293,20 +2349,20 @@ int rpd_launch_cells(hipStream_t st, int form, const ClipLaunch &L) {
     const int S = L.V <= 64 ? 1 : (L.V <= 128 ? 2 : 4);
     // kernel A: the bisector loop of every cell
     {
-        const size_t stride = finish_wave_lds(L.P, S, 0, form == RPD_PREC_FP64 ? 32 : 16);  // planes in R
+        const size_t stride = cells_wave_lds(form, L.P, S);
         a.lds_stride = int(stride);
         // one wave per workgroup: each cell's wave starts and ends on its own
-        const int wpb = 1;
-        const unsigned blocks = unsigned((L.n_ids + wpb - 1) / wpb);
-        const size_t shm = stride * wpb;
+        const unsigned blocks = unsigned(L.n_ids);
+        const dim3 tb(64);
+        const size_t shm = stride;
 #define RPD_CLIP_A1(R, RP, F, B)                                                      \
     do {                                                                              \
         if (S == 1)                                                                   \
-            clip_cells_kernel<R, RP, F, 1, B><<<blocks, dim3(64 * wpb), shm, st>>>(a);\
+            clip_cells_kernel<R, RP, F, 1, B><<<blocks, tb, shm, st>>>(a);            \
         else if (S == 2)                                                              \
-            clip_cells_kernel<R, RP, F, 2, B><<<blocks, dim3(64 * wpb), shm, st>>>(a);\
+            clip_cells_kernel<R, RP, F, 2, B><<<blocks, tb, shm, st>>>(a);            \
         else                                                                          \
-            clip_cells_kernel<R, RP, F, 4, B><<<blocks, dim3(64 * wpb), shm, st>>>(a);\
+            clip_cells_kernel<R, RP, F, 4, B><<<blocks, tb, shm, st>>>(a);            \
     } while (0)
 #define RPD_CLIP_A(R, RP, F)              \
     do {                                  \

@@ -16,11 +16,17 @@ __device__ __forceinline__ int lane_id() {
     return __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
 }
 
-__device__ __forceinline__ uint64_t ballot(bool p) { return __ballot(p); }
+// The lanes where p holds.  (Of one comparison it is the comparison's own
+// mask; a compound condition costs a select and another comparison, so
+// conditions are combined as masks: ballot(x) & ballot(y) & m.)
+__device__ __forceinline__ uint64_t ballot(bool p) { return __builtin_amdgcn_ballot_w64(p); }
 
-// number of set bits of m strictly below this lane
-__device__ __forceinline__ int mbcnt(uint64_t m) {
-    return __builtin_amdgcn_mbcnt_hi(uint32_t(m >> 32), __builtin_amdgcn_mbcnt_lo(uint32_t(m), 0u));
+// whether this lane's bit of the wave-uniform mask m is set
+__device__ __forceinline__ bool in_mask(uint64_t m) { return __builtin_amdgcn_inverse_ballot_w64(m); }
+
+// base plus the number of set bits of m strictly below this lane
+__device__ __forceinline__ int mbcnt(uint64_t m, int base = 0) {
+    return __builtin_amdgcn_mbcnt_hi(uint32_t(m >> 32), __builtin_amdgcn_mbcnt_lo(uint32_t(m), uint32_t(base)));
 }
 
 __device__ __forceinline__ int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
@@ -116,6 +122,20 @@ template <typename T>
 __device__ __forceinline__ T wave_min(T v) {
     return rlane(wave_incl_scan_op(v, T(INFINITY), [](T a, T b) { return a < b ? a : b; }), 63);
 }
+// Maximum over the wave of values >= 0 (their bits order as unsigned integers,
+// whose maximum takes one DPP instruction a step).
+__device__ __forceinline__ float wave_max_pos(float v) {
+    uint32_t x = __float_as_uint(v);
+    x = max(x, uint32_t(__builtin_amdgcn_update_dpp(0, int(x), kDppRowShr1, 0xf, 0xf, true)));
+    x = max(x, uint32_t(__builtin_amdgcn_update_dpp(0, int(x), kDppRowShr2, 0xf, 0xf, true)));
+    x = max(x, uint32_t(__builtin_amdgcn_update_dpp(0, int(x), kDppRowShr4, 0xf, 0xf, true)));
+    x = max(x, uint32_t(__builtin_amdgcn_update_dpp(0, int(x), kDppRowShr8, 0xf, 0xf, true)));
+    x = max(x, uint32_t(__builtin_amdgcn_update_dpp(0, int(x), kDppRowBcast15, 0xa, 0xf, true)));
+    x = max(x, uint32_t(__builtin_amdgcn_update_dpp(0, int(x), kDppRowBcast31, 0xc, 0xf, true)));
+    return __uint_as_float(rlane(x, 63));
+}
+__device__ __forceinline__ double wave_max_pos(double v) { return wave_max(v); }
+
 // exclusive prefix sum across the wave
 __device__ __forceinline__ int wave_excl_scan(int v) {
     return wave_incl_scan_op(v, 0, [](int a, int b) { return a + b; }) - v;

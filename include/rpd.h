@@ -52,7 +52,7 @@ enum rpd_status {
 enum rpd_precision {
     RPD_PREC_FP64 = 0,   /* all-FP64 clip + integration (USE_DOUBLE build)    */
     RPD_PREC_MIXED = 1,  /* FP32 seed-local clip with a certified error filter;
-                            flagged cells recomputed in FP64; FP64 moment
+                            flagged tests decided in FP64; FP64 moment
                             accumulation across domain pieces                */
     RPD_PREC_FP32 = 2    /* FP32 seed-local clip, no filter, no FP64 redo     */
 };
@@ -192,7 +192,9 @@ typedef struct {
                                        loop kernel / restriction+integration */
     int32_t status_hist[RPD_STATUS_NUM];  /* final status per cell           */
     int32_t passes;                 /* clip passes run                       */
-    int32_t fallback_cells;         /* cells recomputed in FP64 (mixed form) */
+    int32_t fallback_cells;         /* cells recomputed in FP64 (mixed form:
+                                       those a test decided in place does not
+                                       settle)                               */
     int32_t final_K, final_P, final_V, final_T;
     int32_t dim;                    /* kNN grid resolution                   */
     int32_t queued_first;           /* pass 1 cells that reached the finish
