@@ -710,11 +710,12 @@ struct RecHeader {
 //
 // Minimum waves per SIMD the bisector kernel is compiled for (one vertex slot
 // per lane): occupancy pays more than the few registers the compiler then
-// spills, all in the code of open tests (FP64 7 waves, 71 VGPRs; mixed 8, 64
-// VGPRs; FP32 form 8, 50; mixed at 7 waves 2% slower).  Wider cells (S > 1,
+// spills, all in the code of open tests.  At 8 waves the compiler has 78 scalar
+// registers and spills more of them than at 7 (94): mixed 1.16 against 1.10 ms,
+// 1M cospherical seeds 7.9 against 7.6, FP64 the same.  Wider cells (S > 1,
 // re-queue passes) are left unconstrained.
 template <typename R, int S>
-constexpr int kClipWaves = S > 1 ? 1 : (sizeof(R) == 8 ? 7 : 8);
+constexpr int kClipWaves = S > 1 ? 1 : 7;
 
 template <typename R, typename RP, bool FILTER, int S, bool BATCH>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kClipWaves<R, S>)))
@@ -2444,7 +2445,11 @@ int rpd_launch_finish(hipStream_t st, int form, const ClipLaunch &L, int nq, int
     const bool vox = L.vox && form != RPD_PREC_FP32 && a.apex_mode == 1;
     // waves per cell from the cells that share the device: this queue's and
     // those of finish kernels running beside it (the Hessian variant: one wave
-    // per cell)
+    // per cell).  Every wave of a cell sets the cell up anew, so one wave is
+    // best as soon as the queue fills the chip (4,096 waves at 4 a SIMD;
+    // 20,676 blue-noise cells at two waves 0.28, at one 0.21 ms); 8 up to half
+    // of that (947 cells that meet hundreds of strips: 8 waves 0.91, 2 waves
+    // 0.98 ms for the solve).
     const int64_t load = int64_t(nq) + std::max(beside, 0);
     auto launch = [&](bool vx, bool hs) -> int {
         const size_t wstride =
@@ -2453,7 +2458,7 @@ int rpd_launch_finish(hipStream_t st, int form, const ClipLaunch &L, int nq, int
             (hs ? hessian_wave_lds(L.P + (vx ? 1 : 0), S) : 0);
         const size_t kLdsMax = lds_limit();
         if (finish_cell_stride(a.T, 1) + wstride > kLdsMax) return RPD_E_LIMIT;
-        int W = hs || a.count_only || load > 32768 ? 1 : (load <= 2048 ? 8 : (load <= 8192 ? 4 : 2));
+        int W = hs || a.count_only || load > 4096 ? 1 : (load <= 2048 ? 8 : 2);
         while (W > 1 && finish_cell_stride(a.T, W) + W * wstride > kLdsMax) W >>= 1;
         a.lds_stride = int(wstride);
         a.cell_stride = int(finish_cell_stride(a.T, W));
