@@ -32,6 +32,7 @@
 #include <hip/hip_runtime.h>
 
 #include <chrono>
+#include <cmath>
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
@@ -80,6 +81,20 @@ constexpr int kPinCounters = 16;
 constexpr int kPinBinFlag = kPinCounters - 4;
 // smallest triangle cap a solve uses
 constexpr int kTriangleFloor = 256;
+// With strips, the cap goes by the size of a cell, (g^3 / n)^(2/3) voxels
+// squared: 12 strips for each, up to kStripFloor.  Where cells are many voxels
+// wide the largest meet several hundred (1,000 seeds, sphere in 96^3: 96 of 947
+// cells above 256, which took two further passes: solve 910 -> 570 us; a batch
+// of 16 requests of up to 100,003 seeds in 96^3: 638, a pass of 1.6 ms, 10.06
+// -> 9.28 ms).  Where cells are small the room only costs residency: 1M seeds,
+// torus in 128^3, finish kernel of 16 cells a CU 0.53 ms (FP64 0.60), with room
+// for 1,024 strips 0.58 (0.71).
+constexpr int kStripFloor = 1024;
+constexpr double kStripsPerArea = 12.0;
+static int strip_floor(int g, int64_t n) {
+    const double w2 = std::cbrt(double(g) * g * g / double(n)) * std::cbrt(double(g) * g * g / double(n));
+    return int(std::min<double>(kStripFloor, std::max<double>(kTriangleFloor, kStripsPerArea * w2)));
+}
 // smallest neighbour cap a solve uses (with re-queue passes, FP64 and mixed)
 constexpr int kNeighbourFloor = 64;
 // the plane cap a solve raises a lower one to, where that costs no residency
@@ -960,7 +975,16 @@ static int solve_impl(rpd_ctx *c, rpd_domain *dom, const rpd_params *prm, rpd_st
     // with re-queue passes allowed: without them an overflow is the answer.
     if (prm->max_extra_steps > 0 && !hess && P < kPlaneFloor)
         P = rpd_clip_plane_room(form0, P, V, std::max(T, kTriangleFloor), kPlaneFloor);
-    T = std::max(T, std::min(kTriangleFloor, rpd_clip_max_T(form0, P, V, hess)));
+    // the restriction goes by voxel faces when every domain has them
+    bool vox = !dom || dom->dev.vface;
+    int t_floor = dom ? strip_floor(dom->dev.g, n) : kTriangleFloor;
+    for (const auto &q : c->batch) {
+        if (!q.dom) continue;
+        vox = vox && q.dom->dev.vface;
+        t_floor = std::max(t_floor, strip_floor(q.dom->dev.g, q.n));
+    }
+    if (!vox || form0 == RPD_PREC_FP32) t_floor = kTriangleFloor;
+    T = std::max(T, std::min(t_floor, rpd_clip_max_T(form0, P, V, hess)));
     // Likewise the vertex cap is the room of the vertex slots it needs
     // (64 per slot): a cap below it saves nothing.
     V = V <= 64 ? 64 : (V <= 128 ? 128 : 256);
@@ -1050,9 +1074,6 @@ static int solve_impl(rpd_ctx *c, rpd_domain *dom, const rpd_params *prm, rpd_st
                                    : nullptr;
     };
     const DomainDev *dd = dom ? &dom->dev : nullptr;
-    // the restriction goes by voxel faces when every domain has them
-    bool vox = !dd || dd->vface;
-    for (const auto &q : c->batch) vox = vox && (!q.dom || q.dom->dev.vface);
     // the weight minimum the kernels subtract, and whether there are walls
     // (border seeds): known here unless the minima are new (then at settle)
     double wmin = 0;
@@ -1378,8 +1399,8 @@ static int solve_impl(rpd_ctx *c, rpd_domain *dom, const rpd_params *prm, rpd_st
         // the restriction (a flagged test, or the triangle, vertex or plane
         // cap met by the cone clips).  Their bisector loop is done,
         // certified, and in pass 1's records, which are the FP64 form's
-        // records too, so the FP64 finish kernel runs over those records
-        // with the grown caps; a full FP64 recomputation would rebuild the
+        // records too, so the finish kernel runs over those records again,
+        // with the grown caps (the FP64 one for flagged tests); a full FP64 recomputation would rebuild the
         // same records first.  The FP32 form's records hold FP32 planes (16
         // bytes, a different layout): its cells take the full pass.
         if (ch.from_finish && ch.k == 0 && ch.n_res == 0 && ch.n_scr > 0 && form0 != RPD_PREC_FP32 &&
@@ -1389,7 +1410,9 @@ static int solve_impl(rpd_ctx *c, rpd_domain *dom, const rpd_params *prm, rpd_st
             ch.pz = Pass{};
             ch.pz.slot = ch.sl;
             ch.pz.index = 1;
-            ch.pz.form = RPD_PREC_FP64;
+            // Overflows alone need no FP64 tests: the same form again, so a
+            // cell's bits do not depend on the cap that it first met.
+            ch.pz.form = n_exact > 0 ? RPD_PREC_FP64 : form0;
             ch.pz.n_ids = ch.n_scr;
             ch.pz.caps[0] = ch.cap.K;
             ch.pz.caps[1] = ch.cap.P;
@@ -1414,7 +1437,7 @@ static int solve_impl(rpd_ctx *c, rpd_domain *dom, const rpd_params *prm, rpd_st
             L.dcnt = dcnt_of(1);
             ch.pz.finish_only = true;
             if (hipEventRecord(c->ev[ch.sl][1], s) != hipSuccess) return RPD_E_DEVICE;
-            int r = rpd_launch_finish(s, RPD_PREC_FP64, L, int(ch.n_scr), 0);
+            int r = rpd_launch_finish(s, ch.pz.form, L, int(ch.n_scr), 0);
             if (r != RPD_OK) return r;
             if (hipEventRecord(c->ev[ch.sl][3], s) != hipSuccess || !copy_counts(ch.nxt, s)) return RPD_E_DEVICE;
             ch.end = s;

@@ -593,15 +593,14 @@ struct WaveCell {
 
 // LDS of one wave: nvs[64S] and 64 spare words | adj[64S] (8 bytes) | chunk /
 // cone planes cpl[64] | go_out flags[16] | planes[P] | plane sources src[P]
-// (int32) | nxt, sta, end [P rounded up to 16 each] | tu[T] (finish kernel) |
-// tail (finish kernel: triangle corners tcor[16][9] and the vertex copy; mixed
-// bisector kernel: FP64 planes).  The parts of a fixed size come first: their
+// (int32) | nxt, sta, end [P rounded up to 16 each] | tail (finish kernel:
+// triangle corners tcor[16][9] and the vertex copy; mixed bisector kernel: FP64
+// planes).  The parts of a fixed size come first: their
 // addresses are constants in the bisector kernel.
 __host__ __device__ constexpr size_t up16(size_t b) { return (b + 15) & ~size_t(15); }
 template <typename R, typename RP, bool FILTER, int S, typename PS>
-__device__ __forceinline__ void bind_lds(char *L, int P, int T, WaveCell<R, RP, FILTER, S, PS> &c,
-                                         int **src = nullptr, int **tu = nullptr, Pl<PS> **cpl = nullptr,
-                                         int **goo = nullptr, char **tail = nullptr) {
+__device__ __forceinline__ void bind_lds(char *L, int P, WaveCell<R, RP, FILTER, S, PS> &c, int **src = nullptr,
+                                         Pl<PS> **cpl = nullptr, int **goo = nullptr, char **tail = nullptr) {
     c.nvs = reinterpret_cast<uint32_t *>(L);
     size_t off = 4 * (64 * S + 64);
     c.adj = reinterpret_cast<uint2 *>(L + off);
@@ -618,8 +617,6 @@ __device__ __forceinline__ void bind_lds(char *L, int P, int T, WaveCell<R, RP, 
     c.sta = c.nxt + up16(P);
     c.end = c.sta + up16(P);
     off += 3 * up16(P);
-    if (tu) *tu = reinterpret_cast<int *>(L + off);
-    off += up16(4 * size_t(T));
     if (tail) *tail = L + off;
 }
 
@@ -635,30 +632,34 @@ constexpr size_t kVtxRecBytes = 40;  // sizeof(VtxRec<double>), the larger one
 
 // LDS bytes of one wave (pl: bytes of one stored plane; tail: bytes after the
 // cone planes and flags)
-__host__ __device__ constexpr size_t wave_lds(int P, int S, int T, size_t pl, size_t tail) {
+__host__ __device__ constexpr size_t wave_lds(int P, int S, size_t pl, size_t tail) {
     return 4 * (64 * size_t(S) + 64) + 8 * 64 * size_t(S) + 64 * pl + 64 + up16(P * pl) + up16(4 * size_t(P)) +
-           3 * up16(P) + up16(4 * size_t(T)) + up16(tail);
+           3 * up16(P) + up16(tail);
 }
 // (the bisector kernel; planes in the test precision, the mixed form with room
 // for the FP64 planes)
 __host__ __device__ constexpr size_t cells_wave_lds(int form, int P, int S) {
-    return wave_lds(P, S, 0, form == RPD_PREC_FP64 ? 32 : 16, form == RPD_PREC_MIXED ? 32 * size_t(P) : 0);
+    return wave_lds(P, S, form == RPD_PREC_FP64 ? 32 : 16, form == RPD_PREC_MIXED ? 32 * size_t(P) : 0);
 }
 // (corners: the finish kernel's triangle corners and vertex copy)
-__host__ __device__ constexpr size_t finish_wave_lds(int P, int S, int T, size_t pl, bool corners = false) {
-    return wave_lds(P, S, T, pl, corners ? 16 * 9 * 8 + 64 * size_t(S) * kVtxRecBytes : 0);
+__host__ __device__ constexpr size_t finish_wave_lds(int P, int S, size_t pl, bool corners = false) {
+    return wave_lds(P, S, pl, corners ? 16 * 9 * 8 + 64 * size_t(S) * kVtxRecBytes : 0);
 }
 // The voxel form of the finish kernel: room for one plane more (a strip has
 // five cone planes, a triangle four), no corners, the vertex copy in the test
 // precision (vr bytes each).
-__host__ __device__ constexpr size_t finish_vox_wave_lds(int P, int S, int T, size_t vr) {
-    return wave_lds(P + 1, S, T, 32, 64 * size_t(S) * vr);
+__host__ __device__ constexpr size_t finish_vox_wave_lds(int P, int S, size_t vr) {
+    return wave_lds(P + 1, S, 32, 64 * size_t(S) * vr);
 }
 // LDS the Hessian adds to a finish-kernel wave: per plane 4 sums, per vertex
 // slot 4 values and a plane id
 __host__ __device__ constexpr size_t hessian_wave_lds(int P, int S) {
     return 32 * size_t(P) + 8 * size_t(P) + 64 * 32;
 }
+
+// Units (strips of voxel faces, triangles) that a wave of the finish kernel
+// tests at once: a lane per cone plane, 5 or 4 a unit.
+constexpr int kStripBatch = 12, kTriBatch = 16;
 
 // Power bisector of the seed S0 and neighbour B in the seed-local frame
 // (CCNewPlane, ConvexCell.cl:314-333): unit normal -b/|b|, offset
@@ -732,7 +733,7 @@ void clip_cells_kernel(ClipArgs a) {
     Pl<R> *chunk = nullptr;  // planes of the current 64 neighbours
     int *src = nullptr;
     char *tail = nullptr;
-    bind_lds(lds_raw, a.P, 0, c, &src, nullptr, &chunk, nullptr, &tail);
+    bind_lds(lds_raw, a.P, c, &src, &chunk, nullptr, &tail);
     c.P = a.P;
     c.V = a.V;
     c.lane = lane;
@@ -1195,13 +1196,13 @@ __device__ __forceinline__ uint64_t box_near(int x, int y, int z, const int *mn,
 //
 // W waves share one cell (W = 1 for large queues, up to 8 for the short
 // re-queue passes whose run time is set by their heaviest cell): every wave
-// rebuilds the cell and its triangle list, wave w takes the triangles
-// k = w, w + W, ...  Each triangle starts from the same backed-up cell, so its
-// contribution does not depend on which wave computes it.  The contributions
-// are summed in increasing k, one after another: with W = 1 as they come (a
-// wave-uniform running sum), with W > 1 from LDS, where the waves put them by
-// triangle index, by wave 0.  Both make the same additions, so the result of
-// a cell is the same bit for bit for every W and every batch it is in.
+// rebuilds the cell and its list of triangles (or strips), the batches of 16
+// (12) units go round the waves.  Each unit starts from the same backed-up
+// cell, so its contribution does not depend on which wave computes it.  A
+// batch's contributions are added in increasing order, and the batches' sums
+// in the batches' order: with W = 1 as they come, with W > 1 from LDS by wave
+// 0.  Both make the same additions, so the result of a cell is the same bit
+// for bit for every W and every packed batch it is in.
 //
 // Cone planes are built lane-parallel, 16 triangles x 4 planes per batch.  A
 // triangle one of whose four planes removes every vertex of the cell with a
@@ -1220,9 +1221,11 @@ __device__ __forceinline__ uint64_t box_near(int x, int y, int z, const int *mn,
 // planes have two components, and five clips and one integration serve two
 // triangles or more.  The apex lies in the middle of the cell's box, not in
 // its first voxel: cones then only meet the cell where the boundary does.
-// Alone on 1M seeds / torus 128^3 the launch went from 1.43 to 0.87 ms
-// (mixed); 1,000 seeds in a sphere at 96^3, where a cell meets hundreds of
-// triangles, from 3.3 to 1.16 ms for the whole solve.
+// 1M seeds, torus in 128^3, mixed: the launch went from 1.43 to 0.67 ms with
+// strips, later to 0.61, and to 0.53 ms with batches of equal work and with
+// integer and folded wave reductions (VALU-bound: about 1,500 instructions a
+// cell before those); 1,000 seeds, sphere in 96^3, where a cell meets hundreds
+// of triangles: the whole solve from 3.3 to 1.16 ms with strips.
 // ---------------------------------------------------------------------------
 template <typename R, typename RP, bool FILTER, int S, bool HESS, bool BATCH, bool VOX>
 // 4 waves per SIMD for S = 1 (128 VGPRs): measured at 1M seeds against 5 and
@@ -1244,16 +1247,18 @@ void finish_cells_kernel(ClipArgs a, int nq, int W) {
 
     char *cell_l = lds_raw + size_t(ci) * a.cell_stride;
     int *fails = reinterpret_cast<int *>(cell_l);                  // [W][2]
-    double4 *contrib = reinterpret_cast<double4 *>(cell_l + 64);  // [T], W > 1 only
+    // the units (triangles or strips) that the cell meets: collected by every
+    // wave of the cell for itself, all writing the same values
+    int *tu = reinterpret_cast<int *>(cell_l + 64);  // [T]
+    double *bsum = reinterpret_cast<double *>(cell_l + 64 + up16(4 * size_t(a.T)));  // [4] a batch, W > 1 only
     WaveCell<R, RP, FILTER, S> c;
-    int *tu = nullptr, *goo = nullptr;
+    int *goo = nullptr;
     Pl<RP> *cpl = nullptr;
     char *tail = nullptr;
     // VOX: a strip's fifth cone plane has room of its own, so that no cap is
     // met earlier than with triangles
     const int P = VOX ? a.P + 1 : a.P;
-    bind_lds(lds_raw + size_t(cpb) * a.cell_stride + size_t(wv) * a.lds_stride, P, a.T, c, nullptr, &tu,
-             &cpl, &goo, &tail);
+    bind_lds(lds_raw + size_t(cpb) * a.cell_stride + size_t(wv) * a.lds_stride, P, c, nullptr, &cpl, &goo, &tail);
     double *tcor = reinterpret_cast<double *>(tail);  // (not VOX)
     c.P = P;
     c.V = a.V;
@@ -1314,8 +1319,9 @@ void finish_cells_kernel(ClipArgs a, int nq, int W) {
         }
     };
 
-    // ---- integration (CCExportBaryVolume): factor/6 * (volume, moments) of
-    // the current cell in the local frame, FP64 wave sums --------------------
+    // ---- integration (CCExportBaryVolume): factor/6 * (moments, volume) of
+    // the current cell in the local frame, FP64 wave sums; every lane of row r
+    // (16 lanes) of the wave returns component r (x, y, z moment, volume) ----
     const RP vol_eps2 = sizeof(RP) == 8 ? RP(1e-12) : RP(1e-6);  // voronoi.cpp:919-922
     // the vertex copy of the skip tests
     VtxRec<R> *vtx = reinterpret_cast<VtxRec<R> *>(VOX ? tcor : tcor + 16 * 9);
@@ -1335,7 +1341,7 @@ void finish_cells_kernel(ClipArgs a, int nq, int W) {
         for (int i = lane; i < nbk; i += 64) hmask[i] = 0;
         wsync();
     }
-    auto integrate = [&](double factor) -> double4 {
+    auto integrate = [&](double factor) -> double {
         RP sw = 0, sx = 0, sy = 0, sz = 0;
 #pragma unroll
         for (int s = 0; s < S; ++s) {
@@ -1505,48 +1511,54 @@ void finish_cells_kernel(ClipArgs a, int nq, int W) {
                 }
             }
         }
-        const double f = factor / 6.0;
-        return make_double4(f * wave_sum(double(sx)), f * wave_sum(double(sy)), f * wave_sum(double(sz)),
-                            f * wave_sum(double(sw)));
+        return factor / 6.0 * wave_sum4(double(sx), double(sy), double(sz), double(sw));
     };
 
     // ---- restriction to the domain grid --------------------------------------
     bool add_volume = true;
     int ntri = 0;
-    double rcell = 0;  // largest distance of a vertex from the seed (FP64)
+    double rcell = 0;  // largest distance of a vertex from the seed (upper bound)
     double P0x = 0, P0y = 0, P0z = 0;  // apex, global frame
     int vmx[3] = {0, 0, 0};
     if (a.g > 0) {
         const int g = a.g;
         const double vs = a.vs;
-        double bmn[3] = {1000.0, 1000.0, 1000.0}, bmx[3] = {0.0, 0.0, 0.0}, vr2 = 0.0;
+        // Box of the vertices in voxels, starting from 1000 and 0 as the
+        // reference does, (int)(b / vs) clamped to [0, g-1]
+        // (ConvexCell.cl:939-940); clamped in floating point first so that
+        // inf/NaN from a degenerate vertex cannot produce an out-of-grid range.
+        // Division, clamp and truncation are monotone, so the wave reduces
+        // integers: the position in 1/1024 voxels, whose high bits are the
+        // voxel, as unsigned maxima of one DPP instruction a step (7 FP64
+        // reductions had been 245 of the 1,500 VALU instructions of a cell;
+        // 1M seeds, torus in 128^3).
+        const double top = double(g - 1), x1000 = 1000.0 / vs;
+        uint32_t qn[3] = {0, 0, 0}, qx[3] = {0, 0, 0};  // (lows complemented)
+        double vr2 = 0.0;
 #pragma unroll
         for (int s = 0; s < S; ++s) {
             if (!in_mask(c.valid[s])) continue;
             RP lx, ly, lz;
             vertex_rp(s, lx, ly, lz);
             vr2 = fmax(vr2, double(lx) * double(lx) + double(ly) * double(ly) + double(lz) * double(lz));
-            const double gx = S0.x + double(lx), gy = S0.y + double(ly), gz = S0.z + double(lz);
-            bmn[0] = fmin(bmn[0], gx);
-            bmn[1] = fmin(bmn[1], gy);
-            bmn[2] = fmin(bmn[2], gz);
-            bmx[0] = fmax(bmx[0], gx);
-            bmx[1] = fmax(bmx[1], gy);
-            bmx[2] = fmax(bmx[2], gz);
+            const double v[3] = {(S0.x + double(lx)) / vs, (S0.y + double(ly)) / vs, (S0.z + double(lz)) / vs};
+#pragma unroll
+            for (int d = 0; d < 3; ++d) {
+                qn[d] = max(qn[d], ~uint32_t(fmin(fmax(fmin(x1000, v[d]), 0.0), top) * 1024.0));
+                qx[d] = max(qx[d], uint32_t(fmin(fmax(v[d], 0.0), top) * 1024.0));
+            }
         }
-        rcell = sqrt(wave_max(vr2));
+        // (rounded up: an upper bound is what the tests below need)
+        rcell = sqrt(double(wave_max_pos(float(vr2) * (1.0f + 0x1.0p-22f))));
         int vmn[3];
         double mid[3];  // middle of the box, in voxels (VOX)
 #pragma unroll
         for (int d = 0; d < 3; ++d) {
-            // (int)(b / vs) clamped to [0, g-1] (ConvexCell.cl:939-940); the
-            // clamp is applied in floating point first so that inf/NaN from a
-            // degenerate vertex cannot produce an out-of-grid range
-            const double lo = wave_min(bmn[d]) / vs, hi = wave_max(bmx[d]) / vs;
-            vmn[d] = uni(int(fmin(fmax(lo, 0.0), double(g - 1))));
-            vmx[d] = uni(int(fmin(fmax(hi, 0.0), double(g - 1))));
+            const uint32_t lo = ~wave_max_u32(qn[d]), hi = wave_max_u32(qx[d]);
+            vmn[d] = int(lo >> 10);
+            vmx[d] = int(hi >> 10);
             if (vmx[d] < vmn[d]) vmx[d] = vmn[d];
-            mid[d] = fmin(fmax(0.5 * (lo + hi), double(vmn[d])), double(vmx[d]));
+            mid[d] = fmin(fmax((double(lo) + double(hi)) * (0.5 / 1024.0), double(vmn[d])), double(vmx[d]));
         }
         if constexpr (VOX) {
             // ---- voxel domain: every boundary face is a voxel face, and the
@@ -1829,7 +1841,7 @@ void finish_cells_kernel(ClipArgs a, int nq, int W) {
             add_volume = in_domain == 2;
         }
     }
-    double4 cadd = make_double4(0.0, 0.0, 0.0, 0.0);
+    double cadd = 0.0;  // the whole cell's term
     if (add_volume && sub == 0) cadd = integrate(1.0);
 
     // The reference clips the triangles in increasing id order and stops at
@@ -1837,7 +1849,9 @@ void finish_cells_kernel(ClipArgs a, int nq, int W) {
     // id.  Triangles are visited here in list order, so after a failure only
     // triangles of smaller id are still clipped.
     int fail_t = 0x7fffffff, fail_st = 0;
-    double sm = 0, sx = 0, sy = 0, sz = 0;  // running sums of the contributions (W = 1; wave-uniform)
+    constexpr int kUB = VOX ? kStripBatch : kTriBatch;  // units of a batch
+    const int nbat = (ntri + kUB - 1) / kUB;
+    double sum = 0.0;  // running sum of the batches (W = 1)
     if (ntri > 0) {
         // backup (ConvexCell.cl:692-715): the vertex registers, their adjacency
         // and the plane count
@@ -1850,7 +1864,6 @@ void finish_cells_kernel(ClipArgs a, int nq, int W) {
             return nullptr;
         };
         constexpr int kPl = VOX ? 5 : 4;    // cone planes of a unit (strip or triangle)
-        constexpr int kUB = VOX ? 12 : 16;  // units of a batch
         constexpr uint64_t kUm = (1ull << kPl) - 1;
         const bool may_skip = c.nb_plane + kPl <= P && nvalid + (VOX ? 8 : 6) <= a.V;
         const double lx0 = P0x - S0.x, ly0 = P0y - S0.y, lz0 = P0z - S0.z;
@@ -1873,12 +1886,17 @@ void finish_cells_kernel(ClipArgs a, int nq, int W) {
         // removes every vertex (kept side n.y + d >= 0), with a margin far
         // above the rounding of d and rcell.
         const double rsk = rcell * (1.0 + 1e-9) + 1e-9;
-        // VOX: wave sub takes the batches sub, sub + W, ... of 12 strips in
-        // list order; else the triangles sub, sub + W, ...
-        for (int jb = VOX ? sub * kUB : sub; jb < ntri; jb += kUB * W) {
+        // Batch jb is the units jb, jb + nbat, ...: neighbours in the list, of
+        // which either all or none are near the cell, go to different batches,
+        // so that the batches and with them the waves that take them (sub, sub
+        // + W, ...) have about the same number to clip.  Which units a batch
+        // has does not depend on W, and the batches' sums are added in order:
+        // the result is the same for every W.
+        for (int jb = sub; jb < nbat; jb += W) {
+            double bs = 0.0;  // the batch's sum
             // cone planes, lane = kPl * unit + plane
             const int i = VOX ? lane / 5 : lane >> 2, f = VOX ? lane - 5 * i : lane & 3;
-            const int k = VOX ? (i < kUB ? jb + i : ntri) : jb + W * i;
+            const int k = i < kUB ? jb + nbat * i : ntri;
             Pl<RP> pl{RP(0), RP(0), RP(0), RP(0)};
             uint64_t gom = 0;  // VOX: strips whose region counts positive, at lane 5 * strip
             // VOX: the strip in the local frame, across axis ax at rc, from
@@ -2098,19 +2116,15 @@ void finish_cells_kernel(ClipArgs a, int nq, int W) {
             uint32_t todo = 0;
 #pragma unroll
             for (int t = 0; t < kUB; ++t)
-                if (jb + (VOX ? t : W * t) < ntri && ((skipm >> (kPl * t)) & kUm) == 0) todo |= 1u << t;
-            if (W > 1 && lane < kUB && jb + (VOX ? lane : W * lane) < ntri)
-                contrib[jb + (VOX ? lane : W * lane)] = make_double4(0.0, 0.0, 0.0, 0.0);
-            // in increasing k: the running sums add the contributions in order
-            // (a skipped triangle adds +0, which leaves them unchanged)
+                if (jb + nbat * t < ntri && ((skipm >> (kPl * t)) & kUm) == 0) todo |= 1u << t;
+            // in increasing order (a skipped unit adds nothing)
             while (todo) {
                 const int t = __builtin_ctz(todo);
                 todo &= todo - 1;
-                const int kk = jb + (VOX ? t : W * t);
+                const int kk = jb + nbat * t;
                 // (a strip stands for several triangles: its place in the list)
                 const int tid = VOX ? kk : uni(tu[kk]);
                 if (tid > fail_t) continue;
-                double4 ck = make_double4(0.0, 0.0, 0.0, 0.0);
                 int res = kNoClip;
                 // each cone plane read from LDS just before its clip: the four
                 // held at once would take 32 registers through the clips
@@ -2130,21 +2144,17 @@ void finish_cells_kernel(ClipArgs a, int nq, int W) {
                     fail_t = tid;
                     fail_st = res;
                 } else if (res != RPD_EMPTY_CELL) {
-                    ck = integrate((VOX ? ((gom >> (kPl * t)) & 1) != 0 : goo[t] != 0) ? 1.0 : -1.0);
+                    bs += integrate((VOX ? ((gom >> (kPl * t)) & 1) != 0 : goo[t] != 0) ? 1.0 : -1.0);
                 }
                 c = bk;
 #pragma unroll
                 for (int s = 0; s < S; ++s) c.adj[s * 64 + lane] = bk_adj[s];
                 wsync();
-                if (W == 1) {
-                    sx = uni(sx + ck.x);
-                    sy = uni(sy + ck.y);
-                    sz = uni(sz + ck.z);
-                    sm = uni(sm + ck.w);
-                } else if (lane == 0) {
-                    contrib[kk] = ck;
-                }
             }
+            if (W == 1)
+                sum += bs;
+            else if ((lane & 15) == 0)
+                bsum[4 * jb + (lane >> 4)] = bs;
             wsync();  // the next batch overwrites cpl / goo
         }
     }
@@ -2170,18 +2180,11 @@ void finish_cells_kernel(ClipArgs a, int nq, int W) {
         fail(fs);
         return;
     }
-    // fixed summation order: the contributions in increasing k, then the
-    // whole-cell term
-    if (W > 1) {
-        for (int k = 0; k < ntri; ++k) {
-            const double4 q = contrib[k];
-            sx += q.x;
-            sy += q.y;
-            sz += q.z;
-            sm += q.w;
-        }
-    }
-    const double acc_m = cadd.w + sm, acc_x = cadd.x + sx, acc_y = cadd.y + sy, acc_z = cadd.z + sz;
+    // fixed summation order: the batches in order, then the whole-cell term
+    if (W > 1)
+        for (int k = 0; k < nbat; ++k) sum += bsum[4 * k + (lane >> 4)];
+    sum += cadd;
+    const double acc_x = rlane(sum, 0), acc_y = rlane(sum, 16), acc_z = rlane(sum, 32), acc_m = rlane(sum, 48);
     // Hessian entries (ConvexCell.cl:1133-1151): the record's planes towards
     // a seed whose face keeps more than 0.2 of area, in plane order, with the
     // neighbours' original indices; more than H: hessian_overflow, the first
@@ -2233,7 +2236,9 @@ using namespace rpd;
 // Bytes of one stored plane: the planes of the FP64 and mixed forms are FP64.
 static size_t plane_bytes(int form) { return form == RPD_PREC_FP32 ? 16 : 32; }
 
-// LDS bytes a workgroup may use on the current device.
+// LDS of a gfx950 CU, shared by the resident workgroups
+constexpr size_t kLdsPerCu = 160 * 1024;
+
 // LDS a workgroup may use on the current device (asked once per device)
 static size_t lds_limit() {
     static std::atomic<int> cached[64];
@@ -2246,14 +2251,16 @@ static size_t lds_limit() {
     return size_t(v);
 }
 
-// LDS of the cell part of a finish-kernel workgroup: fail slots, then, when
-// W > 1 waves share the cell, its contributions (T).
-static size_t finish_cell_stride(int T, int W) { return W > 1 ? (64 + 32 * size_t(T) + 15) & ~size_t(15) : 64; }
+// LDS of the cell part of a finish-kernel workgroup: fail slots, the units it
+// meets (T) and, when W > 1 waves share the cell, the sums of its batches.
+static size_t finish_cell_stride(int T, int W) {
+    return 64 + up16(4 * size_t(T)) + (W > 1 ? 32 * ((size_t(T) + kStripBatch - 1) / kStripBatch) : 0);
+}
 
 // LDS of one finish-kernel cell handled by a single wave.
 static size_t finish_cell_lds(int form, int P, int V, int T, bool hess) {
     const int S = V <= 64 ? 1 : (V <= 128 ? 2 : 4);
-    return finish_cell_stride(T, 1) + finish_wave_lds(P, S, T, plane_bytes(form), true) +
+    return finish_cell_stride(T, 1) + finish_wave_lds(P, S, plane_bytes(form), true) +
            (hess ? hessian_wave_lds(P, S) : 0);
 }
 
@@ -2272,8 +2279,6 @@ int rpd_clip_max_T(int form, int P, int V, bool hess) {
 }
 
 int rpd_clip_plane_room(int form, int P, int V, int T, int floor) {
-    // LDS of a gfx950 CU, shared by the resident workgroups
-    constexpr size_t kLdsPerCu = 160 * 1024;
     const int S = V <= 64 ? 1 : (V <= 128 ? 2 : 4);
     if (S != 1) return P;
     // cells per CU at the kernels' residency: 4 waves per SIMD for the
@@ -2469,13 +2474,13 @@ int rpd_launch_finish(hipStream_t st, int form, const ClipLaunch &L, int nq, int
     // per cell).  Every wave of a cell sets the cell up anew, so one wave is
     // best as soon as the queue fills the chip (4,096 waves at 4 a SIMD;
     // 20,676 blue-noise cells at two waves 0.28, at one 0.21 ms); 8 up to half
-    // of that (947 cells that meet hundreds of strips: 8 waves 0.91, 2 waves
-    // 0.98 ms for the solve).
+    // of that (947 cells that meet hundreds of strips, those above 256 in
+    // further passes: 8 waves 0.91, 2 waves 0.98 ms for the solve).
     const int64_t load = int64_t(nq) + std::max(beside, 0);
     auto launch = [&](bool vx, bool hs) -> int {
         const size_t wstride =
-            (vx ? finish_vox_wave_lds(L.P, S, a.T, form == RPD_PREC_FP64 ? sizeof(VtxRec<double>) : sizeof(VtxRec<float>))
-                : finish_wave_lds(L.P, S, a.T, pl, true)) +
+            (vx ? finish_vox_wave_lds(L.P, S, form == RPD_PREC_FP64 ? sizeof(VtxRec<double>) : sizeof(VtxRec<float>))
+                : finish_wave_lds(L.P, S, pl, true)) +
             (hs ? hessian_wave_lds(L.P + (vx ? 1 : 0), S) : 0);
         const size_t kLdsMax = lds_limit();
         if (finish_cell_stride(a.T, 1) + wstride > kLdsMax) return RPD_E_LIMIT;

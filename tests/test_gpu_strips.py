@@ -69,3 +69,22 @@ def test_strips_match_triangle_lists(rpd, ctx, kind, g, n, prec):
     assert (~same).sum() <= n // 100
     assert np.abs(f0[same][:, :, 3] - f1[same][:, :, 3]).max() <= 1e-10 * face
     assert np.abs(f0[same][:, :, :3] - f1[same][:, :, :3]).max() <= 1e-10 * face * 1000.0
+
+
+@pytest.mark.parametrize("prec", [0, 1])
+@pytest.mark.parametrize("g,n", [(24, 6), (16, 40)])
+def test_strip_cap_does_not_change_cells(rpd, ctx, g, n, prec):
+    """Cells that meet more strips than the cap take a pass over the same
+    records with a larger one; batches of strips are the same for every cap
+    and number of waves: the same bits as with room from the beginning."""
+    x = rpd.generate_seeds(rpd.SEEDS_UNIFORM, n, seed=n, wmax=0.0)
+    dom = ctx.domain(rpd.Grid.voxels(_mask("random", g)))
+    ctx.set_seeds(x)
+    out = []
+    for T in (10, 1500, 20000):
+        st = ctx.solve(dom, K=64, P=60, V=64, T=T, precision=prec)
+        out.append((ctx.moments(), ctx.status(), st["passes"]))
+    dom.close()
+    assert out[0][2] > out[2][2], "no cell above the smallest cap"
+    for m, s, _ in out[1:]:
+        assert np.array_equal(m, out[0][0]) and np.array_equal(s, out[0][1])
