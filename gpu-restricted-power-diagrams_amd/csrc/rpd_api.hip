@@ -171,7 +171,8 @@ struct rpd_ctx {
     hipEvent_t evb[2] = {};    // a solve's binning (and weight minima): before, after
     int *pin = nullptr;        // kPinWords pinned host words
     int *pin_dev = nullptr;    // their device address (nullptr: copies go through the copy engine)
-    double *pin_red = nullptr;  // 2 x kWminBlocks pinned doubles: per-block weight minima
+    double *pin_red = nullptr;  // pinned: the weight minima
+    double *pin_red_dev = nullptr;  // its device address (nullptr: a copy)
     // smallest weight of the non-border seeds and of all seeds, for the
     // current seeds (valid once wmin_ok)
     bool wmin_ok = false;
@@ -193,16 +194,17 @@ static void *g_scratch_ptr[kMaxDevices] = {};
 
 namespace {
 
-// Up to 12 device int arrays cleared by one single-workgroup launch: the
-// counters a solve starts from, without one fill launch each.
+// Up to 16 device int arrays cleared by one launch: the counters a solve
+// starts from, without one fill launch each.
 struct ZeroSet {
-    int *p[12];
-    int n[12];
+    int *p[16];
+    int n[16];
     int k;
 };
-__global__ void zero_words_kernel(ZeroSet z) {
+constexpr int kZeroBlocks = 256;
+__global__ __launch_bounds__(256) void zero_words_kernel(ZeroSet z) {
     for (int j = 0; j < z.k; ++j)
-        for (int i = int(threadIdx.x); i < z.n[j]; i += int(blockDim.x)) z.p[j][i] = 0;
+        for (int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x; i < z.n[j]; i += kZeroBlocks * 256) z.p[j][i] = 0;
 }
 
 // Resolves the current device's copy of `scratch` once (device current).
@@ -240,56 +242,57 @@ int set_err(rpd_ctx *c, int code, const char *fmt, ...) {
         if (r_ != RPD_OK) return set_err(ctx, r_, "%s failed (%d)", what, r_); \
     } while (0)
 
-// per-block minimum of the weights of non-border seeds (out[b]) and of all
-// weights (out[gridDim.x + b])
+// The minimum weight of the non-border seeds and of all seeds, to out[0],
+// out[1] (for the kernels queued before the host has them) and to out_host
+// (mapped host memory, unless null).  part: the blocks' minima; the block that
+// finishes last (left: zero before the launch) reduces them.
 __global__ __launch_bounds__(256) void wmin_kernel(const double4 *__restrict__ seeds, int64_t n,
-                                                   double *__restrict__ out) {
+                                                   double *__restrict__ part, int *__restrict__ left,
+                                                   double *__restrict__ out, double *__restrict__ out_host) {
     __shared__ double red[2][256];
+    __shared__ int last;
     double m = INFINITY, ma = INFINITY;
+    auto reduce = [&]() {
+        red[0][threadIdx.x] = m;
+        red[1][threadIdx.x] = ma;
+        __syncthreads();
+        for (int o = 128; o > 0; o >>= 1) {
+            if (threadIdx.x < o) {
+                red[0][threadIdx.x] = fmin(red[0][threadIdx.x], red[0][threadIdx.x + o]);
+                red[1][threadIdx.x] = fmin(red[1][threadIdx.x], red[1][threadIdx.x + o]);
+            }
+            __syncthreads();
+        }
+    };
     for (int64_t i = blockIdx.x * int64_t(blockDim.x) + threadIdx.x; i < n; i += int64_t(gridDim.x) * blockDim.x) {
         const double w = seeds[i].w;
         if (w > RPD_NO_CELL_LIMITS) m = fmin(m, w);
         ma = fmin(ma, w);
     }
-    red[0][threadIdx.x] = m;
-    red[1][threadIdx.x] = ma;
-    __syncthreads();
-    for (int o = 128; o > 0; o >>= 1) {
-        if (threadIdx.x < o) {
-            red[0][threadIdx.x] = fmin(red[0][threadIdx.x], red[0][threadIdx.x + o]);
-            red[1][threadIdx.x] = fmin(red[1][threadIdx.x], red[1][threadIdx.x + o]);
-        }
-        __syncthreads();
-    }
+    reduce();
     if (threadIdx.x == 0) {
-        out[blockIdx.x] = red[0][0];
-        out[gridDim.x + blockIdx.x] = red[1][0];
+        __hip_atomic_store(part + blockIdx.x, red[0][0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(part + gridDim.x + blockIdx.x, red[1][0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __threadfence();
+        last = atomicAdd(left, 1) == int(gridDim.x) - 1;
     }
-}
-
-// The two minima over the nb blocks' partials (non-border seeds, all seeds)
-// to out[0], out[1]: for the kernels queued before the host has them.
-__global__ __launch_bounds__(256) void wmin_final_kernel(const double *__restrict__ part, int nb,
-                                                         double *__restrict__ out) {
-    __shared__ double red[2][256];
-    double m = INFINITY, ma = INFINITY;
-    for (int i = threadIdx.x; i < nb; i += 256) {
-        m = fmin(m, part[i]);
-        ma = fmin(ma, part[nb + i]);
-    }
-    red[0][threadIdx.x] = m;
-    red[1][threadIdx.x] = ma;
     __syncthreads();
-    for (int o = 128; o > 0; o >>= 1) {
-        if (threadIdx.x < o) {
-            red[0][threadIdx.x] = fmin(red[0][threadIdx.x], red[0][threadIdx.x + o]);
-            red[1][threadIdx.x] = fmin(red[1][threadIdx.x], red[1][threadIdx.x + o]);
-        }
-        __syncthreads();
+    if (!last) return;
+    __threadfence();
+    m = ma = INFINITY;
+    for (int i = int(threadIdx.x); i < int(gridDim.x); i += 256) {
+        m = fmin(m, __hip_atomic_load(part + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+        ma = fmin(ma, __hip_atomic_load(part + gridDim.x + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
     }
+    reduce();
     if (threadIdx.x == 0) {
         out[0] = red[0][0];
         out[1] = red[1][0];
+        if (out_host) {
+            out_host[0] = red[0][0];
+            out_host[1] = red[1][0];
+            __threadfence_system();
+        }
     }
 }
 
@@ -558,7 +561,8 @@ __global__ __launch_bounds__(256) void mark_neighbours_kernel(const char *__rest
 }
 
 // Bins the seeds in key precision prec unless they are.  With pending set
-// the binning is only queued: *pending tells whether it was, and the caller,
+// the binning is only queued, in scratch that the caller has prepared and
+// cleared (rpd_bin_prepare): *pending tells whether it was, and the caller,
 // once it has synchronised the stream, finishes it with finish_binning.
 int ensure_binning(rpd_ctx *c, int prec, bool *pending = nullptr) {
     if (pending) *pending = false;
@@ -574,7 +578,7 @@ int ensure_binning(rpd_ctx *c, int prec, bool *pending = nullptr) {
     if (pending) {
         RPDCHK(c,
                rpd_bin_seeds_async(c->stream, c->seeds.as<double4>(), n, prec, dim, c->bin_scratch,
-                                   c->pin + kPinBinFlag, c->perm.as<int>(), c->counters.as<int>(), c->stored.ptr,
+                                   c->pin + kPinBinFlag, c->pin_dev ? c->pin_dev + kPinBinFlag : nullptr, c->perm.as<int>(), c->counters.as<int>(), c->stored.ptr,
                                    c->stored64.as<double4>()),
                "binning");
         *pending = true;
@@ -671,11 +675,14 @@ int rpd_create_streams(int device, int n_streams, rpd_ctx **out) {
         (void)hipGetLastError();
         c->pin_dev = nullptr;
     }
-    if (hipHostMalloc(reinterpret_cast<void **>(&c->pin_red), 2 * kWminBlocks * sizeof(double),
-                      hipHostMallocDefault) != hipSuccess) {
+    if (hipHostMalloc(reinterpret_cast<void **>(&c->pin_red), 2 * sizeof(double), hipHostMallocDefault) != hipSuccess) {
         c->pin_red = nullptr;
         rpd_destroy(c);
         return RPD_E_DEVICE;
+    }
+    if (hipHostGetDevicePointer(reinterpret_cast<void **>(&c->pin_red_dev), c->pin_red, 0) != hipSuccess) {
+        (void)hipGetLastError();
+        c->pin_red_dev = nullptr;
     }
     *out = c;
     return RPD_OK;
@@ -992,31 +999,8 @@ static int solve_impl(rpd_ctx *c, rpd_domain *dom, const rpd_params *prm, rpd_st
     st.n = n;
     auto t_start = std::chrono::steady_clock::now();
 
-    HIPCHK(c, hipEventRecord(c->evb[0], c->stream));
-    // The weight minima of new seeds (over the non-border seeds, and over
-    // all, whose sign tells whether there are walls) and the binning are
-    // queued, and nothing waits for them here: the cover test reads the
-    // minima on the device (wdev), and the host reads them, with the
-    // binning's crowded-cell flag, after the solve's first wait (settle
-    // below), which the kNN launch has already overlapped.
-    const bool new_wmin = !batch && prm->security_mode == 0 && !c->wmin_ok;
-    const double *wdev = nullptr;
-    if (new_wmin) {
-        RPDCHK(c, c->wred.ensure((2 * kWminBlocks + 2) * sizeof(double)), "alloc wred");
-        double *wr = c->wred.as<double>();
-        wmin_kernel<<<kWminBlocks, 256, 0, c->stream>>>(c->seeds.as<double4>(), n, wr);
-        wmin_final_kernel<<<1, 256, 0, c->stream>>>(wr, kWminBlocks, wr + 2 * kWminBlocks);
-        HIPCHK(c, hipMemcpyAsync(c->pin_red, wr + 2 * kWminBlocks, 2 * sizeof(double), hipMemcpyDeviceToHost,
-                                 c->stream));
-        wdev = wr + 2 * kWminBlocks;
-    }
-    if (batch) {
-        if (c->bin_prec != kprec) return set_err(c, RPD_E_STATE, "rpd_solve_batch: binned in another precision");
-    }
-    bool bin_pending = false;
-    if (!batch) RPDCHK(c, ensure_binning(c, kprec, &bin_pending), "binning");
-    HIPCHK(c, hipEventRecord(c->evb[1], c->stream));
-
+    if (batch && c->bin_prec != kprec)
+        return set_err(c, RPD_E_STATE, "rpd_solve_batch: binned in another precision");
     RPDCHK(c, c->out.ensure(size_t(n) * 32), "alloc out");
     RPDCHK(c, c->status.ensure(size_t(n) * 4), "alloc status");
     RPDCHK(c, c->kused.ensure(size_t(n) * 4), "alloc kused");
@@ -1031,8 +1015,13 @@ static int solve_impl(rpd_ctx *c, rpd_domain *dom, const rpd_params *prm, rpd_st
     RPDCHK(c, c->cnt.ensure(64), "alloc cnt");
     for (auto &b : c->pb) RPDCHK(c, b.q.ensure(2 * sizeof(int)), "alloc queue counter");
     RPDCHK(c, c->pb1.q.ensure(2 * sizeof(int)), "alloc queue counter");
+    const bool new_wmin = !batch && prm->security_mode == 0 && !c->wmin_ok;
+    RPDCHK(c, c->wred.ensure((2 * kWminBlocks + 3) * sizeof(double)), "alloc wred");
+    int *wleft = reinterpret_cast<int *>(c->wred.as<double>() + 2 * kWminBlocks + 2);
+    HIPCHK(c, hipEventRecord(c->evb[0], c->stream));
     // The counters the solve starts from, cleared by one launch: the final
-    // status histogram's, every failure list's and the queue counters.  A
+    // status histogram's, every failure list's and the queue counters, and
+    // what the weight minima, the binning and the cover test count with.  A
     // list stays "fresh" (known zero) until a pass writes it; clearing a fresh
     // one is skipped.
     bool fresh_fl[6];
@@ -1049,9 +1038,46 @@ static int solve_impl(rpd_ctx *c, rpd_domain *dom, const rpd_params *prm, rpd_st
             z.p[z.k] = b->q.as<int>();
             z.n[z.k++] = 2;
         }
-        zero_words_kernel<<<1, 64, 0, c->stream>>>(z);
+        if (new_wmin) {
+            z.p[z.k] = wleft;
+            z.n[z.k++] = 1;
+        }
+        if (!batch && c->bin_prec != kprec) {
+            RPDCHK(c, rpd_bin_prepare(c->stream, n, rpd_knn_dim(n), c->bin_scratch, &z.p[z.k], &z.n[z.k]),
+                   "alloc binning");
+            ++z.k;
+        }
+        if (dom || batch) {
+            RPDCHK(c, rpd_cover_prepare(int(std::max<size_t>(c->batch.size(), 1)), n, c->cull_scratch, &z.p[z.k],
+                                        &z.n[z.k]),
+                   "alloc domain cover");
+            ++z.k;
+        }
+        zero_words_kernel<<<kZeroBlocks, 256, 0, c->stream>>>(z);
         HIPCHK(c, hipGetLastError());
     }
+    // The weight minima of new seeds (over the non-border seeds, and over
+    // all, whose sign tells whether there are walls) and the binning are
+    // queued, and nothing waits for them here: the cover test reads the
+    // minima on the device (wdev), and the host reads them, with the
+    // binning's crowded-cell flag, after the solve's first wait (settle
+    // below), which the kNN launch has already overlapped.
+    const double *wdev = nullptr;
+    if (new_wmin) {
+        double *wr = c->wred.as<double>();
+        double *host = c->pin_red_dev;
+        wmin_kernel<<<kWminBlocks, 256, 0, c->stream>>>(c->seeds.as<double4>(), n, wr, wleft, wr + 2 * kWminBlocks,
+                                                        host);
+        HIPCHK(c, hipGetLastError());
+        if (!host)
+            HIPCHK(c, hipMemcpyAsync(c->pin_red, wr + 2 * kWminBlocks, 2 * sizeof(double), hipMemcpyDeviceToHost,
+                                     c->stream));
+        wdev = wr + 2 * kWminBlocks;
+    }
+    bool bin_pending = false;
+    if (!batch) RPDCHK(c, ensure_binning(c, kprec, &bin_pending), "binning");
+    HIPCHK(c, hipEventRecord(c->evb[1], c->stream));
+
     c->hess_H = hess ? prm->H : 0;
     c->hess_HC = hess ? prm->HC : 1;
     if (hess) {
@@ -1156,7 +1182,7 @@ static int solve_impl(rpd_ctx *c, rpd_domain *dom, const rpd_params *prm, rpd_st
         HIPCHK(c, hipEventRecord(c->ev[1][0], c->stream));
         RPDCHK(c,
                rpd_cover_skip(c->stream, cov.data(), int(cov.size()), n, c->cull_scratch, c->ids1.as<int>(), cover_pin,
-                              &cover_count),
+                              c->pin_dev ? c->pin_dev + (cover_pin - c->pin) : nullptr, &cover_count),
                "domain cover");
         HIPCHK(c, hipEventRecord(c->ev[1][1], c->stream));
         ids1 = c->ids1.as<int>();

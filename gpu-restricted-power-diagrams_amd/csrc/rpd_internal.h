@@ -77,11 +77,15 @@ int rpd_bin_seeds(hipStream_t st, const double4 *seeds, int64_t n, int prec, int
 int rpd_bin_seeds_in(hipStream_t st, const double4 *seeds, int64_t n, int prec, int dim, void *scratch,
                      size_t scratch_bytes, int *flag_host, int *perm, int *counters, void *stored, double4 *stored64);
 size_t rpd_bin_scratch_bytes(hipStream_t st, int64_t n, int dim);
-// The binning queued without a wait: the crowded-cell flag goes to
-// flag_pinned (pinned host memory).  Once the stream has been synchronised, a
-// set flag calls for rpd_bin_seeds_redo (the crowded-cell path; it waits).
+// The binning queued without a wait, in the scratch that rpd_bin_prepare has
+// sized and whose words [zero, zero + zero_words) the caller has cleared: the
+// crowded-cell flag goes to flag_pinned (pinned host memory; flag_dev: its
+// device address, or null, then it is copied).  Once the stream has been
+// synchronised, a set flag calls for rpd_bin_seeds_redo (the crowded-cell
+// path; it waits).
+int rpd_bin_prepare(hipStream_t st, int64_t n, int dim, DevBuf &scratch, int **zero, int *zero_words);
 int rpd_bin_seeds_async(hipStream_t st, const double4 *seeds, int64_t n, int prec, int dim, DevBuf &scratch,
-                        int *flag_pinned, int *perm, int *counters, void *stored, double4 *stored64);
+                        int *flag_pinned, int *flag_dev, int *perm, int *counters, void *stored, double4 *stored64);
 int rpd_bin_seeds_redo(hipStream_t st, const double4 *seeds, int64_t n, int prec, int dim, DevBuf &scratch,
                        int *perm, void *stored, double4 *stored64);
 // Several diagrams in one launch (a packed batch): request r owns the
@@ -250,13 +254,16 @@ struct CoverArgs {
     int *status;
     int *kused;
 };
-// Writes the outputs of the skipped cells and the stored ids of the others,
-// ascending, to ids_out (n_total entries); *n_out = their number.  The
-// requests' ranges lie in [0, n_total).  count_dev null: synchronizes st.
-// Else nothing waits: *count_dev receives the device copy of the number and
-// *n_out (pinned host memory) is written by a copy queued on st.
+// Scratch for nreq requests over n_total ids, whose words [zero, zero +
+// zero_words) are to be cleared before rpd_cover_skip.
+int rpd_cover_prepare(int nreq, int64_t n_total, DevBuf &scratch, int **zero, int *zero_words);
+// Queues: the outputs of the skipped cells, and the stored ids of the others,
+// ascending, to ids_out (n_total entries).  The requests' ranges follow each
+// other and cover [0, n_total).  *count_dev receives the device copy of the
+// number of ids, *n_out (pinned host memory; n_out_dev: its device address, or
+// null, then it is copied) the number.
 int rpd_cover_skip(hipStream_t st, const CoverArgs *reqs, int nreq, int64_t n_total, DevBuf &scratch, int *ids_out,
-                   int *n_out, const int **count_dev = nullptr);
+                   int *n_out, int *n_out_dev, const int **count_dev);
 
 // Bytes of one queued-cell record.
 size_t rpd_clip_record_bytes(int form, int P, int V);

@@ -3,8 +3,8 @@
 // Replaces the reference's KNearests (knearests.cpp:48-315) and
 // build_knearests (knearests.cl:36-78):
 //   * binning: cell = floor(p * dim / 1000) per axis (knearests.cpp:35-46) in
-//     the seed precision; a stable radix sort of (cell, original index) gives
-//     the permutation, so seeds keep original order inside a cell;
+//     the seed precision; the permutation is the stable sort by cell (a
+//     counting sort), so seeds keep original order inside a cell;
 //   * query: one wavefront per query seed over the sorted array.  Candidate
 //     cells are visited shell by shell (Chebyshev rings with per-axis bounds);
 //     each row of a shell is one contiguous range of the sorted array, so the
@@ -19,7 +19,6 @@
 #include <hip/hip_runtime.h>
 #include <cstring>
 #include <rocprim/device/device_radix_sort.hpp>
-#include <rocprim/device/device_scan.hpp>
 
 #include "rpd_internal.h"
 #include "rpd_wave.h"
@@ -62,37 +61,99 @@ __global__ void bin_cells_kernel(const double4 *__restrict__ seeds, int64_t n, i
     rank[i] = atomicAdd(&counts[c], 1);  // a place in the cell, in no set order
 }
 
-// Seed i to its place in its cell's range of perm (order within a cell set
-// by the atomics; sort_cells_kernel fixes it).
-__global__ void scatter_cells_kernel(const int *__restrict__ cell, const int *__restrict__ rank, int64_t n,
-                                     const int *__restrict__ counters, int *__restrict__ perm) {
-    const int64_t i = blockIdx.x * int64_t(blockDim.x) + threadIdx.x;
-    if (i >= n) return;
-    perm[counters[cell[i]] + rank[i]] = int(i);
+// The cells' counts to the ends before them: an exclusive prefix sum, one
+// workgroup a tile of 2,048 (the library's takes two launches).
+constexpr int kScanTile = 2048;
+__global__ __launch_bounds__(256) void scan_cells_kernel(const int *__restrict__ counts, int64_t m,
+                                                         int *__restrict__ counters,
+                                                         unsigned long long *__restrict__ state,
+                                                         int *__restrict__ ticket) {
+    __shared__ int tile_s, before_s, wsum[4];
+    const int lane = lane_id(), wv = uni(int(threadIdx.x >> 6));
+    if (threadIdx.x == 0) tile_s = atomicAdd(ticket, 1);
+    __syncthreads();
+    const int tile = uni(tile_s);
+    const int64_t i0 = int64_t(tile) * kScanTile + int64_t(threadIdx.x) * 8;
+    int v[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+    if (i0 + 8 <= m) {
+        const int4 x = *reinterpret_cast<const int4 *>(counts + i0), y = *reinterpret_cast<const int4 *>(counts + i0 + 4);
+        v[0] = x.x, v[1] = x.y, v[2] = x.z, v[3] = x.w;
+        v[4] = y.x, v[5] = y.y, v[6] = y.z, v[7] = y.w;
+    } else {
+        for (int j = 0; j < 8; ++j)
+            if (i0 + j < m) v[j] = counts[i0 + j];
+    }
+    int sum = 0;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) sum += v[j];
+    int at = wave_excl_scan(sum);
+    if (lane == 63) wsum[wv] = at + sum;
+    __syncthreads();
+    if (wv == 0) {
+        const int b = tile_prefix(state, tile, wsum[0] + wsum[1] + wsum[2] + wsum[3]);
+        if (lane == 0) before_s = b;
+    }
+    __syncthreads();
+    at += before_s;
+    for (int w = 0; w < wv; ++w) at += wsum[w];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        if (i0 + j < m) counters[i0 + j] = at;
+        at += v[j];
+    }
 }
 
-// Each cell's range of perm in increasing original index, so that perm is
-// the stable sort of the seeds by cell.  Ranges longer than kSortRun are
-// left to the caller (*big set): a clustered input goes to the radix sort.
+// Seed i to its cell's range of members, in the order set by the atomics.
+__global__ void scatter_cells_kernel(const int *__restrict__ cell, const int *__restrict__ rank, int64_t n,
+                                     const int *__restrict__ counters, int *__restrict__ members) {
+    const int64_t i = blockIdx.x * int64_t(blockDim.x) + threadIdx.x;
+    if (i >= n) return;
+    members[counters[cell[i]] + rank[i]] = int(i);
+}
+
+// Each member to its final place: perm is the stable sort of the seeds by
+// cell, so a seed's place in its cell's range is the number of members with a
+// smaller index.  The seed's copies go with it: one launch, where sorting each
+// cell's range by one thread and gathering afterwards took two (100,000 seeds:
+// 11.4 + 3.7 us).  A thread takes a member, not a seed: its reads of the seed
+// are scattered, but its writes stay within a cell of its neighbours' (by
+// seed, 1M seeds: weight minima and binning 156 us, by member 127).  Ranges longer than kSortRun
+// are left in members' order and *big is set (and big_host, mapped host
+// memory, unless null): a clustered input goes to the radix sort.
 constexpr int kSortRun = 32;
-__global__ void sort_cells_kernel(const int *__restrict__ counters, int64_t nc, int *__restrict__ perm,
-                                  int *__restrict__ big) {
-    const int64_t c = blockIdx.x * int64_t(blockDim.x) + threadIdx.x;
-    if (c >= nc) return;
+template <typename R>
+__global__ __launch_bounds__(256) void place_seeds_kernel(const double4 *__restrict__ seeds, int64_t n,
+                                                          const int *__restrict__ cell,
+                                                          const int *__restrict__ counters,
+                                                          const int *__restrict__ members, int *__restrict__ perm,
+                                                          typename Vec4T<R>::T *__restrict__ stored,
+                                                          double4 *__restrict__ stored64, int *__restrict__ big,
+                                                          int *__restrict__ big_host) {
+    const int64_t p = blockIdx.x * int64_t(blockDim.x) + threadIdx.x;
+    if (p >= n) return;
+    const int i = members[p];
+    const double4 s = seeds[i];
+    const int c = cell[i];
     const int lo = counters[c], hi = counters[c + 1];
+    int at = lo;
     if (hi - lo > kSortRun) {
+        at = int(p);
         *big = 1;
-        return;
-    }
-    for (int j = lo + 1; j < hi; ++j) {
-        const int v = perm[j];
-        int k = j - 1;
-        while (k >= lo && perm[k] > v) {
-            perm[k + 1] = perm[k];
-            --k;
+        if (big_host) {
+            *big_host = 1;
+            __threadfence_system();
         }
-        perm[k + 1] = v;
+    } else {
+        for (int j = lo; j < hi; ++j) at += members[j] < i ? 1 : 0;
     }
+    perm[at] = i;
+    typename Vec4T<R>::T v;
+    v.x = R(s.x);
+    v.y = R(s.y);
+    v.z = R(s.z);
+    v.w = R(s.w);
+    stored[at] = v;
+    if (stored64) stored64[at] = s;
 }
 
 __global__ void iota_kernel(int *__restrict__ out, int64_t n) {
@@ -746,41 +807,48 @@ int rpd_knn_dim(int64_t n) {
 // a counting sort whose cells are then sorted by index, or, when a cell holds
 // more than kSortRun seeds, a radix sort of (cell, index).  Waits for the
 // stream.
-// Bytes of binning scratch for n seeds on a dim^3 grid (0 on a HIP error).
-// Layout: cell_in, cell_out, rank / orig (n ints each), counts (dim^3 + 1),
-// the crowded-cell flag, rocPRIM temporary storage.
-
-// Layout of the binning's scratch: cell ids (in, out), ranks, per-cell
-// counts, the crowded-cell flag, the library sort's / scan's temporary.
+//
+// Layout of the binning's scratch: cell ids, members (cell ids out in the radix
+// sort), ranks, per-cell counts, and, cleared with them, the crowded-cell flag,
+// the scan's ticket and its tiles' words; the library sort's temporary.
 struct BinLayout {
-    size_t off_cell_out, off_rank, off_counts, off_flag, off_tmp, sort_bytes, scan_bytes, need;
+    size_t off_cell_out, off_rank, off_counts, off_flag, off_state, off_tmp, sort_bytes, need;
     unsigned end_bit;
 };
-static int bin_layout(hipStream_t st, int64_t n, int dim, BinLayout &b) {
-    const int64_t nc = int64_t(dim) * dim * dim;
+static int bin_layout(hipStream_t st, int64_t n, int64_t nc, BinLayout &b) {
     const size_t bytes_cell = size_t(n) * 4;
     int *null_i = nullptr;
     b.end_bit = 1;
     while ((int64_t(1) << b.end_bit) < nc) ++b.end_bit;
-    b.sort_bytes = b.scan_bytes = 0;
+    b.sort_bytes = 0;
     if (rocprim::radix_sort_pairs(nullptr, b.sort_bytes, null_i, null_i, null_i, null_i, n, 0u, b.end_bit, st) !=
-        hipSuccess)
-        return RPD_E_DEVICE;
-    if (rocprim::exclusive_scan(nullptr, b.scan_bytes, null_i, null_i, 0, size_t(nc + 1), rocprim::plus<int>(), st) !=
         hipSuccess)
         return RPD_E_DEVICE;
     b.off_cell_out = bytes_cell;
     b.off_rank = 2 * bytes_cell;
-    b.off_counts = 3 * bytes_cell;
+    b.off_counts = (3 * bytes_cell + 255) & ~size_t(255);
     b.off_flag = (b.off_counts + size_t(nc + 1) * 4 + 255) & ~size_t(255);
-    b.off_tmp = b.off_flag + 256;
-    b.need = b.off_tmp + std::max(b.sort_bytes, b.scan_bytes) + 256;
+    b.off_state = b.off_flag + 16;
+    b.off_tmp = (b.off_state + size_t((nc + kScanTile) / kScanTile) * 8 + 255) & ~size_t(255);
+    b.need = b.off_tmp + b.sort_bytes + 256;
     return RPD_OK;
 }
 
+static int64_t cells_of(int dim) { return int64_t(dim) * dim * dim; }
+
+// Bytes of binning scratch for n seeds on a dim^3 grid (0 on a HIP error).
 size_t rpd_bin_scratch_bytes(hipStream_t st, int64_t n, int dim) {
     BinLayout b;
-    return bin_layout(st, n, dim, b) == RPD_OK ? b.need : 0;
+    return bin_layout(st, n, cells_of(dim), b) == RPD_OK ? b.need : 0;
+}
+
+int rpd_bin_prepare(hipStream_t st, int64_t n, int dim, DevBuf &scratch, int **zero, int *zero_words) {
+    BinLayout b;
+    if (bin_layout(st, n, cells_of(dim), b) != RPD_OK) return RPD_E_DEVICE;
+    if (scratch.ensure(b.need) != RPD_OK) return RPD_E_NOMEM;
+    *zero = reinterpret_cast<int *>(static_cast<char *>(scratch.ptr) + b.off_counts);
+    *zero_words = int((b.off_tmp - b.off_counts) / 4);
+    return RPD_OK;
 }
 
 template <typename R>
@@ -791,40 +859,42 @@ static void gather_seeds(hipStream_t st, const double4 *seeds, const int *perm, 
     gather_seeds_kernel<R><<<nb, tb, 0, st>>>(seeds, perm, n, static_cast<typename Vec4T<R>::T *>(stored), stored64);
 }
 
-// Queues the binning; its crowded-cell flag is copied to flag_host.
+// Queues the binning; its crowded-cell flag is copied to flag_host, or, with
+// flag_dev, the flag's device address, written there (clear until then).
+// zeroed: the scratch's counts and what follows them are cleared already.
 static int bin_queue(hipStream_t st, const double4 *seeds, int64_t n, int prec, int dim, void *scratch_ptr,
-                     size_t scratch_bytes, int *flag_host, int *perm, int *counters, void *stored,
-                     double4 *stored64) {
+                     size_t scratch_bytes, int *flag_host, int *flag_dev, bool zeroed, int *perm, int *counters,
+                     void *stored, double4 *stored64) {
     BinLayout b;
-    if (bin_layout(st, n, dim, b) != RPD_OK) return RPD_E_DEVICE;
+    const int64_t nc = cells_of(dim);
+    if (bin_layout(st, n, nc, b) != RPD_OK) return RPD_E_DEVICE;
     if (b.need > scratch_bytes) return RPD_E_LIMIT;
-    const int64_t nc = int64_t(dim) * dim * dim;
     char *base = static_cast<char *>(scratch_ptr);
-    int *cell_in = reinterpret_cast<int *>(base);
+    int *cell = reinterpret_cast<int *>(base);
+    int *members = reinterpret_cast<int *>(base + b.off_cell_out);
     int *rank = reinterpret_cast<int *>(base + b.off_rank);
     int *counts = reinterpret_cast<int *>(base + b.off_counts);
-    int *big = reinterpret_cast<int *>(base + b.off_flag);
-    void *tmp = base + b.off_tmp;
-    // the counts and the flag, which follows them, cleared at once
-    if (hipMemsetAsync(counts, 0, b.off_flag + sizeof(int) - b.off_counts, st) != hipSuccess) return RPD_E_DEVICE;
+    int *big = reinterpret_cast<int *>(base + b.off_flag), *ticket = big + 1;
+    auto *state = reinterpret_cast<unsigned long long *>(base + b.off_state);
+    if (!zeroed && hipMemsetAsync(counts, 0, b.off_tmp - b.off_counts, st) != hipSuccess) return RPD_E_DEVICE;
+    if (flag_dev) *flag_host = 0;
     const int tb = 256;
     const unsigned nb = unsigned((n + tb - 1) / tb);
     if (prec == 0)
-        bin_cells_kernel<float><<<nb, tb, 0, st>>>(seeds, n, dim, cell_in, counts, rank);
+        bin_cells_kernel<float><<<nb, tb, 0, st>>>(seeds, n, dim, cell, counts, rank);
     else
-        bin_cells_kernel<double><<<nb, tb, 0, st>>>(seeds, n, dim, cell_in, counts, rank);
-    size_t scb = b.scan_bytes;
-    if (rocprim::exclusive_scan(tmp, scb, counts, counters, 0, size_t(nc + 1), rocprim::plus<int>(), st) !=
-        hipSuccess)
-        return RPD_E_DEVICE;
-    scatter_cells_kernel<<<nb, tb, 0, st>>>(cell_in, rank, n, counters, perm);
-    sort_cells_kernel<<<unsigned((nc + tb - 1) / tb), tb, 0, st>>>(counters, nc, perm, big);
-    // gathered at once; a crowded cell (rare) sorts and gathers again
+        bin_cells_kernel<double><<<nb, tb, 0, st>>>(seeds, n, dim, cell, counts, rank);
+    scan_cells_kernel<<<unsigned((nc + kScanTile) / kScanTile), 256, 0, st>>>(counts, nc + 1, counters, state, ticket);
+    scatter_cells_kernel<<<nb, tb, 0, st>>>(cell, rank, n, counters, members);
+    // placed at once; a crowded cell (rare) sorts and gathers again
     if (prec == 0)
-        gather_seeds<float>(st, seeds, perm, n, stored, stored64);
+        place_seeds_kernel<float><<<nb, tb, 0, st>>>(seeds, n, cell, counters, members, perm,
+                                                     static_cast<float4 *>(stored), stored64, big, flag_dev);
     else
-        gather_seeds<double>(st, seeds, perm, n, stored, stored64);
-    if (hipMemcpyAsync(flag_host, big, sizeof(int), hipMemcpyDeviceToHost, st) != hipSuccess) return RPD_E_DEVICE;
+        place_seeds_kernel<double><<<nb, tb, 0, st>>>(seeds, n, cell, counters, members, perm,
+                                                      static_cast<double4 *>(stored), stored64, big, flag_dev);
+    if (!flag_dev && hipMemcpyAsync(flag_host, big, sizeof(int), hipMemcpyDeviceToHost, st) != hipSuccess)
+        return RPD_E_DEVICE;
     return hipGetLastError() == hipSuccess ? RPD_OK : RPD_E_DEVICE;
 }
 
@@ -833,7 +903,7 @@ static int bin_queue(hipStream_t st, const double4 *seeds, int64_t n, int prec, 
 static int bin_redo(hipStream_t st, const double4 *seeds, int64_t n, int prec, int dim, void *scratch_ptr,
                     int *perm, void *stored, double4 *stored64) {
     BinLayout b;
-    if (bin_layout(st, n, dim, b) != RPD_OK) return RPD_E_DEVICE;
+    if (bin_layout(st, n, cells_of(dim), b) != RPD_OK) return RPD_E_DEVICE;
     char *base = static_cast<char *>(scratch_ptr);
     int *cell_in = reinterpret_cast<int *>(base);
     int *cell_out = reinterpret_cast<int *>(base + b.off_cell_out);
@@ -863,19 +933,17 @@ int rpd_bin_seeds(hipStream_t st, const double4 *seeds, int64_t n, int prec, int
 }
 int rpd_bin_seeds_in(hipStream_t st, const double4 *seeds, int64_t n, int prec, int dim, void *scratch_ptr,
                      size_t scratch_bytes, int *flag_host, int *perm, int *counters, void *stored, double4 *stored64) {
-    const int r = bin_queue(st, seeds, n, prec, dim, scratch_ptr, scratch_bytes, flag_host, perm, counters, stored,
-                            stored64);
+    const int r = bin_queue(st, seeds, n, prec, dim, scratch_ptr, scratch_bytes, flag_host, nullptr, false, perm,
+                            counters, stored, stored64);
     if (r != RPD_OK) return r;
     if (hipStreamSynchronize(st) != hipSuccess) return RPD_E_DEVICE;
     if (*flag_host) return bin_redo(st, seeds, n, prec, dim, scratch_ptr, perm, stored, stored64);
     return RPD_OK;
 }
 int rpd_bin_seeds_async(hipStream_t st, const double4 *seeds, int64_t n, int prec, int dim, DevBuf &scratch,
-                        int *flag_pinned, int *perm, int *counters, void *stored, double4 *stored64) {
-    const size_t need = rpd_bin_scratch_bytes(st, n, dim);
-    if (need == 0) return RPD_E_DEVICE;
-    if (scratch.ensure(need) != RPD_OK) return RPD_E_NOMEM;
-    return bin_queue(st, seeds, n, prec, dim, scratch.ptr, need, flag_pinned, perm, counters, stored, stored64);
+                        int *flag_pinned, int *flag_dev, int *perm, int *counters, void *stored, double4 *stored64) {
+    return bin_queue(st, seeds, n, prec, dim, scratch.ptr, scratch.bytes, flag_pinned, flag_dev, true, perm, counters,
+                     stored, stored64);
 }
 int rpd_bin_seeds_redo(hipStream_t st, const double4 *seeds, int64_t n, int prec, int dim, DevBuf &scratch,
                        int *perm, void *stored, double4 *stored64) {

@@ -221,4 +221,34 @@ __device__ __forceinline__ uint64_t shr_lane1(uint64_t v, uint64_t first) {
 // index of the lowest set bit (m != 0)
 __device__ __forceinline__ int lowest_bit(uint64_t m) { return __ffsll((long long)m) - 1; }
 
+// Sum of the totals of the tiles before `tile`, found by one wave of the tile's
+// workgroup (decoupled lookback).  state: a zeroed word per tile, which becomes
+// (1, total), then (2, sum up to and with the tile), value in the low half:
+// one 64-bit word, so nothing else is ordered by it.  Tiles are numbered by a
+// ticket that a workgroup takes when it starts: the tiles before it have
+// started too, and post their totals without waiting for anyone, so every wait
+// ends.
+__device__ __forceinline__ int tile_prefix(unsigned long long *state, int tile, int total) {
+    const int lane = lane_id();
+    auto post = [&](unsigned long long kind, int v) {
+        if (lane == 0)
+            __hip_atomic_store(state + tile, (kind << 32) | uint32_t(v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    };
+    post(tile == 0 ? 2 : 1, total);
+    int before = 0;
+    for (int j0 = tile - 1; j0 >= 0; j0 -= 64) {
+        const int j = j0 - lane;
+        unsigned long long v = 2ull << 32;  // before the first tile: nothing
+        if (j >= 0)
+            while (((v = __hip_atomic_load(state + j, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) >> 32) == 0)
+                __builtin_amdgcn_s_sleep(1);
+        const uint64_t whole = ballot((v >> 32) == 2);
+        const int last = whole ? lowest_bit(whole) : 63;
+        before += wave_sum(lane <= last ? int(uint32_t(v)) : 0);
+        if (whole) break;
+    }
+    if (tile > 0) post(2, before + total);
+    return before;
+}
+
 }  // namespace rpd
