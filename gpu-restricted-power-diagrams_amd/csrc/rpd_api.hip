@@ -146,12 +146,11 @@ struct rpd_ctx {
     struct BatchReq {
         rpd_domain *dom = nullptr;
         int64_t base = 0, n = 0;
-        double wmin = 0, wall = 0;
         int dim = 0;
         int64_t coff = 0;
     };
     std::vector<BatchReq> batch;
-    DevBuf req_desc, knn_req, req_of;
+    DevBuf req_desc, knn_req, req_of, req_wmin;
     // pass work buffers: up to three passes may run at once, one per stream;
     // pass 1's own (its records keep the states of its resumable cells and
     // serve the finish failures' first pass)
@@ -1161,10 +1160,12 @@ static int solve_impl(rpd_ctx *c, rpd_domain *dom, const rpd_params *prm, rpd_st
         return ca;
     };
     if (batch) {
-        for (const auto &q : c->batch)
+        for (const auto &q : c->batch) {
             cov.push_back(cover_of(q.dom ? &q.dom->dev : nullptr, c->counters.as<int>() + q.coff, q.dim, q.base, q.n,
-                                   prm->security_mode == 0 && q.wmin < INFINITY ? q.wmin : 0.0,
-                                   prm->security_mode != 0 || q.wall <= RPD_NO_CELL_LIMITS));
+                                   0.0, prm->security_mode != 0));
+            // (the device tells walls from none)
+            cov.back().wdev = c->req_wmin.as<double>() + 2 * (cov.size() - 1);
+        }
     } else if (dd) {
         // new minima: the device tells walls (no cover test) from none
         cov.push_back(cover_of(dd, c->counters.as<int>(), c->dim, 0, n, wmin, new_wmin ? false : border_seeds));
@@ -1823,14 +1824,6 @@ int rpd_solve_batch(rpd_ctx *c, int32_t nreq, rpd_domain *const *doms, const dou
         q.n = ns[r];
         q.dim = rpd_knn_dim(q.n);
         q.coff = coff;
-        // weight minima over the non-border seeds and over all, on the host
-        q.wmin = q.wall = INFINITY;
-        const double *x = xyzw[r];
-        for (int64_t i = 0; i < q.n; ++i) {
-            const double w = x[4 * i + 3];
-            if (w > RPD_NO_CELL_LIMITS) q.wmin = std::min(q.wmin, w);
-            q.wall = std::min(q.wall, w);
-        }
         base += q.n;
         coff += int64_t(q.dim) * q.dim * q.dim + 1;
         if (coff > INT32_MAX) return set_err(c, RPD_E_LIMIT, "rpd_solve_batch: kNN grids too large");
@@ -1844,30 +1837,16 @@ int rpd_solve_batch(rpd_ctx *c, int32_t nreq, rpd_domain *const *doms, const dou
     RPDCHK(c, c->req_of.ensure(size_t(total) * 2), "alloc request map");
     RPDCHK(c, c->req_desc.ensure(size_t(nreq) * sizeof(ReqDesc)), "alloc request descriptors");
     RPDCHK(c, c->knn_req.ensure(size_t(nreq) * sizeof(KnnReq)), "alloc request descriptors");
+    RPDCHK(c, c->req_wmin.ensure(size_t(nreq) * 2 * sizeof(double)), "alloc request minima");
     hipStream_t s = c->stream;
     std::vector<ReqDesc> desc(static_cast<size_t>(nreq));
     std::vector<KnnReq> kdesc(static_cast<size_t>(nreq));
     for (int r = 0; r < nreq; ++r) {
         const auto &q = reqs[size_t(r)];
-        double4 *sd = c->seeds.as<double4>() + q.base;
-        HIPCHK(c, hipMemcpyAsync(sd, xyzw[r], size_t(q.n) * 32, hipMemcpyHostToDevice, s));
-        // the request's own binning (as alone), then its ids made global
-        int *perm = c->perm.as<int>() + q.base;
-        int *cnt = c->counters.as<int>() + q.coff;
-        const int64_t nc = int64_t(q.dim) * q.dim * q.dim;
-        RPDCHK(c,
-               rpd_bin_seeds(s, sd, q.n, kprec, q.dim, c->bin_scratch, perm, cnt,
-                             static_cast<char *>(c->stored.ptr) + size_t(q.base) * vsz,
-                             c->stored64.as<double4>() + q.base),
-               "rpd_solve_batch: binning");
-        RPDCHK(c, rpd_add_base(s, perm, q.n, int(q.base)), "rpd_solve_batch: binning");
-        RPDCHK(c, rpd_add_base(s, cnt, nc + 1, int(q.base)), "rpd_solve_batch: binning");
-        HIPCHK(c, hipMemsetD16Async(reinterpret_cast<hipDeviceptr_t>(c->req_of.as<uint16_t>() + q.base),
-                                    uint16_t(r), size_t(q.n), s));
+        HIPCHK(c, hipMemcpyAsync(c->seeds.as<double4>() + q.base, xyzw[r], size_t(q.n) * 32, hipMemcpyHostToDevice, s));
         ReqDesc &d = desc[size_t(r)];
         d = ReqDesc{};
         d.n_seeds = q.n;
-        d.wmin = prm->security_mode == 0 && q.wmin < INFINITY ? q.wmin : 0.0;
         if (q.dom) {
             const DomainDev &dv = q.dom->dev;
             d.g = dv.g;
@@ -1885,11 +1864,23 @@ int rpd_solve_batch(rpd_ctx *c, int32_t nreq, rpd_domain *const *doms, const dou
             d.vface = dv.vface;
             d.dist = prm->cull ? dv.dist : nullptr;
         }
-        kdesc[size_t(r)] = KnnReq{cnt, q.dim};
+        kdesc[size_t(r)] = KnnReq{c->counters.as<int>() + q.coff, q.dim, q.base};
     }
     HIPCHK(c, hipMemcpyAsync(c->req_desc.ptr, desc.data(), desc.size() * sizeof(ReqDesc), hipMemcpyHostToDevice, s));
     HIPCHK(c, hipMemcpyAsync(c->knn_req.ptr, kdesc.data(), kdesc.size() * sizeof(KnnReq), hipMemcpyHostToDevice, s));
-    HIPCHK(c, hipStreamSynchronize(s));  // the host vectors above are pageable
+    // The requests' weight minima and binnings (each as alone) at once: 16
+    // requests of up to 100,003 seeds took 8 launches and a wait apiece and the
+    // minima a pass on the host, 8.1 ms for the call; so, 6.8.
+    // The wait in rpd_bin_batch covers the copies from the (pageable) vectors.
+    RPDCHK(c,
+           rpd_batch_wmin(s, c->seeds.as<double4>(), c->knn_req.as<KnnReq>(), c->req_desc.as<ReqDesc>(), nreq,
+                          prm->security_mode == 0, c->req_wmin.as<double>()),
+           "rpd_solve_batch: weight minima");
+    RPDCHK(c,
+           rpd_bin_batch(s, c->seeds.as<double4>(), total, kprec, coff, c->knn_req.as<KnnReq>(), nreq,
+                         c->req_of.as<uint16_t>(), c->bin_scratch, c->pin + kPinBinFlag, c->perm.as<int>(),
+                         c->counters.as<int>(), c->stored.ptr, c->stored64.as<double4>()),
+           "rpd_solve_batch: binning");
     c->n = total;
     c->bin_prec = kprec;
     c->dim = 0;

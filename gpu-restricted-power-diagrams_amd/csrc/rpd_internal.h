@@ -96,7 +96,19 @@ int rpd_bin_seeds_redo(hipStream_t st, const double4 *seeds, int64_t n, int prec
 struct KnnReq {
     const int *counters;  // dim^3 + 1 entries, global stored ids
     int dim;
+    int64_t base;         // base_r
 };
+// The requests' binnings at once: their seeds lie one after the other, their
+// counters too (n_counters in all, kreqs[r].counters points into them).  Fills
+// req_of as well.  Waits for the stream.
+int rpd_bin_batch(hipStream_t st, const double4 *seeds, int64_t n, int prec, int64_t n_counters, const KnnReq *kreqs,
+                  int nreq, uint16_t *req_of, DevBuf &scratch, int *flag_pinned, int *perm, int *counters,
+                  void *stored, double4 *stored64);
+// The requests' minimum weights (non-border seeds, all) to pairs[2r], pairs[2r
+// + 1]; desc[r].wmin becomes the first (power, and one is there) or 0.
+struct ReqDesc;
+int rpd_batch_wmin(hipStream_t st, const double4 *seeds, const KnnReq *kreqs, ReqDesc *desc, int nreq, bool power,
+                   double *pairs);
 // K nearest of each query (stored ids ids[0..n_ids), nullptr: all), or, with
 // lower set, the K after the neighbour lower[q] (stored-id indexed).  With
 // kreqs set, each query searches the grid of its request (req_of) instead of
@@ -109,8 +121,6 @@ int rpd_launch_knn(hipStream_t st, int prec, const void *stored, const int *perm
                    const int *ids, int64_t n_ids, int K, int *out, const int *lower = nullptr,
                    const KnnReq *kreqs = nullptr, const uint16_t *req_of = nullptr, const int *n_dev = nullptr,
                    bool narrow = false);
-// adds base to n ints (binning of one request of a packed batch)
-int rpd_add_base(hipStream_t st, int *v, int64_t n, int base);
 
 // ---- clip (rpd_clip.hip) --------------------------------------------------
 struct DomainDev {

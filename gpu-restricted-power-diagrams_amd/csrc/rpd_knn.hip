@@ -49,14 +49,34 @@ __device__ __forceinline__ int cell_coord(double c, int dim) {
     return max(0, min(i, dim - 1));
 }
 
+// A packed batch (kreqs): the requests' seeds lie one after the other, and so
+// do their grids' cells, each with one more that stays empty, whose place in
+// the sums is the end of the request's last cell.  req_of[i] becomes seed i's
+// request.
 template <typename R>
 __global__ void bin_cells_kernel(const double4 *__restrict__ seeds, int64_t n, int dim, int *__restrict__ cell,
-                                 int *__restrict__ counts, int *__restrict__ rank) {
+                                 int *__restrict__ counts, int *__restrict__ rank,
+                                 const KnnReq *__restrict__ kreqs, int nreq, const int *__restrict__ counters,
+                                 uint16_t *__restrict__ req_of) {
     const int64_t i = blockIdx.x * int64_t(blockDim.x) + threadIdx.x;
     if (i >= n) return;
     const double4 s = seeds[i];
     const R x = R(s.x), y = R(s.y), z = R(s.z);
-    const int c = cell_coord(x, dim) + cell_coord(y, dim) * dim + cell_coord(z, dim) * dim * dim;
+    int c = 0;
+    if (kreqs) {
+        int lo = 0, hi = nreq - 1;  // the last request that starts at or before i
+        while (lo < hi) {
+            const int m = (lo + hi + 1) >> 1;
+            if (kreqs[m].base <= i)
+                lo = m;
+            else
+                hi = m - 1;
+        }
+        req_of[i] = uint16_t(lo);
+        dim = kreqs[lo].dim;
+        c = int(kreqs[lo].counters - counters);
+    }
+    c += cell_coord(x, dim) + cell_coord(y, dim) * dim + cell_coord(z, dim) * dim * dim;
     cell[i] = c;
     rank[i] = atomicAdd(&counts[c], 1);  // a place in the cell, in no set order
 }
@@ -862,11 +882,13 @@ static void gather_seeds(hipStream_t st, const double4 *seeds, const int *perm, 
 // Queues the binning; its crowded-cell flag is copied to flag_host, or, with
 // flag_dev, the flag's device address, written there (clear until then).
 // zeroed: the scratch's counts and what follows them are cleared already.
-static int bin_queue(hipStream_t st, const double4 *seeds, int64_t n, int prec, int dim, void *scratch_ptr,
-                     size_t scratch_bytes, int *flag_host, int *flag_dev, bool zeroed, int *perm, int *counters,
-                     void *stored, double4 *stored64) {
+// kreqs (on the device, nullable): a packed batch of nreq requests with nc
+// cells in all but the last one's empty cell (then dim is not read).
+static int bin_queue(hipStream_t st, const double4 *seeds, int64_t n, int prec, int dim, int64_t nc,
+                     void *scratch_ptr, size_t scratch_bytes, int *flag_host, int *flag_dev, bool zeroed, int *perm,
+                     int *counters, void *stored, double4 *stored64, const KnnReq *kreqs = nullptr, int nreq = 0,
+                     uint16_t *req_of = nullptr) {
     BinLayout b;
-    const int64_t nc = cells_of(dim);
     if (bin_layout(st, n, nc, b) != RPD_OK) return RPD_E_DEVICE;
     if (b.need > scratch_bytes) return RPD_E_LIMIT;
     char *base = static_cast<char *>(scratch_ptr);
@@ -881,9 +903,9 @@ static int bin_queue(hipStream_t st, const double4 *seeds, int64_t n, int prec, 
     const int tb = 256;
     const unsigned nb = unsigned((n + tb - 1) / tb);
     if (prec == 0)
-        bin_cells_kernel<float><<<nb, tb, 0, st>>>(seeds, n, dim, cell, counts, rank);
+        bin_cells_kernel<float><<<nb, tb, 0, st>>>(seeds, n, dim, cell, counts, rank, kreqs, nreq, counters, req_of);
     else
-        bin_cells_kernel<double><<<nb, tb, 0, st>>>(seeds, n, dim, cell, counts, rank);
+        bin_cells_kernel<double><<<nb, tb, 0, st>>>(seeds, n, dim, cell, counts, rank, kreqs, nreq, counters, req_of);
     scan_cells_kernel<<<unsigned((nc + kScanTile) / kScanTile), 256, 0, st>>>(counts, nc + 1, counters, state, ticket);
     scatter_cells_kernel<<<nb, tb, 0, st>>>(cell, rank, n, counters, members);
     // placed at once; a crowded cell (rare) sorts and gathers again
@@ -900,10 +922,10 @@ static int bin_queue(hipStream_t st, const double4 *seeds, int64_t n, int prec, 
 
 // The crowded-cell path: the permutation of a radix sort of (cell, index),
 // then the gather again; waits for the stream.
-static int bin_redo(hipStream_t st, const double4 *seeds, int64_t n, int prec, int dim, void *scratch_ptr,
+static int bin_redo(hipStream_t st, const double4 *seeds, int64_t n, int prec, int64_t nc, void *scratch_ptr,
                     int *perm, void *stored, double4 *stored64) {
     BinLayout b;
-    if (bin_layout(st, n, cells_of(dim), b) != RPD_OK) return RPD_E_DEVICE;
+    if (bin_layout(st, n, nc, b) != RPD_OK) return RPD_E_DEVICE;
     char *base = static_cast<char *>(scratch_ptr);
     int *cell_in = reinterpret_cast<int *>(base);
     int *cell_out = reinterpret_cast<int *>(base + b.off_cell_out);
@@ -933,33 +955,74 @@ int rpd_bin_seeds(hipStream_t st, const double4 *seeds, int64_t n, int prec, int
 }
 int rpd_bin_seeds_in(hipStream_t st, const double4 *seeds, int64_t n, int prec, int dim, void *scratch_ptr,
                      size_t scratch_bytes, int *flag_host, int *perm, int *counters, void *stored, double4 *stored64) {
-    const int r = bin_queue(st, seeds, n, prec, dim, scratch_ptr, scratch_bytes, flag_host, nullptr, false, perm,
-                            counters, stored, stored64);
+    const int r = bin_queue(st, seeds, n, prec, dim, cells_of(dim), scratch_ptr, scratch_bytes, flag_host, nullptr, false,
+                            perm, counters, stored, stored64);
     if (r != RPD_OK) return r;
     if (hipStreamSynchronize(st) != hipSuccess) return RPD_E_DEVICE;
-    if (*flag_host) return bin_redo(st, seeds, n, prec, dim, scratch_ptr, perm, stored, stored64);
+    if (*flag_host) return bin_redo(st, seeds, n, prec, cells_of(dim), scratch_ptr, perm, stored, stored64);
     return RPD_OK;
 }
 int rpd_bin_seeds_async(hipStream_t st, const double4 *seeds, int64_t n, int prec, int dim, DevBuf &scratch,
                         int *flag_pinned, int *flag_dev, int *perm, int *counters, void *stored, double4 *stored64) {
-    return bin_queue(st, seeds, n, prec, dim, scratch.ptr, scratch.bytes, flag_pinned, flag_dev, true, perm, counters,
-                     stored, stored64);
+    return bin_queue(st, seeds, n, prec, dim, cells_of(dim), scratch.ptr, scratch.bytes, flag_pinned, flag_dev, true,
+                     perm, counters, stored, stored64);
 }
 int rpd_bin_seeds_redo(hipStream_t st, const double4 *seeds, int64_t n, int prec, int dim, DevBuf &scratch,
                        int *perm, void *stored, double4 *stored64) {
-    return bin_redo(st, seeds, n, prec, dim, scratch.ptr, perm, stored, stored64);
+    return bin_redo(st, seeds, n, prec, cells_of(dim), scratch.ptr, perm, stored, stored64);
+}
+
+int rpd_bin_batch(hipStream_t st, const double4 *seeds, int64_t n, int prec, int64_t n_counters, const KnnReq *kreqs,
+                  int nreq, uint16_t *req_of, DevBuf &scratch, int *flag_pinned, int *perm, int *counters,
+                  void *stored, double4 *stored64) {
+    BinLayout b;
+    if (bin_layout(st, n, n_counters - 1, b) != RPD_OK) return RPD_E_DEVICE;
+    if (scratch.ensure(b.need) != RPD_OK) return RPD_E_NOMEM;
+    const int r = bin_queue(st, seeds, n, prec, 0, n_counters - 1, scratch.ptr, b.need, flag_pinned, nullptr, false, perm,
+                            counters, stored, stored64, kreqs, nreq, req_of);
+    if (r != RPD_OK) return r;
+    if (hipStreamSynchronize(st) != hipSuccess) return RPD_E_DEVICE;
+    if (*flag_pinned) return bin_redo(st, seeds, n, prec, n_counters - 1, scratch.ptr, perm, stored, stored64);
+    return RPD_OK;
 }
 
 namespace rpd {
-__global__ void add_base_kernel(int *__restrict__ v, int64_t n, int base) {
-    const int64_t i = blockIdx.x * int64_t(blockDim.x) + threadIdx.x;
-    if (i < n) v[i] += base;
+// One workgroup a request: the minimum weight of its non-border seeds and of
+// all, to pairs[2r], pairs[2r + 1], and what the clip kernels subtract.
+__global__ __launch_bounds__(1024) void batch_wmin_kernel(const double4 *__restrict__ seeds,
+                                                          const KnnReq *__restrict__ kreqs, ReqDesc *__restrict__ desc,
+                                                          int power, double *__restrict__ pairs) {
+    __shared__ double red[2][16];
+    const int r = int(blockIdx.x), lane = lane_id(), wv = int(threadIdx.x >> 6);
+    const int64_t base = kreqs[r].base, n = desc[r].n_seeds;
+    double m = INFINITY, ma = INFINITY;
+    for (int64_t i = threadIdx.x; i < n; i += 1024) {
+        const double w = seeds[base + i].w;
+        if (w > RPD_NO_CELL_LIMITS) m = fmin(m, w);
+        ma = fmin(ma, w);
+    }
+    m = wave_min(m);
+    ma = wave_min(ma);
+    if (lane == 0) {
+        red[0][wv] = m;
+        red[1][wv] = ma;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < 16; ++w) {
+            m = fmin(m, red[0][w]);
+            ma = fmin(ma, red[1][w]);
+        }
+        pairs[2 * r] = m;
+        pairs[2 * r + 1] = ma;
+        desc[r].wmin = power && m < INFINITY ? m : 0.0;
+    }
 }
 }  // namespace rpd
 
-int rpd_add_base(hipStream_t st, int *v, int64_t n, int base) {
-    if (n <= 0 || base == 0) return RPD_OK;
-    add_base_kernel<<<unsigned((n + 255) / 256), 256, 0, st>>>(v, n, base);
+int rpd_batch_wmin(hipStream_t st, const double4 *seeds, const KnnReq *kreqs, ReqDesc *desc, int nreq, bool power,
+                   double *pairs) {
+    batch_wmin_kernel<<<unsigned(nreq), 1024, 0, st>>>(seeds, kreqs, desc, power ? 1 : 0, pairs);
     return hipGetLastError() == hipSuccess ? RPD_OK : RPD_E_DEVICE;
 }
 

@@ -37,3 +37,34 @@ def test_kept_cells_are_the_whole_diagram(rpd, ctx, n):
     dom.close()
     assert out[0][1] > 0 and out[0][1] + out[0][2] == n and out[1][1] == 0
     assert np.array_equal(out[0][0], out[1][0])
+
+
+@pytest.mark.parametrize("prec", [0, 1])
+@pytest.mark.parametrize("crowded", [False, True])
+def test_batch_is_binned_as_alone(rpd, ctx, prec, crowded):
+    """The requests' binnings in one go: each request's permutation and weight
+    minima as alone, also when a cell of one of them holds more seeds than a
+    run that is sorted in place."""
+    rng = np.random.default_rng(5)
+    reqs = []
+    for k, n in enumerate((2, 700, 3001, 40000, 17)):
+        x = rpd.generate_seeds(rpd.SEEDS_UNIFORM, n, seed=n, wmax=10.0 * k)
+        if crowded and n == 3001:
+            x[:200, :3] = 300.0 + rng.random((200, 3))
+        reqs.append(x)
+    dom = ctx.domain(rpd.Grid.shape(0, 24, (0.5, 0.5, 0.5, 0.4)))
+    caps = dict(K=64, P=48, V=64, precision=prec)
+    alone, perms = [], []
+    base = 0
+    for x in reqs:
+        ctx.set_seeds(x)
+        ctx.solve(dom, **caps)
+        alone.append(ctx.moments())
+        perms.append(ctx.perm() + base)
+        base += x.shape[0]
+    _, outs = ctx.solve_batch([(dom, x) for x in reqs], **caps)
+    perm = ctx.perm()
+    dom.close()
+    assert np.array_equal(perm, np.concatenate(perms))
+    for k, (o, m) in enumerate(zip(outs, alone)):
+        assert np.array_equal(o, m), "request %d" % k
