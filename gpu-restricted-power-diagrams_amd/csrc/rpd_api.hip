@@ -193,17 +193,29 @@ static void *g_scratch_ptr[kMaxDevices] = {};
 
 namespace {
 
-// Up to 16 device int arrays cleared by one launch: the counters a solve
-// starts from, without one fill launch each.
-struct ZeroSet {
-    int *p[16];
-    int n[16];
-    int k;
+// Up to 20 device int arrays filled by one launch: the counters a solve starts
+// from, without one launch each, and the outputs of the cells that the cover
+// test leaves out (16-byte aligned arrays, 16 bytes a store).
+struct FillSet {
+    int *p[20];
+    int64_t n[20];
+    int v[20];
+    int k = 0;
+    void add(int *ptr, int64_t words, int value = 0) {
+        p[k] = ptr;
+        n[k] = words;
+        v[k++] = value;
+    }
 };
-constexpr int kZeroBlocks = 256;
-__global__ __launch_bounds__(256) void zero_words_kernel(ZeroSet z) {
-    for (int j = 0; j < z.k; ++j)
-        for (int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x; i < z.n[j]; i += kZeroBlocks * 256) z.p[j][i] = 0;
+constexpr int kFillBlocks = 512;
+__global__ __launch_bounds__(256) void fill_words_kernel(FillSet z) {
+    const int64_t t = int64_t(blockIdx.x) * 256 + threadIdx.x;
+    for (int j = 0; j < z.k; ++j) {
+        const int64_t n4 = z.n[j] >> 2;
+        const int v = z.v[j];
+        for (int64_t i = t; i < n4; i += kFillBlocks * 256) reinterpret_cast<int4 *>(z.p[j])[i] = make_int4(v, v, v, v);
+        if (t < (z.n[j] & 3)) z.p[j][4 * n4 + t] = v;
+    }
 }
 
 // Resolves the current device's copy of `scratch` once (device current).
@@ -1016,6 +1028,7 @@ static int solve_impl(rpd_ctx *c, rpd_domain *dom, const rpd_params *prm, rpd_st
     RPDCHK(c, c->pb1.q.ensure(2 * sizeof(int)), "alloc queue counter");
     const bool new_wmin = !batch && prm->security_mode == 0 && !c->wmin_ok;
     RPDCHK(c, c->wred.ensure((2 * kWminBlocks + 3) * sizeof(double)), "alloc wred");
+    const bool may_cover = (dom || batch) && prm->cull && prm->security_mode == 0;
     int *wleft = reinterpret_cast<int *>(c->wred.as<double>() + 2 * kWminBlocks + 2);
     HIPCHK(c, hipEventRecord(c->evb[0], c->stream));
     // The counters the solve starts from, cleared by one launch: the final
@@ -1025,34 +1038,28 @@ static int solve_impl(rpd_ctx *c, rpd_domain *dom, const rpd_params *prm, rpd_st
     // one is skipped.
     bool fresh_fl[6];
     {
-        ZeroSet z{};
-        z.p[z.k] = c->cnt.as<int>();
-        z.n[z.k++] = 16;
+        FillSet z{};
+        z.add(c->cnt.as<int>(), 16);
         for (int i = 0; i < 6; ++i) {
-            z.p[z.k] = c->fl[i].cnt.as<int>();
-            z.n[z.k++] = kFailCounters;
+            z.add(c->fl[i].cnt.as<int>(), kFailCounters);
             fresh_fl[i] = true;
         }
-        for (PassBufs *b : {&c->pb1, &c->pb[0], &c->pb[1], &c->pb[2], &c->pb[3]}) {
-            z.p[z.k] = b->q.as<int>();
-            z.n[z.k++] = 2;
-        }
-        if (new_wmin) {
-            z.p[z.k] = wleft;
-            z.n[z.k++] = 1;
-        }
+        for (PassBufs *b : {&c->pb1, &c->pb[0], &c->pb[1], &c->pb[2], &c->pb[3]}) z.add(b->q.as<int>(), 2);
+        if (new_wmin) z.add(wleft, 1);
+        int *zp = nullptr, zn = 0;
         if (!batch && c->bin_prec != kprec) {
-            RPDCHK(c, rpd_bin_prepare(c->stream, n, rpd_knn_dim(n), c->bin_scratch, &z.p[z.k], &z.n[z.k]),
-                   "alloc binning");
-            ++z.k;
+            RPDCHK(c, rpd_bin_prepare(c->stream, n, rpd_knn_dim(n), c->bin_scratch, &zp, &zn), "alloc binning");
+            z.add(zp, zn);
         }
-        if (dom || batch) {
-            RPDCHK(c, rpd_cover_prepare(int(std::max<size_t>(c->batch.size(), 1)), n, c->cull_scratch, &z.p[z.k],
-                                        &z.n[z.k]),
+        if (may_cover) {
+            RPDCHK(c, rpd_cover_prepare(int(std::max<size_t>(c->batch.size(), 1)), n, c->cull_scratch, &zp, &zn),
                    "alloc domain cover");
-            ++z.k;
+            z.add(zp, zn);
+            z.add(c->out.as<int>(), 8 * n);
+            z.add(c->status.as<int>(), n, RPD_SUCCESS);
+            z.add(c->kused.as<int>(), n);
         }
-        zero_words_kernel<<<kZeroBlocks, 256, 0, c->stream>>>(z);
+        fill_words_kernel<<<kFillBlocks, 256, 0, c->stream>>>(z);
         HIPCHK(c, hipGetLastError());
     }
     // The weight minima of new seeds (over the non-border seeds, and over
@@ -1139,12 +1146,11 @@ static int solve_impl(rpd_ctx *c, rpd_domain *dom, const rpd_params *prm, rpd_st
                         bool walls) {
         CoverArgs ca{};
         ca.stored64 = c->stored64.as<double4>();
-        ca.perm = c->perm.as<int>();
         ca.counters = counters;
         ca.dim = dim;
         ca.base = base;
         ca.n = cnt;
-        ca.apply = d && prm->cull && prm->security_mode == 0 && !walls;
+        ca.apply = d && may_cover && !walls;
         if (d) {
             ca.dvox = d->dvox;
             ca.n_dvox = d->n_dvox;
@@ -1154,9 +1160,6 @@ static int solve_impl(rpd_ctx *c, rpd_domain *dom, const rpd_params *prm, rpd_st
         }
         ca.wmin = wm;
         ca.wdev = walls ? nullptr : wdev;
-        ca.out = c->out.as<double4>();
-        ca.status = c->status.as<int>();
-        ca.kused = c->kused.as<int>();
         return ca;
     };
     if (batch) {

@@ -245,7 +245,6 @@ constexpr int kDcStride = RPD_DCOUNT_INTS;
 // One per request: its cells are the stored ids [base, base + n).
 struct CoverArgs {
     const double4 *stored64;  // sorted seeds, FP64 (every request)
-    const int *perm;          // stored -> original (every request)
     const int *counters;      // the request's kNN grid: dim^3 + 1 exclusive prefix, global stored ids
     int dim;
     int64_t base, n;
@@ -260,15 +259,12 @@ struct CoverArgs {
     // minimum over all) replacing wmin; a second one <= RPD_NO_CELL_LIMITS
     // (walls) turns the test off
     const double *wdev;
-    double4 *out;             // original order: skipped cells get 0
-    int *status;
-    int *kused;
 };
 // Scratch for nreq requests over n_total ids, whose words [zero, zero +
 // zero_words) are to be cleared before rpd_cover_skip.
 int rpd_cover_prepare(int nreq, int64_t n_total, DevBuf &scratch, int **zero, int *zero_words);
-// Queues: the outputs of the skipped cells, and the stored ids of the others,
-// ascending, to ids_out (n_total entries).  The requests' ranges follow each
+// Queues: the stored ids of the cells that are not provably empty, ascending,
+// to ids_out (n_total entries; the others' outputs are the caller's).  The requests' ranges follow each
 // other and cover [0, n_total).  *count_dev receives the device copy of the
 // number of ids, *n_out (pinned host memory; n_out_dev: its device address, or
 // null, then it is copied) the number.
