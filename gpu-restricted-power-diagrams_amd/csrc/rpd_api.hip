@@ -90,6 +90,8 @@ constexpr int kTriangleFloor = 256;
 // torus in 128^3, finish kernel of 16 cells a CU 0.53 ms (FP64 0.60), with room
 // for 1,024 strips 0.58 (0.71).
 constexpr int kStripFloor = 1024;
+// recomputed cells of the FP32 form up to which they list 256 neighbours
+constexpr int kShortQueue = 4096;
 constexpr double kStripsPerArea = 12.0;
 static int strip_floor(int g, int64_t n) {
     const double w2 = std::cbrt(double(g) * g * g / double(n)) * std::cbrt(double(g) * g * g / double(n));
@@ -1497,7 +1499,13 @@ static int solve_impl(rpd_ctx *c, rpd_domain *dom, const rpd_params *prm, rpd_st
         // as many of them would run out of neighbours again as in the
         // previous pass (one more pass for them); the loop reads only the
         // neighbours it needs
-        ch.pz.caps[0] = std::min(256, nc.K);
+        // The FP32 form keeps no states, so its cells that ran out come here
+        // too: a short queue lists all 256 at once (its kNN is a matter of
+        // latency, and another pass for the few cells that need more than
+        // twice K takes longer: FP32, 2,000 seeds 570 -> 470 us, 10,000 715 ->
+        // 592; from 20,000 seeds on neither is better)
+        ch.pz.caps[0] = form0 == RPD_PREC_FP32 && ch.n_scr <= kShortQueue ? int(std::min<int64_t>(256, n - 1))
+                                                                           : std::min(256, nc.K);
         ch.pr.caps[1] = ch.pz.caps[1] = nc.P;
         ch.pr.caps[2] = ch.pz.caps[2] = nc.V;
         ch.pr.caps[3] = ch.pz.caps[3] = nc.T;
