@@ -978,10 +978,14 @@ static int solve_impl(rpd_ctx *c, rpd_domain *dom, const rpd_params *prm, rpd_st
     // further passes (100,000 seeds in a torus at 100^3, K = 20: 87% of the
     // cells a second time; solve 1.46 -> 0.98 ms, K = 25 0.90 of 1.29 ms,
     // 300,000 seeds at K = 50 4.9 -> 4.7 ms).
-    // Only with re-queue passes allowed: without them, running out is the
-    // answer; and not in the FP32 form, whose re-queue passes are FP64.
-    if (prm->max_extra_steps > 0 && form0 != RPD_PREC_FP32 && K < kNeighbourFloor)
-        K = int(std::min<int64_t>(kNeighbourFloor, n - 1));
+    // Not in the FP32 form, whose re-queue passes are FP64.  The number of
+    // neighbours a cell may use in all stays what K and the passes allow
+    // (k_reach: K doubled, by at most 256, once a pass): running out of them
+    // is an answer, not a matter of how they were listed.
+    int64_t k_reach = K;
+    for (int k = 0; k < prm->max_extra_steps && k_reach < n - 1; ++k)
+        k_reach = std::min<int64_t>(n - 1, k_reach + std::min<int64_t>(k_reach, 256));
+    if (form0 != RPD_PREC_FP32 && K < kNeighbourFloor && k_reach > kNeighbourFloor) K = kNeighbourFloor;
     // The triangle cap is raised to kTriangleFloor where it is lower: a cell
     // done by one wave keeps 4 bytes of LDS per union entry, which costs the
     // finish kernel no residency, and a cell's result does not depend on the
@@ -1343,8 +1347,16 @@ static int solve_impl(rpd_ctx *c, rpd_domain *dom, const rpd_params *prm, rpd_st
         // so a cell may go on past 256 neighbours in all (a cell bounded by
         // walls reaches twice as far as its bisectors); a recomputed cell
         // lists at most 256
-        if (h[RPD_SECURITY_RADIUS_NOT_REACHED])
-            nc.K = int(std::min<int64_t>(n - 1, int64_t(cap.K) + std::min(cap.K, 256)));
+        // The FP32 form keeps no states in its first pass, so its cells that
+        // ran out are computed anew: a short queue lists 256 at once (its kNN
+        // is a matter of latency, and another pass for the few cells that need
+        // more than twice K takes longer: FP32, 2,000 seeds 570 -> 470 us,
+        // 10,000 715 -> 592; from 20,000 seeds on neither is better).
+        if (h[RPD_SECURITY_RADIUS_NOT_REACHED]) {
+            nc.K = cap.K + std::min(cap.K, 256);
+            if (form0 == RPD_PREC_FP32 && cnt[0] + cnt[1] <= kShortQueue) nc.K = std::max(nc.K, 256);
+            nc.K = int(std::min<int64_t>(nc.K, k_reach));
+        }
         if (h[RPD_TRIANGLE_OVERFLOW]) nc.T = std::max(int(cap.T * 1.5) + 1, cnt[13]);
         nc.T = std::min(nc.T, rpd_clip_max_T(RPD_PREC_FP64, nc.P, nc.V, hess));
         return nc;
@@ -1488,8 +1500,11 @@ static int solve_impl(rpd_ctx *c, rpd_domain *dom, const rpd_params *prm, rpd_st
         ch.pr.index = ch.pz.index = 1 + ch.k;
         // resumed cells of a mixed solve go on in the mixed form, which decides
         // its open tests in FP64 in place (the reference stop, whose near
-        // cases it leaves to the FP64 form, and the Hessian go on in FP64)
-        ch.pr.form = form0 == RPD_PREC_MIXED && prm->security_mode == 0 && !hess ? RPD_PREC_MIXED : RPD_PREC_FP64;
+        // cases it leaves to the FP64 form, and the Hessian go on in FP64);
+        // with the last neighbours they may use, in FP64, whose stop test has
+        // no margin
+        ch.pr.form = form0 == RPD_PREC_MIXED && prm->security_mode == 0 && !hess && nc.K < k_reach ? RPD_PREC_MIXED
+                                                                                                  : RPD_PREC_FP64;
         ch.pz.form = RPD_PREC_FP64;
         ch.pr.n_ids = ch.n_res;
         ch.pz.n_ids = ch.n_scr;
@@ -1499,13 +1514,7 @@ static int solve_impl(rpd_ctx *c, rpd_domain *dom, const rpd_params *prm, rpd_st
         // as many of them would run out of neighbours again as in the
         // previous pass (one more pass for them); the loop reads only the
         // neighbours it needs
-        // The FP32 form keeps no states, so its cells that ran out come here
-        // too: a short queue lists all 256 at once (its kNN is a matter of
-        // latency, and another pass for the few cells that need more than
-        // twice K takes longer: FP32, 2,000 seeds 570 -> 470 us, 10,000 715 ->
-        // 592; from 20,000 seeds on neither is better)
-        ch.pz.caps[0] = form0 == RPD_PREC_FP32 && ch.n_scr <= kShortQueue ? int(std::min<int64_t>(256, n - 1))
-                                                                           : std::min(256, nc.K);
+        ch.pz.caps[0] = std::min(256, nc.K);
         ch.pr.caps[1] = ch.pz.caps[1] = nc.P;
         ch.pr.caps[2] = ch.pz.caps[2] = nc.V;
         ch.pr.caps[3] = ch.pz.caps[3] = nc.T;

@@ -68,3 +68,22 @@ def test_batch_is_binned_as_alone(rpd, ctx, prec, crowded):
     assert np.array_equal(perm, np.concatenate(perms))
     for k, (o, m) in enumerate(zip(outs, alone)):
         assert np.array_equal(o, m), "request %d" % k
+
+
+@pytest.mark.parametrize("prec", [0, 1, 2])
+@pytest.mark.parametrize("K,steps,reach", [(20, 1, 40), (7, 2, 28), (30, 2, 120)])
+def test_neighbours_in_all_are_what_the_caps_allow(rpd, ctx, prec, K, steps, reach):
+    """However the first list is sized, a cell may use K neighbours, doubled
+    once a pass: the cells that run out are those of one list of that length
+    (the FP32 form goes on in FP64)."""
+    x = rpd.generate_seeds(rpd.SEEDS_UNIFORM, 3000, seed=9, wmax=0.0)
+    x[:, :3] = 200.0 + 0.6 * x[:, :3]  # cells of the outer seeds reach far
+    dom = ctx.domain(rpd.Grid.shape(0, 16, (0.5, 0.5, 0.5, 0.45)))
+    ctx.set_seeds(x)
+    ctx.solve(dom, K=K, P=100, V=128, precision=prec, max_extra_steps=steps)
+    got = ctx.status()
+    ctx.solve(dom, K=reach, P=100, V=128, precision=0, max_extra_steps=0)
+    ref = ctx.status()
+    dom.close()
+    assert (ref != 4).any()
+    assert np.array_equal(got, ref)
