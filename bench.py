@@ -392,7 +392,7 @@ def main():
     roofline = roofline_cells = None
     if flop is not None:
         ka = "clip_cells_kernel<float, double, true, 1, false>"
-        kb = "finish_cells_kernel<float, double, true, 1, false, false>"
+        kb = "finish_cells_kernel<float, double, true, 1, false, false, true>"
         roofline_cells = valu_roofline(*flop["mixed"]["cells"], n, t_cells, ka + " (mixed form, pass 1)",
                                        measured_traffic(ka))
         roofline = valu_roofline(*flop["mixed"]["finish"], n, t_finish, kb + " (mixed form, pass 1)",
