@@ -153,8 +153,11 @@ typedef struct {
                                      at least 256, V to its vertex slots'
                                      room (64/128/256) and, with
                                      max_extra_steps > 0, P toward 48 and (FP64
-                                     and mixed forms) K to at least 64.  A
-                                     cell's result does not depend on the cap
+                                     and mixed forms) K to 64 where K, doubled
+                                     by at most 256 a step, gets past it (the
+                                     neighbours in all stay as many).  T is
+                                     raised further, to at most 1,024, where
+                                     cells are many voxels wide.  A cell's result does not depend on the cap
                                      it succeeds with; the caps a solve used
                                      are in rpd_stats.final_* / pass_caps    */
     int32_t precision;            /* enum rpd_precision                       */
