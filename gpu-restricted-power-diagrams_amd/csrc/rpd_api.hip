@@ -1501,10 +1501,11 @@ static int solve_impl(rpd_ctx *c, rpd_domain *dom, const rpd_params *prm, rpd_st
         // resumed cells of a mixed solve go on in the mixed form, which decides
         // its open tests in FP64 in place (the reference stop, whose near
         // cases it leaves to the FP64 form, and the Hessian go on in FP64);
-        // with the last neighbours they may use, in FP64, whose stop test has
-        // no margin
-        ch.pr.form = form0 == RPD_PREC_MIXED && prm->security_mode == 0 && !hess && nc.K < k_reach ? RPD_PREC_MIXED
-                                                                                                  : RPD_PREC_FP64;
+        // with the last neighbours they may use, and on the last step, in
+        // FP64, whose stop test has no margin
+        const bool more = nc.K < k_reach && ch.k + 1 < prm->max_extra_steps;
+        ch.pr.form = form0 == RPD_PREC_MIXED && prm->security_mode == 0 && !hess && more ? RPD_PREC_MIXED
+                                                                                          : RPD_PREC_FP64;
         ch.pz.form = RPD_PREC_FP64;
         ch.pr.n_ids = ch.n_res;
         ch.pz.n_ids = ch.n_scr;

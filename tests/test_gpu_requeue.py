@@ -1,0 +1,63 @@
+"""Re-queue passes of a solve: which form a cell's last pass has, and that no
+pass repeats what cannot change."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _sphere(m):
+    """m directions, evenly spread."""
+    k = np.arange(m) + 0.5
+    z, a = 1 - 2 * k / m, np.pi * (1 + 5 ** 0.5) * k
+    r = np.sqrt(1 - z * z)
+    return np.stack((r * np.cos(a), r * np.sin(a), z), 1)
+
+
+def _radius(u, d):
+    """Largest vertex distance of the polytope {y: u_i . y <= d_i / 2}."""
+    n = len(d)
+    i, j, k = (t.reshape(-1) for t in np.meshgrid(*(np.arange(n),) * 3, indexing="ij"))
+    keep = (i < j) & (j < k)
+    i, j, k = i[keep], j[keep], k[keep]
+    a = np.stack((u[i], u[j], u[k]), 1)
+    ok = np.abs(np.linalg.det(a)) > 1e-9
+    a, b = a[ok], np.stack((d[i], d[j], d[k]), 1)[ok] / 2
+    y = np.linalg.solve(a, b[..., None])[..., 0]
+    y = y[(y @ u.T <= d / 2 * (1 + 1e-12)).all(1)]
+    return float(np.sqrt((y * y).sum(1).max()))
+
+
+@pytest.mark.parametrize("steps", [2, 3])
+@pytest.mark.parametrize("prec", [0, 1])
+def test_the_last_step_has_no_margin(rpd, ctx, prec, steps):
+    """One cell: its 60 faces overflow the planes in pass 1, the recomputation
+    runs out of the 64 neighbours listed, and the 128th, the last that the next
+    pass lists, lies between the cell's exact stop radius and the FP32 radius's
+    margin over it.  The neighbours past the 60th lie behind others and cut
+    nothing; those far out (their cells miss the domain) are there so that the
+    list does not hold every seed."""
+    m, D = 60, 200.0
+    u = _sphere(m)
+    d = D * (1 + 1e-3 * np.arange(m) / m)
+    R = _radius(u, d)
+    assert 2 * R > D * 1.03
+    more = np.linspace(D * 1.005, D * 1.02, 67)
+    v = u[np.arange(67) % m]
+    last = 2 * R * (1 + 1e-5)
+    far = _sphere(300)
+    p = np.concatenate((np.zeros((1, 3)), u * d[:, None], v * more[:, None], u[:1] * last,
+                        far * np.linspace(2.2 * D, 2.4 * D, 300)[:, None]))
+    x = np.zeros((p.shape[0], 4))
+    x[:, :3] = 500.0 + p
+    mask = np.zeros((64, 64, 64), np.uint8)
+    mask[31:33, 31:33, 31:33] = 1
+    dom = ctx.domain(rpd.Grid.voxels(mask.reshape(-1)))
+    ctx.set_seeds(x)
+    st = ctx.solve(dom, K=64, P=50, V=256, precision=prec, max_extra_steps=steps)
+    status, mom = ctx.status(), ctx.moments()
+    dom.close()
+    assert st["pass_cells"][:3] == [1, 1, 1]  # (the other cells miss the domain)
+    assert [c[0] for c in st["pass_caps"][:3]] == [64, 64, 64]  # the third lists the 64 neighbours after those
+    assert status[0] == 4
+    assert abs(mom[0, 3] - 31.25 ** 3) < 1e-9 * 31.25 ** 3
