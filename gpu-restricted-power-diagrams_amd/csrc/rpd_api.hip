@@ -1225,11 +1225,17 @@ static int solve_impl(rpd_ctx *c, rpd_domain *dom, const rpd_params *prm, rpd_st
     // same records (FP64 planes), its finish kernel decides in FP64, in
     // place, the tests its filter leaves open and those of ill-conditioned
     // vertices, so a cell gets the FP64 form's combinatorics for less work.
+    // The cells that come back with an exact-predicate failure finish in FP64:
+    // the mixed form would mostly fail them again, on every step left (corner
+    // apex, 10,000 to 300,000 seeds in a torus at 100^3, where 0.5% of the
+    // cells have cone planes through lattice points: 6 passes instead of 4).
     const int finish_form_fp64 = form0 == RPD_PREC_MIXED && !hess ? RPD_PREC_MIXED : RPD_PREC_FP64;
     // A re-queue pass's kernels: kNN, bisector kernel and finish kernel (over
     // every cell of the pass: those the bisector kernel did not queue are left
-    // out on the device, so nothing waits for a count).
-    auto pass_run = [&](Pass &ps, const int *ids, int fl_out, const Resume &rz, int beside, ClipLaunch &L) -> int {
+    // out on the device, so nothing waits for a count).  The first n_exact of
+    // its cells are exact-predicate failures.
+    auto pass_run = [&](Pass &ps, const int *ids, int64_t n_exact, int fl_out, const Resume &rz, int beside,
+                        ClipLaunch &L) -> int {
         const int sl = ps.slot;
         hipStream_t s = c->streams[sl];
         PassBufs &b = c->pb[sl];
@@ -1285,8 +1291,15 @@ static int solve_impl(rpd_ctx *c, rpd_domain *dom, const rpd_params *prm, rpd_st
         L.reqs = reqs;
         L.req_of = req_of;
         r = rpd_launch_cells(s, ps.form, L);
-        if (r == RPD_OK)
-            r = rpd_launch_finish(s, ps.form == RPD_PREC_FP64 ? finish_form_fp64 : ps.form, L, int(ps.n_ids), beside);
+        const int fin = ps.form == RPD_PREC_FP64 ? finish_form_fp64 : ps.form;
+        const int64_t n64 = fin == RPD_PREC_FP64 ? 0 : n_exact;
+        if (r == RPD_OK && n64 > 0)
+            r = rpd_launch_finish(s, RPD_PREC_FP64, L, int(n64), beside + int(ps.n_ids - n64));
+        if (r == RPD_OK && n64 < ps.n_ids) {
+            ClipLaunch Lf = L;  // the records after those
+            Lf.rec = static_cast<char *>(L.rec) + size_t(n64) * rpd_clip_record_bytes(ps.form, P_, V_);
+            r = rpd_launch_finish(s, fin, Lf, int(ps.n_ids - n64), beside + int(n64));
+        }
         if (r != RPD_OK) return r;
         return hipEventRecord(c->ev[sl][3], s) == hipSuccess ? RPD_OK : RPD_E_DEVICE;
     };
@@ -1530,14 +1543,14 @@ static int solve_impl(rpd_ctx *c, rpd_domain *dom, const rpd_params *prm, rpd_st
             rr.in = ch.left.rec;
             rr.in_stride = ch.left.stride;
             rr.in_P = ch.left.P;
-            r = pass_run(ch.pr, c->fl[ch.cur].sec.as<int>(), ch.nxt, rr, beside, ch.Lr);
+            r = pass_run(ch.pr, c->fl[ch.cur].sec.as<int>(), 0, ch.nxt, rr, beside, ch.Lr);
             if (r != RPD_OK) return r;
         }
         if (ch.n_scr > 0) {
             Resume rr = ch.rz;
             rr.out_base = int(ch.n_res);
             // exact entries and (when recomputed) the overflows are one range
-            r = pass_run(ch.pz, c->fl[ch.cur].eo.as<int>() + n - n_exact, ch.nxt, rr, beside, ch.Lz);
+            r = pass_run(ch.pz, c->fl[ch.cur].eo.as<int>() + n - n_exact, n_exact, ch.nxt, rr, beside, ch.Lz);
             if (r == RPD_OK) r = pass_lists(ch.pz, ch.Lz, c->pb[ch.sl2], ch.nxt, ch.n_res == 0, nullptr);
             if (r != RPD_OK) return r;
             ch.end = s2;

@@ -61,3 +61,21 @@ def test_the_last_step_has_no_margin(rpd, ctx, prec, steps):
     assert [c[0] for c in st["pass_caps"][:3]] == [64, 64, 64]  # the third lists the 64 neighbours after those
     assert status[0] == 4
     assert abs(mom[0, 3] - 31.25 ** 3) < 1e-9 * 31.25 ** 3
+
+
+@pytest.mark.parametrize("n", [10000, 100000])
+def test_exact_failures_end_in_fp64(rpd, ctx, n):
+    """The corner apex puts cone planes through lattice points, which leaves
+    the cavities of some cells inconsistent in FP64.  The mixed form ends them
+    with the FP64 form's status, and takes at most one pass more to find out."""
+    x = rpd.generate_seeds(rpd.SEEDS_UNIFORM, n, seed=5, wmax=0.0)
+    dom = ctx.domain(rpd.Grid.shape(rpd.SHAPE_TORUS, 100, (0.5, 0.5, 0.5, 0.3, 0.12)))
+    ctx.set_seeds(x)
+    out = []
+    for prec in (0, 1):
+        st = ctx.solve(dom, K=50, P=30, V=40, precision=prec, apex_mode=0)
+        out.append((ctx.status(), st["passes"]))
+    dom.close()
+    assert (out[0][0] == 2).any()
+    assert np.array_equal(out[0][0], out[1][0])
+    assert out[1][1] <= out[0][1] + 1
