@@ -1457,7 +1457,7 @@ static int solve_impl(rpd_ctx *c, rpd_domain *dom, const rpd_params *prm, rpd_st
         // cap met by the cone clips).  Their bisector loop is done,
         // certified, and in pass 1's records, which are the FP64 form's
         // records too, so the finish kernel runs over those records again,
-        // with the grown caps (the FP64 one for flagged tests); a full FP64 recomputation would rebuild the
+        // with the grown caps; a full FP64 recomputation would rebuild the
         // same records first.  The FP32 form's records hold FP32 planes (16
         // bytes, a different layout): its cells take the full pass.
         if (ch.from_finish && ch.k == 0 && ch.n_res == 0 && ch.n_scr > 0 && form0 != RPD_PREC_FP32 &&
@@ -1467,9 +1467,6 @@ static int solve_impl(rpd_ctx *c, rpd_domain *dom, const rpd_params *prm, rpd_st
             ch.pz = Pass{};
             ch.pz.slot = ch.sl;
             ch.pz.index = 1;
-            // Overflows alone need no FP64 tests: the same form again, so a
-            // cell's bits do not depend on the cap that it first met.
-            ch.pz.form = n_exact > 0 ? RPD_PREC_FP64 : form0;
             ch.pz.n_ids = ch.n_scr;
             ch.pz.caps[0] = ch.cap.K;
             ch.pz.caps[1] = ch.cap.P;
@@ -1484,7 +1481,6 @@ static int solve_impl(rpd_ctx *c, rpd_domain *dom, const rpd_params *prm, rpd_st
             L.P = nc.P;
             L.V = nc.V;
             L.T = nc.T;
-            L.slots = c->fslot.as<int>() + n - n_exact;  // the failures' range of the list, in place
             L.fl_slot = nullptr;
             L.fl_cnt = c->fl[ch.nxt].cnt.as<int>();
             L.fl_eo = c->fl[ch.nxt].eo.as<int>() + n;
@@ -1494,7 +1490,28 @@ static int solve_impl(rpd_ctx *c, rpd_domain *dom, const rpd_params *prm, rpd_st
             L.dcnt = dcnt_of(1);
             ch.pz.finish_only = true;
             if (hipEventRecord(c->ev[ch.sl][1], s) != hipSuccess) return RPD_E_DEVICE;
-            int r = rpd_launch_finish(s, ch.pz.form, L, int(ch.n_scr), 0);
+            // The list's two ranges, in place: flagged tests in FP64, overflows
+            // in the form they had, so that a cell's bits depend neither on
+            // the cap that it first met nor on other cells (or requests).  On
+            // the last step no FP64 pass is left for a cavity that the mixed
+            // form then finds inconsistent: such a cell keeps what an FP64
+            // launch has written before.
+            const int n_again = int(ch.n_scr) - n_exact;
+            int r = RPD_OK;
+            if (n_exact > 0) {
+                L.slots = c->fslot.as<int>() + n - n_exact;
+                r = rpd_launch_finish(s, RPD_PREC_FP64, L, n_exact, 0);
+            }
+            L.slots = c->fslot.as<int>() + n;
+            L.keep_exact = form0 == RPD_PREC_MIXED && ch.k + 1 >= prm->max_extra_steps;
+            if (r == RPD_OK && n_again > 0 && L.keep_exact) {
+                ClipLaunch L64 = L;
+                L64.keep_exact = false;
+                L64.fl_cnt = nullptr;
+                L64.dcnt = nullptr;
+                r = rpd_launch_finish(s, RPD_PREC_FP64, L64, n_again, 0);
+            }
+            if (r == RPD_OK && n_again > 0) r = rpd_launch_finish(s, form0, L, n_again, 0);
             if (r != RPD_OK) return r;
             if (hipEventRecord(c->ev[ch.sl][3], s) != hipSuccess || !copy_counts(ch.nxt, s)) return RPD_E_DEVICE;
             ch.end = s;

@@ -125,6 +125,7 @@ struct ClipArgs {
     int *hids;
     int H, hc;
     int *dcnt;  // debug counters of this pass (kDcStride ints), nullable
+    int keep_exact;  // finish kernel: an exact-predicate failure leaves the outputs as they are
     int count_only;  // finish kernel, triangle lists: only the union counters of the cells whose union fits
     // packed batch (nullable): the fields of request req_of[sid] replace
     // n_seeds, wmin and the domain's
@@ -1298,7 +1299,9 @@ void finish_cells_kernel(ClipArgs a, int nq, int W) {
             note_failure(a, sid, st, slot);
         }
     };
-    auto fail = [&](int st) { finish(st, 0.0, 0.0, 0.0, 0.0); };
+    auto fail = [&](int st) {
+        if (!(a.keep_exact && exact_failure(st))) finish(st, 0.0, 0.0, 0.0, 0.0);
+    };
 
     // vertex coordinates in the geometry precision RP: the registers when
     // R == RP, else recomputed from the stored RP planes
@@ -2364,6 +2367,7 @@ static int make_args(int form, const ClipLaunch &L, ClipArgs &a) {
     a.req_of = L.req_of;
     a.slots = L.slots;
     a.fl_slot = L.fl_slot;
+    a.keep_exact = L.keep_exact ? 1 : 0;
     return RPD_OK;
 }
 

@@ -212,6 +212,9 @@ struct ClipLaunch {
     // out as fl_eo)
     const int *slots;
     int *fl_slot;
+    // finish kernel: a cell that ends with an exact-predicate failure leaves
+    // its outputs as they are
+    bool keep_exact;
     // finish kernel: the P and V the records were written with (0: P, V)
     int rec_P, rec_V;
 };

@@ -3,6 +3,8 @@ pass repeats what cannot change."""
 import numpy as np
 import pytest
 
+from meshes import icosphere
+
 pytestmark = pytest.mark.gpu
 
 
@@ -79,3 +81,27 @@ def test_exact_failures_end_in_fp64(rpd, ctx, n):
     assert (out[0][0] == 2).any()
     assert np.array_equal(out[0][0], out[1][0])
     assert out[1][1] <= out[0][1] + 1
+
+
+@pytest.mark.parametrize("steps", [1, 5])
+def test_overflows_do_not_see_other_requests_failures(rpd, ctx, steps):
+    """Cells that meet more triangles than the cap finish in a second pass, in
+    the form of the first; a batch's other request, whose cells fail the exact
+    predicates there, changes none of their bits."""
+    P, T = icosphere(4, radius=2.0, rot_seed=11)
+    mesh = ctx.domain(rpd.Grid.mesh(P, T, 64))
+    vox = ctx.domain(rpd.Grid.shape(rpd.SHAPE_SPHERE, 32, (0.5, 0.5, 0.5, 0.45)))
+    x = rpd.generate_seeds(rpd.SEEDS_UNIFORM, 300, seed=1, wmax=0.0)
+    y = rpd.generate_seeds(rpd.SEEDS_UNIFORM, 20000, seed=2, wmax=0.0)
+    caps = dict(K=128, P=100, V=64, precision=1, apex_mode=0, max_extra_steps=steps)
+    ctx.set_seeds(y)
+    assert ctx.solve(vox, **caps)["fallback_cells"] > 0
+    ctx.set_seeds(x)
+    st = ctx.solve(mesh, **caps)
+    alone, status = ctx.moments(), ctx.status()
+    _, (got, _) = ctx.solve_batch([(mesh, x), (vox, y)], **caps)
+    both = ctx.status()[:300]
+    mesh.close()
+    vox.close()
+    assert st["passes"] > 1 and st["fallback_cells"] == 0 and st["pass_caps"][1][3] > st["pass_caps"][0][3]
+    assert np.array_equal(status, both) and np.array_equal(got, alone)
