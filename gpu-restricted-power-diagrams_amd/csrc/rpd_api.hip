@@ -999,8 +999,9 @@ static int solve_impl(rpd_ctx *c, rpd_domain *dom, const rpd_params *prm, rpd_st
     // with re-queue passes allowed: without them an overflow is the answer.
     if (prm->max_extra_steps > 0 && !hess && P < kPlaneFloor)
         P = rpd_clip_plane_room(form0, P, V, std::max(T, kTriangleFloor), kPlaneFloor);
-    // the restriction goes by voxel faces when every domain has them
-    bool vox = !dom || dom->dev.vface;
+    // the restriction goes by voxel faces when every domain has them, but for
+    // the reference's corner apex and the FP32 form's own passes
+    bool vox = (!dom || dom->dev.vface) && prm->apex_mode == 1;
     int t_floor = dom ? strip_floor(dom->dev.g, n) : kTriangleFloor;
     for (const auto &q : c->batch) {
         if (!q.dom) continue;

@@ -2468,11 +2468,11 @@ int rpd_launch_finish(hipStream_t st, int form, const ClipLaunch &L, int nq, int
     // (re-queue passes) spread each cell over W waves.
     const size_t pl = plane_bytes(form);
     const bool hess = a.H > 0;
-    // Domains of voxel faces (of every request of a batch) restrict by strips;
-    // the FP32 form and the reference's corner apex take the triangle lists.
+    // Domains of voxel faces restrict by strips (L.vox); the FP32 form takes
+    // the triangle lists.
     // The debug counters count triangles: with strips, a launch of the
     // triangle form for the union's counters alone follows.
-    const bool vox = L.vox && form != RPD_PREC_FP32 && a.apex_mode == 1;
+    const bool vox = L.vox && form != RPD_PREC_FP32;
     // waves per cell from the cells that share the device: this queue's and
     // those of finish kernels running beside it (the Hessian variant: one wave
     // per cell).  Every wave of a cell sets the cell up anew, so one wave is

@@ -182,7 +182,8 @@ struct ClipLaunch {
     double wmin;
     bool cull;
     const DomainDev *dom;  // nullptr: no domain
-    bool vox;              // every domain of the launch has voxel faces (DomainDev::vface)
+    bool vox;              // by strips of voxel faces (every domain of the launch has them: DomainDev::vface;
+                           // not with the reference's corner apex)
     double4 *out;          // original order
     int *status;           // original order
     int *kused;            // original order (nullable)
