@@ -999,16 +999,23 @@ static int solve_impl(rpd_ctx *c, rpd_domain *dom, const rpd_params *prm, rpd_st
     // with re-queue passes allowed: without them an overflow is the answer.
     if (prm->max_extra_steps > 0 && !hess && P < kPlaneFloor)
         P = rpd_clip_plane_room(form0, P, V, std::max(T, kTriangleFloor), kPlaneFloor);
-    // the restriction goes by voxel faces when every domain has them, but for
-    // the reference's corner apex and the FP32 form's own passes
-    bool vox = (!dom || dom->dev.vface) && prm->apex_mode == 1;
-    int t_floor = dom ? strip_floor(dom->dev.g, n) : kTriangleFloor;
-    for (const auto &q : c->batch) {
-        if (!q.dom) continue;
-        vox = vox && q.dom->dev.vface;
-        t_floor = std::max(t_floor, strip_floor(q.dom->dev.g, q.n));
-    }
-    if (!vox || form0 == RPD_PREC_FP32) t_floor = kTriangleFloor;
+    // Domains of voxel faces are restricted by them, others by their triangle
+    // lists (so are all with the reference's corner apex and in the FP32
+    // form's own passes), in a batch each request as alone.
+    bool vox = false, lists = false;
+    int t_floor = kTriangleFloor;
+    auto add_domain = [&](const rpd_domain *d, int64_t seeds) {
+        if (!d) return;
+        if (!d->dev.vface || prm->apex_mode != 1) {
+            lists = true;
+            return;
+        }
+        vox = true;
+        if (form0 != RPD_PREC_FP32) t_floor = std::max(t_floor, strip_floor(d->dev.g, seeds));
+    };
+    add_domain(dom, n);
+    for (const auto &q : c->batch) add_domain(q.dom, q.n);
+    if (!lists && prm->apex_mode == 1) vox = true;  // (no domain at all: the kernel with less LDS a cell)
     T = std::max(T, std::min(t_floor, rpd_clip_max_T(form0, P, V, hess)));
     // Likewise the vertex cap is the room of the vertex slots it needs
     // (64 per slot): a cap below it saves nothing.
@@ -1266,6 +1273,7 @@ static int solve_impl(rpd_ctx *c, rpd_domain *dom, const rpd_params *prm, rpd_st
         L.cull = prm->cull != 0;
         L.dom = dd;
         L.vox = vox;
+        L.lists = lists;
         L.out = c->out.as<double4>();
         L.status = c->status.as<int>();
         L.kused = c->kused.as<int>();
@@ -1695,6 +1703,7 @@ static int solve_impl(rpd_ctx *c, rpd_domain *dom, const rpd_params *prm, rpd_st
         L.cull = prm->cull != 0;
         L.dom = dd;
         L.vox = vox;
+        L.lists = lists;
         L.out = c->out.as<double4>();
         L.status = c->status.as<int>();
         L.kused = c->kused.as<int>();

@@ -126,6 +126,9 @@ struct ClipArgs {
     int H, hc;
     int *dcnt;  // debug counters of this pass (kDcStride ints), nullable
     int keep_exact;  // finish kernel: an exact-predicate failure leaves the outputs as they are
+    // finish kernel, a batch with both kinds of domains: 1 only the cells of
+    // requests with voxel faces (or no domain), 2 only the others
+    int only;
     int count_only;  // finish kernel, triangle lists: only the union counters of the cells whose union fits
     // packed batch (nullable): the fields of request req_of[sid] replace
     // n_seeds, wmin and the domain's
@@ -1268,7 +1271,10 @@ void finish_cells_kernel(ClipArgs a, int nq, int W) {
     const char *rec = a.rec + size_t(slot) * size_t(a.rec_stride);
     const RecHeader hd = *reinterpret_cast<const RecHeader *>(rec);
     const int sid = uni(hd.sid);
-    if constexpr (BATCH) bind_request(a, sid);
+    if constexpr (BATCH) {
+        bind_request(a, sid);
+        if (a.only && (a.only == 1) != (a.vface != nullptr || a.g == 0)) return;
+    }
     const int kused = uni(hd.kused);
     const int nent = uni(hd.nent);
     c.nb_plane = uni(hd.nb_plane);
@@ -2469,7 +2475,9 @@ int rpd_launch_finish(hipStream_t st, int form, const ClipLaunch &L, int nq, int
     const size_t pl = plane_bytes(form);
     const bool hess = a.H > 0;
     // Domains of voxel faces restrict by strips (L.vox); the FP32 form takes
-    // the triangle lists.
+    // the triangle lists.  A batch with both kinds takes two launches: in one,
+    // by triangle lists, its voxel requests' bits and speed would depend on
+    // what they are packed with.
     // The debug counters count triangles: with strips, a launch of the
     // triangle form for the union's counters alone follows.
     const bool vox = L.vox && form != RPD_PREC_FP32;
@@ -2536,13 +2544,19 @@ int rpd_launch_finish(hipStream_t st, int form, const ClipLaunch &L, int nq, int
 #undef RPD_CLIP_B2
         return RPD_OK;
     };
-    const int rl = launch(vox, hess);
-    if (rl != RPD_OK) return rl;
-    if (vox && a.dcnt) {
+    const bool both = vox && L.lists;
+    a.only = both ? 1 : 0;
+    int rl = launch(vox, hess);
+    if (rl == RPD_OK && both) {
+        a.only = 2;
+        rl = launch(false, hess);
+    }
+    if (rl == RPD_OK && vox && a.dcnt) {
+        a.only = both ? 1 : 0;
         a.count_only = 1;
         a.T = 0;
-        const int rc = launch(false, false);
-        if (rc != RPD_OK) return rc;
+        rl = launch(false, false);
     }
+    if (rl != RPD_OK) return rl;
     return hipGetLastError() == hipSuccess ? RPD_OK : RPD_E_DEVICE;
 }

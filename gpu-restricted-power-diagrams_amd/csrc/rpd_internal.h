@@ -182,8 +182,8 @@ struct ClipLaunch {
     double wmin;
     bool cull;
     const DomainDev *dom;  // nullptr: no domain
-    bool vox;              // by strips of voxel faces (every domain of the launch has them: DomainDev::vface;
-                           // not with the reference's corner apex)
+    bool vox, lists;       // domains of the launch that are restricted by strips of voxel faces
+                           // (DomainDev::vface), and by triangle lists; a batch may have both
     double4 *out;          // original order
     int *status;           // original order
     int *kused;            // original order (nullable)
