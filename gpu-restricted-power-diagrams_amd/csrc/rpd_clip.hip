@@ -2488,6 +2488,12 @@ int rpd_launch_finish(hipStream_t st, int form, const ClipLaunch &L, int nq, int
     // 20,676 blue-noise cells at two waves 0.28, at one 0.21 ms); 8 up to half
     // of that (947 cells that meet hundreds of strips, those above 256 in
     // further passes: 8 waves 0.91, 2 waves 0.98 ms for the solve).
+    // With triangle lists the heaviest cells cost several times as much, and
+    // they set the launch's time for longer: more waves up to eight times the
+    // queue (uniform seeds, the solve: 30,000 in a torus mesh at 100^3 590 ->
+    // 525 us, FP64 695 -> 592; FP32, 30,000 in a voxel torus 1,185 -> 925;
+    // 20,000 blue-noise seeds in a sphere mesh, whose cells are all alike, 404
+    // -> 426).
     const int64_t load = int64_t(nq) + std::max(beside, 0);
     auto launch = [&](bool vx, bool hs) -> int {
         const size_t wstride =
@@ -2496,7 +2502,9 @@ int rpd_launch_finish(hipStream_t st, int form, const ClipLaunch &L, int nq, int
             (hs ? hessian_wave_lds(L.P + (vx ? 1 : 0), S) : 0);
         const size_t kLdsMax = lds_limit();
         if (finish_cell_stride(a.T, 1) + wstride > kLdsMax) return RPD_E_LIMIT;
-        int W = hs || a.count_only || load > 4096 ? 1 : (load <= 2048 ? 8 : 2);
+        int W = 1;
+        if (!hs && !a.count_only)
+            W = load <= 2048 ? 8 : (vx ? (load <= 4096 ? 2 : 1) : (load <= 8192 ? 4 : (load <= 32768 ? 2 : 1)));
         while (W > 1 && finish_cell_stride(a.T, W) + W * wstride > kLdsMax) W >>= 1;
         a.lds_stride = int(wstride);
         a.cell_stride = int(finish_cell_stride(a.T, W));
