@@ -1237,12 +1237,13 @@ static int solve_impl(rpd_ctx *c, rpd_domain *dom, const rpd_params *prm, rpd_st
     // the mixed form would mostly fail them again, on every step left (corner
     // apex, 10,000 to 300,000 seeds in a torus at 100^3, where 0.5% of the
     // cells have cone planes through lattice points: 6 passes instead of 4).
+    // So do, with the corner apex, all cells computed again.
     const int finish_form_fp64 = form0 == RPD_PREC_MIXED && !hess ? RPD_PREC_MIXED : RPD_PREC_FP64;
     // A re-queue pass's kernels: kNN, bisector kernel and finish kernel (over
     // every cell of the pass: those the bisector kernel did not queue are left
-    // out on the device, so nothing waits for a count).  The first n_exact of
-    // its cells are exact-predicate failures.
-    auto pass_run = [&](Pass &ps, const int *ids, int64_t n_exact, int fl_out, const Resume &rz, int beside,
+    // out on the device, so nothing waits for a count).  The first n_fp64 of
+    // its cells finish in FP64.
+    auto pass_run = [&](Pass &ps, const int *ids, int64_t n_fp64, int fl_out, const Resume &rz, int beside,
                         ClipLaunch &L) -> int {
         const int sl = ps.slot;
         hipStream_t s = c->streams[sl];
@@ -1301,7 +1302,7 @@ static int solve_impl(rpd_ctx *c, rpd_domain *dom, const rpd_params *prm, rpd_st
         L.req_of = req_of;
         r = rpd_launch_cells(s, ps.form, L);
         const int fin = ps.form == RPD_PREC_FP64 ? finish_form_fp64 : ps.form;
-        const int64_t n64 = fin == RPD_PREC_FP64 ? 0 : n_exact;
+        const int64_t n64 = fin == RPD_PREC_FP64 ? 0 : n_fp64;
         if (r == RPD_OK && n64 > 0)
             r = rpd_launch_finish(s, RPD_PREC_FP64, L, int(n64), beside + int(ps.n_ids - n64));
         if (r == RPD_OK && n64 < ps.n_ids) {
@@ -1586,7 +1587,8 @@ static int solve_impl(rpd_ctx *c, rpd_domain *dom, const rpd_params *prm, rpd_st
             Resume rr = ch.rz;
             rr.out_base = int(ch.n_res);
             // exact entries and (when recomputed) the overflows are one range
-            r = pass_run(ch.pz, c->fl[ch.cur].eo.as<int>() + n - n_exact, n_exact, ch.nxt, rr, beside, ch.Lz);
+            r = pass_run(ch.pz, c->fl[ch.cur].eo.as<int>() + n - n_exact, prm->apex_mode == 1 ? n_exact : ch.n_scr,
+                         ch.nxt, rr, beside, ch.Lz);
             if (r == RPD_OK) r = pass_lists(ch.pz, ch.Lz, c->pb[ch.sl2], ch.nxt, ch.n_res == 0, nullptr);
             if (r != RPD_OK) return r;
             ch.end = s2;
