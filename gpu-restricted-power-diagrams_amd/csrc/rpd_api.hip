@@ -2091,57 +2091,89 @@ int compact_device(rpd_ctx *c, double keep_volume, int32_t keep_distance) {
         HIPCHK(c, hipMemcpyAsync(&cnt, c->cnt.ptr, sizeof(int), hipMemcpyDeviceToHost, s));
         HIPCHK(c, hipStreamSynchronize(s));
         if (cnt <= 0) break;
-        int K = std::min<int64_t>(std::max(c->last_K, 1), n - 1), P = c->last_P, V = c->last_V;
-        for (int step = 0; cnt > 0 && step <= std::max(c->last_steps, 0); ++step) {
-            PassBufs &b = c->pb[0];
+        // A pass lists at most 256 neighbours (the kNN's limit).  Cells that
+        // overflow are computed again with grown caps, those whose list runs
+        // out go on from their states (as in a solve's re-queue passes, but
+        // one stream): the failures of a pass go to list fl[1 - cur], its
+        // states to rs[1 - cur], where the next pass finds them.
+        int K = int(std::min<int64_t>({int64_t(std::max(c->last_K, 1)), int64_t(256), n - 1}));
+        int P = c->last_P, V = c->last_V;
+        int n_scr = cnt, n_res = 0, cur = 0, more = 0, in_P = 0;
+        size_t in_stride = 0;
+        const int *ids = c->ids1.as<int>();
+        for (int step = 0; n_scr + n_res > 0 && step <= std::max(c->last_steps, 0); ++step) {
             const size_t stride = rpd_clip_record_bytes(RPD_PREC_FP64, P, V);
-            RPDCHK(c, b.ensure(cnt, K, stride), "alloc records");
-            HIPCHK(c, hipMemsetAsync(c->fl[0].cnt.ptr, 0, kFailCounters * sizeof(int), s));
-            RPDCHK(c,
-                   rpd_launch_knn(s, c->bin_prec, c->stored.ptr, c->perm.as<int>(), c->counters.as<int>(), c->dim,
-                                  c->ids1.as<int>(), cnt, K, b.knn.as<int>()),
-                   "bordering knn");
-            ClipLaunch L{};
-            L.seeds = c->stored64.as<double4>();
-            L.perm = c->perm.as<int>();
-            L.ids = c->ids1.as<int>();
-            L.knn = b.knn.as<int>();
-            L.n_ids = cnt;
-            L.n_seeds = n;
-            L.K = K;
-            L.P = P;
-            L.V = V;
-            L.T = 1;
-            L.apex_mode = 1;
-            L.security_mode = c->last_sm;
-            L.wmin = c->wmin_ok && c->wmin < INFINITY ? c->wmin : 0.0;
-            L.cull = false;
-            L.dom = nullptr;
-            L.out = c->bout.as<double4>();
-            L.status = c->bstatus.as<int>();
-            L.rec = b.rec.ptr;
-            L.code = b.code.as<uint8_t>();
-            RPDCHK(c, rpd_launch_cells(s, RPD_PREC_FP64, L), "bordering cells");
-            RPDCHK(c,
-                   rpd_launch_lists(s, L, FailLists{c->fl[0].cnt.as<int>(), c->fl[0].eo.as<int>() + n,
-                                                    c->fl[0].sec.as<int>(), b.q.as<int>(), nullptr, nullptr}),
-                   "bordering cells");
-            HIPCHK(c, hipMemcpyAsync(c->pin + kPinCounters, c->fl[0].cnt.ptr, kFailCounters * sizeof(int),
+            const int nxt = 1 - cur;
+            FailBufs &fl = c->fl[nxt];
+            RPDCHK(c, c->rs[nxt].ensure(size_t(n_scr + n_res) * stride), "alloc bordering states");
+            HIPCHK(c, hipMemsetAsync(fl.cnt.ptr, 0, kFailCounters * sizeof(int), s));
+            auto pass = [&](const int *pass_ids, int np, int Kp, bool resume, int base) -> int {
+                PassBufs &b = c->pb[0];
+                if (np <= 0) return RPD_OK;
+                RPDCHK(c, b.ensure(np, Kp, stride), "alloc records");
+                RPDCHK(c,
+                       rpd_launch_knn(s, c->bin_prec, c->stored.ptr, c->perm.as<int>(), c->counters.as<int>(), c->dim,
+                                      pass_ids, np, Kp, b.knn.as<int>(), resume ? c->lastnb.as<int>() : nullptr),
+                       "bordering knn");
+                ClipLaunch L{};
+                L.seeds = c->stored64.as<double4>();
+                L.perm = c->perm.as<int>();
+                L.ids = pass_ids;
+                L.knn = b.knn.as<int>();
+                L.n_ids = np;
+                L.n_seeds = n;
+                L.K = Kp;
+                L.P = P;
+                L.V = V;
+                L.T = 1;
+                L.apex_mode = 1;
+                L.security_mode = c->last_sm;
+                L.wmin = c->wmin_ok && c->wmin < INFINITY ? c->wmin : 0.0;
+                L.cull = false;
+                L.dom = nullptr;
+                L.out = c->bout.as<double4>();
+                L.status = c->bstatus.as<int>();
+                L.rec = b.rec.ptr;
+                L.code = b.code.as<uint8_t>();
+                L.rs_out = static_cast<char *>(c->rs[nxt].ptr);
+                L.rs_out_stride = int(stride);
+                L.rs_base = base;
+                L.rslot = c->rslot.as<int>();
+                L.lastnb = c->lastnb.as<int>();
+                if (resume) {
+                    L.rs_in = static_cast<const char *>(c->rs[cur].ptr);
+                    L.rs_in_stride = int(in_stride);
+                    L.rs_in_P = in_P;
+                }
+                RPDCHK(c, rpd_launch_cells(s, RPD_PREC_FP64, L), "bordering cells");
+                RPDCHK(c,
+                       rpd_launch_lists(s, L, FailLists{fl.cnt.as<int>(), fl.eo.as<int>() + n, fl.sec.as<int>(),
+                                                        b.q.as<int>(), nullptr, nullptr}),
+                       "bordering cells");
+                const int S = V <= 64 ? 1 : (V <= 128 ? 2 : 4);
+                mark_neighbours_kernel<<<unsigned((np + 3) / 4), 256, 0, s>>>(
+                    static_cast<const char *>(b.rec.ptr), int(stride), P, S, np, c->used.as<int>(), k + 1);
+                HIPCHK(c, hipGetLastError());
+                return RPD_OK;
+            };
+            int r = pass(c->fl[cur].sec.as<int>(), n_res, more, true, 0);
+            if (r == RPD_OK) r = pass(ids, n_scr, std::min(K, 256), false, n_res);
+            if (r != RPD_OK) return r;
+            HIPCHK(c, hipMemcpyAsync(c->pin + kPinCounters, fl.cnt.ptr, kFailCounters * sizeof(int),
                                      hipMemcpyDeviceToHost, s));
-            const int S = V <= 64 ? 1 : (V <= 128 ? 2 : 4);
-            mark_neighbours_kernel<<<unsigned((cnt + 3) / 4), 256, 0, s>>>(
-                static_cast<const char *>(b.rec.ptr), int(stride), P, S, cnt, c->used.as<int>(), k + 1);
             HIPCHK(c, hipStreamSynchronize(s));
-            // cells that overflowed or ran out of neighbours: again with grown caps
+            in_stride = stride;
+            in_P = P;
             const int *h = c->pin + kPinCounters + 2;
-            const int n_over = c->pin[kPinCounters + 1];
-            if (n_over <= 0) break;
             if (h[RPD_VERTEX_OVERFLOW]) V = std::min(256, int(V * 1.5));
             if (h[RPD_PLANE_OVERFLOW]) P = std::min(255, int(P * 1.5));
-            if (h[RPD_SECURITY_RADIUS_NOT_REACHED]) K = int(std::min<int64_t>(n - 1, std::min(256, 2 * K)));
-            HIPCHK(c, hipMemcpyAsync(c->ids1.ptr, c->fl[0].eo.as<int>() + n, size_t(n_over) * 4,
-                                     hipMemcpyDeviceToDevice, s));
-            cnt = n_over;
+            // (the list holds at most 256 more, and every other seed in all)
+            more = int(std::min<int64_t>(n - 1, std::min(256, K)));
+            K = int(std::min<int64_t>(n - 1, int64_t(K) + more));
+            n_res = c->pin[kPinCounters + 14];
+            n_scr = c->pin[kPinCounters + 1];
+            ids = fl.eo.as<int>() + n;
+            cur = nxt;
         }
         HIPCHK(c, hipStreamSynchronize(s));
     }
