@@ -950,6 +950,75 @@ int rpd_knn_device_noalloc(rpd_ctx *c, const double *d_xyzw, int64_t n, int32_t 
     return RPD_OK;
 }
 
+// The caps of a solve's first pass, over n seeds: those of the parameters,
+// raised where that costs nothing (the triangle cap apart), and the number of
+// neighbours a cell may use in all.
+struct FirstCaps {
+    int K, P, V;
+    int64_t k_reach;
+};
+static FirstCaps first_caps(const rpd_params *prm, int64_t n) {
+    const int form0 = prm->precision;
+    int K = int(std::min<int64_t>(prm->K, n - 1)), P = prm->P, V = prm->V;
+    // The neighbour cap is raised to a wavefront's 64 where it is lower: the
+    // kNN of 64 neighbours uses the same selection buffer as that of 20 (59
+    // against 48 us for 21,000 FP64 queries), the bisector kernel loads 64
+    // neighbours at once in any case, and a lower cap only sends cells to
+    // further passes (100,000 seeds in a torus at 100^3, K = 20: 87% of the
+    // cells a second time; solve 1.46 -> 0.98 ms, K = 25 0.90 of 1.29 ms,
+    // 300,000 seeds at K = 50 4.9 -> 4.7 ms).
+    // Not in the FP32 form, whose re-queue passes are FP64.  The number of
+    // neighbours a cell may use in all stays what K and the passes allow
+    // (k_reach: K doubled, by at most 256, once a pass): running out of them
+    // is an answer, not a matter of how they were listed.
+    int64_t k_reach = K;
+    for (int k = 0; k < prm->max_extra_steps && k_reach < n - 1; ++k)
+        k_reach = std::min<int64_t>(n - 1, k_reach + std::min<int64_t>(k_reach, 256));
+    if (form0 != RPD_PREC_FP32 && K < kNeighbourFloor && k_reach > kNeighbourFloor) K = kNeighbourFloor;
+    // The plane cap is raised toward kPlaneFloor as far as the bisector and
+    // finish kernels keep their residency: the restriction's cone clips add
+    // up to 4 planes to a cell, which pushed the cells closest to the cap
+    // into an FP64 finish pass of their own (6 cells at P = 40 at the 1M
+    // torus, which also grew the bisector failures' pass to P = 60).  Only
+    // with re-queue passes allowed: without them an overflow is the answer.
+    if (prm->max_extra_steps > 0 && prm->H <= 0 && P < kPlaneFloor)
+        P = rpd_clip_plane_room(form0, P, V, std::max(prm->T, kTriangleFloor), kPlaneFloor);
+    // Likewise the vertex cap is the room of the vertex slots it needs
+    // (64 per slot): a cap below it saves nothing.
+    V = V <= 64 ? 64 : (V <= 128 ? 128 : 256);
+    return FirstCaps{K, P, V, k_reach};
+}
+
+// Device bytes that a solve of n seeds holds at its peak, as a server counts a
+// request.  Per seed: the seeds (32) and their two sorted copies (64),
+// permutation and kNN grid (6), outputs, status and K used (40), pass 1's ids
+// (4), six failure lists (72) and the record slots of one (8), resume slots and
+// last neighbours (8), the request (2), binning scratch (24); pass 1's kNN
+// list, record and code; then, for the cells that go on, a list of twice the
+// neighbours, an FP64 record and the kept state, with the next larger room for
+// vertices where more than one step may follow.  Those are counted for half of
+// the cells where the first list holds a wavefront's neighbours, for every
+// cell where it is shorter (20 neighbours: 98% of uniform seeds go on) and
+// half as many again where they may go on twice; and 24 MB for what some 40
+// allocations round up to.  Measured (10^6 uniform seeds in a cube, bytes a
+// seed, counted and held): K 25, mixed 5,823 and 3,223; K 20, one step, FP64
+// 7,295 and 7,109; K 25, FP32 10,480 and 7,632.
+extern "C" int64_t rpd_solve_bytes(int64_t n, const rpd_params *prm) {
+    rpd_params p = *prm;  // (not checked yet)
+    p.precision = std::max(0, std::min(2, p.precision));
+    p.K = std::max(1, std::min(256, p.K));
+    p.P = std::max(7, std::min(255, p.P));
+    p.V = std::max(8, std::min(256, p.V));
+    p.T = std::max(0, p.T);
+    const FirstCaps fc = first_caps(&p, INT32_MAX);  // (a batch has more seeds than the request)
+    const int64_t first = 4 * fc.K + int64_t(rpd_clip_record_bytes(p.precision, fc.P, fc.V)) + 1;
+    const int V2 = p.max_extra_steps > 1 ? std::min(256, 2 * fc.V) : fc.V;
+    const int64_t rec2 = int64_t(rpd_clip_record_bytes(RPD_PREC_FP64, fc.P, V2));
+    const int64_t again = 4 * std::min(256, 2 * fc.K) + rec2 + 1 + rec2;
+    const int64_t half = p.max_extra_steps <= 0 ? 0 : (fc.K >= kNeighbourFloor ? 1 : (p.max_extra_steps > 1 ? 3 : 2));
+    return n * (260 + first) + n * half * again / 2 + (int64_t(24) << 20);
+}
+
 // The solve of the context's seeds: one diagram (against dom), or the packed
 // batch rpd_solve_batch has set up (dom null, each request's domain in its
 // descriptor).
@@ -970,35 +1039,14 @@ static int solve_impl(rpd_ctx *c, rpd_domain *dom, const rpd_params *prm, rpd_st
     const int64_t n = c->n;
     const int form0 = prm->precision;
     const int kprec = form0 == RPD_PREC_FP64 ? 1 : 0;
-    int K = std::min<int64_t>(prm->K, n - 1), P = prm->P, V = prm->V, T = prm->T;
-    // The neighbour cap is raised to a wavefront's 64 where it is lower: the
-    // kNN of 64 neighbours uses the same selection buffer as that of 20 (59
-    // against 48 us for 21,000 FP64 queries), the bisector kernel loads 64
-    // neighbours at once in any case, and a lower cap only sends cells to
-    // further passes (100,000 seeds in a torus at 100^3, K = 20: 87% of the
-    // cells a second time; solve 1.46 -> 0.98 ms, K = 25 0.90 of 1.29 ms,
-    // 300,000 seeds at K = 50 4.9 -> 4.7 ms).
-    // Not in the FP32 form, whose re-queue passes are FP64.  The number of
-    // neighbours a cell may use in all stays what K and the passes allow
-    // (k_reach: K doubled, by at most 256, once a pass): running out of them
-    // is an answer, not a matter of how they were listed.
-    int64_t k_reach = K;
-    for (int k = 0; k < prm->max_extra_steps && k_reach < n - 1; ++k)
-        k_reach = std::min<int64_t>(n - 1, k_reach + std::min<int64_t>(k_reach, 256));
-    if (form0 != RPD_PREC_FP32 && K < kNeighbourFloor && k_reach > kNeighbourFloor) K = kNeighbourFloor;
+    const FirstCaps fc = first_caps(prm, n);
+    const int64_t k_reach = fc.k_reach;
+    int K = fc.K, P = fc.P, V = fc.V, T = prm->T;
     // The triangle cap is raised to kTriangleFloor where it is lower: a cell
     // done by one wave keeps 4 bytes of LDS per union entry, which costs the
     // finish kernel no residency, and a cell's result does not depend on the
     // cap it succeeds with; a lower cap only sends cells to re-queue passes.
     const bool hess = prm->H > 0;
-    // The plane cap likewise, toward kPlaneFloor as far as the bisector and
-    // finish kernels keep their residency: the restriction's cone clips add
-    // up to 4 planes to a cell, which pushed the cells closest to the cap
-    // into an FP64 finish pass of their own (6 cells at P = 40 at the 1M
-    // torus, which also grew the bisector failures' pass to P = 60).  Only
-    // with re-queue passes allowed: without them an overflow is the answer.
-    if (prm->max_extra_steps > 0 && !hess && P < kPlaneFloor)
-        P = rpd_clip_plane_room(form0, P, V, std::max(T, kTriangleFloor), kPlaneFloor);
     // Domains of voxel faces are restricted by them, others by their triangle
     // lists (so are all with the reference's corner apex and in the FP32
     // form's own passes), in a batch each request as alone.
@@ -1017,9 +1065,6 @@ static int solve_impl(rpd_ctx *c, rpd_domain *dom, const rpd_params *prm, rpd_st
     for (const auto &q : c->batch) add_domain(q.dom, q.n);
     if (!lists && prm->apex_mode == 1) vox = true;  // (no domain at all: the kernel with less LDS a cell)
     T = std::max(T, std::min(t_floor, rpd_clip_max_T(form0, P, V, hess)));
-    // Likewise the vertex cap is the room of the vertex slots it needs
-    // (64 per slot): a cap below it saves nothing.
-    V = V <= 64 ? 64 : (V <= 128 ? 128 : 256);
     rpd_stats st{};
     st.n = n;
     auto t_start = std::chrono::steady_clock::now();

@@ -37,6 +37,7 @@
 
 int rpd_ctx_device(const rpd_ctx *ctx);                            // rpd_api.hip
 int rpd_create_streams(int device, int n_streams, rpd_ctx **out);  // rpd_api.hip
+extern "C" int64_t rpd_solve_bytes(int64_t n, const rpd_params *prm);  // rpd_api.hip
 
 namespace {
 
@@ -56,26 +57,11 @@ struct Request {
     double lat_ms = 0;
 };
 
-// Device bytes one solve of n seeds holds at its peak, per seed: the seeds
-// (32) and their two sorted copies (64), permutation (4), outputs, status and
-// K used (40), the pass-1 id list (4), six failure lists (72), resume slots
-// and last neighbours (8), cover flags (1), binning scratch (16), kNN lists
-// and cell records of pass 1 and, bounded by the same size, of the re-queue
-// passes that run beside it; plus the kept states of pass 1's cells whose
-// list ran out (room for 2/5 of the cells, plus 1024).
 // Seeds of one batch: requests are packed up to this total (a larger request
 // runs alone), so that the queue spreads over the slots and each batch fills
 // the device in its first pass while its re-queue tail overlaps the other
 // slots' work.
 constexpr int64_t kBatchMaxSeeds = int64_t(1) << 19;
-
-int64_t footprint_bytes(int64_t n, const rpd_params &p) {
-    const int64_t K = std::max(1, p.K), P = std::max(1, p.P);
-    const int64_t S = p.V <= 64 ? 1 : (p.V <= 128 ? 2 : 4);
-    const int64_t rec = 16 + P * 36 + 256 * S;
-    return n * (32 + 64 + 4 + 40 + 4 + 72 + 8 + 1 + 16 + 2 * (4 * K + rec)) +
-           (std::min(n, n * 2 / 5 + 1024)) * rec + (int64_t(1) << 20);
-}
 
 }  // namespace
 
@@ -231,7 +217,7 @@ int rpd_server_submit(rpd_server *s, rpd_domain *dom, const double *xyzw, int64_
     r->prm.H = 0;
     r->prm.HC = 1;
     r->seeds.assign(xyzw, xyzw + size_t(n) * 4);
-    r->footprint = footprint_bytes(n, r->prm);
+    r->footprint = rpd_solve_bytes(n, &r->prm);
     r->t_submit = Clock::now();
     {
         std::lock_guard<std::mutex> lk(s->mu);
