@@ -346,35 +346,54 @@ void domain_distance(const rpd_grid_desc *g, std::vector<uint8_t> &dist) {
 // The faces of a domain made of voxel faces (DomainDev::vface), or false: the
 // triangles are not exactly the two halves of lattice squares (corner
 // coordinates i * vs, bit for bit), oriented alike, each in the lists of the
-// voxels on both sides; or a voxel's class is unknown.  The finish kernel then
-// keeps to the triangle lists.
+// voxels on both sides; a voxel's class is unknown; or the faces are not those
+// between voxels of different class (the frame's outside counts as outside),
+// with the normal into the voxel inside: the strips take another apex than the
+// triangle lists, which makes no difference only if faces and classes agree.
+// The finish kernel then keeps to the triangle lists.
 bool voxel_faces(const rpd_grid_desc *g, const std::vector<int> &tvoffs, const std::vector<uint32_t> &tvox,
                  std::vector<int> &offs, std::vector<uint32_t> &faces) {
     const int G = g->size;
     if (!g->centre || G > 1023) return false;
-    const size_t nv = size_t(G) * G * G, nt = size_t(g->num_triangles);
-    for (size_t v = 0; v < nv; ++v)
-        if (g->centre[v] != 0 && g->centre[v] != 2) return false;
-    const double vs = 1000.0 / double(G);
+    const size_t gg = size_t(G), nv = gg * gg * gg, nt = size_t(g->num_triangles);
+    const int8_t *const cls = g->centre;
+    // every class 0 or 2; the faces between voxels of different class
+    unsigned other = 0;
+    for (size_t v = 0; v < nv; ++v) other |= uint8_t(cls[v]) & ~2u;
+    if (other) return false;
+    size_t between = 0;
+    for (size_t z = 0; z < gg; ++z)
+        for (size_t y = 0; y < gg; ++y) {
+            const int8_t *const row = cls + gg * (y + gg * z);
+            // (the row past the last one: outside)
+            const int8_t *const ry = y + 1 < gg ? row + gg : nullptr, *const rz = z + 1 < gg ? row + gg * gg : nullptr;
+            unsigned k = (row[0] != 0) + (row[gg - 1] != 0);
+            for (size_t x = 0; x + 1 < gg; ++x) k += row[x] != row[x + 1];
+            for (size_t x = 0; x < gg; ++x) {
+                k += ry ? row[x] != ry[x] : row[x] != 0;
+                k += rz ? row[x] != rz[x] : row[x] != 0;
+                k += (y == 0 && row[x] != 0) + (z == 0 && row[x] != 0);
+            }
+            between += k;
+        }
+    if (2 * between != nt) return false;
+    const double vs = 1000.0 / double(G), iv = double(G) / 1000.0;
     // lattice coordinates of the points
     std::vector<uint16_t> pt(3 * size_t(g->num_points));
     for (size_t p = 0; p < size_t(g->num_points); ++p)
         for (int k = 0; k < 3; ++k) {
             const double x = g->points[4 * p + size_t(k)];
             if (!(x >= 0.0 && x <= 1000.0 + vs)) return false;
-            const int i = int(std::lround(x / vs));
+            const int i = int(x * iv + 0.5);
             if (i > G || i * vs != x) return false;
             pt[3 * p + size_t(k)] = uint16_t(i);
         }
-    // each triangle: its face (lowest corner, axis), the corner of its right
-    // angle (2 bits) and the sign of its normal
-    const size_t G1 = size_t(G) + 1;
-    struct Half {
-        uint32_t at;  // x | y << 10 | z << 20 | axis << 30
-        uint8_t corner, up;
-    };
-    std::vector<Half> half(nt);
-    offs.assign(G1 * G1 * G1 + 1, 0);
+    // Per lattice point and axis, the face whose lowest corner it is: 0 none,
+    // kHalf and the corner of the right angle of the one half seen, or kWhole;
+    // kUp with either: the normal along the axis.
+    constexpr uint8_t kUp = 4, kHalf = 8, kWhole = 16;
+    const size_t G1 = gg + 1, np = G1 * G1 * G1;
+    std::vector<uint8_t> face(3 * np, 0);
     for (size_t t = 0; t < nt; ++t) {
         int p[3][3], lo[3], hi[3];
         for (int c = 0; c < 3; ++c)
@@ -402,67 +421,65 @@ bool voxel_faces(const rpd_grid_desc *g, const std::vector<int> &tvoffs, const s
         const int cr = (p[1][u] - p[0][u]) * (p[2][v] - p[0][v]) - (p[1][v] - p[0][v]) * (p[2][u] - p[0][u]);
         // (e_u x e_v is +e_axis for x and z, -e_axis for y)
         const bool up = (cr > 0) != (ax == 1);
-        // in the lists of the voxels on both sides
+        // the voxels on both sides: the normal points to the one inside, the
+        // other is outside, and both list the triangle
         for (int side = 0; side < 2; ++side) {
             int w[3] = {lo[0], lo[1], lo[2]};
             w[ax] -= side;
-            if (w[ax] < 0 || w[ax] >= G) continue;
+            const bool in_frame = w[ax] >= 0 && w[ax] < G;
+            if ((in_frame ? int(cls[size_t(w[0]) + gg * (size_t(w[1]) + gg * size_t(w[2]))]) : 0) !=
+                (up == (side == 0) ? 2 : 0))
+                return false;
+            if (!in_frame) continue;
             const uint32_t pv = (uint32_t(w[2]) << 20) | (uint32_t(w[1]) << 10) | uint32_t(w[0]);
             if (!std::binary_search(tvox.begin() + tvoffs[t], tvox.begin() + tvoffs[t + 1], pv)) return false;
         }
-        half[t] = Half{(uint32_t(lo[2]) << 20) | (uint32_t(lo[1]) << 10) | uint32_t(lo[0]) | (uint32_t(ax) << 30),
-                       uint8_t(missing), uint8_t(up)};
+        // two halves a face, of one orientation, with opposite right angles
+        uint8_t &f = face[3 * (size_t(lo[0]) + G1 * (size_t(lo[1]) + G1 * size_t(lo[2]))) + size_t(ax)];
+        const uint8_t mine = uint8_t(missing | (up ? kUp : 0) | kHalf);
+        if (f == 0)
+            f = mine;
+        else if (f == (mine ^ 3))
+            f = uint8_t(kWhole | (up ? kUp : 0));
+        else
+            return false;
     }
-    auto point_of = [&](uint32_t at) {
-        return size_t(at & 1023u) + G1 * (size_t((at >> 10) & 1023u) + G1 * size_t((at >> 20) & 1023u));
-    };
-    // the halves by lattice point
-    for (const Half &h : half) offs[point_of(h.at) + 1]++;
-    for (size_t i = 0; i + 1 < offs.size(); ++i) offs[i + 1] += offs[i];
-    std::vector<int> cur(offs.begin(), offs.end() - 1), by(nt);
-    for (size_t t = 0; t < nt; ++t) by[size_t(cur[point_of(half[t].at)]++)] = int(t);
-    // two halves each, of one orientation, with opposite right angles
+    // (as many halves as the faces between have, none met twice: every face is
+    // whole unless some have one half and others are missing)
     faces.clear();
     faces.reserve(nt);
-    std::vector<int> foffs(offs.size(), 0);
-    for (size_t i = 0; i + 1 < offs.size(); ++i) {
-        for (uint32_t ax = 0; ax < 3; ++ax) {
-            const Half *h[2] = {nullptr, nullptr};
-            int n = 0;
-            for (int q = offs[i]; q < offs[i + 1]; ++q) {
-                const Half &x = half[size_t(by[size_t(q)])];
-                if (x.at >> 30 != ax) continue;
-                if (n == 2) return false;
-                h[n++] = &x;
+    offs.resize(np + 1);
+    offs[0] = 0;
+    size_t i = 0;
+    for (size_t z = 0; z < G1; ++z)
+        for (size_t y = 0; y < G1; ++y)
+            for (size_t x = 0; x < G1; ++x, ++i) {
+                const uint8_t *f = &face[3 * i];
+                if (f[0] | f[1] | f[2])
+                    for (uint32_t ax = 0; ax < 3; ++ax) {
+                        if (f[ax] == 0) continue;
+                        if (!(f[ax] & kWhole)) return false;
+                        faces.push_back((uint32_t(z) << 20) | (uint32_t(y) << 10) | uint32_t(x) | (ax << 30));
+                        faces.push_back(f[ax] & kUp ? 1u : 0u);
+                    }
+                offs[i + 1] = int(faces.size() / 2);
             }
-            if (n == 0) continue;
-            if (n != 2 || h[0]->up != h[1]->up || (h[0]->corner ^ h[1]->corner) != 3) return false;
-            faces.push_back(h[0]->at);
-            faces.push_back(h[0]->up ? 1u : 0u);
-        }
-        foffs[i + 1] = int(faces.size() / 2);
-    }
-    offs.swap(foffs);
     // runs along x (faces across y or z) or y (faces across x), from the end
-    auto find = [&](size_t i, uint32_t ax) -> int {
-        for (int q = offs[i]; q < offs[i + 1]; ++q)
-            if (faces[2 * size_t(q)] >> 30 == ax) return q;
-        return -1;
-    };
-    for (size_t i = offs.size() - 1; i-- > 0;)
-        for (int q = offs[i]; q < offs[i + 1]; ++q) {
-            const uint32_t at = faces[2 * size_t(q)], ax = at >> 30;
-            const size_t next = i + (ax == 0 ? G1 : 1);
-            uint32_t run = 1;
-            if (((ax == 0 ? at >> 10 : at) & 1023u) < uint32_t(G)) {
-                const int r = find(next, ax);
-                if (r >= 0 && (faces[2 * size_t(r) + 1] & 1u) == (faces[2 * size_t(q) + 1] & 1u)) {
-                    run += faces[2 * size_t(r) + 1] >> 2;
-                    faces[2 * size_t(r) + 1] |= 2u;
-                }
+    for (size_t q = faces.size() / 2; q-- > 0;) {
+        const uint32_t at = faces[2 * q], ax = at >> 30;
+        const size_t here = size_t(at & 1023u) + G1 * (size_t((at >> 10) & 1023u) + G1 * size_t((at >> 20) & 1023u));
+        uint32_t run = 1;
+        if (((ax == 0 ? at >> 10 : at) & 1023u) < uint32_t(G)) {
+            const size_t next = here + (ax == 0 ? G1 : 1);
+            const uint8_t *f = &face[3 * next];
+            if (f[ax] == face[3 * here + ax]) {
+                const size_t r = size_t(offs[next]) + (ax > 0 && f[0]) + (ax > 1 && f[1]);
+                run += faces[2 * r + 1] >> 2;
+                faces[2 * r + 1] |= 2u;
             }
-            faces[2 * size_t(q) + 1] |= run << 2;
         }
+        faces[2 * q + 1] |= run << 2;
+    }
     return true;
 }
 

@@ -1,5 +1,7 @@
 """Which way a call's cells are restricted: by strips of voxel faces or by
 triangle lists, and with which caps."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -51,3 +53,41 @@ def test_batch_of_both_kinds_of_domains(rpd, ctx, prec, apex):
     assert np.array_equal(got, np.concatenate(status))
     for k, (o, m) in enumerate(zip(outs, alone)):
         assert np.array_equal(o, m, equal_nan=True), "request %d" % k
+
+
+@pytest.mark.parametrize("prec", [0, 1])
+@pytest.mark.parametrize("what", ["class", "open"])
+def test_faces_that_do_not_bound_the_classes(rpd, ctx, prec, what):
+    """Strips take another apex than the triangle lists, which is the same cell
+    only if the faces are those between inside and outside voxels.  Where they
+    are not (a class that says otherwise, a surface with holes) the result is
+    that of the lists: of the same domain with a point off the lattice."""
+    g, n = 8, 300
+    x = rpd.generate_seeds(rpd.SEEDS_UNIFORM, n, seed=n, wmax=0.0)
+    rng = np.random.default_rng(1)
+    mask = np.ones((g, g, g), np.uint8)
+    mask[2:6, 3:5, 1:4] = 0
+    flips = rng.choice(g ** 3, 60, replace=False)
+    ctx.set_seeds(x)
+    out = []
+    for off in (False, True):
+        grid = rpd.Grid.voxels(mask.reshape(-1))
+        d = grid.desc
+        if what == "class":
+            c = np.ctypeslib.as_array(ctypes.cast(d.centre, ctypes.POINTER(ctypes.c_int8)), (g ** 3,))
+            c[flips] = 2 - c[flips]
+        else:  # faces turned over: as many triangles, all in the lists
+            t = np.ctypeslib.as_array(ctypes.cast(d.triangles, ctypes.POINTER(ctypes.c_int32)), (d.num_triangles, 3))
+            k = rng.choice(d.num_triangles // 2, 40, replace=False) if not off else k
+            for i in (2 * k, 2 * k + 1):
+                t[i] = t[i][:, [1, 0, 2]]
+        if off:
+            p = ctypes.cast(d.points, ctypes.POINTER(ctypes.c_double))
+            p[0] = np.nextafter(p[0], 500.0)
+        dom = ctx.domain(grid)
+        ctx.solve(dom, K=64, P=60, V=64, T=2000, precision=prec)
+        out.append((ctx.moments(), ctx.status()))
+        dom.close()
+    v = 1e9 / n
+    assert np.array_equal(out[0][1], out[1][1])
+    assert np.abs(out[0][0][:, 3] - out[1][0][:, 3]).max() <= 1e-11 * v
