@@ -1306,7 +1306,7 @@ void finish_cells_kernel(ClipArgs a, int nq, int W) {
         }
     };
     auto fail = [&](int st) {
-        if (!(a.keep_exact && exact_failure(st))) finish(st, 0.0, 0.0, 0.0, 0.0);
+        if (!(exact_failure(st) && cold_args()->keep_exact)) finish(st, 0.0, 0.0, 0.0, 0.0);
     };
 
     // vertex coordinates in the geometry precision RP: the registers when
