@@ -362,19 +362,18 @@ bool voxel_faces(const rpd_grid_desc *g, const std::vector<int> &tvoffs, const s
     for (size_t v = 0; v < nv; ++v) other |= uint8_t(cls[v]) & ~2u;
     if (other) return false;
     size_t between = 0;
+    const std::vector<int8_t> outside(gg, 0);
+    auto differ = [&](const int8_t *p, const int8_t *q, size_t m) {
+        unsigned k = 0;
+        for (size_t x = 0; x < m; ++x) k += p[x] != q[x];
+        return k;
+    };
     for (size_t z = 0; z < gg; ++z)
         for (size_t y = 0; y < gg; ++y) {
-            const int8_t *const row = cls + gg * (y + gg * z);
-            // (the row past the last one: outside)
-            const int8_t *const ry = y + 1 < gg ? row + gg : nullptr, *const rz = z + 1 < gg ? row + gg * gg : nullptr;
-            unsigned k = (row[0] != 0) + (row[gg - 1] != 0);
-            for (size_t x = 0; x + 1 < gg; ++x) k += row[x] != row[x + 1];
-            for (size_t x = 0; x < gg; ++x) {
-                k += ry ? row[x] != ry[x] : row[x] != 0;
-                k += rz ? row[x] != rz[x] : row[x] != 0;
-                k += (y == 0 && row[x] != 0) + (z == 0 && row[x] != 0);
-            }
-            between += k;
+            const int8_t *const row = cls + gg * (y + gg * z), *const out = outside.data();
+            between += differ(row, row + 1, gg - 1) + (row[0] != 0) + (row[gg - 1] != 0);
+            between += differ(row, y > 0 ? row - gg : out, gg) + (y + 1 == gg ? differ(row, out, gg) : 0);
+            between += differ(row, z > 0 ? row - gg * gg : out, gg) + (z + 1 == gg ? differ(row, out, gg) : 0);
         }
     if (2 * between != nt) return false;
     const double vs = 1000.0 / double(G), iv = double(G) / 1000.0;
@@ -450,20 +449,26 @@ bool voxel_faces(const rpd_grid_desc *g, const std::vector<int> &tvoffs, const s
     faces.reserve(nt);
     offs.resize(np + 1);
     offs[0] = 0;
-    size_t i = 0;
-    for (size_t z = 0; z < G1; ++z)
-        for (size_t y = 0; y < G1; ++y)
-            for (size_t x = 0; x < G1; ++x, ++i) {
-                const uint8_t *f = &face[3 * i];
-                if (f[0] | f[1] | f[2])
-                    for (uint32_t ax = 0; ax < 3; ++ax) {
-                        if (f[ax] == 0) continue;
-                        if (!(f[ax] & kWhole)) return false;
-                        faces.push_back((uint32_t(z) << 20) | (uint32_t(y) << 10) | uint32_t(x) | (ax << 30));
-                        faces.push_back(f[ax] & kUp ? 1u : 0u);
-                    }
-                offs[i + 1] = int(faces.size() / 2);
+    for (size_t row = 0; row < G1 * G1; ++row) {
+        const uint8_t *f = &face[3 * G1 * row];
+        int *o = &offs[G1 * row + 1];
+        unsigned any = 0;
+        for (size_t x = 0; x < 3 * G1; ++x) any |= f[x];
+        if (!any) {
+            std::fill(o, o + G1, int(faces.size() / 2));
+            continue;
+        }
+        const uint32_t yz = (uint32_t(row / G1) << 20) | (uint32_t(row % G1) << 10);
+        for (size_t x = 0; x < G1; ++x, f += 3) {
+            for (uint32_t ax = 0; ax < 3; ++ax) {
+                if (f[ax] == 0) continue;
+                if (!(f[ax] & kWhole)) return false;
+                faces.push_back(yz | uint32_t(x) | (ax << 30));
+                faces.push_back(f[ax] & kUp ? 1u : 0u);
             }
+            o[x] = int(faces.size() / 2);
+        }
+    }
     // runs along x (faces across y or z) or y (faces across x), from the end
     for (size_t q = faces.size() / 2; q-- > 0;) {
         const uint32_t at = faces[2 * q], ax = at >> 30;
