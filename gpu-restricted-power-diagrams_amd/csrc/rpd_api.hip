@@ -4,28 +4,30 @@
 // Pass policy (replaces VoroAlgo::launch, voronoi.cpp:1244-1376):
 //   pass 1: every cell, caps K/P/V/T of rpd_params, in the requested form;
 //   then up to max_extra_steps re-queue passes over the failed cells only,
-//   which the kernels append to device lists:
+//   from device lists:
 //     * vertex/plane overflow -> that cap x1.5 (as the reference);
 //     * security radius not reached -> K x2 (the reference: x1.5);
 //     * triangle overflow -> T = the largest triangle union the finish
 //       kernel counted, at least T x1.5 (the reference: x1.5), within the
 //       LDS of one finish-kernel cell;
 //     * needs_exact_predicates, inconsistent_boundary and
-//       find_another_beginning_vertex from an FP32 form -> recomputed (the
-//       reference drops cells flagged only for exact predicates,
-//       voronoi.cpp:1349-1356; here they are always recomputed); from the
-//       FP64 form they are final (a recomputation fails the same way);
+//       find_another_beginning_vertex from an FP32 or the mixed form ->
+//       recomputed and finished in FP64 (the reference drops cells flagged
+//       only for exact predicates, voronoi.cpp:1349-1356); from the FP64 form
+//       they are final (a recomputation fails the same way);
 //     * empty_cell is final (volume 0);
-//   every re-queue pass runs in the FP64 form, in two chains that run at
+//   the re-queue passes are FP64, but those of a mixed solve finish in the
+//   mixed form (other than exact-predicate failures) and resume cells in it
+//   up to the last neighbours and the last step; they run in two chains at
 //   once, each growing its own caps: the failures of pass 1's bisector
 //   kernel (and theirs, and so on), whose first pass is queued before pass
 //   1's finish kernel, and the failures of that finish kernel.  The host
 //   drives both by polling their streams; small counters come back through
-//   pinned memory, so that no copy waits for a busy stream.  A cell's result does not
-//   depend on the caps it succeeds with.  A cell whose list ran out keeps its
-//   state (planes, vertices, last neighbour) when there is room; the next
-//   pass lists only the neighbours after that one and clips on from the
-//   state, which is the clip sequence of one run with the longer list.
+//   pinned memory, so that no copy waits for a busy stream.  A cell's result
+//   does not depend on the caps it succeeds with.  A cell whose list ran out
+//   keeps its state (planes, vertices, last neighbour); the next pass lists
+//   only the neighbours after that one and clips on from the state, which is
+//   the clip sequence of one run with the longer list.
 // Boundary cells are processed in the same pass as interior cells (the
 // reference defers them with a T = 0 first pass and recomputes them).
 
@@ -1287,7 +1289,7 @@ static int solve_impl(rpd_ctx *c, rpd_domain *dom, const rpd_params *prm, rpd_st
         int nq = 0;    // queued cells (pass 1)
         bool finish_only = false;  // a finish kernel over earlier records (events 1 and 3 only)
     };
-    // resumable cells: records read (in, FP64 passes) and written (out)
+    // resumable cells: records read (in) and written (out)
     struct Resume {
         const char *in = nullptr;  // the cells of this pass resume from here
         int in_stride = 0, in_P = 0;
@@ -1474,8 +1476,8 @@ static int solve_impl(rpd_ctx *c, rpd_domain *dom, const rpd_params *prm, rpd_st
     // pass 1's finish kernel run at once.  Each pass takes the failures of
     // the previous one (list cur, counters cnt): the cells whose state was
     // kept resume on stream sl (their kNN lists only the neighbours after the
-    // last one used), the others are recomputed in FP64 on stream sl2, both
-    // at once.  Pass k writes its failures to list outs[k % 2] and the states
+    // last one used), the others are recomputed, clipped in FP64, on stream
+    // sl2, both at once.  Pass k writes its failures to list outs[k % 2] and the states
     // of its resumable cells to rs buffer rsb[k % 2].
     struct Chain {
         int sl = 0, sl2 = 0, dep = 0;
@@ -1515,8 +1517,8 @@ static int solve_impl(rpd_ctx *c, rpd_domain *dom, const rpd_params *prm, rpd_st
         const int n_exact = cnt[0], n_over = cnt[1], n_sec = cnt[14];
         const Caps nc = grow(cnt, ch.cap);
         const bool caps_changed = nc.K != ch.cap.K || nc.P != ch.cap.P || nc.V != ch.cap.V || nc.T != ch.cap.T;
-        // exact-predicate failures (only listed from the FP32 forms) always
-        // go to FP64; overflows only when a cap grew; kept states when K grew
+        // exact-predicate failures (not listed from the FP64 form) always go
+        // to FP64; overflows only when a cap grew; kept states when K grew
         // (else they would run out again: they end as they are)
         ch.n_res = n_sec > 0 && ch.left.rec && nc.K > ch.cap.K ? n_sec : 0;
         ch.n_scr = n_exact + (caps_changed ? n_over : 0);

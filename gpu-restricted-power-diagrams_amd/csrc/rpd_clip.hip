@@ -21,12 +21,12 @@
 // Two kernels per pass:
 //   clip_cells_kernel   the bisector loop for every cell (light, high
 //                       occupancy).  A cell that provably misses the domain
-//                       ends there with volume 0; a finished cell is appended
-//                       to a queue as a compact record (FP64 planes + vertex
-//                       triples);
+//                       ends there with volume 0; a finished cell leaves a
+//                       compact record at its item's slot (FP64 planes, vertex
+//                       triples and adjacency);
 //   finish_cells_kernel restriction to the domain (bbox, voxels, apex, cone
-//                       clips per boundary triangle) and the integration, for
-//                       the queued cells only.
+//                       clips per strip of voxel faces or boundary triangle)
+//                       and the integration, for the cells with a record.
 //
 // Everything is in the seed-local frame (origin at the seed, FP64 inputs):
 // planes n.y + d with d = (|b|^2 + w_B - w_s) / (2|b|), b = B - s.
@@ -39,7 +39,7 @@
 // decides it: the finish kernel has FP64 planes in LDS, the bisector kernel
 // FP32 planes, beside which it makes FP64 ones when a test first needs them.
 // A cavity that such decisions leave inconsistent ends the cell with a status
-// that the host re-runs in FP64.  The records' planes are FP64; the
+// that the host re-runs in FP64 to its end.  The records' planes are FP64; the
 // cell geometry that produces the results
 // (bbox, cone planes, volume and moments) is evaluated in FP64 from them, so
 // an unflagged mixed cell has the FP64 combinatorics and FP64 geometry.  FP32
@@ -111,8 +111,8 @@ struct ClipArgs {
     // rs_out_stride bytes; the slot is kept in rslot[sid]), the stored id of
     // its last neighbour to lastnb[sid].  rs_out may be rec itself (rs_base
     // 0): an item has one record, for the finish kernel or to resume from.
-    // rs_out null: a plain overflow.  With rs_in set (FP64 form), every cell
-    // resumes from record rs_in[rslot[sid]] (written with rs_in_P planes) and
+    // rs_out null: a plain overflow.  With rs_in set (FP64 and mixed forms:
+    // records of FP64 planes), every cell resumes from record rs_in[rslot[sid]] (written with rs_in_P planes) and
     // its list holds only the neighbours after the ones it has used.
     char *rs_out;
     int rs_out_stride, rs_base;
@@ -1205,8 +1205,8 @@ __device__ __forceinline__ uint64_t box_near(int x, int y, int z, const int *mn,
 // cell, so its contribution does not depend on which wave computes it.  A
 // batch's contributions are added in increasing order, and the batches' sums
 // in the batches' order: with W = 1 as they come, with W > 1 from LDS by wave
-// 0.  Both make the same additions, so the result of a cell is the same bit
-// for bit for every W and every packed batch it is in.
+// 0.  Both make the same additions, so the result of a cell in this form is the
+// same bit for bit for every W and every packed batch it is in.
 //
 // Cone planes are built lane-parallel, 16 triangles x 4 planes per batch.  A
 // triangle one of whose four planes removes every vertex of the cell with a
@@ -1259,8 +1259,11 @@ void finish_cells_kernel(ClipArgs a, int nq, int W) {
     int *goo = nullptr;
     Pl<RP> *cpl = nullptr;
     char *tail = nullptr;
-    // VOX: a strip's fifth cone plane has room of its own, so that no cap is
-    // met earlier than with triangles
+    // VOX: a strip's fifth cone plane has room of its own, so that the plane
+    // cap is met no earlier than with triangles.  (The vertex cap is met less
+    // often: of 3,600 cells of 62 vertices in random domains, without passes
+    // to grow the cap, 362 by lists and none by strips, whose cones' planes
+    // meet in the middle of the cell, so that the first halves it.)
     const int P = VOX ? a.P + 1 : a.P;
     bind_lds(lds_raw + size_t(cpb) * a.cell_stride + size_t(wv) * a.lds_stride, P, c, nullptr, &cpl, &goo, &tail);
     double *tcor = reinterpret_cast<double *>(tail);  // (not VOX)

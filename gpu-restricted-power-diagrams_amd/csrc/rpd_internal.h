@@ -196,7 +196,7 @@ struct ClipLaunch {
     // resumable cells (security radius not reached), see ClipArgs in rpd_clip.hip
     char *rs_out;          // records written by this pass (nullable), item t's at slot rs_base + t
     int rs_out_stride, rs_base;
-    const char *rs_in;     // records this pass resumes from (nullable; FP64 form)
+    const char *rs_in;     // records this pass resumes from (nullable; FP64 and mixed forms)
     int rs_in_stride, rs_in_P;
     int *rslot, *lastnb;   // per stored id
     // Hessian (H > 0): per original seed H entries of hc values, neighbours'

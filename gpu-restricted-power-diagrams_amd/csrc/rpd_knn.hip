@@ -824,8 +824,8 @@ int rpd_knn_dim(int64_t n) {
 // perm[n], counters[dim^3+1], stored (float4 or double4 by prec) and stored64.
 // perm is the stable sort of the seeds by cell (knearests.cpp:129-191 sorts
 // by cell with a counting sort; here the order within a cell is fixed too):
-// a counting sort whose cells are then sorted by index, or, when a cell holds
-// more than kSortRun seeds, a radix sort of (cell, index).  Waits for the
+// a counting sort whose members then find their rank in the cell, or, when a
+// cell holds more than kSortRun seeds, a radix sort of (cell, index).  Waits for the
 // stream.
 //
 // Layout of the binning's scratch: cell ids, members (cell ids out in the radix

@@ -164,8 +164,10 @@ typedef struct {
     int32_t max_extra_steps;      /* re-queue passes over failed cells with
                                      grown caps (ref: 5)                      */
     int32_t apex_mode;            /* 0 reference corner apex, 1 (default)
-                                     centre of the first voxel of the cell's
-                                     bbox whose centre class is known         */
+                                     inside a voxel of the cell's bbox whose
+                                     centre class is known: the first one, or,
+                                     where the domain is one of voxel faces,
+                                     the one in the middle                    */
     int32_t security_mode;        /* 0 (default) exact power-diagram stop:
                                      d*(d - 2R) >= w_s - w_min; 1 reference
                                      stop d^2 > 4R^2 (ConvexCell.cl:364-382),
