@@ -1073,21 +1073,20 @@ static int solve_impl(rpd_ctx *c, rpd_domain *dom, const rpd_params *prm, rpd_st
     const bool hess = prm->H > 0;
     // Domains of voxel faces are restricted by them, others by their triangle
     // lists (so are all with the reference's corner apex and in the FP32
-    // form's own passes), in a batch each request as alone.
+    // form's own passes), in a batch each request as alone; cells of no domain
+    // take the strips' kernel, which has less LDS a cell.
     bool vox = false, lists = false;
     int t_floor = kTriangleFloor;
     auto add_domain = [&](const rpd_domain *d, int64_t seeds) {
-        if (!d) return;
-        if (!d->dev.vface || prm->apex_mode != 1) {
+        if (prm->apex_mode != 1 || (d && !d->dev.vface)) {
             lists = true;
             return;
         }
         vox = true;
-        if (form0 != RPD_PREC_FP32) t_floor = std::max(t_floor, strip_floor(d->dev.g, seeds));
+        if (d && form0 != RPD_PREC_FP32) t_floor = std::max(t_floor, strip_floor(d->dev.g, seeds));
     };
-    add_domain(dom, n);
+    if (!batch) add_domain(dom, n);
     for (const auto &q : c->batch) add_domain(q.dom, q.n);
-    if (!lists && prm->apex_mode == 1) vox = true;  // (no domain at all: the kernel with less LDS a cell)
     T = std::max(T, std::min(t_floor, rpd_clip_max_T(form0, P, V, hess)));
     rpd_stats st{};
     st.n = n;

@@ -33,11 +33,12 @@
 //
 // Forms: FP64 (all double); mixed: the plane-side tests and the vertex
 // registers are FP32 and each test also evaluates a certified bound on its
-// FP32 error against the FP64 planes, 2^-18 * sum of |terms| of the det4x4
-// expansion.  A test inside the bound, and every test of an ill-conditioned
-// vertex, is decided in FP64 from the vertex's planes, as the FP64 form
-// decides it: the finish kernel has FP64 planes in LDS, the bisector kernel
-// FP32 planes, beside which it makes FP64 ones when a test first needs them.
+// FP32 error against the FP64 planes, 2^-18 * (at least the sum of |terms| of
+// the det4x4 expansion).  A test inside the bound, and every test of an
+// ill-conditioned vertex, is decided in FP64 from the vertex's planes, as the
+// FP64 form decides it: the finish kernel has FP64 planes in LDS, the bisector
+// kernel FP32 planes, beside which it makes FP64 ones when a test first needs
+// them.
 // A cavity that such decisions leave inconsistent ends the cell with a status
 // that the host re-runs in FP64 to its end.  The records' planes are FP64; the
 // cell geometry that produces the results

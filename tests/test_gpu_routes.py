@@ -24,14 +24,16 @@ def test_strip_room_is_for_strips(rpd, ctx, prec, apex, strips):
 
 @pytest.mark.parametrize("prec", [0, 1, 2])
 @pytest.mark.parametrize("apex", [0, 1])
-def test_batch_of_both_kinds_of_domains(rpd, ctx, prec, apex):
+@pytest.mark.parametrize("kinds", ["all", "mesh and none", "voxel and none"])
+def test_batch_of_both_kinds_of_domains(rpd, ctx, prec, apex, kinds):
     """A voxel domain, a mesh and no domain in one batch, each request as
     alone: the same bits, and over all passes (which pass counts a cell depends
     on the cap, the batch's largest) the same largest union of triangles."""
     P, T = icosphere(3, radius=2.0, rot_seed=11)
     doms = [ctx.domain(rpd.Grid.shape(rpd.SHAPE_SPHERE, 24, (0.5, 0.5, 0.5, 0.4))),
             ctx.domain(rpd.Grid.mesh(P, T, 40)), None]
-    reqs = [(doms[k % 3], rpd.generate_seeds(rpd.SEEDS_UNIFORM, n, seed=n, wmax=0.0))
+    kinds = {"all": (0, 1, 2), "mesh and none": (1, 2), "voxel and none": (0, 2)}[kinds]
+    reqs = [(doms[kinds[k % len(kinds)]], rpd.generate_seeds(rpd.SEEDS_UNIFORM, n, seed=n, wmax=0.0))
             for k, n in enumerate((5000, 3000, 700, 40, 20000, 17, 200))]
     caps = dict(precision=prec, apex_mode=apex, debug_counters=1)
     alone, status, most = [], [], 0
